@@ -20,7 +20,8 @@
 //            checkpoints) -> B4 knot gradients and parameter reductions.
 // Per-step coefficients: when every clock step of a chunk is within 2^-16 / (2 max|mu|) of the chunk mean
 // (a uniform clock in float32), coefficients are first-order Taylor models in h around the mean (error
-// below float32 rounding); otherwise they are evaluated exactly per step.
+// below float32 rounding); else, while every step is small (2 max|u| |h| <= kPolyR), they are polynomials in h whose
+// coefficients each lane forms once (PolyCoef); otherwise they are evaluated exactly per step.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -125,11 +126,6 @@ __device__ __forceinline__ void load_chunk(const DiagArgs& a, int b, int t0, int
   const float* th = a.clock + (size_t)b * a.L + t0;
   for (int k = threadIdx.x; k < Tc; k += st) s_h[k] = th[k + 1] - th[k];
 }
-__device__ __forceinline__ void load_clock(const DiagArgs& a, int b, int t0, int Tc, float* s_h) {
-  const float* th = a.clock + (size_t)b * a.L + t0;
-  for (int k = threadIdx.x; k < Tc; k += blockDim.x) s_h[k] = th[k + 1] - th[k];
-}
-
 // ------------------------------------------------------------------------------------------- coefficients
 template <class T> struct Coef {
   T rho, phi_j, phi_k, IA, IB, lamA, lamB;
@@ -209,6 +205,64 @@ __device__ __forceinline__ void lin_coef(const Coef<T>& c0, const CoefD<T>& q, f
   }
 }
 
+// Small-step model (ews_numerics.h kPolyR): the lane's coefficients as polynomials in the clock step, formed once per
+// chunk. A step is 2 (3 kPolyPhi + 2 kPolyD) multiply-adds and a handful of complex products; the exact evaluation's
+// two 13-term series with their node derivatives and five complex exponentials were 2-3 thousand instructions, most of
+// a non-uniform chunk's time (d = 16 planes, B = 32, L = 1751, an irregular clock with its gradient: the kernels of a
+// training step 5.9 -> 0.24 ms with the inversion adjoint and the chunk length below, the adjoint 4.74 -> 0.09). The
+// flows follow from phi: e^x = 1 + x phi(x), and the pair flows are products of the planes' (cached flows: at the
+// shared step).
+template <class T, bool CPLX, int N> struct PolyCoef {
+  T uj, uk, ph[kPolyPhi + 1], phk[kPolyPhi + 1], B[kPolyD + 1], A[kPolyD + 1];
+  bool per_int;
+  T crho, crhok;  // cached flows
+  __device__ __forceinline__ void init(T u, T w, bool per_interval, float href) {
+    uj = u;
+    uk = w;
+    per_int = per_interval;
+    crho = crhok = zero<T>();
+    poly_phi(u, ph);
+    if (!per_int) crho = expv(href * u);
+    if constexpr (N == 2) {
+      poly_phi(w, phk);
+      poly_dd3(u, u + w, B);
+      if constexpr (CPLX) poly_dd3(u, u + conjc(w), A);
+      if (!per_int) crhok = expv(href * w);
+    }
+  }
+  static __device__ __forceinline__ T flow(T u, const T* c, float h) { return (h * u) * poly_val<kPolyPhi>(c, h) + 1.0f; }
+  // DH: also the derivatives in h that the clock gradient needs
+  template <bool DH> __device__ __forceinline__ void at(float h, Coef<T>& c, CoefD<T>& q) const {
+    if constexpr (DH) {
+      c.phi_j = poly_val_d<kPolyPhi>(ph, h, q.phi_j1);
+    } else {
+      c.phi_j = poly_val<kPolyPhi>(ph, h);
+    }
+    c.rho = per_int ? (h * uj) * c.phi_j + 1.0f : crho;
+    if constexpr (DH) q.rho1 = per_int ? c.rho * uj : zero<T>();
+    if constexpr (N == 2) {
+      c.phi_k = poly_val<kPolyPhi>(phk, h);
+      c.rho_k = per_int ? (h * uk) * c.phi_k + 1.0f : crhok;
+      c.lamB = c.rho * c.rho_k;
+      if constexpr (DH) {
+        c.IB = poly_val_d<kPolyD>(B, h, q.IB1);
+        q.lamB1 = per_int ? c.lamB * (uj + uk) : zero<T>();
+      } else {
+        c.IB = poly_val<kPolyD>(B, h);
+      }
+      if constexpr (CPLX) {
+        c.lamA = c.rho * conjc(c.rho_k);
+        if constexpr (DH) {
+          c.IA = poly_val_d<kPolyD>(A, h, q.IA1);
+          q.lamA1 = per_int ? c.lamA * (uj + conjc(uk)) : zero<T>();
+        } else {
+          c.IA = poly_val<kPolyD>(A, h);
+        }
+      }
+    }
+  }
+};
+
 // One forward Chen step of the lane's elements.
 template <class T, bool CPLX, int N>
 __device__ __forceinline__ void fwd_step(const Coef<T>& c, T pj, T pk, T& S1, T& SA, T& SB) {
@@ -221,32 +275,29 @@ __device__ __forceinline__ void fwd_step(const Coef<T>& c, T pj, T pk, T& S1, T&
   S1 = cj + c.phi_j * pj;
 }
 
-// Chunk setup shared by all chunk kernels: the uniform-clock test and the reference step.
+// Chunk setup shared by all chunk kernels: the chunk's class and its reference step. The class is decided once, by the
+// forward's first summary pass (or the pair-group forward), and kept in the residual: flag bit 0 uniform steps, bit 1
+// the steps may be inverted, bit 3 small steps (the polynomial model applies), and the mean step hbar.
+constexpr int kFlagUniform = 1, kFlagInvert = 2, kFlagSmall = 8;
 struct ChunkClock {
   float hbar, href;
   bool fast, per_int;
   bool inv_ok;  // stepping the recursion backwards amplifies errors by at most 2 over the chunk
+  bool small;   // every step inside the polynomial model's radius
 };
 
-template <class T>
-__device__ __forceinline__ ChunkClock chunk_clock(const DiagArgs& a, int b, int Tc, const float* s_h) {
-  ChunkClock cc;
-  float s = 0.0f;
-  for (int t = 0; t < Tc; ++t) s += s_h[t];
-  cc.hbar = s / (float)Tc;
-  float dmax = 0.0f;
-  bool finite = true;
-  for (int t = 0; t < Tc; ++t) {
-    const float dl = fabsf(s_h[t] - cc.hbar);
-    dmax = fmaxf(dmax, dl);
-    finite = finite && (dl <= 3.0e38f);
-  }
-  float R = 0.0f;
-  T dummy{};
-  for (int j = 0; j < a.K; ++j) R = fmaxf(R, absv(load_u(a.params, j, &dummy)));
-  // with the pair-group kernels active (a.fast_ok) they own every uniform chunk; the chunks left here take exact
-  // per-step coefficients, so that the FAST instantiations have no work and are not launched
-  cc.fast = finite && (dmax * 2.0f * R < 1.52587890625e-5f) && !a.fast_ok;  // 2^-16
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, lanes::dpp<lanes::kXor1>(v));
+  v = fmaxf(v, lanes::dpp<lanes::kXor2>(v));
+  v = fmaxf(v, lanes::dpp<lanes::kHalfMirror>(v));
+  v = fmaxf(v, lanes::dpp<lanes::kMirror>(v));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+__device__ __forceinline__ void chunk_ref(const DiagArgs& a, int b, ChunkClock& cc) {
   cc.per_int = a.flow_mode == EWS_FLOW_PER_INTERVAL;
   const float* th = a.clock + (size_t)b * a.L;
   if (a.flow_mode == EWS_FLOW_CACHED) {
@@ -256,12 +307,57 @@ __device__ __forceinline__ ChunkClock chunk_clock(const DiagArgs& a, int b, int 
   } else {
     cc.href = 0.0f;
   }
-  // largest contraction rate Re(-u_j) (the damping d_j of a plane, lambda_j of a real channel); a level-2
-  // element contracts at most at twice that rate, so the inverse step grows errors by e^{2 Dmax tau}
-  float Dmax = 0.0f;
-  for (int j = 0; j < a.K; ++j) Dmax = fmaxf(Dmax, -re(load_u(a.params, j, &dummy)));
+}
+
+// The classification (a lane per step and per generator entry, every wavefront the same result).
+template <class T>
+__device__ __forceinline__ ChunkClock chunk_classify(const DiagArgs& a, int b, int Tc, const float* s_h) {
+  ChunkClock cc;
+  chunk_ref(a, b, cc);
+  const int lane = threadIdx.x & 63;
+  float s = 0.0f;
+  for (int t = lane; t < Tc; t += 64) s += s_h[t];
+  s = lanes::sum64(s);
+  cc.hbar = s / (float)Tc;
+  float dmax = 0.0f, hmax = 0.0f, bad = 0.0f;
+  for (int t = lane; t < Tc; t += 64) {
+    const float dl = fabsf(s_h[t] - cc.hbar);
+    dmax = fmaxf(dmax, dl);
+    hmax = fmaxf(hmax, fabsf(s_h[t]));
+    if (!(dl <= 3.0e38f)) bad = 1.0f;
+  }
+  // R: largest |u|; Dmax: largest contraction rate Re(-u_j) (the damping d_j of a plane, lambda_j of a real channel);
+  // a level-2 element contracts at most at twice that rate, so the inverse step grows errors by e^{2 Dmax tau}
+  float R = 0.0f, Dmax = 0.0f;
+  T dummy{};
+  for (int j = lane; j < a.K; j += 64) {
+    const T u = load_u(a.params, j, &dummy);
+    const float au = absv(u);
+    if (!(au <= 3.0e38f)) bad = 1.0f;
+    R = fmaxf(R, au);
+    Dmax = fmaxf(Dmax, -re(u));
+  }
+  dmax = wave_max(dmax);
+  hmax = wave_max(hmax);
+  bad = wave_max(bad);
+  R = wave_max(R);
+  Dmax = wave_max(Dmax);
+  const bool finite = bad == 0.0f && isfinite(s);
+  cc.fast = finite && (dmax * 2.0f * R < 1.52587890625e-5f);  // 2^-16
+  cc.small = finite && poly_order_ok(a.sq1, a.sq2) && 2.0f * R * hmax <= kPolyR;
   const float tau = cc.per_int ? s : fabsf(cc.href) * (float)Tc;
   cc.inv_ok = finite && (2.0f * Dmax * tau <= 0.69314718f);
+  return cc;
+}
+// The class as the forward left it.
+__device__ __forceinline__ ChunkClock chunk_class(const DiagArgs& a, int b, int c) {
+  ChunkClock cc;
+  chunk_ref(a, b, cc);
+  const int f = a.cflag[b * a.C + c];
+  cc.hbar = a.chbar[b * a.C + c];
+  cc.fast = (f & kFlagUniform) != 0;
+  cc.inv_ok = (f & kFlagInvert) != 0;
+  cc.small = (f & kFlagSmall) != 0;
   return cc;
 }
 
@@ -355,19 +451,26 @@ __global__ __launch_bounds__(MAXT) void k_chunk_fwd(DiagArgs a) {
   float* s_v = smem;
   float* s_h = s_v + a.T * a.d;
   const int c = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  if (a.fast_ok && (a.cflag[b * a.C + c] & 1)) return;  // a pair-group kernel owns this chunk
-  // generic chunks: the first summary pass (FAST) classifies every chunk and writes its class (bit 0 uniform,
-  // bit 1 invertible); every later kernel reads it and leaves a chunk it does not own before staging anything
+  // the first summary pass (FAST) classifies every chunk and writes its class; every later kernel reads it and leaves
+  // a chunk it does not own before staging anything
   constexpr bool kClassify = MODE == MODE_SUMMARY && FAST;
-  if (!kClassify && !a.fast_ok && ((a.cflag[b * a.C + c] & 1) != 0) != FAST) return;
+  if (!kClassify && ((a.cflag[b * a.C + c] & kFlagUniform) != 0) != FAST) return;
   const int t0 = c * a.T;
   const int Tc = min(a.T, a.n_int - t0);
   load_chunk(a, b, t0, Tc, s_v, s_h);
   __syncthreads();
   const LaneMap m = lane_map(a, tid);
-  const ChunkClock cc = chunk_clock<T>(a, b, Tc, s_h);
-  if (kClassify && !a.fast_ok && tid == 0) a.cflag[b * a.C + c] = (cc.fast ? 1 : 0) | (cc.inv_ok ? 2 : 0);
-  if (cc.fast != FAST) return;  // the other instantiation owns this chunk
+  ChunkClock cc;
+  if constexpr (kClassify) {
+    cc = chunk_classify<T>(a, b, Tc, s_h);
+    if (tid == 0) {
+      a.cflag[b * a.C + c] = (cc.fast ? kFlagUniform : 0) | (cc.inv_ok ? kFlagInvert : 0) | (cc.small ? kFlagSmall : 0);
+      a.chbar[b * a.C + c] = cc.hbar;
+    }
+    if (!cc.fast) return;  // the other instantiation owns this chunk
+  } else {
+    cc = chunk_class(a, b, c);
+  }
   if (!m.active) return;
   T dummy{};
   const T uj = load_u(a.params, m.j, &dummy);
@@ -404,23 +507,15 @@ __global__ __launch_bounds__(MAXT) void k_chunk_fwd(DiagArgs a) {
     arg[i] = 0;
   }
 
-  for (int t = 0; t < Tc; ++t) {
-    const float h = s_h[t];
-    Coef<T> co;
-    if constexpr (FAST) {
-      lin_coef<T, CPLX, N>(c0, q, h - cc.hbar, cc.per_int, co);
-    } else {
-      CoefD<T> qq;
-      eval_coef<T, CPLX, N, false>(a.sq1, a.sq2, h, cc.href, cc.per_int, uj, uk, co, qq);
-    }
+  auto step = [&](int t, const Coef<T>& co) {
     const T pj = lds_p<T>(s_v, t, a.d, m.j);
     const T pk = (N == 2) ? lds_p<T>(s_v, t, a.d, m.k) : zero<T>();
     fwd_step<T, CPLX, N>(co, pj, pk, S1, SA, SB);
-    if (MODE == MODE_SUMMARY) continue;
+    if (MODE == MODE_SUMMARY) return;
     if (logrows) {  // LogEWS row: level 1, then S2[a,b] - S1_a S1_b / 2 at the Lyndon words a < b
       S1k = co.rho_k * S1k + co.phi_k * pk;
       write_log_row<CPLX>(a, m, b, t0 + t, S1, S1k, SA, SB);
-      continue;
+      return;
     }
     // the lane's output values in the row layout
     float v[6];
@@ -474,6 +569,29 @@ __global__ __launch_bounds__(MAXT) void k_chunk_fwd(DiagArgs a) {
           acc[i] += v[i];
         }
       }
+    }
+  };
+  if constexpr (FAST) {
+    for (int t = 0; t < Tc; ++t) {
+      Coef<T> co;
+      lin_coef<T, CPLX, N>(c0, q, s_h[t] - cc.hbar, cc.per_int, co);
+      step(t, co);
+    }
+  } else if (cc.small) {
+    PolyCoef<T, CPLX, N> pc;
+    pc.init(uj, uk, cc.per_int, cc.href);
+    for (int t = 0; t < Tc; ++t) {
+      Coef<T> co;
+      CoefD<T> qq;
+      pc.template at<false>(s_h[t], co, qq);
+      step(t, co);
+    }
+  } else {
+    for (int t = 0; t < Tc; ++t) {
+      Coef<T> co;
+      CoefD<T> qq;
+      eval_coef<T, CPLX, N, false>(a.sq1, a.sq2, s_h[t], cc.href, cc.per_int, uj, uk, co, qq);
+      step(t, co);
     }
   }
 
@@ -709,7 +827,7 @@ __global__ __launch_bounds__(MAXT) void k_chunk_mix(DiagArgs a, MixEpi e) {
   load_chunk(a, b, t0, Tc, s_v, s_h);
   __syncthreads();
   const LaneMap m = lane_map(a, tid);  // lanes past the pairs join the barriers of the mixer blocks
-  const ChunkClock cc = chunk_clock<T>(a, b, Tc, s_h);
+  const ChunkClock cc = chunk_class(a, b, c);
   T dummy{};
   const T uj = load_u(a.params, m.j, &dummy);
   const T uk = load_u(a.params, m.k, &dummy);
@@ -1356,15 +1474,11 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_local(DiagArgs a) {
   int* s_am = reinterpret_cast<int*>(smem + Lo.am);
   float* s_red = smem + Lo.g;
   const int c = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  if (a.fast_ok && (a.cflag[b * a.C + c] & 1)) return;  // a pair-group kernel owns this chunk
-  if (!a.fast_ok && ((a.cflag[b * a.C + c] & 1) != 0) != FAST) return;  // the forward's chunk class
+  if (((a.cflag[b * a.C + c] & kFlagUniform) != 0) != FAST) return;  // the forward's chunk class
   const int t0 = c * a.T;
   const int Tc = min(a.T, a.n_int - t0);
   const bool prefix = a.readout == EWS_READOUT_PREFIX;
-  load_clock(a, b, t0, Tc, s_h);
-  __syncthreads();
-  const ChunkClock cc = chunk_clock<T>(a, b, Tc, s_h);
-  if (cc.fast != FAST) return;  // the other instantiation owns this chunk
+  const ChunkClock cc = chunk_class(a, b, c);
   load_chunk(a, b, t0, Tc, s_v, s_h);
   if (!prefix) stage_vec(a, b, s_gv, s_am);
   const int nblk = (Tc + kGBL - 1) / kGBL;
@@ -1379,6 +1493,8 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_local(DiagArgs a) {
   Coef<T> c0;
   CoefD<T> q;
   if constexpr (FAST) eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q);
+  PolyCoef<T, CPLX, N> pc;
+  if constexpr (!FAST) pc.init(uj, uk, cc.per_int, cc.href);
   T L1 = zero<T>(), LA = zero<T>(), LB = zero<T>();
   for (int blk = nblk - 1; blk >= 0; --blk) {
     const int buf = (nblk - 1 - blk) & 1;
@@ -1402,7 +1518,8 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_local(DiagArgs a) {
             lin_coef<T, CPLX, N>(c0, q, h - cc.hbar, cc.per_int, co);
           } else {
             CoefD<T> qq;
-            eval_coef<T, CPLX, N, false>(a.sq1, a.sq2, h, cc.href, cc.per_int, uj, uk, co, qq);
+            if (cc.small) pc.template at<false>(h, co, qq);
+            else eval_coef<T, CPLX, N, false>(a.sq1, a.sq2, h, cc.href, cc.per_int, uj, uk, co, qq);
           }
           T toC = zero<T>();
           if constexpr (N == 2) {
@@ -1455,6 +1572,21 @@ template <class T> struct BwdAcc {
   T Gx, GyA, GyB, Gxp;             // node cotangents times h (per-interval coefficients)
   T Sflow, SflowA, SflowB;         // summed flow cotangents (cached flows)
 };
+// Moments of the coefficient cotangents under the small-step model: X[m] = sum_t h_t^(m+1) g_t (one multiply-add per
+// real component and power instead of the node derivatives of every step; poly_*_node contracts them at the end).
+template <class T> struct PolyMom {
+  T ph[kPolyPhi], A[kPolyD], B[kPolyD];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int m = 0; m < kPolyPhi; ++m) ph[m] = zero<T>();
+#pragma unroll
+    for (int m = 0; m < kPolyD; ++m) A[m] = B[m] = zero<T>();
+  }
+};
+template <int M, class T> __device__ __forceinline__ void add_moments(T* X, const float* hp, T g) {
+#pragma unroll
+  for (int m = 0; m < M; ++m) X[m] = fma_r(hp[m], g, X[m]);
+}
 struct RedLds {
   float *rC, *rP, *cS, *cP;        // LDS row/column sums (multi-wave workgroups)
 };
@@ -1463,11 +1595,18 @@ struct RedLds {
 // adjoint of the Chen step with the state S(t-1) = (H1, HA, HB), writes dv[tg] for the plane lanes and the
 // step's dh partial to s_dh, and moves acc's cotangents from S(t) to S(t-1).
 // DH: the clock gradient is requested; without it the step's dh terms are not formed.
-template <bool CPLX, int N, bool WAVE, bool ALLRED, bool DH, class T>
+// POLY: the coefficients come from the small-step model; their cotangents go to the moments mom.
+template <bool CPLX, int N, bool WAVE, bool ALLRED, bool DH, bool POLY, class T>
 __device__ __forceinline__ void bwd_step(const DiagArgs& a, const LaneMap& m, const GammaSrc& gs, int s, int t, int tg,
                                          float h, const float* s_v, bool per_int, const Coef<T>& co,
-                                         const CoefD<T>& qq, BwdAcc<T>& acc, T H1, T HA, T HB, const RedLds& red,
-                                         float* s_dh) {
+                                         const CoefD<T>& qq, BwdAcc<T>& acc, PolyMom<T>& mom, T H1, T HA, T HB,
+                                         const RedLds& red, float* s_dh) {
+  float hp[POLY ? kPolyD : 1];
+  hp[0] = h;
+  if constexpr (POLY) {
+#pragma unroll
+    for (int i = 1; i < kPolyD; ++i) hp[i] = hp[i - 1] * h;
+  }
   const int tid = threadIdx.x, NW = (blockDim.x + 63) / 64, wid = tid / 64, b = blockIdx.y;
   float* s_rC = red.rC;
   float* s_rP = red.rP;
@@ -1492,8 +1631,12 @@ __device__ __forceinline__ void bwd_step(const DiagArgs& a, const LaneMap& m, co
           toPk = conjc(pj) * gf;
           const T gIB = conjc(pj * pk) * acc.LB;
           const T gLB = conjc(HB) * acc.LB;
-          acc.Gx += h * (gIB * conjc(qq.DxB));
-          acc.GyB += h * (gIB * conjc(qq.DyB));
+          if constexpr (POLY) {
+            add_moments<kPolyD>(mom.B, hp, gIB);
+          } else {
+            acc.Gx += h * (gIB * conjc(qq.DxB));
+            acc.GyB += h * (gIB * conjc(qq.DyB));
+          }
           if constexpr (DH) dhp += redot(gIB, qq.IB1);
           if (per_int) {
             acc.GyB += h * (gLB * conjc(co.lamB));
@@ -1509,8 +1652,12 @@ __device__ __forceinline__ void bwd_step(const DiagArgs& a, const LaneMap& m, co
             toPk += conjc(ge) * pj;
             const T gIA = conjc(pj * conjc(pk)) * acc.LA;
             const T gLA = conjc(HA) * acc.LA;
-            acc.Gx += h * (gIA * conjc(qq.DxA));
-            acc.GyA += h * (gIA * conjc(qq.DyA));
+            if constexpr (POLY) {
+              add_moments<kPolyD>(mom.A, hp, gIA);
+            } else {
+              acc.Gx += h * (gIA * conjc(qq.DxA));
+              acc.GyA += h * (gIA * conjc(qq.DyA));
+            }
             if constexpr (DH) dhp += redot(gIA, qq.IA1);
             if (per_int) {
               acc.GyA += h * (gLA * conjc(co.lamA));
@@ -1586,7 +1733,8 @@ __device__ __forceinline__ void bwd_step(const DiagArgs& a, const LaneMap& m, co
           }
           const T grho = conjc(H1) * gc;
           const T gphi = conjc(pj) * gs1;
-          acc.Gxp += h * (gphi * conjc(qq.dphi_j));
+          if constexpr (POLY) add_moments<kPolyPhi>(mom.ph, hp, gphi);
+          else acc.Gxp += h * (gphi * conjc(qq.dphi_j));
           if constexpr (DH) dhp += redot(gphi, qq.phi_j1);
           if (per_int) {
             acc.Gxp += h * (grho * conjc(co.rho));
@@ -1703,6 +1851,23 @@ __device__ __forceinline__ void bwd_epilogue(const DiagArgs& a, const LaneMap& m
   }
 }
 
+// The moments' share of the node cotangents.
+template <bool CPLX, int N, class T>
+__device__ __forceinline__ void fold_moments(const LaneMap& m, const PolyMom<T>& mom, T uj, T ua, T ub, BwdAcc<T>& acc) {
+  if (m.plane) acc.Gxp += poly_phi_node(uj, mom.ph);
+  if constexpr (N == 2) {
+    T gx, gy;
+    poly_dd3_node(uj, ub, mom.B, gx, gy);
+    acc.Gx += gx;
+    acc.GyB += gy;
+    if constexpr (CPLX) {
+      poly_dd3_node(uj, ua, mom.A, gx, gy);
+      acc.Gx += gx;
+      acc.GyA += gy;
+    }
+  }
+}
+
 // State loads of the lane from a float64 kernel-layout row / cotangent loads from a float32 row.
 template <bool CPLX, int N, class T>
 __device__ __forceinline__ void load_state_d(const DiagArgs& a, const LaneMap& m, const double* cr, T& S1, T& SA, T& SB) {
@@ -1735,25 +1900,14 @@ __device__ __forceinline__ void load_cot(const DiagArgs& a, const LaneMap& m, co
   }
 }
 
-// Shared prologue: clock steps, ownership test, increments, per-sample cotangent, first staged block.
+// Shared prologue: ownership test (the forward's chunk class), increments, per-sample cotangent, first staged block.
 #define EWS_BWD_PROLOGUE(OWNS, ROWS)                                                                              \
   const int tid = threadIdx.x;                                                                             \
-  if (a.fast_ok && (a.cflag[b * a.C + c] & 3) == 3) return; /* a pair-group kernel owns this chunk */      \
-  if (!a.fast_ok) { /* the forward's chunk class: leave a chunk this kernel does not own before staging */ \
-    const int gf = a.cflag[b * a.C + c];                                                                   \
-    ChunkClock cc;                                                                                         \
-    cc.fast = (gf & 1) != 0;                                                                               \
-    cc.inv_ok = (gf & 2) != 0;                                                                             \
-    if (!(OWNS)) return;                                                                                   \
-  }                                                                                                        \
+  const ChunkClock cc = chunk_class(a, b, c);                                                              \
+  if (!(OWNS)) return; /* before anything is staged */                                                     \
   const int t0 = c * a.T;                                                                                  \
   const int Tc = min(a.T, a.n_int - t0);                                                                   \
   const bool prefix = a.readout == EWS_READOUT_PREFIX;                                                     \
-  load_clock(a, b, t0, Tc, s_h);                                                                           \
-  __syncthreads();                                                                                         \
-  ChunkClock cc = chunk_clock<T>(a, b, Tc, s_h);                                                           \
-  if (a.fast_ok) cc.inv_ok = (a.cflag[b * a.C + c] & 2) != 0; /* one invertibility test for every kernel */ \
-  if (!(OWNS)) return;                                                                                     \
   load_chunk(a, b, t0, Tc, s_v, s_h);                                                                      \
   if (!prefix) stage_vec(a, b, s_gv, s_am);                                                                \
   const int nblk = (Tc + (ROWS) - 1) / (ROWS);                                                             \
@@ -1767,11 +1921,16 @@ __device__ __forceinline__ void load_cot(const DiagArgs& a, const LaneMap& m, co
   const T uk = load_u(a.params, m.k, &dummy);                                                              \
   const T ua = uj + conjc(uk), ub = uj + uk;
 
-// (a) Uniform-clock chunks whose decay allows it: the states S(t-1) come from inverting the steps backwards from
-// the chunk's end state (c_j = S1(t) - s1_j(t) is exact; then divide by the flows), so nothing is recomputed
-// forward and no history is kept.
-template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
-__global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
+// Which full adjoint owns a chunk of class f: the inversion adjoint under the first-order model (the pair-group
+// kernels at d = 16) or the small-step model, else the recomputing one.
+__device__ __forceinline__ bool inv_lin(int f) { return (f & 3) == 3; }
+__device__ __forceinline__ bool inv_poly(int f) { return (f & (kFlagUniform | kFlagInvert | kFlagSmall)) == (kFlagInvert | kFlagSmall); }
+
+// (a) Chunks whose decay allows it, under the first-order model (uniform steps) or the small-step model (POLY): the
+// states S(t-1) come from inverting the steps backwards from the chunk's end state (c_j = S1(t) - s1_j(t) is exact;
+// then divide by the flows), so nothing is recomputed forward and no history is kept.
+template <bool CPLX, int N, int MAXT, bool WAVE, bool DH, bool POLY>
+__device__ __forceinline__ void chunk_bwd_inv(const DiagArgs& a, const int c, const int b) {
   using T = typename Types<CPLX>::T;
   extern __shared__ float smem[];
   const BwdLds Lo = bwd_lds_layout(a.T, a.d, a.W, blockDim.x, 0, WAVE, true, kGB);
@@ -1784,16 +1943,19 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
                    smem + Lo.red + 6 * blockDim.x};
   float* s_dh = smem + Lo.dh;
   float* s_g = smem + Lo.g;
-  const int c = blockIdx.x, b = blockIdx.y;
-  EWS_BWD_PROLOGUE(cc.fast && cc.inv_ok, kGB)
+  EWS_BWD_PROLOGUE(POLY ? (!cc.fast && cc.small && cc.inv_ok) : (cc.fast && cc.inv_ok), kGB)
   Coef<T> c0;
   CoefD<T> q0;
-  eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q0);
-  // d/dh of the inverse flows 1/rho = e^{-x}, 1/lambda = e^{-y} at hbar
+  PolyCoef<T, CPLX, N> pc;
+  if constexpr (POLY) pc.init(uj, uk, cc.per_int, cc.href);
+  else eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q0);
+  // the inverse flows 1/rho = e^{-x}, 1/lambda = e^{-y}: at hbar and their d/dh (uniform steps), or at the shared
+  // step (POLY, cached flows; a small step's own inverse flow is 1 - x phi(-x))
   const T irho0 = expv(-(cc.per_int ? cc.hbar : cc.href) * uj);
   const T irho1 = cc.per_int ? -(irho0 * uj) : zero<T>();
+  const T irhok0 = POLY ? expv(-cc.href * uk) : zero<T>();
   T ilB0 = zero<T>(), ilB1 = zero<T>(), ilA0 = zero<T>(), ilA1 = zero<T>();
-  if constexpr (N == 2) {
+  if constexpr (N == 2 && !POLY) {
     const float hf = cc.per_int ? cc.hbar : cc.href;
     ilB0 = expv(-hf * ub);
     ilB1 = cc.per_int ? -(ilB0 * ub) : zero<T>();
@@ -1806,6 +1968,8 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
   load_state_d<CPLX, N>(a, m, a.carries + ((size_t)b * (a.C + 1) + c + 1) * a.D, S1, SA, SB);
   BwdAcc<T> acc;
   load_cot<CPLX, N>(a, m, a.mt + ((size_t)b * a.C + c) * a.D, acc);
+  PolyMom<T> mom;
+  if constexpr (POLY) mom.clear();
   for (int blk = nblk - 1; blk >= 0; --blk) {
     const int buf = (nblk - 1 - blk) & 1;
     const bool more = prefix && blk > 0;
@@ -1816,23 +1980,39 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
     for (int s = kGB - 1; s >= 0; --s) {
       const int t = blk * kGB + s;
       if (t < Tc) {
-        const float dlt = s_h[t] - cc.hbar;
+        const float h = s_h[t], dlt = h - cc.hbar;
         Coef<T> co;
-        lin_coef<T, CPLX, N>(c0, q0, dlt, cc.per_int, co);
+        CoefD<T> qp;
+        T irho, ilB = zero<T>(), ilA = zero<T>();
+        if constexpr (POLY) {
+          pc.template at<DH>(h, co, qp);
+          irho = cc.per_int ? pc.flow(uj, pc.ph, -h) : irho0;
+          if constexpr (N == 2) {
+            const T irk = cc.per_int ? pc.flow(uk, pc.phk, -h) : irhok0;
+            ilB = irho * irk;
+            if constexpr (CPLX) ilA = irho * conjc(irk);
+          }
+        } else {
+          lin_coef<T, CPLX, N>(c0, q0, dlt, cc.per_int, co);
+          irho = irho0 + irho1 * dlt;
+          if constexpr (N == 2) {
+            ilB = ilB0 + ilB1 * dlt;
+            if constexpr (CPLX) ilA = ilA0 + ilA1 * dlt;
+          }
+        }
         const T pj = lds_p<T>(s_v, t, a.d, m.j);
         const T pk = (N == 2) ? lds_p<T>(s_v, t, a.d, m.k) : zero<T>();
         // invert step t: S(t) -> S(t-1)
         const T cj = S1 - co.phi_j * pj;
-        const T H1 = (irho0 + irho1 * dlt) * cj;
+        const T H1 = irho * cj;
         T HA = zero<T>(), HB = zero<T>();
         if constexpr (N == 2) {
           const T s1k = co.phi_k * pk;
-          HB = (ilB0 + ilB1 * dlt) * (SB - cj * s1k - co.IB * (pj * pk));
-          if constexpr (CPLX) HA = (ilA0 + ilA1 * dlt) * (SA - cj * conjc(s1k) - co.IA * (pj * conjc(pk)));
+          HB = ilB * (SB - cj * s1k - co.IB * (pj * pk));
+          if constexpr (CPLX) HA = ilA * (SA - cj * conjc(s1k) - co.IA * (pj * conjc(pk)));
         }
-        bwd_step<CPLX, N, WAVE, MAXT == 1024, DH>(a, m, gs, s, t, t0 + t, s_h[t], s_v, cc.per_int, co, q0, acc, H1, HA,
-                                                  HB, red,
-                                s_dh);
+        bwd_step<CPLX, N, WAVE, MAXT == 1024, DH, POLY>(a, m, gs, s, t, t0 + t, h, s_v, cc.per_int, co, POLY ? qp : q0,
+                                                        acc, mom, H1, HA, HB, red, s_dh);
         S1 = H1;
         SA = HA;
         SB = HB;
@@ -1841,7 +2021,36 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
     if (more) lds_dma_wait();
     __syncthreads();
   }
+  if constexpr (POLY) fold_moments<CPLX, N>(m, mom, uj, ua, ub, acc);
   bwd_epilogue<CPLX, N, WAVE, DH>(a, m, cc, acc, uj, ua, ub, Tc, t0, s_dh, s_g, c, b);
+}
+
+template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
+__global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
+  chunk_bwd_inv<CPLX, N, MAXT, WAVE, DH, false>(a, blockIdx.x, blockIdx.y);
+}
+// Chunks blockIdx.x, blockIdx.x + gridDim.x, ... of sample blockIdx.y whose class OWNS accepts: the classes of 64
+// candidate chunks are read at once (one lane each), so that a launch whose chunks all belong to other kernels (the
+// host does not know the clock) needs few workgroups and ends in a few rounds. The ballot is the same in every
+// wavefront of the workgroup.
+template <class OWNS, class F> __device__ __forceinline__ void visit_chunks(const DiagArgs& a, OWNS&& owns, F&& f) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  for (int base = blockIdx.x; base < a.C; base += 64 * gridDim.x) {
+    const int cl = base + gridDim.x * lane;
+    unsigned long long mask = __ballot(cl < a.C && owns(a.cflag[b * a.C + min(cl, a.C - 1)]));
+    while (mask) {
+      const int i = __ffsll((long long)mask) - 1;
+      mask &= mask - 1;
+      f(base + gridDim.x * i, b);
+      __syncthreads();
+    }
+  }
+}
+// (two wavefronts per SIMD: with the registers left free it took 279 and ran alone)
+template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
+__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(2))) void k_chunk_bwd_inv_small(DiagArgs a) {
+  visit_chunks(a, [](int f) { return inv_poly(f); },
+               [&](int c, int b) { chunk_bwd_inv<CPLX, N, MAXT, WAVE, DH, true>(a, c, b); });
 }
 
 // (b) Every other chunk: forward states recomputed from the chunk's float64 carry (checkpoints every kb steps; each
@@ -1866,12 +2075,28 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
   const RedLds red{smem + Lo.red, smem + Lo.red + 2 * NT, smem + Lo.red + 4 * NT, smem + Lo.red + 6 * NT};
   float* s_dh = smem + Lo.dh;
   float* s_g = smem + Lo.g;
-  EWS_BWD_PROLOGUE(!(cc.fast && cc.inv_ok), kb)
+  EWS_BWD_PROLOGUE(!(cc.inv_ok && (cc.fast || cc.small)), kb)
   // uniform chunks (too contractive to invert) take the first-order model at the mean step, as every other
-  // kernel does for them; the others evaluate each step's exact coefficients
+  // kernel does for them, small-step chunks the polynomial model; the others evaluate each step's exact coefficients
   Coef<T> c0;
   CoefD<T> q0;
+  PolyCoef<T, CPLX, N> pc;
+  const bool poly = !cc.fast && cc.small;
   if (cc.fast) eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q0);
+  if (poly) pc.init(uj, uk, cc.per_int, cc.href);
+  PolyMom<T> mom;
+  mom.clear();
+  // the coefficients of the forward recomputation, and with the derivatives the adjoint needs
+  auto coef_fwd = [&](int t, Coef<T>& co) {
+    CoefD<T> qq;
+    if (poly) {
+      pc.template at<false>(s_h[t], co, qq);
+    } else if (cc.fast) {
+      lin_coef<T, CPLX, N>(c0, q0, s_h[t] - cc.hbar, cc.per_int, co);
+    } else {
+      eval_coef<T, CPLX, N, false>(a.sq1, a.sq2, s_h[t], cc.href, cc.per_int, uj, uk, co, qq);
+    }
+  };
   auto coef_at = [&](int t, Coef<T>& co, CoefD<T>& qq) {
     if (cc.fast) {
       lin_coef<T, CPLX, N>(c0, q0, s_h[t] - cc.hbar, cc.per_int, co);
@@ -1910,8 +2135,7 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
   for (int t = 0; t < Tc; ++t) {
     if ((t % kb) == 0) st_store(s_ck + (size_t)(t / kb) * NS * NT, S1, SA, SB);
     Coef<T> co;
-    CoefD<T> qq;
-    coef_at(t, co, qq);
+    coef_fwd(t, co);
     const T pj = lds_p<T>(s_v, t, a.d, m.j);
     const T pk = (N == 2) ? lds_p<T>(s_v, t, a.d, m.k) : zero<T>();
     fwd_step<T, CPLX, N>(co, pj, pk, S1, SA, SB);
@@ -1932,8 +2156,7 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
       if (t >= Tc) break;
       st_store(s_hist + (size_t)s * NS * NT, S1, SA, SB);
       Coef<T> co;
-      CoefD<T> qq;
-      coef_at(t, co, qq);
+      coef_fwd(t, co);
       const T pj = lds_p<T>(s_v, t, a.d, m.j);
       const T pk = (N == 2) ? lds_p<T>(s_v, t, a.d, m.k) : zero<T>();
       fwd_step<T, CPLX, N>(co, pj, pk, S1, SA, SB);
@@ -1946,35 +2169,27 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
         st_load(s_hist + (size_t)s * NS * NT, H1, HA, HB);
         Coef<T> co;
         CoefD<T> qq;
-        coef_at(t, co, qq);
-        bwd_step<CPLX, N, WAVE, MAXT == 1024, DH>(a, m, gs, s, t, t0 + t, s_h[t], s_v, cc.per_int, co, qq, acc, H1, HA, HB,
-                                              red, s_dh);
+        if (poly) {
+          pc.template at<DH>(s_h[t], co, qq);
+          bwd_step<CPLX, N, WAVE, MAXT == 1024, DH, true>(a, m, gs, s, t, t0 + t, s_h[t], s_v, cc.per_int, co, qq, acc,
+                                                          mom, H1, HA, HB, red, s_dh);
+        } else {
+          coef_at(t, co, qq);
+          bwd_step<CPLX, N, WAVE, MAXT == 1024, DH, false>(a, m, gs, s, t, t0 + t, s_h[t], s_v, cc.per_int, co, qq, acc,
+                                                           mom, H1, HA, HB, red, s_dh);
+        }
       }
     }
     if (more) lds_dma_wait();
     __syncthreads();
   }
+  if (poly) fold_moments<CPLX, N>(m, mom, uj, ua, ub, acc);
   bwd_epilogue<CPLX, N, WAVE, DH>(a, m, cc, acc, uj, ua, ub, Tc, t0, s_dh, s_g, c, b);
 }
-// Chunks blockIdx.x, blockIdx.x + gridDim.x, ... of sample blockIdx.y: with the pair kernels active the grid is
-// small (most chunks belong to them), otherwise one chunk per workgroup. The ownership flags of 64 candidate
-// chunks are read at once (one lane each: the pair kernels' flags, or the generic chunk class written by the first
-// summary pass) and only the chunks left to this kernel are visited.
 template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
 __global__ __launch_bounds__(MAXT) void k_chunk_bwd_full(DiagArgs a) {
-  const int b = blockIdx.y, lane = threadIdx.x & 63;
-  for (int base = blockIdx.x; base < a.C; base += 64 * gridDim.x) {
-    const int cl = base + gridDim.x * lane;
-    // a pair-group kernel (fast_ok) or the inversion adjoint (generic class: uniform and invertible) owns the others
-    const bool need = cl < a.C && (a.cflag[b * a.C + cl] & 3) != 3;
-    unsigned long long mask = __ballot(need);  // the same in every wavefront of the workgroup
-    while (mask) {
-      const int i = __ffsll((long long)mask) - 1;
-      mask &= mask - 1;
-      chunk_bwd_full<CPLX, N, MAXT, WAVE, DH>(a, base + gridDim.x * i, b);
-      __syncthreads();
-    }
-  }
+  visit_chunks(a, [](int f) { return !inv_lin(f) && !inv_poly(f); },
+               [&](int c, int b) { chunk_bwd_full<CPLX, N, MAXT, WAVE, DH>(a, c, b); });
 }
 
 // ------------------------------------------------------------------------------------------- B0 (log rows)
@@ -2006,12 +2221,12 @@ __global__ __launch_bounds__(256) void k_log_cot(DiagArgs a, const float* __rest
 
 // ------------------------------------------------------------------------------------------- B4
 // Knot gradients from interval gradients: dX_t = dv_{t-1} - dv_t, dtheta_t = dh_{t-1} - dh_t (+ the shared flow
-// step's gradient for cached flows). One workgroup per (chunk, sample): the chunk's first knot always, its interior
+// step's gradient for cached flows), a wavefront per (chunk, sample): the chunk's first knot always, its interior
 // knots unless a pair-group adjoint already wrote them (it leaves dv / dh of its first and last interval for the
-// boundary knots); workgroup C handles the last knot L-1.
-__global__ void k_knot_grads(DiagArgs a) {
-  const int c = blockIdx.x, b = blockIdx.y;
-  const int dp1 = a.d + 1;
+// boundary knots); chunk C handles the last knot L-1. A chunk's knots are one contiguous run of a sample's floats, so
+// element e is dv[e - d] - dv[e] with no index arithmetic, four loads in flight.
+__device__ __forceinline__ void knot_grads(const DiagArgs& a, int c, int b) {
+  const int lane = threadIdx.x & 63;
   int k0, k1;  // knot range [k0, k1)
   if (c == a.C) {
     k0 = a.n_int;
@@ -2022,30 +2237,36 @@ __global__ void k_knot_grads(DiagArgs a) {
     k1 = owned ? k0 + 1 : min(k0 + a.T, a.n_int);
   }
   const float* dvb = a.dv + (size_t)b * a.n_int * a.d;
-  const float* dhb = a.dh + (size_t)b * a.n_int;
-  for (int i = threadIdx.x; i < (k1 - k0) * dp1; i += blockDim.x) {
-    const int t = k0 + i / dp1, ch = i % dp1;
-    const size_t bt = (size_t)b * a.L + t;
-    if (ch < a.d) {
-      float g = 0.0f;
-      if (t >= 1) g += dvb[(size_t)(t - 1) * a.d + ch];
-      if (t < a.n_int) g -= dvb[(size_t)t * a.d + ch];
-      a.dpath[bt * a.d + ch] = g;
-    } else if (a.dclock) {  // null: the clock gradient is not requested
-      float g = 0.0f;
-      if (t >= 1) g += dhb[t - 1];
-      if (t < a.n_int) g -= dhb[t];
-      if (a.flow_mode != EWS_FLOW_PER_INTERVAL) {
-        // shared flow step href = theta[r+1] - theta[r]
-        const int r = (a.flow_mode == EWS_FLOW_CACHED) ? 0 : 1;
-        if (t == r || t == r + 1) {
-          double hs = 0.0;
-          for (int cc = 0; cc < a.C; ++cc) hs += (double)a.gph[(size_t)b * a.C + cc];
-          g += (t == r + 1) ? (float)hs : -(float)hs;
-        }
-      }
-      a.dclock[bt] = g;
+  float* dpb = a.dpath + (size_t)b * a.L * a.d;
+  const long e1 = (long)k1 * a.d, last = (long)a.n_int * a.d;
+  for (long e = (long)k0 * a.d + lane; e < e1; e += 4 * 64) {
+    float g0[4], g1[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long x = e + 64 * u;
+      g0[u] = x < e1 && x >= a.d ? dvb[x - a.d] : 0.0f;
+      g1[u] = x < e1 && x < last ? dvb[x] : 0.0f;
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (e + 64 * u < e1) dpb[e + 64 * u] = g0[u] - g1[u];
+  }
+  if (!a.dclock) return;  // null: the clock gradient is not requested
+  const float* dhb = a.dh + (size_t)b * a.n_int;
+  for (int t = k0 + lane; t < k1; t += 64) {
+    float g = 0.0f;
+    if (t >= 1) g += dhb[t - 1];
+    if (t < a.n_int) g -= dhb[t];
+    if (a.flow_mode != EWS_FLOW_PER_INTERVAL) {
+      // shared flow step href = theta[r+1] - theta[r]
+      const int r = (a.flow_mode == EWS_FLOW_CACHED) ? 0 : 1;
+      if (t == r || t == r + 1) {
+        double hs = 0.0;
+        for (int cc = 0; cc < a.C; ++cc) hs += (double)a.gph[(size_t)b * a.C + cc];
+        g += (t == r + 1) ? (float)hs : -(float)hs;
+      }
+    }
+    a.dclock[(size_t)b * a.L + t] = g;
   }
 }
 
@@ -2053,12 +2274,11 @@ __global__ void k_knot_grads(DiagArgs a) {
 // range of the (B C, npar) partials in float64 (thread (r, p) takes rows r, r + R, ...: coalesced), then one
 // workgroup adds the block sums in order.
 constexpr int kParamBlocks = 128;
-__global__ __launch_bounds__(256) void k_param_partial(DiagArgs a) {
-  __shared__ double red[256];
+__device__ __forceinline__ void param_partial(const DiagArgs& a, int blk, double* red) {
   const int np = a.npar, R = 256 / np;
   const int r = threadIdx.x / np, p = threadIdx.x % np;
   const int n = a.B * a.C, per = (n + kParamBlocks - 1) / kParamBlocks;
-  const int r0 = blockIdx.x * per, r1 = min(n, r0 + per);
+  const int r0 = blk * per, r1 = min(n, r0 + per);
   double s = 0.0;
   if (r < R) {
     int bc = r0 + r;
@@ -2074,7 +2294,20 @@ __global__ __launch_bounds__(256) void k_param_partial(DiagArgs a) {
   if (threadIdx.x < np) {
     double t = 0.0;
     for (int rr = 0; rr < R; ++rr) t += red[rr * np + threadIdx.x];
-    a.gpart[(size_t)blockIdx.x * np + threadIdx.x] = t;
+    a.gpart[(size_t)blk * np + threadIdx.x] = t;
+  }
+}
+// The knot gradients and the first stage of the parameter sums, independent of each other, in one launch: workgroups
+// [0, xk) of a sample take four chunks each (a wavefront a chunk), the others the parameter blocks.
+__global__ __launch_bounds__(256) void k_knot_param(DiagArgs a, int xk) {
+  __shared__ double red[256];
+  const int x = blockIdx.x, b = blockIdx.y;
+  if (x < xk) {
+    const int c = 4 * x + (threadIdx.x >> 6);
+    if (c <= a.C) knot_grads(a, c, b);
+  } else {
+    const int blk = (x - xk) * a.B + b;
+    if (blk < kParamBlocks) param_partial(a, blk, red);
   }
 }
 __global__ __launch_bounds__(256) void k_param_grads(DiagArgs a) {
@@ -2213,6 +2446,23 @@ int make_plan(const ews_diag_desc* s, Plan& p) {
   p.lds_carry = (size_t)p.scan_cb * p.K * CW * 8 + (size_t)p.scan_cb * p.D * 4;
   p.lds_adjoint = (size_t)p.scan_cb * p.K * CW * 16 + (size_t)p.NT * CW * 8 + (size_t)p.scan_cb * p.D * 4;
   return EWS_OK;
+}
+
+// The chunk length that suits the number of intervals (a caller that leaves the choice open asks for it and puts it
+// into the descriptor's chunk). A chunk is a sequential chain, so while there are too few chunks to fill the chip its
+// length is the time; with enough of them shorter chunks only add carries. Kernel time of a training step at T = 64 /
+// 32 / 16 (us), by chunks at T = 64: pair-group planes (a wavefront takes two or four chunks) 47: 168 / 145 / 124,
+// 500: 197 / 172 / 161, 880 on an irregular clock: 443 / 346 / 307, 2250: 244 / 289 / 342; generic kernels (a
+// workgroup a chunk) at d = 24, 47: 323 / 230 / 201, 282: 378 / 317 / 344, 1560: 731 / 754 / 919.
+int suited_chunk(const Plan& p) {
+  const int enough = p.fast ? 2048 : 512;
+  int T = p.T;
+  while (T > 16 && (long)p.B * ((p.n_int + T - 1) / T) < enough) {
+    const int C2 = (p.n_int + T / 2 - 1) / (T / 2);
+    if (!p.fast && p.NG == 1 && C2 > p.scan_cb) break;  // a second chunk group costs two launches
+    T /= 2;
+  }
+  return T;
 }
 
 struct WsLayout {
@@ -2417,22 +2667,26 @@ template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
 int full_adjoints(const Plan& p, const DiagArgs& a, hipStream_t st) {
   dim3 grid(p.C, p.B), blkb(p.NTb);
   if (set_lds(&k_chunk_bwd_inv<CPLX, N, MAXT, WAVE, DH>, p.lds_bwd_inv) != EWS_OK) return EWS_ERR_LAUNCH;
+  if (set_lds(&k_chunk_bwd_inv_small<CPLX, N, MAXT, WAVE, DH>, p.lds_bwd_inv) != EWS_OK) return EWS_ERR_LAUNCH;
   if (set_lds(&k_chunk_bwd_full<CPLX, N, MAXT, WAVE, DH>, p.lds_bwd_full) != EWS_OK) return EWS_ERR_LAUNCH;
   if (!p.fast) {  // k_chunk_bwd_inv owns only FAST chunks
     hipLaunchKernelGGL((k_chunk_bwd_inv<CPLX, N, MAXT, WAVE, DH>), grid, blkb, p.lds_bwd_inv, st, a);
     EWS_LAUNCH_CHECK();
   }
-  // the recomputing adjoint's LDS leaves about one workgroup per CU, so up to eight chunks per workgroup (strided,
-  // visited only when owned) cost no parallelism while 512 or more workgroups remain, and spare the launch most of
-  // its exiting workgroups when the other kernels own the chunks
-  const int gx = p.fast ? min(p.C, 8) : min(p.C, max((p.C + 7) / 8, (512 + p.B - 1) / p.B));
+  // Both visit the chunks of their class: up to eight chunks per workgroup while 2048 workgroups remain (512 for the
+  // recomputing adjoint, whose LDS leaves about one workgroup per CU), so that a launch that owns every chunk still
+  // fills the chip and one that owns none has few workgroups to drain.
+  const int gs = min(p.C, max((p.C + 7) / 8, (2048 + p.B - 1) / p.B));
+  hipLaunchKernelGGL((k_chunk_bwd_inv_small<CPLX, N, MAXT, WAVE, DH>), dim3(gs, p.B), blkb, p.lds_bwd_inv, st, a);
+  EWS_LAUNCH_CHECK();
+  const int gx = min(p.C, max((p.C + 7) / 8, (512 + p.B - 1) / p.B));
   hipLaunchKernelGGL((k_chunk_bwd_full<CPLX, N, MAXT, WAVE, DH>), dim3(gx, p.B), blkb, p.lds_bwd_full, st, a);
   EWS_LAUNCH_CHECK();
   return EWS_OK;
 }
 
-// Backward passes: 0 chunk-local adjoints, 1 reverse adjoint scan, 2 full chunk adjoints, 3 knot gradients,
-// 4 parameter reduction.
+// Backward passes: 0 chunk-local adjoints, 1 reverse adjoint scan, 2 full chunk adjoints, 3 knot gradients and the
+// parameter partials' block sums, 4 the sum of those.
 template <bool CPLX, int N, int MAXT, bool WAVE>
 int backward_pass(const Plan& p, DiagArgs a, hipStream_t st, int pass) {
   dim3 grid(p.C, p.B), blkb(p.NTb);
@@ -2468,11 +2722,12 @@ int backward_pass(const Plan& p, DiagArgs a, hipStream_t st, int pass) {
       if (a.dclock) return full_adjoints<CPLX, N, MAXT, WAVE, true>(p, a, st);
       return full_adjoints<CPLX, N, MAXT, WAVE, false>(p, a, st);
     case 3:
-      hipLaunchKernelGGL(k_knot_grads, dim3(p.C + 1, p.B), dim3(64), 0, st, a);
+    {
+      const int xk = (p.C + 1 + 3) / 4, xp = (kParamBlocks + p.B - 1) / p.B;
+      hipLaunchKernelGGL(k_knot_param, dim3(xk + xp, p.B), dim3(256), 0, st, a, xk);
       break;
+    }
     case 4:
-      hipLaunchKernelGGL(k_param_partial, dim3(kParamBlocks), dim3(256), 0, st, a);
-      EWS_LAUNCH_CHECK();
       hipLaunchKernelGGL(k_param_grads, dim3(1), dim3(256), 0, st, a);
       break;
     default:
@@ -2656,6 +2911,13 @@ int ews_diag_backward(const ews_diag_desc* desc, const void* path, const float* 
 }
 
 int ews_diag_num_passes(int direction) { return direction == 0 ? kForwardPasses : kBackwardPasses; }
+
+int ews_diag_suited_chunk(const ews_diag_desc* desc) {
+  Plan p;
+  const int rc = make_plan(desc, p);
+  if (rc != EWS_OK) return rc;
+  return desc->chunk != 0 || p.seq ? desc->chunk : suited_chunk(p);
+}
 
 int ews_diag_uses_chunk_kernels(const ews_diag_desc* desc) {
   Plan p;

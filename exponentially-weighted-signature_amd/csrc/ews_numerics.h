@@ -263,4 +263,75 @@ template <class T, bool DERIV> EWS_HD DD3<T> dd3q(T x, T y, int q) {
   return o;
 }
 
+// Small steps: while 2 max|u| |h| <= kPolyR every coefficient is a polynomial in the clock step h whose coefficients
+// depend on the generator alone, phi(h u) = sum_m h^m u^m / (m+1)! and exp[0, h u, h v] = sum_m h^m h_m(u, v) / (m+2)!,
+// cut at degrees kPolyPhi and kPolyD (remainders below 1e-9 and 2e-8 of the value, their node derivatives below
+// 1e-7): a lane forms the coefficients once and each step is a Horner chain in the real h instead of two 13-term
+// series and five complex exponentials. A series leaf whose order reaches these degrees is the same polynomial.
+constexpr float kPolyR = 0.4f;
+constexpr int kPolyPhi = 6, kPolyD = 7;
+
+EWS_HD bool poly_order_ok(int q1, int q2) { return (q1 == 0 || q1 >= kPolyPhi) && (q2 == 0 || q2 >= kPolyD); }
+
+template <class T> EWS_HD void poly_phi(T u, T* c) {  // c[m] = u^m / (m+1)!
+  c[0] = one<T>();
+#pragma unroll
+  for (int m = 1; m <= kPolyPhi; ++m) c[m] = c[m - 1] * u * (1.0f / (float)(m + 1));
+}
+template <class T> EWS_HD void poly_dd3(T u, T v, T* c) {  // c[m] = h_m(u, v) / (m+2)!
+  T a = 0.5f * one<T>();
+  c[0] = a;
+#pragma unroll
+  for (int m = 1; m <= kPolyD; ++m) {
+    a = a * u * (1.0f / (float)(m + 2));
+    c[m] = v * c[m - 1] * (1.0f / (float)(m + 2)) + a;
+  }
+}
+EWS_HD float fma_r(float h, float a, float c) { return fmaf(h, a, c); }
+EWS_HD cf fma_r(float h, cf a, cf c) { return cf{fmaf(h, a.re, c.re), fmaf(h, a.im, c.im)}; }
+template <int M, class T> EWS_HD T poly_val(const T* c, float h) {
+  T r = c[M];
+#pragma unroll
+  for (int m = M - 1; m >= 0; --m) r = fma_r(h, r, c[m]);
+  return r;
+}
+template <int M, class T> EWS_HD T poly_val_d(const T* c, float h, T& d) {  // the value, and d/dh in d
+  T r = c[M];
+  d = zero<T>();
+#pragma unroll
+  for (int m = M - 1; m >= 0; --m) {
+    d = fma_r(h, d, r);
+    r = fma_r(h, r, c[m]);
+  }
+  return r;
+}
+
+// The node cotangents of the small-step polynomials from the moments M[m] = sum_t h_t^(m+1) g_t of a coefficient's
+// cotangents g_t: sum_t h_t g_t conj(d phi / dx) and sum_t h_t g_t conj(dD/dx), conj(dD/dy) at the steps' nodes.
+template <class T> EWS_HD T poly_phi_node(T u, const T* M) {
+  T a = 0.5f * one<T>(), g = M[0] * conj(a);  // (m+1) u^m / (m+2)!
+#pragma unroll
+  for (int m = 1; m < kPolyPhi; ++m) {
+    a = a * u * (1.0f / (float)(m + 2));
+    g += (float)(m + 1) * (M[m] * conj(a));
+  }
+  return g;
+}
+template <class T> EWS_HD void poly_dd3_node(T u, T v, const T* M, T& gx, T& gy) {
+  const float s6 = 1.0f / 6.0f;
+  T bx = s6 * one<T>(), by = bx, hx = bx, hy = bx;  // u^m / (m+3)!, v^m / (m+3)!, h_m(u,u,v) and h_m(u,v,v) over (m+3)!
+  gx = M[0] * conj(hx);
+  gy = gx;
+#pragma unroll
+  for (int m = 1; m < kPolyD; ++m) {
+    const float r3 = 1.0f / (float)(m + 3);
+    bx = bx * u * r3;
+    by = by * v * r3;
+    hx = v * hx * r3 + (float)(m + 1) * bx;
+    hy = u * hy * r3 + (float)(m + 1) * by;
+    gx += M[m] * conj(hx);
+    gy += M[m] * conj(hy);
+  }
+}
+
 }  // namespace ews

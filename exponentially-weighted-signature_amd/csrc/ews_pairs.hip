@@ -449,7 +449,8 @@ __device__ __forceinline__ void fwd_coef(const DiagArgs& a, const Lane& l, float
 
 // ------------------------------------------------------------------------------------------------ classification
 // Chunk c of sample b: flag bit 0 = uniform steps (coefficients at the mean step hbar), bit 1 = the steps may be
-// inverted backwards (stepping back amplifies errors by e^{2 Dmax tau} <= 2 over the chunk). Evaluated by the 16
+// inverted backwards (stepping back amplifies errors by e^{2 Dmax tau} <= 2 over the chunk), bit 2 = the coefficient
+// table applies, bit 3 = small steps (2 max|u| |h| <= kPolyR: the coefficients as polynomials in h). Evaluated by the 16
 // lanes of the chunk's group, each over every 16th step, then combined with DPP inside the group.
 __device__ __forceinline__ float row_max16(float v) {
   v = fmaxf(v, EWS_ROR(v, 8));
@@ -473,13 +474,14 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   const float th0 = th[0];
   const float tau = th[Tc] - th0;
   hb = tau / (float)Tc;
-  float dev = 0.0f, drift = 0.0f, bad = 0.0f;
+  float dev = 0.0f, drift = 0.0f, bad = 0.0f, hmax = 0.0f;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int t = gl + 16 * u;
     if (t < Tc) {
       const float h = x1[u] - x0[u];
       if (!isfinite(h)) bad = 1.0f;
+      hmax = fmaxf(hmax, fabsf(h));
       dev = fmaxf(dev, fabsf(h - hb));
       drift = fmaxf(drift, fabsf((x1[u] - th0) - (float)(t + 1) * hb));
     }
@@ -487,12 +489,14 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   dev = row_max16(dev);
   drift = row_max16(drift);
   bad = row_max16(bad);
+  hmax = row_max16(hmax);
   const bool fin = bad == 0.0f && isfinite(tau) && isfinite(R);
   const float lim = 4.76837158e-7f;  // 2^-21
   const bool uni = fin && R * dev <= lim && R * drift <= lim;
   const bool inv = fin && 2.0f * Dm * fabsf(tau) <= 0.69314718f;
   const bool tab = uni && R * fabsf(hb - a.ctab[0]) <= 0.5f * lim;  // the coefficient table applies
-  return (uni ? 1 : 0) | (inv ? 2 : 0) | (tab ? 4 : 0);
+  const bool small = fin && 2.0f * R * hmax <= kPolyR;
+  return (uni ? 1 : 0) | (inv ? 2 : 0) | (tab ? 4 : 0) | (small ? 8 : 0);
 }
 
 // ------------------------------------------------------------------------------------------------ carries
@@ -851,11 +855,11 @@ __global__ __launch_bounds__(64) void k_bwd_local(DiagArgs a) {
   const Lane l = lane_of<KP>(threadIdx.x);
   const int b = blockIdx.y, cb = blockIdx.x * GPW, c = cb + l.gi;
   const int nblk = (a.T + SB - 1) / SB;
-  if constexpr (SKIP_INV) {  // nothing to do when every chunk of the workgroup is left to the full local adjoint
+  {  // nothing to do when every chunk of the workgroup is left to another kernel
     bool any = false;
     for (int i = 0; i < GPW && cb + i < a.C; ++i) {
       const int fl = a.cflag[b * a.C + cb + i];
-      any = any || ((fl & 1) && (fl & 3) != 3);
+      any = any || ((fl & 1) && !(SKIP_INV && (fl & 3) == 3));
     }
     if (!any) return;
   }
@@ -1008,6 +1012,7 @@ __global__ __launch_bounds__(64) void k_bwd_full(DiagArgs a) {
   __syncthreads();
   const int ci = b * a.C + (c < a.C ? c : 0);
   const bool active = c < a.C && (a.cflag[ci] & 3) == 3;
+  if (!__any(active)) return;  // both chunks left to the generic kernels (one wavefront: uniform)
   const int t0 = c * a.T, Tc = active ? min(a.T, a.n_int - t0) : 0;
   const float hb = active ? a.chbar[ci] : 0.0f;
   // coefficients at hbar
@@ -2139,50 +2144,116 @@ __device__ __forceinline__ void lb_summary_cf(const DiagArgs& a, int b, int c, f
   __syncthreads();  // the LDS scratch is reused by the next chunk
 }
 
-// A chunk of a quad that holds a non-uniform chunk, one lane per pair (lane = 8 j + k), every step's coefficients at
-// its own clock step; the lane's full-scale states S1 (of plane j), SA, SB (of pair (j, k)) go in and out. OUT:
-// the lane writes level 1 (k = 0) and its 2 x 2 block of every prefix row.
-template <bool OUT, bool BF16>
-__device__ __forceinline__ void lb_pairwise(const DiagArgs& a, int b, int c, int j, int k, dc& S1d, dc& SAd,
-                                            dc& SBd) {
-  const int t0 = c * a.T, Tc = min(a.T, a.n_int - t0);
+// A chunk of a quad that holds a non-uniform chunk, one lane per pair (lane = 8 j + k): the lane's full-scale states S1
+// (of plane j), SA, SB (of pair (j, k)) go in and out. OUT: the lane writes level 1 (k = 0) and its 2 x 2 block of
+// every prefix row. The chunk's increments are staged in LDS by the lanes (lane = step, both knots loaded a chunk
+// ahead) and the clock step of step t is lane t's register, so no load sits on the recursion. Small steps take the
+// polynomial coefficients (PwCoef, formed once per quad: about 60 multiply-adds a step), the others each step's exact
+// ones, two 13-term series and five exponentials.
+struct PwCoef {
+  cf uj, uk, ph[kPolyPhi + 1], phk[kPolyPhi + 1], B[kPolyD + 1], A[kPolyD + 1];
+};
+__device__ __forceinline__ void pw_init(const DiagArgs& a, int j, int k, PwCoef& p) {
+  p.uj = load_u(a.params, j);
+  p.uk = load_u(a.params, k);
+  poly_phi(p.uj, p.ph);
+  poly_phi(p.uk, p.phk);
+  poly_dd3(p.uj, p.uj + p.uk, p.B);
+  poly_dd3(p.uj, p.uj + conj(p.uk), p.A);
+}
+// the lane's knots and clock step of one chunk (lane = step); lanes past the chunk hold zeros
+template <bool BF16> struct PwIn {
+  float x0[DIM], x1[DIM], h;
+};
+template <bool BF16> __device__ __forceinline__ void pw_load(const DiagArgs& a, int b, int c, PwIn<BF16>& in) {
+  const int l = threadIdx.x, t0 = c * a.T, Tc = min(a.T, a.n_int - t0);
   const float* th = a.clock + (size_t)b * a.L + t0;
-  const cf uj = load_u(a.params, j), uk = load_u(a.params, k);
-  const cf ub = uj + uk, ua = uj + conj(uk);
-  cf S1{(float)S1d.re, (float)S1d.im}, SA{(float)SAd.re, (float)SAd.im}, SBv{(float)SBd.re, (float)SBd.im};
+#pragma unroll
+  for (int i = 0; i < DIM; ++i) in.x0[i] = in.x1[i] = 0.0f;
+  in.h = 0.0f;
+  if (l < Tc) {
+    load_knot<BF16>(a, b, t0 + l, in.x0);
+    load_knot<BF16>(a, b, t0 + l + 1, in.x1);
+    in.h = th[l + 1] - th[l];
+  }
+}
+template <bool BF16> __device__ __forceinline__ void pw_stage(const PwIn<BF16>& in, float (*s_p)[DIM]) {
+#pragma unroll
+  for (int i = 0; i < DIM; i += 4)
+    *reinterpret_cast<f4a*>(&s_p[threadIdx.x][i]) =
+        f4a{in.x1[i] - in.x0[i], in.x1[i + 1] - in.x0[i + 1], in.x1[i + 2] - in.x0[i + 2], in.x1[i + 3] - in.x0[i + 3]};
+}
+template <bool OUT, bool SMALL>
+__device__ __forceinline__ void lb_pairwise(const DiagArgs& a, int b, int c, int j, int k, const PwCoef& p, float hl,
+                                            const float (*s_p)[DIM], PairSt& z) {
+  const int t0 = c * a.T, Tc = min(a.T, a.n_int - t0);
+  const cf uj = p.uj, uk = p.uk, ub = uj + uk, ua = uj + conj(uk);
+  cf S1{(float)z.S1.re, (float)z.S1.im}, SA{(float)z.SA.re, (float)z.SA.im}, SBv{(float)z.SB.re, (float)z.SB.im};
+  float* row = OUT ? a.out + ((size_t)b * a.n_int + t0) * a.W : nullptr;
   for (int t = 0; t < Tc; ++t) {
-    const size_t ix = (size_t)b * a.L + t0 + t;
-    cf pj, pk;
-    if constexpr (!BF16) {
-      const float* x = reinterpret_cast<const float*>(a.path) + ix * DIM;
-      pj = cf{x[DIM + 2 * j] - x[2 * j], x[DIM + 2 * j + 1] - x[2 * j + 1]};
-      pk = cf{x[DIM + 2 * k] - x[2 * k], x[DIM + 2 * k + 1] - x[2 * k + 1]};
+    const float h = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hl), t));
+    const float2 vj = *reinterpret_cast<const float2*>(&s_p[t][2 * j]), vk = *reinterpret_cast<const float2*>(&s_p[t][2 * k]);
+    const cf pj{vj.x, vj.y}, pk{vk.x, vk.y};
+    cf rho, phj, phk, LB, LA, IB, IA;
+    if constexpr (SMALL) {
+      phj = poly_val<kPolyPhi>(p.ph, h);
+      phk = poly_val<kPolyPhi>(p.phk, h);
+      rho = (h * uj) * phj + 1.0f;
+      const cf rk = (h * uk) * phk + 1.0f;
+      LB = rho * rk;
+      LA = rho * conj(rk);
+      IB = poly_val<kPolyD>(p.B, h);
+      IA = poly_val<kPolyD>(p.A, h);
     } else {
-      const unsigned short* x = reinterpret_cast<const unsigned short*>(a.path) + ix * DIM;
-      auto bf = [](unsigned short v) { return __uint_as_float((unsigned)v << 16); };
-      pj = cf{bf(x[DIM + 2 * j]) - bf(x[2 * j]), bf(x[DIM + 2 * j + 1]) - bf(x[2 * j + 1])};
-      pk = cf{bf(x[DIM + 2 * k]) - bf(x[2 * k]), bf(x[DIM + 2 * k + 1]) - bf(x[2 * k + 1])};
+      const cf xj = h * uj;
+      const Node1<cf> nj = node1(xj);
+      rho = nj.e;
+      phj = nj.p;
+      phk = node1(h * uk).p;
+      LB = expv(h * ub);
+      LA = expv(h * ua);
+      IB = dd3<cf, false>(xj, h * ub).d;
+      IA = dd3<cf, false>(xj, h * ua).d;
     }
-    const float h = th[t + 1] - th[t];
-    const cf xj = h * uj;
-    const Node1<cf> nj = node1(xj);
-    const cf s1k = node1(h * uk).p * pk;
-    const cf cj = nj.e * S1;
-    SBv = expv(h * ub) * SBv + cj * s1k + dd3<cf, false>(xj, h * ub).d * (pj * pk);
-    SA = expv(h * ua) * SA + cj * conj(s1k) + dd3<cf, false>(xj, h * ua).d * (pj * conj(pk));
-    S1 = cj + nj.p * pj;
+    const cf s1k = phk * pk;
+    const cf cj = rho * S1;
+    SBv = LB * SBv + cj * s1k + IB * (pj * pk);
+    SA = LA * SA + cj * conj(s1k) + IA * (pj * conj(pk));
+    S1 = cj + phj * pj;
     if constexpr (OUT) {
-      float* row = a.out + ((size_t)b * a.n_int + t0 + t) * a.W;
       if (a.lvl0 && j == 0 && k == 0) row[0] = 1.0f;
       if (k == 0) *reinterpret_cast<f2u*>(row + a.off1 + 2 * j) = f2u{S1.re, S1.im};
       float* r0 = row + a.off2 + (2 * j) * DIM + 2 * k;
       *reinterpret_cast<f2u*>(r0) = f2u{0.5f * (SA.re + SBv.re), 0.5f * (SBv.im - SA.im)};
       *reinterpret_cast<f2u*>(r0 + DIM) = f2u{0.5f * (SA.im + SBv.im), 0.5f * (SA.re - SBv.re)};
+      row += a.W;
     }
   }
-  S1d = dc{(double)S1.re, (double)S1.im};
-  SAd = dc{(double)SA.re, (double)SA.im};
-  SBd = dc{(double)SBv.re, (double)SBv.im};
+  z.S1 = dc{(double)S1.re, (double)S1.im};
+  z.SA = dc{(double)SA.re, (double)SA.im};
+  z.SB = dc{(double)SBv.re, (double)SBv.im};
+}
+// The nc chunks of a quad in turn: from the zero state to their summaries (OUT false: s_row[i] written), or from the
+// carries in s_row[i] to the prefix rows.
+// SMALL: every chunk of the quad has small steps.
+template <bool OUT, bool BF16, bool SMALL>
+__device__ __forceinline__ void lb_pairwise_quad(const DiagArgs& a, int b, int cb, int nc, int j, int k,
+                                                 float (*s_p)[DIM], float (*s_row)[RBUF]) {
+  PwCoef p;
+  pw_init(a, j, k, p);
+  PwIn<BF16> in;
+  pw_load<BF16>(a, b, cb, in);
+  for (int i = 0; i < nc; ++i) {
+    __syncthreads();  // the previous chunk's increments have been read (and, first, the classes written)
+    pw_stage<BF16>(in, s_p);
+    const float hl = in.h;
+    __syncthreads();
+    if (i + 1 < nc) pw_load<BF16>(a, b, cb + i + 1, in);
+    PairSt z{};
+    if (OUT) z = load_st_f(s_row[i], j, k);
+    lb_pairwise<OUT, SMALL>(a, b, cb + i, j, k, p, hl, s_p, z);
+    if (!OUT) store_st_f(s_row[i], j, k, z);
+  }
 }
 
 template <bool BF16>
@@ -2222,6 +2293,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     }
   }
   const bool quad_uni = __all(!act || (flag & 1));  // wavefront-uniform: the staging is shared
+  const bool quad_small = __all(!act || (flag & 8));
+  float(*s_p)[DIM] = reinterpret_cast<float(*)[DIM]>(&s_v[0][0]);  // a non-uniform quad's increments, chunk by chunk
   const int t0 = act ? c * a.T : 0, Tc = act ? min(a.T, a.n_int - t0) : 0;
   if (quad_uni) {  // the summaries in closed form, chunk by chunk (lane = step); the next chunk's loads in flight
     __shared__ float s_tot[DIM];
@@ -2235,11 +2308,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
       in = nx;
     }
   } else {
-    for (int i = 0; i < nc; ++i) {
-      PairSt z{};
-      lb_pairwise<false, BF16>(a, b, cb + i, jj, kk, z.S1, z.SA, z.SB);
-      store_st_f(s_row[i], jj, kk, z);
-    }
+    if (quad_small) lb_pairwise_quad<false, BF16, true>(a, b, cb, nc, jj, kk, s_p, s_row);
+    else lb_pairwise_quad<false, BF16, false>(a, b, cb, nc, jj, kk, s_p, s_row);
   }
   if (tid < 8 * nc) s_F[tid >> 3][tid & 7] = span_flow(a, b, cb + (tid >> 3), cb + (tid >> 3) + 1, tid & 7);
   __syncthreads();
@@ -2315,10 +2385,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     wave_order();
     lb_steps<true, BF16>(a, l, b, cb, t0, Tc, f, S1, SA, SB_, s_v, s_row[l.gi]);
   } else {
-    for (int i = 0; i < nc; ++i) {
-      PairSt z = load_st_f(s_row[i], jj, kk);
-      lb_pairwise<true, BF16>(a, b, cb + i, jj, kk, z.S1, z.SA, z.SB);
-    }
+    if (quad_small) lb_pairwise_quad<true, BF16, true>(a, b, cb, nc, jj, kk, s_p, s_row);
+    else lb_pairwise_quad<true, BF16, false>(a, b, cb, nc, jj, kk, s_p, s_row);
   }
 }
 

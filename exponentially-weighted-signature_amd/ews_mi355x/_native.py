@@ -85,6 +85,7 @@ EXPORTED = (
     "ews_token1_scan",
     "ews_token1_scan_backward",
     "ews_diag_mixer_forward",
+    "ews_diag_suited_chunk",
     "ews_diag_uses_chunk_kernels",
 )
 
@@ -366,6 +367,8 @@ def load():
     lib.ews_chain_backward.restype = i32
     lib.ews_diag_mixer_forward.argtypes = [dp, ctypes.POINTER(MixerDesc), vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.ews_diag_mixer_forward.restype = i32
+    lib.ews_diag_suited_chunk.argtypes = [dp]
+    lib.ews_diag_suited_chunk.restype = i32
     lib.ews_diag_uses_chunk_kernels.argtypes = [dp]
     lib.ews_diag_uses_chunk_kernels.restype = i32
     t1p = ctypes.POINTER(Token1Desc)

@@ -40,6 +40,14 @@ def _aligned(x):
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _suited_chunk(lib, B, L, d, N, structure, flow_mode, readout, level0, dt, chunk, leaf, series_q):
+    """The library's chunk length for this many intervals where the caller leaves it open (chunk 0)."""
+    if chunk:
+        return chunk
+    desc = make_desc(B, L, d, N, structure, flow_mode, readout, level0, dt, 0, leaf, series_q)
+    return max(0, int(lib.ews_diag_suited_chunk(ctypes.byref(desc))))  # an invalid descriptor: the call reports it
+
+
 class DiagScan(torch.autograd.Function):
     """out = EWS readout of (path, clock) under a diagonal / rotation-plane generator with parameters
     ``params`` ((d/2, 2) rows (d_j, w_j) for planes, (d,) for a real diagonal)."""
@@ -53,6 +61,7 @@ class DiagScan(torch.autograd.Function):
         params = params.contiguous()
         B, L, d = path.shape
         dt = nat.DTYPE_BF16 if path.dtype == torch.bfloat16 else nat.DTYPE_F32
+        chunk = _suited_chunk(lib, B, L, d, N, structure, flow_mode, readout, level0, dt, chunk, leaf, series_q)
         desc = make_desc(B, L, d, N, structure, flow_mode, readout, level0, dt, chunk, leaf, series_q)
         D = d + (d * d if N == 2 else 0)
         W = D + (1 if level0 else 0)
@@ -607,7 +616,8 @@ class ScanMixerFn(torch.autograd.Function):
         B, L, d = path.shape
         hidden = weight.shape[0]
         dt = nat.DTYPE_BF16 if path.dtype == torch.bfloat16 else nat.DTYPE_F32
-        sdesc = make_desc(B, L, d, N, structure, flow_mode, "prefix", True, dt, 0, leaf, series_q)
+        chunk = _suited_chunk(lib, B, L, d, N, structure, flow_mode, "prefix", True, dt, 0, leaf, series_q)
+        sdesc = make_desc(B, L, d, N, structure, flow_mode, "prefix", True, dt, chunk, leaf, series_q)
         eps3 = (ctypes.c_float * 3)(*[float(x) for x in (list(eps) + [0.0] * 3)[:3]])
         mdesc = nat.MixerDesc(B, L - 1, d, N, 1, hidden, nat.GRADED_VARIANTS[variant], int(prepend), int(prescale),
                               eps3)

@@ -464,6 +464,13 @@ int ews_mixer_backward_weight(const ews_mixer_desc* desc, const float* rows, con
                               const void* residual, const float* grad_out, float* grad_rows, float* row_dots,
                               float* grad_weight, void* workspace, ews_stream_t stream);
 
+/* The intervals per chunk that suit this descriptor's batch and length, for a caller that leaves the choice open: the
+ * default chunk for many intervals, down to 16 for few (a chunk is a sequential chain; too few of them leave the chip
+ * idle). The descriptor's own chunk when it is not 0; 0 where the per-sample sequential kernels run; a negative error
+ * code for an invalid descriptor. Put it into chunk before the size queries: they and every call must agree on it. No
+ * counterpart in the reference. */
+int ews_diag_suited_chunk(const ews_diag_desc* desc);
+
 /* 1 when ews_diag_forward runs this configuration on the chunk kernels (where ews_diag_mixer_forward applies), 0
  * otherwise (the pair-group planes, the per-sample sequential kernels, an invalid descriptor). No counterpart in
  * the reference: it tells a caller which route of the block's epilogue to take. */
