@@ -36,7 +36,8 @@ from typing import Optional
 import torch
 
 from . import ops
-from .params import AParamConstant, block_sizes_of, diagonal_structure, is_rotation_planes, jordan_chains_of
+from .params import (AParamConstant, block_sizes_of, diagonal_structure, is_rotation_planes, jordan_chains_of,
+                     kernel_rows)
 
 LEAF_KINDS = ("van_loan", "series", "plane_closed", "block_series", "jordan_closed", "jordan_closed_tables")
 COMBINE_KINDS = ("assoc", "lean", "block_kernel", "dense_kernel")
@@ -143,11 +144,30 @@ class EWS(torch.nn.Module):
             return "cached_basepoint"
         return "per_interval"
 
-    def _diag_params(self, A):
-        """Kernel parameters read off the materialised A as ews/core/leaf.py:130-131 reads them."""
+    @staticmethod
+    def _scaled(A, a_scale, device):
+        """A times a_scale in float32 (a plain number needs no tensor on the device, and 1 no product). A has to be on
+        the path's device."""
+        A = A.to(torch.float32)
+        if device.type != "cpu" and A.device != device:
+            raise RuntimeError("Expected all tensors to be on the same device, but found the generator on "
+                               f"{A.device} and the path on {device}")
+        if isinstance(a_scale, (int, float)):
+            return A if a_scale == 1 else A * float(a_scale)
+        return A * torch.as_tensor(a_scale, dtype=torch.float32, device=device)
+
+    def _diag_params(self, device, a_scale):
+        """Kernel parameters as ews/core/leaf.py:130-131 reads them off the materialised A times a_scale: straight from
+        the parametrisation where it holds them, else off A (row 0 of every 2 x 2 block, or the diagonal). a_scale
+        None: unscaled, moved to the path's device."""
+        rows = kernel_rows(self.A_param)
+        A = self.A_param() if rows is None else rows
+        A = A.to(device, torch.float32) if a_scale is None else self._scaled(A, a_scale, device)
+        if rows is not None:
+            return A.contiguous()
         if self.structure == "planes":
-            ii = torch.arange(0, self.d, 2, device=A.device)
-            return torch.stack([A[ii, ii], A[ii, ii + 1]], -1).contiguous()
+            K = self.d // 2
+            return A.reshape(K, 2, K, 2).diagonal(dim1=0, dim2=2)[0].t().contiguous()
         return torch.diagonal(A).contiguous()
 
     def _chain_form(self):
@@ -222,7 +242,15 @@ class EWS(torch.nn.Module):
         engine = self._engine_check()
         if self.dtype != torch.float32:
             raise TypeError("the MI355X kernels compute in float32 (dtype=torch.float32)")
-        A = self.A_param().to(torch.float32) * torch.as_tensor(a_scale, dtype=torch.float32, device=path.device)
+        if engine == "diag":
+            params = self._diag_params(path.device, a_scale)
+            if path.dtype != torch.bfloat16:
+                path = path.to(torch.float32)
+            clock = clock.to(torch.float32)
+            leaf = self.leaf if self.leaf in ("series", "block_series") else "plane_closed"
+            return ops.diag_scan(path, clock, params, self.N, self.structure, self._flow_mode(readout), readout,
+                                 level0, chunk=0, leaf=leaf, series_q=self.series_q or 0)
+        A = self._scaled(self.A_param(), a_scale, path.device)
         if engine == "chain":
             kind, size, q, step = self._chain_form()
             kr = readout if readout in ("prefix", "terminal") else "prefix"
@@ -233,38 +261,30 @@ class EWS(torch.nn.Module):
             if readout == "max":
                 return out.max(1).values
             return out
-        if engine == "dense":
-            chen = "exact" if self.jordan_flows else self.chen_expm  # closed-form chain flows are exact
-            if self.leaf in JORDAN_LEAVES or (self.leaf == "plane_closed" and self.structure == "planes"):
-                # the chains' closed-form local terms at any step (a rotation plane is a complex chain of one
-                # coordinate), the flows of chen_expm, the dense combine
-                kind, size = jordan_chains_of(self.A_param) if self.leaf in JORDAN_LEAVES else ("complex", 2)
-                return ops.jordan_scan(path.to(torch.float32), clock.to(torch.float32),
-                                       A.to(path.device).contiguous(), self.N, kind, size, self._flow_mode(readout),
-                                       readout, level0, chen_expm=chen)
-            if self.leaf == "block_series":
-                # the block-series leaf (general blocks, or planes / diagonals under approximate flows): the exact
-                # level 1 G v at any step and the blockwise order-series_q series at level 2, as the reference
-                # computes them (ews/core/leaf.py:138-175, blockdiag_engine.py:88-155)
-                leaf = ops.DenseLeaf("block_series", q=self.series_q or 0, chen_expm=chen)
-                return ops.dense_scan(path.to(torch.float32), clock.to(torch.float32),
-                                      A.to(path.device).contiguous(), self.N, leaf.q, self._flow_mode(readout),
-                                      readout, level0, leaf=leaf, keep=self._keep_dense())
-            if self.leaf == "van_loan":
-                leaf = ops.DenseLeaf("van_loan", M=self.M, van_loan_expm=self.van_loan_expm,
-                                     reweighting_mode=self.reweighting_mode, chen_expm=chen)
-            else:
-                leaf = ops.DenseLeaf("series", q=self.series_q, chen_expm=chen)
-            return ops.dense_scan(path.to(torch.float32), clock.to(torch.float32), A.to(path.device).contiguous(),
-                                  self.N, leaf.q, self._flow_mode(readout), readout, level0, leaf=leaf,
-                                  keep=self._keep_dense())
-        params = self._diag_params(A.to(path.device))
-        if path.dtype != torch.bfloat16:
-            path = path.to(torch.float32)
-        clock = clock.to(torch.float32)
-        leaf = self.leaf if self.leaf in ("series", "block_series") else "plane_closed"
-        return ops.diag_scan(path, clock, params, self.N, self.structure, self._flow_mode(readout), readout,
-                             level0, chunk=0, leaf=leaf, series_q=self.series_q or 0)
+        chen = "exact" if self.jordan_flows else self.chen_expm  # closed-form chain flows are exact
+        if self.leaf in JORDAN_LEAVES or (self.leaf == "plane_closed" and self.structure == "planes"):
+            # the chains' closed-form local terms at any step (a rotation plane is a complex chain of one
+            # coordinate), the flows of chen_expm, the dense combine
+            kind, size = jordan_chains_of(self.A_param) if self.leaf in JORDAN_LEAVES else ("complex", 2)
+            return ops.jordan_scan(path.to(torch.float32), clock.to(torch.float32),
+                                   A.to(path.device).contiguous(), self.N, kind, size, self._flow_mode(readout),
+                                   readout, level0, chen_expm=chen)
+        if self.leaf == "block_series":
+            # the block-series leaf (general blocks, or planes / diagonals under approximate flows): the exact
+            # level 1 G v at any step and the blockwise order-series_q series at level 2, as the reference
+            # computes them (ews/core/leaf.py:138-175, blockdiag_engine.py:88-155)
+            leaf = ops.DenseLeaf("block_series", q=self.series_q or 0, chen_expm=chen)
+            return ops.dense_scan(path.to(torch.float32), clock.to(torch.float32),
+                                  A.to(path.device).contiguous(), self.N, leaf.q, self._flow_mode(readout),
+                                  readout, level0, leaf=leaf, keep=self._keep_dense())
+        if self.leaf == "van_loan":
+            leaf = ops.DenseLeaf("van_loan", M=self.M, van_loan_expm=self.van_loan_expm,
+                                 reweighting_mode=self.reweighting_mode, chen_expm=chen)
+        else:
+            leaf = ops.DenseLeaf("series", q=self.series_q, chen_expm=chen)
+        return ops.dense_scan(path.to(torch.float32), clock.to(torch.float32), A.to(path.device).contiguous(),
+                              self.N, leaf.q, self._flow_mode(readout), readout, level0, leaf=leaf,
+                              keep=self._keep_dense())
 
     def _log_prefix_fused(self, path, clock):
         """LogEWS prefix rows computed inside the scan (rotation planes or a real diagonal, depth 2, the diagonal
@@ -277,8 +297,7 @@ class EWS(torch.nn.Module):
             return None
         if self.dtype != torch.float32:
             raise TypeError("the MI355X kernels compute in float32 (dtype=torch.float32)")
-        A = self.A_param().to(torch.float32)
-        params = self._diag_params(A.to(path.device))
+        params = self._diag_params(path.device, None)
         if path.dtype != torch.bfloat16:
             path = path.to(torch.float32)
         leaf = self.leaf if self.leaf in ("series", "block_series") else "plane_closed"
@@ -296,8 +315,7 @@ class EWS(torch.nn.Module):
         if mixer.d != self.d or mixer.N != self.N or mixer.hidden_dim > 64 or self._engine_check() != "diag":
             return None
         self._check_batch(path, clock)
-        A = self.A_param().to(torch.float32) * torch.as_tensor(a_scale, dtype=torch.float32, device=path.device)
-        params = self._diag_params(A.to(path.device))
+        params = self._diag_params(path.device, a_scale)
         if path.dtype != torch.bfloat16:
             path = path.to(torch.float32)
         leaf = self.leaf if self.leaf in ("series", "block_series") else "plane_closed"

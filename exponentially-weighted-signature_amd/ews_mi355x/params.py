@@ -267,14 +267,12 @@ class AParamDampedRotation(torch.nn.Module):
 
 
 def _planes_to_dense(dw):
-    """(P, 2) rows (d_j, w_j) -> block-diagonal (2P, 2P) with blocks [[d, w], [-w, d]]."""
+    """(P, 2) rows (d_j, w_j) -> block-diagonal (2P, 2P) with blocks [[d, w], [-w, d]]. The four entries of every
+    block lie on the diagonal of a (2, 2, P, P) view, so one diagonal embedding places them (its gradient is a view;
+    four indexed writes and their gathers were forty launches of a training step)."""
     P = dw.shape[0]
-    A = torch.zeros((2 * P, 2 * P), dtype=dw.dtype, device=dw.device)
-    i = torch.arange(P, device=dw.device)
-    A = A.index_put((2 * i, 2 * i), dw[:, 0])
-    A = A.index_put((2 * i + 1, 2 * i + 1), dw[:, 0])
-    A = A.index_put((2 * i, 2 * i + 1), dw[:, 1])
-    A = A.index_put((2 * i + 1, 2 * i), -dw[:, 1])
+    d, w = dw.unbind(-1)
+    A = torch.diag_embed(torch.stack([d, w, -w, d]).reshape(2, 2, P)).permute(2, 0, 3, 1).reshape(2 * P, 2 * P)
     A._ews_chain = ("complex", 2)  # rotation planes by construction (read without a device-to-host copy)
     return A
 
@@ -294,6 +292,27 @@ def block_sizes_of(a_param):
 def is_rotation_planes(a_param):
     """combine.py:61-63."""
     return type(a_param).__name__ in ROTATION_CLASSES
+
+
+def _hooked(module):
+    from torch.nn.modules import module as m
+
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+                module._backward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks or
+                m._global_backward_hooks or m._global_backward_pre_hooks)
+
+
+def kernel_rows(a_param):
+    """The diagonal kernels' parameters, (d/2, 2) plane rows (d_j, w_j) or the (d,) diagonal, straight from a
+    parametrisation whose forward is one of this module's own (the exact class, no hooks), without forming A; None
+    for any other, whose A has to be read."""
+    if _hooked(a_param):
+        return None
+    if type(a_param) in (AParamBoundedRotation, AParamDampedRotation):
+        return a_param.plane_params()
+    if type(a_param) is AParamEFM:
+        return a_param.diagonal()
+    return None
 
 
 def diagonal_structure(a_param):
