@@ -20,8 +20,8 @@
 // runs of chunks composed in parallel, then chained), the chunk's flow taken in closed form over its clock span (the
 // chain's flows commute); the rows from the carries. Adjoint: each chunk's own rows from a zero cotangent (its
 // cotangent on the carry-in state), a float64 reverse scan over chunks (the same parallel scan), then each chunk
-// from the cotangent at its end with the states recomputed from its carry into LDS: dv, dh and the chain-parameter
-// partials (c, eps), summed in a fixed order (deterministic). Gradients of A land on the entries the chain is read
+// from the cotangent at its end with the states by inverting its steps (or recomputed from its carry): the knot
+// gradients and the chain-parameter partials (c, eps), summed in a fixed order (deterministic). Gradients of A land on the entries the chain is read
 // from (A[f, f], A[f+1, f] and the coupling A[f, f+1] or A[f, f+2], f the chain's first row), as the reference's
 // closed-form leaf and jordan_flows read them; a parametrisation of uniform chains gets its exact parameter gradient
 // from them.
@@ -69,9 +69,12 @@ __device__ __forceinline__ zd zexp(zd a) {
   return zd{m * c, m * s};
 }
 
-constexpr int kTaylor = 28;       // terms of the phi^(r) series (|x| <= 2: the tail is below 1e-20)
+// terms of the phi^(r) series by |x|: the tails are below 1e-20 (2^-9: x^7 / 7! = 2e-23; 1/8: 3e-22; 2: 1e-21)
+constexpr int kTaylor0 = 7, kTaylor1 = 13, kTaylor = 28;
+constexpr double kReach0 = 1.0 / 512, kReach1 = 0.125;
 constexpr double kSwitch = 2.0;   // |x| above which the recurrence from e^x takes over
-constexpr int kMaxT = 64;         // longest chunk (the adjoint's LDS holds a chunk of states per lane)
+constexpr int kMaxT = 64;         // longest chunk
+constexpr double kInvert = 8.0;   // largest log contraction of a chunk whose steps the adjoint inverts
 
 struct CArgs {
   int B, L, n, d, K, size, cplx, M;  // M: coordinates per chain (complex for complex chains)
@@ -86,8 +89,9 @@ struct CArgs {
   double* summ;     // (B, C, K, M) complex: each chunk from a zero state
   double* mu;       // (B, C, K, M) complex: the chunk's own rows' cotangent on its carry-in state
   double* mt;       // (B, C, K, M) complex: the cotangent at the chunk's end from the later chunks
-  float* dv;        // (B, n, d) per-interval increment cotangents
-  float* dh;        // (B, n) per-interval step cotangents (every chain's)
+  float* dvb;       // (B, C, 2, d) increment cotangents of each chunk's first and last interval
+  float* dhb;       // (B, C, 2) step cotangents of those (every chain's)
+  float2* st;       // (B, n, K, M) states before each step, of the chunks whose steps are not inverted
   double* pp;       // (B, C, K, 5): partials of Re c, Im c, eps, and of the reference steps theta1-theta0, theta2-theta1
   float* gpath;
   float* gclock;
@@ -116,9 +120,33 @@ __device__ __forceinline__ double mode_step(const float* th, int L, int t, doubl
   return (double)th[2] - (double)th[1];
 }
 
-// u[r] = phi^(r)(x) / r!, r = 0..R: exact (q = 0) or of the degree-q Taylor polynomial of phi
+// sum_{j < NT} x^j / ((j + r + 1) j! r!), r = 0..R, the constants at compile time
+template <int R, int NT>
+__device__ __forceinline__ void u_series(zd x, zd* u) {
+  zd t = Z(1.0);  // x^j
+  double jf = 1.0, rf[R + 1];
+  rf[0] = 1.0;
+#pragma unroll
+  for (int r = 1; r <= R; ++r) rf[r] = rf[r - 1] * (double)r;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+#pragma unroll
+    for (int r = 0; r <= R; ++r) {
+      const double k = 1.0 / ((double)(j + r + 1) * jf * rf[r]);
+      u[r].re = fma(k, t.re, u[r].re);
+      u[r].im = fma(k, t.im, u[r].im);
+    }
+    t = t * x;
+    jf *= (double)(j + 1);
+  }
+}
+
+// u[r] = phi^(r)(x) / r!, r = 0..R: exact (q = 0) or of the degree-q Taylor polynomial of phi; ex = e^x for q = 0.
+// The exact series takes as many terms as the wavefront's largest |x| needs: a gated clock's steps of 1/L lie far
+// inside 2^-9, where 7 terms serve for 28.
 template <int R>
-__device__ __forceinline__ void u_table(zd x, int q, zd* u) {
+__device__ __forceinline__ void u_table(zd x, int q, zd* u, zd& ex) {
+  ex = Z(1.0);
 #pragma unroll
   for (int r = 0; r <= R; ++r) u[r] = Z(0.0);
   if (q > 0) {
@@ -140,20 +168,14 @@ __device__ __forceinline__ void u_table(zd x, int q, zd* u) {
     return;
   }
   if (x.re * x.re + x.im * x.im <= kSwitch * kSwitch) {
-    zd t = Z(1.0);  // x^j / j!
-    for (int j = 0; j < kTaylor; ++j) {
-#pragma unroll
-      for (int r = 0; r <= R; ++r) u[r] += (1.0 / (double)(j + r + 1)) * t;
-      t = (1.0 / (double)(j + 1)) * (t * x);
-    }
-    double f = 1.0;
-#pragma unroll
-    for (int r = 1; r <= R; ++r) {
-      f *= (double)r;
-      u[r] = (1.0 / f) * u[r];
-    }
+    const double ax2 = x.re * x.re + x.im * x.im;
+    if (!__any(ax2 > kReach0 * kReach0)) u_series<R, kTaylor0>(x, u);
+    else if (!__any(ax2 > kReach1 * kReach1)) u_series<R, kTaylor1>(x, u);
+    else u_series<R, kTaylor>(x, u);
+    ex = Z(1.0) + x * u[0];
   } else {
     const zd e = zexp(x);
+    ex = e;
     zd ph = zdiv(e - Z(1.0), x);
     u[0] = ph;
     double f = 1.0;
@@ -173,15 +195,15 @@ struct Coef {
 };
 template <int M>
 __device__ __forceinline__ void coefs(zd c, double eps, double hl, double hf, int q, Coef<M>& k) {
-  zd u[M];
-  u_table<M - 1>(Z(-hl) * c, q, u);
+  zd u[M], ex;
+  u_table<M - 1>(-hl * c, q, u, ex);
   double hp = 1.0;
 #pragma unroll
   for (int p = 0; p < M; ++p) {
     k.g[p] = hp * u[p];
     hp *= -hl;
   }
-  k.e[0] = zexp(Z(-hf) * c);
+  k.e[0] = q == 0 && hl == hf ? ex : zexp(-hf * c);  // one step for the leaf and the flow: e^x = 1 + x phi(x)
 #pragma unroll
   for (int p = 1; p < M; ++p) k.e[p] = (-hf * eps / (double)p) * k.e[p - 1];
 }
@@ -203,9 +225,24 @@ __device__ __forceinline__ void step(const Coef<M>& k, double eps, const zd* v, 
 // the chunk's flow over a clock span tau: e^{-tau c} sum_p (-tau eps)^p / p! Nil^p
 template <int M>
 __device__ __forceinline__ void span_flow(zd c, double eps, double tau, zd* F) {
-  F[0] = zexp(Z(-tau) * c);
+  F[0] = zexp(-tau * c);
 #pragma unroll
   for (int p = 1; p < M; ++p) F[p] = (-tau * eps / (double)p) * F[p - 1];
+}
+// the flow over one interval's step: e^x from the series of phi while |x| is small (a sine, a cosine and an
+// exponential in float64 otherwise)
+template <int M>
+__device__ __forceinline__ void flow_of(zd c, double eps, double h, zd* F) {
+  const zd x = -h * c;
+  if (x.re * x.re + x.im * x.im <= kReach1 * kReach1) {
+    zd u[1], ex;
+    u_table<0>(x, 0, u, ex);
+    F[0] = ex;
+  } else {
+    F[0] = zexp(x);
+  }
+#pragma unroll
+  for (int p = 1; p < M; ++p) F[p] = (-h * eps / (double)p) * F[p - 1];
 }
 // the flow span of chunk cc under the flow mode
 __device__ __forceinline__ double chunk_span(const CArgs& a, const float* th, int cc) {
@@ -222,6 +259,33 @@ __device__ __forceinline__ void load_knot(const CArgs& a, int b, int t, int j, z
   const float* r = a.path + ((size_t)b * a.L + t) * a.d + (size_t)j * a.size;
 #pragma unroll
   for (int i = 0; i < M; ++i) x[i] = CPLX ? Z((double)r[2 * i], (double)r[2 * i + 1]) : Z((double)r[i]);
+}
+
+// A chain's coordinates of one row as loaded (floats, converted at their use), and stored.
+template <int M, bool CPLX> struct Knot {
+  float x[CPLX ? 2 * M : M];
+  __device__ __forceinline__ void row(const float* r) {
+#pragma unroll
+    for (int i = 0; i < (CPLX ? 2 * M : M); ++i) x[i] = r[i];
+  }
+  __device__ __forceinline__ void load(const CArgs& a, int b, int t, int j) {
+    row(a.path + ((size_t)b * a.L + t) * a.d + (size_t)j * a.size);
+  }
+  __device__ __forceinline__ void get(zd* z) const {
+#pragma unroll
+    for (int i = 0; i < M; ++i) z[i] = CPLX ? Z((double)x[2 * i], (double)x[2 * i + 1]) : Z((double)x[i]);
+  }
+};
+template <int M, bool CPLX> __device__ __forceinline__ void st_row(float* r, const zd* z) {
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    if (CPLX) {
+      r[2 * i] = (float)z[i].re;
+      r[2 * i + 1] = (float)z[i].im;
+    } else {
+      r[i] = (float)z[i].re;
+    }
+  }
 }
 
 struct Lane {
@@ -277,37 +341,37 @@ __device__ __forceinline__ void fwd_body(const CArgs& a) {
     for (int i = 0; i < M; ++i) S[i] = Z(0.0);
   }
   const float* th = a.clock + (size_t)l.b * a.L;
-  zd x0[M], x1[M], v[M];
+  // the knots and clock values run two intervals ahead of their use (the recursion waits on no load)
+  zd x0[M], v[M];
+  Knot<M, CPLX> x1, x2;
   load_knot<M, CPLX>(a, l.b, l.t0, l.j, x0);
+  x1.load(a, l.b, l.t0 + 1, l.j);
   double th0 = (double)th[l.t0];
+  float th1 = th[l.t0 + 1];
   Coef<M> k;
   const bool fixed = a.flow_mode != EWS_FLOW_PER_INTERVAL && a.leaf_mode != EWS_FLOW_PER_INTERVAL;
   if (fixed) coefs<M>(c, eps, mode_step(th, a.L, 1, 0.0, a.leaf_mode), mode_step(th, a.L, 1, 0.0, a.flow_mode), a.q, k);
   for (int s = 0; s < l.Tc; ++s) {
-    const int t = l.t0 + s;
-    load_knot<M, CPLX>(a, l.b, t + 1, l.j, x1);
-    const double th1 = (double)th[t + 1], h = th1 - th0;
+    const int t = l.t0 + s, tn = l.t0 + min(s + 2, l.Tc);
+    x2.load(a, l.b, tn, l.j);
+    const float th2 = th[tn];
+    const double h = (double)th1 - th0;
+    zd xc[M];
+    x1.get(xc);
 #pragma unroll
-    for (int i = 0; i < M; ++i) v[i] = x1[i] - x0[i];
+    for (int i = 0; i < M; ++i) v[i] = xc[i] - x0[i];
     if (!fixed || (t <= 1 && (a.flow_mode == EWS_FLOW_CACHED_BASEPOINT || a.leaf_mode == EWS_FLOW_CACHED_BASEPOINT)))
       coefs<M>(c, eps, mode_step(th, a.L, t, h, a.leaf_mode), mode_step(th, a.L, t, h, a.flow_mode), a.q, k);
     step<M>(k, eps, v, S);
     if (ROWS) {
-      float* row = a.out + ((size_t)l.b * a.n + t) * a.W + a.lvl0 + (size_t)l.j * a.size;
-#pragma unroll
-      for (int i = 0; i < M; ++i) {
-        if (CPLX) {
-          row[2 * i] = (float)S[i].re;
-          row[2 * i + 1] = (float)S[i].im;
-        } else {
-          row[i] = (float)S[i].re;
-        }
-      }
+      st_row<M, CPLX>(a.out + ((size_t)l.b * a.n + t) * a.W + a.lvl0 + (size_t)l.j * a.size, S);
       if (a.lvl0 && l.j == 0) a.out[((size_t)l.b * a.n + t) * a.W] = 1.0f;
     }
 #pragma unroll
-    for (int i = 0; i < M; ++i) x0[i] = x1[i];
-    th0 = th1;
+    for (int i = 0; i < M; ++i) x0[i] = xc[i];
+    x1 = x2;
+    th0 = (double)th1;
+    th1 = th2;
   }
   if (!ROWS) st_state<M>(a.summ + ch_off(a, l.b, l.c, l.j), S);
 }
@@ -328,6 +392,7 @@ __global__ __launch_bounds__(64) void k_rows(CArgs a) {
 // (cotangents). The maps compose as (F2, z2) o (F1, z1) = (F2 F1, F2 z1 + z2) (adjoint: F2^H z1 + z2), the flows
 // being polynomials in Nil that commute.
 constexpr int kCarryThreads = 256;
+constexpr int kGroup = 16;  // runs per group of the chaining
 
 template <int M>
 __device__ __forceinline__ void nil_apply(const zd* F, const zd* S, zd* o) {  // (F S)_i = sum_p F[p] S_{i+p}
@@ -385,6 +450,7 @@ template <int M, bool CPLX, bool BWD>
 __device__ __forceinline__ void carry_scan(const CArgs& a) {
   __shared__ double s_map[kCarryThreads][4 * M];  // each thread's composed map: F, then z (complex)
   __shared__ double s_in[kCarryThreads][2 * M];   // each thread's start state
+  __shared__ double s_grp[kCarryThreads / kGroup][4 * M];
   const int b = blockIdx.x / a.K, j = blockIdx.x % a.K, tid = threadIdx.x;
   zd c;
   double eps;
@@ -409,6 +475,27 @@ __device__ __forceinline__ void carry_scan(const CArgs& a) {
   st_state<M>(&s_map[tid][0], AF);
   st_state<M>(&s_map[tid][2 * M], Az);
   __syncthreads();
+  // the threads' maps chained from the initial state in two levels (a single chain over up to 256 maps was a quarter
+  // of the scan's time): kGroup runs composed per group, the groups' maps chained, the runs of a group from its state
+  const int ng = (nrun + kGroup - 1) / kGroup;
+  if (tid < ng) {
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      AF[i] = Z(i == 0 ? 1.0 : 0.0);
+      Az[i] = Z(0.0);
+    }
+    for (int u = tid * kGroup; u < min(nrun, (tid + 1) * kGroup); ++u) {
+      ld_state<M>(&s_map[u][0], F);
+      ld_state<M>(&s_map[u][2 * M], z);
+      nil_mul<M>(F, AF, t);
+#pragma unroll
+      for (int i = 0; i < M; ++i) AF[i] = t[i];
+      map_apply<M, BWD>(F, z, Az);
+    }
+    st_state<M>(&s_grp[tid][0], AF);
+    st_state<M>(&s_grp[tid][2 * M], Az);
+  }
+  __syncthreads();
   if (tid == 0) {
     zd S[M];
     if (BWD && a.readout == EWS_READOUT_TERMINAL) {
@@ -419,7 +506,18 @@ __device__ __forceinline__ void carry_scan(const CArgs& a) {
 #pragma unroll
       for (int i = 0; i < M; ++i) S[i] = Z(0.0);
     }
-    for (int u = 0; u < nrun; ++u) {  // the threads past nrun own no chunk
+    for (int u = 0; u < ng; ++u) {
+      st_state<M>(&s_in[u * kGroup][0], S);  // the state before the group's first run
+      ld_state<M>(&s_grp[u][0], F);
+      ld_state<M>(&s_grp[u][2 * M], z);
+      map_apply<M, BWD>(F, z, S);
+    }
+  }
+  __syncthreads();
+  if (tid < ng) {
+    zd S[M];
+    ld_state<M>(&s_in[tid * kGroup][0], S);
+    for (int u = tid * kGroup; u < min(nrun, (tid + 1) * kGroup); ++u) {  // the threads past nrun own no chunk
       st_state<M>(&s_in[u][0], S);
       ld_state<M>(&s_map[u][0], F);
       ld_state<M>(&s_map[u][2 * M], z);
@@ -460,13 +558,6 @@ __global__ void k_terminal(CArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------ adjoint
-// the row cotangent of interval t on the chain's coordinates (G = dl/dRe + i dl/dIm for complex coordinates)
-template <int M, bool CPLX>
-__device__ __forceinline__ void load_g(const CArgs& a, int b, int t, int j, zd* g) {
-  const float* r = a.gout + ((size_t)b * a.n + t) * a.W + a.lvl0 + (size_t)j * a.size;
-#pragma unroll
-  for (int i = 0; i < M; ++i) g[i] = CPLX ? Z((double)r[2 * i], (double)r[2 * i + 1]) : Z((double)r[i]);
-}
 // Lam <- E^H Lam
 template <int M>
 __device__ __forceinline__ void adj_flow(const zd* e, zd* Lam) {
@@ -493,14 +584,28 @@ __global__ __launch_bounds__(64) void k_local(CArgs a) {
   zd Lam[M], g[M], e[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) Lam[i] = Z(0.0);
+  // row cotangents and clock values two intervals ahead of their use
+  Knot<M, CPLX> g0, g1, g2;
+  const float* gr = a.gout + (size_t)l.b * a.n * a.W + a.lvl0 + (size_t)l.j * a.size;
+  const int tl = l.t0 + l.Tc - 1;
+  g0.row(gr + (size_t)tl * a.W);
+  g1.row(gr + (size_t)max(tl - 1, l.t0) * a.W);
+  float thu = th[tl + 1], th0 = th[tl], th1 = th[max(tl - 1, l.t0)];
   for (int s = l.Tc - 1; s >= 0; --s) {
-    const int t = l.t0 + s;
-    load_g<M, CPLX>(a, l.b, t, l.j, g);
+    const int t = l.t0 + s, tp = max(t - 2, l.t0);
+    g2.row(gr + (size_t)tp * a.W);
+    const float th2 = th[tp];
+    g0.get(g);
 #pragma unroll
     for (int i = 0; i < M; ++i) Lam[i] += g[i];
-    const double hf = mode_step(th, a.L, t, (double)th[t + 1] - (double)th[t], a.flow_mode);
-    span_flow<M>(c, eps, hf, e);
+    const double hf = mode_step(th, a.L, t, (double)thu - (double)th0, a.flow_mode);
+    flow_of<M>(c, eps, hf, e);
     adj_flow<M>(e, Lam);
+    g0 = g1;
+    g1 = g2;
+    thu = th0;
+    th0 = th1;
+    th1 = th2;
   }
   st_state<M>(a.mu + ch_off(a, l.b, l.c, l.j), Lam);
 }
@@ -512,72 +617,125 @@ __global__ __launch_bounds__(kCarryThreads) void k_carry_bwd(CArgs a) {
   carry_scan<M, CPLX, true>(a);
 }
 
-// each chunk from the cotangent at its end: states from the carry into LDS, then the steps in reverse with dv, dh
-// and the chain-parameter partials
+// Each chunk from the cotangent at its end: the steps in reverse with the increment and step cotangents and the
+// chain-parameter partials. The states S_{t-1} come from inverting each step from the chunk's end state in float64
+// while the whole chunk contracts by less than e^kInvert (errors then stay below 1e-12, where states kept in float32
+// had 6e-8); a wavefront with a stronger contraction first recomputes its states from the carry into st. The sweep keeps the interval after in registers, so
+// a chunk's interior knot gradients dX_{t+1} = dv_t - dv_{t+1} (and the clock's) are written here; the cotangents of
+// its first and last interval go to dvb / dhb for the boundary knots (k_bounds). Bound by float64 issue: at B = 8,
+// L = 49,920, 16 complex chains of two coordinates, 543 us with the 28-term series at every step, the states
+// recomputed into LDS (one wavefront per SIMD) and dv, dh through memory; 171 us now (the step 1.12 -> 0.60 ms).
 template <int M, bool CPLX>
 __global__ __launch_bounds__(64) void k_full(CArgs a) {
-  extern __shared__ float2 s_st[];  // [64 lanes][T][M] states before each step
+  constexpr int NX = CPLX ? 2 * M : M;
   const Lane l = lane_of(a);
   if (!l.group) return;  // the lanes of one chunk stay together: the dh sums exchange across them
   const bool live = l.live;
-  float2* my = s_st + (size_t)threadIdx.x * a.T * M;
   zd c = Z(0.0);
   double eps = 0.0;
   if (live) chain_params(a, l.j, c, eps);
   const float* th = a.clock + (size_t)l.b * a.L;
-  // 1. the states S_{t-1} of the chunk's steps, from its carry
-  zd S[M], x0[M], x1[M], v[M];
-  Coef<M> k;
-  if (live) {
+  const int tl = l.t0 + l.Tc - 1;
+  // the chunk's total flow step, a lane per step
+  double tot = 0.0;
+  for (int s = l.j; s < l.Tc; s += a.KP) {
+    const int t = l.t0 + s;
+    tot += fabs(mode_step(th, a.L, t, (double)th[t + 1] - (double)th[t], a.flow_mode));
+  }
+  for (int o = 1; o < a.KP; o <<= 1) tot += __shfl_xor(tot, o, 64);
+  const bool invert = !__any(live && !((fabs(c.re) + fabs(eps)) * tot <= kInvert));
+  zd S[M], v[M], xc[M], xn[M];
+  Knot<M, CPLX> x1, x2;
+  // the states of the lane's steps, (B, n, K, M) pairs
+  float2* my = a.st + (((size_t)l.b * a.n + l.t0) * a.K + l.j) * M;
+  const size_t my_step = (size_t)a.K * M;
+  if (invert) {
+    if (live) ld_state<M>(a.carries + st_off(a, l.b, l.c + 1, l.j), S);
+  } else if (live) {
+    Coef<M> k;
+    zd x0[M];
     ld_state<M>(a.carries + st_off(a, l.b, l.c, l.j), S);
     load_knot<M, CPLX>(a, l.b, l.t0, l.j, x0);
+    x1.load(a, l.b, l.t0 + 1, l.j);
     double th0 = (double)th[l.t0];
+    float th1 = th[l.t0 + 1];
     for (int s = 0; s < l.Tc; ++s) {
-      const int t = l.t0 + s;
+      const int t = l.t0 + s, tn = l.t0 + min(s + 2, l.Tc);
 #pragma unroll
-      for (int i = 0; i < M; ++i) my[s * M + i] = float2{(float)S[i].re, (float)S[i].im};
-      load_knot<M, CPLX>(a, l.b, t + 1, l.j, x1);
-      const double th1 = (double)th[t + 1], h = th1 - th0;
+      for (int i = 0; i < M; ++i) my[s * my_step + i] = float2{(float)S[i].re, (float)S[i].im};
+      if (s == l.Tc - 1) break;
+      x2.load(a, l.b, tn, l.j);
+      const float th2 = th[tn];
+      x1.get(xc);
+      const double h = (double)th1 - th0;
 #pragma unroll
-      for (int i = 0; i < M; ++i) v[i] = x1[i] - x0[i];
+      for (int i = 0; i < M; ++i) v[i] = xc[i] - x0[i];
       coefs<M>(c, eps, mode_step(th, a.L, t, h, a.leaf_mode), mode_step(th, a.L, t, h, a.flow_mode), a.q, k);
       step<M>(k, eps, v, S);
 #pragma unroll
-      for (int i = 0; i < M; ++i) x0[i] = x1[i];
-      th0 = th1;
+      for (int i = 0; i < M; ++i) x0[i] = xc[i];
+      x1 = x2;
+      th0 = (double)th1;
+      th1 = th2;
     }
   }
-  // 2. the steps in reverse from the cotangent at the chunk's end
+  // 2. the steps in reverse from the cotangent at the chunk's end; knots, row cotangents and clock values two intervals
+  // ahead of their use
+  const bool rows = a.readout != EWS_READOUT_TERMINAL, own_step = a.leaf_mode == a.flow_mode && a.q == 0;
   zd Lam[M], g[M], Gc = Z(0.0);
   double deps = 0.0, dref0 = 0.0, dref1 = 0.0;
+  float dvn[NX], dhn = 0.0f;  // of the interval after
+  Knot<M, CPLX> g0{}, g1{}, g2{};
+  const float* gr = a.gout + (size_t)l.b * a.n * a.W + a.lvl0 + (size_t)l.j * a.size;
+  float thu = th[tl + 1], th0 = th[tl], th1 = th[max(tl - 1, l.t0)];
   if (live) {
     ld_state<M>(a.mt + ch_off(a, l.b, l.c, l.j), Lam);
-    load_knot<M, CPLX>(a, l.b, l.t0 + l.Tc, l.j, x1);
+    load_knot<M, CPLX>(a, l.b, tl + 1, l.j, xn);
+    x1.load(a, l.b, tl, l.j);
+    x2.load(a, l.b, max(tl - 1, l.t0), l.j);
+    if (rows) {
+      g0.row(gr + (size_t)tl * a.W);
+      g1.row(gr + (size_t)max(tl - 1, l.t0) * a.W);
+    }
   }
   for (int s = l.Tc - 1; s >= 0; --s) {
-    const int t = l.t0 + s;
+    const int t = l.t0 + s, tp = max(t - 2, l.t0);
     double dh_own = 0.0;
+    const float th2 = th[tp];
     if (live) {
-      if (a.readout != EWS_READOUT_TERMINAL) {
-        load_g<M, CPLX>(a, l.b, t, l.j, g);
+      Knot<M, CPLX> x3;
+      x3.load(a, l.b, tp, l.j);
+      if (rows) {
+        g2.row(gr + (size_t)tp * a.W);
+        g0.get(g);
 #pragma unroll
         for (int i = 0; i < M; ++i) Lam[i] += g[i];
+        g0 = g1;
+        g1 = g2;
       }
-      load_knot<M, CPLX>(a, l.b, t, l.j, x0);
+      x1.get(xc);
 #pragma unroll
-      for (int i = 0; i < M; ++i) v[i] = x1[i] - x0[i];
-      const double h = (double)th[t + 1] - (double)th[t];
+      for (int i = 0; i < M; ++i) {
+        v[i] = xn[i] - xc[i];
+        xn[i] = xc[i];
+      }
+      x1 = x2;
+      x2 = x3;
+      const double h = (double)thu - (double)th0;
       const double hl = mode_step(th, a.L, t, h, a.leaf_mode), hf = mode_step(th, a.L, t, h, a.flow_mode);
-      zd u[M + 1];
-      u_table<M>(Z(-hl) * c, a.q, u);
+      zd u[M + 1], ex;
+      u_table<M>(-hl * c, a.q, u, ex);
       zd ew[M];  // eps^p, as reals
       ew[0] = Z(1.0);
 #pragma unroll
       for (int p = 1; p < M; ++p) ew[p] = eps * ew[p - 1];
       // leaf: s_i = sum_p z_p eps^p v_{i+p}, z_p = (-hl)^p u_p(-hl c)
-      zd dv[M];
+      zd dv[M], Es[M];  // Es: E S_{t-1} = S_t - s_t
 #pragma unroll
-      for (int i = 0; i < M; ++i) dv[i] = Z(0.0);
+      for (int i = 0; i < M; ++i) {
+        dv[i] = Z(0.0);
+        Es[i] = S[i];
+      }
       double hp = 1.0, hq = 0.0, dhl = 0.0;  // (-hl)^p, (-hl)^(p-1)
 #pragma unroll
       for (int p = 0; p < M; ++p) {
@@ -587,6 +745,7 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
         for (int i = 0; i + p < M; ++i) {
           Gz += cjm(ew[p].re * v[i + p], Lam[i]);
           dv[i + p] += (ew[p].re) * cjm(zp, Lam[i]);
+          Es[i] = Es[i] - zp * (ew[p].re * v[i + p]);
           if (p > 0) deps += (double)p * ew[p - 1].re * redot(Lam[i], zp * v[i + p]);
         }
         // dz_p / dc = -hl (p+1) (-hl)^p u_{p+1}; dz_p / dhl = -p (-hl)^(p-1) u_p - c (p+1) (-hl)^p u_{p+1}
@@ -598,15 +757,30 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
         hp *= -hl;
       }
       // flow: (E S)_i = sum_p e_p S_{i+p}, e_p = e^{-hf c} (-hf eps)^p / p!
-      zd Sp[M];
+      zd Sp[M], e[M];
+      e[0] = own_step ? ex : zexp(-hf * c);
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        const float2 w = my[s * M + i];
-        Sp[i] = Z((double)w.x, (double)w.y);
-      }
-      zd e[M];
-      span_flow<M>(c, eps, hf, e);
+      for (int p = 1; p < M; ++p) e[p] = (-hf * eps / (double)p) * e[p - 1];
       const zd ef = e[0];
+      if (invert) {  // back substitution from the last coordinate
+        const double nrm = 1.0 / fma(ef.re, ef.re, ef.im * ef.im);
+        const zd ei = Z(nrm * ef.re, -nrm * ef.im);
+#pragma unroll
+        for (int i = M - 1; i >= 0; --i) {
+          zd r = Es[i];
+#pragma unroll
+          for (int p = 1; p + i < M; ++p) r = r - e[p] * Sp[i + p];
+          Sp[i] = ei * r;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+          const float2 w = my[s * my_step + i];
+          Sp[i] = Z((double)w.x, (double)w.y);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < M; ++i) S[i] = Sp[i];
       double dhf = 0.0;
       double xp = 1.0, fp = 1.0;  // (-hf eps)^(p-1), (p-1)!
 #pragma unroll
@@ -625,17 +799,25 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
         dhf += redot(Ge, deh);
       }
       adj_flow<M>(e, Lam);
-      // increment cotangent of the interval
-      float* dvr = a.dv + ((size_t)l.b * a.n + t) * a.d + (size_t)l.j * a.size;
+      // increment cotangent of the interval: the knot after it, or the chunk's boundary rows
+      float dvf[NX];
+      st_row<M, CPLX>(dvf, dv);
+      const size_t col = (size_t)l.j * a.size;
+      float* bnd = a.dvb + ((size_t)l.b * a.C + l.c) * 2 * a.d + col;
+      if (s < l.Tc - 1) {
+        float* o = a.gpath + ((size_t)l.b * a.L + t + 1) * a.d + col;
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        if (CPLX) {
-          dvr[2 * i] = (float)dv[i].re;
-          dvr[2 * i + 1] = (float)dv[i].im;
-        } else {
-          dvr[i] = (float)dv[i].re;
-        }
+        for (int i = 0; i < NX; ++i) o[i] = dvf[i] - dvn[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < NX; ++i) bnd[a.d + i] = dvf[i];
       }
+      if (s == 0) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i) bnd[i] = dvf[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NX; ++i) dvn[i] = dvf[i];
       // steps: the interval's own, or the shared reference steps (theta1 - theta0: cached; theta2 - theta1:
       // cached with basepoint, interval 0 none)
       if (a.leaf_mode == EWS_FLOW_PER_INTERVAL) dh_own += dhl;
@@ -644,13 +826,22 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
       if (a.flow_mode == EWS_FLOW_PER_INTERVAL) dh_own += dhf;
       else if (a.flow_mode == EWS_FLOW_CACHED) dref0 += dhf;
       else if (t > 0) dref1 += dhf;
-#pragma unroll
-      for (int i = 0; i < M; ++i) x1[i] = x0[i];
     }
+    thu = th0;
+    th0 = th1;
+    th1 = th2;
+    if (!a.gclock) continue;
     // dh of the interval: every chain of the sample, summed across the chunk's lane group
     double acc = dh_own;
     for (int o = 1; o < a.KP; o <<= 1) acc += __shfl_xor(acc, o, 64);
-    if (l.j == 0) a.dh[(size_t)l.b * a.n + t] = (float)acc;
+    if (l.j == 0) {
+      const float dhf = (float)acc;
+      float* bnd = a.dhb + ((size_t)l.b * a.C + l.c) * 2;
+      if (s < l.Tc - 1) a.gclock[(size_t)l.b * a.L + t + 1] = dhf - dhn;
+      else bnd[1] = dhf;
+      if (s == 0) bnd[0] = dhf;
+      dhn = dhf;
+    }
   }
   if (live) {
     double* pp = a.pp + (((size_t)l.b * a.C + l.c) * a.K + l.j) * 5;
@@ -662,52 +853,37 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
   }
 }
 
-// knot gradients: dX_t = dv_{t-1} - dv_t; dtheta_t = dh_{t-1} - dh_t, plus the reference steps' shares (summed over
-// the sample's chunks and chains in order)
-__device__ __forceinline__ void knot_clock(const CArgs& a, size_t b, size_t t) {
-  double g = (t > 0 ? (double)a.dh[b * a.n + t - 1] : 0.0) - (t < (size_t)a.n ? (double)a.dh[b * a.n + t] : 0.0);
-  if (t <= 2 && (a.flow_mode != EWS_FLOW_PER_INTERVAL || a.leaf_mode != EWS_FLOW_PER_INTERVAL)) {
+// The knots between chunks, and the first and last: dX = dv of the chunk before's last interval - dv of this chunk's
+// first; the clock's likewise, plus the reference steps' shares (summed over the sample's chunks and chains in order)
+// on knots 0 to 2. A thread per (sample, chunk or the last knot, column; column d the clock).
+__global__ void k_bounds(CArgs a) {
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t per = (size_t)(a.C + 1) * (a.d + 1);
+  if (e >= (size_t)a.B * per) return;
+  const size_t b = e / per, r = e % per, c = r / (a.d + 1), ch = r % (a.d + 1);
+  const size_t t = c < (size_t)a.C ? c * a.T : (size_t)a.n;
+  const size_t row = b * a.C + c;  // this chunk's boundary rows
+  if (ch < (size_t)a.d) {
+    const float lo = c > 0 ? a.dvb[((row - 1) * 2 + 1) * a.d + ch] : 0.0f;
+    const float hi = c < (size_t)a.C ? a.dvb[row * 2 * a.d + ch] : 0.0f;
+    a.gpath[(b * a.L + t) * a.d + ch] = lo - hi;
+    return;
+  }
+  if (!a.gclock) return;
+  double g = (c > 0 ? (double)a.dhb[(row - 1) * 2 + 1] : 0.0) - (c < (size_t)a.C ? (double)a.dhb[row * 2] : 0.0);
+  const bool shared = a.flow_mode != EWS_FLOW_PER_INTERVAL || a.leaf_mode != EWS_FLOW_PER_INTERVAL;
+  if (shared && t <= 2) {
     double r0 = 0.0, r1 = 0.0;
     for (size_t i = 0; i < (size_t)a.C * a.K; ++i) {
       r0 += a.pp[(b * a.C * a.K + i) * 5 + 3];
       r1 += a.pp[(b * a.C * a.K + i) * 5 + 4];
     }
-    if (t == 1) g += r0 - r1;
-    else if (t == 0) g -= r0;
-    else g += r1;
+    g += t == 0 ? -r0 : t == 1 ? r0 - r1 : r1;
+    if (t == 0)  // knots 1 and 2 where they lie inside chunk 0 (its adjoint wrote them)
+      for (int k = 1; k <= 2; ++k)
+        if (k < a.n && k % a.T != 0) a.gclock[b * a.L + k] += (float)(k == 1 ? r0 - r1 : r1);
   }
   a.gclock[b * a.L + t] = (float)g;
-}
-__global__ void k_knots(CArgs a) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t per = (size_t)a.L * (a.d + 1);
-  if (e >= (size_t)a.B * per) return;
-  const size_t b = e / per, r = e % per, t = r / (a.d + 1), ch = r % (a.d + 1);
-  if (ch < (size_t)a.d) {
-    const float lo = t > 0 ? a.dv[(b * a.n + t - 1) * a.d + ch] : 0.0f;
-    const float hi = t < (size_t)a.n ? a.dv[(b * a.n + t) * a.d + ch] : 0.0f;
-    a.gpath[(b * a.L + t) * a.d + ch] = lo - hi;
-  } else if (a.gclock) {
-    knot_clock(a, b, t);
-  }
-}
-// the same for d % 4 == 0 and 16-byte aligned rows: the path columns four at a time (a thread per sample, knot and
-// float4), then the clock column, a thread per (sample, knot), in threads B L d / 4 ..
-__global__ void k_knots4(CArgs a) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t d4 = (size_t)a.d / 4, np = (size_t)a.B * a.L * d4;
-  if (e < np) {
-    const size_t b = e / ((size_t)a.L * d4), r = e % ((size_t)a.L * d4), t = r / d4, q = r % d4;
-    const float4* dv4 = reinterpret_cast<const float4*>(a.dv);
-    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const float4 lo = t > 0 ? dv4[(b * a.n + t - 1) * d4 + q] : z;
-    const float4 hi = t < (size_t)a.n ? dv4[(b * a.n + t) * d4 + q] : z;
-    reinterpret_cast<float4*>(a.gpath)[(b * a.L + t) * d4 + q] =
-        make_float4(lo.x - hi.x, lo.y - hi.y, lo.z - hi.z, lo.w - hi.w);
-  } else if (a.gclock && e < np + (size_t)a.B * a.L) {
-    const size_t k = e - np;
-    knot_clock(a, k / a.L, k % a.L);
-  }
 }
 
 // grad_A: zero, then each chain's entries from the partials (one workgroup per chain and component, float64 sums in
@@ -716,16 +892,25 @@ __global__ void k_zero_a(CArgs a) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e < a.d * a.d) a.gA[e] = 0.0f;
 }
-__global__ __launch_bounds__(256) void k_params(CArgs a) {
-  __shared__ double red[256];
+constexpr int kParamThreads = 1024;
+__global__ __launch_bounds__(kParamThreads) void k_params(CArgs a) {
+  __shared__ double red[kParamThreads];
   const int j = blockIdx.x / 3, comp = blockIdx.x % 3, tid = threadIdx.x;
   if ((!a.cplx && comp == 1) || (comp == 2 && a.M == 1)) return;  // uniform across the workgroup
   const size_t tot = (size_t)a.B * a.C;
   double acc = 0.0;
-  for (size_t it = tid; it < tot; it += 256) acc += a.pp[(it * a.K + j) * 5 + comp];
+  for (size_t it = tid; it < tot; it += 4 * kParamThreads) {  // four loads in flight
+    double x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const size_t i = it + (size_t)u * kParamThreads;
+      x[u] = i < tot ? a.pp[(i * a.K + j) * 5 + comp] : 0.0;
+    }
+    acc += (x[0] + x[1]) + (x[2] + x[3]);
+  }
   red[tid] = acc;
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
+  for (int o = kParamThreads / 2; o > 0; o >>= 1) {
     if (tid < o) red[tid] += red[tid + o];
     __syncthreads();
   }
@@ -774,11 +959,16 @@ CArgs chain_args(const ews_chain_desc* s) {
   a.cplx = s->kind == EWS_JORDAN_COMPLEX;
   a.M = a.cplx ? s->size / 2 : s->size;
   a.K = s->dim / s->size;
-  a.T = s->chunk ? s->chunk : 32;
-  a.C = (a.n + a.T - 1) / a.T;
   a.KP = 1;
   while (a.KP < a.K) a.KP <<= 1;
   a.CPW = 64 / a.KP;
+  // 32 intervals a chunk, or down to 8 while that leaves under 512 wavefronts (a chunk is a sequential chain; kernels of
+  // a training step at K = 16, T = 32 / 16 / 8: 24 wavefronts at T = 32 158 / 100 / 77 us, 312: 163 / 127 / 135, 3120:
+  // 394 / 436 / 553)
+  a.T = s->chunk ? s->chunk : 32;
+  if (!s->chunk)
+    while (a.T > 8 && (long)a.B * ((a.n + a.T - 1) / a.T) < 512L * a.CPW) a.T /= 2;
+  a.C = (a.n + a.T - 1) / a.T;
   a.flow_mode = s->flow_mode;
   a.leaf_mode = s->leaf_mode;
   a.readout = s->readout;
@@ -792,9 +982,9 @@ size_t al256c(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t carries_bytes(const CArgs& a) { return al256c((size_t)a.B * (a.C + 1) * a.K * a.M * 16); }
 size_t chunk_state_bytes(const CArgs& a) { return al256c((size_t)a.B * a.C * a.K * a.M * 16); }
 
-// the workspace: summaries (forward); mu, mt, dv, dh and the partials (backward)
+// the workspace: summaries (forward); mu, mt, the boundary cotangents and the partials (backward)
 struct WsOff {
-  size_t summ, mu, mt, dv, dh, pp, total;
+  size_t summ, mu, mt, dvb, dhb, pp, st, total;
 };
 WsOff ws_off(const CArgs& a) {
   WsOff w{};
@@ -802,9 +992,10 @@ WsOff ws_off(const CArgs& a) {
   w.summ = o; o += chunk_state_bytes(a);
   w.mu = o; o += chunk_state_bytes(a);
   w.mt = o; o += chunk_state_bytes(a);
-  w.dv = o; o += al256c((size_t)a.B * a.n * a.d * 4);
-  w.dh = o; o += al256c((size_t)a.B * a.n * 4);
+  w.dvb = o; o += al256c((size_t)a.B * a.C * 2 * a.d * 4);
+  w.dhb = o; o += al256c((size_t)a.B * a.C * 2 * 4);
   w.pp = o; o += al256c((size_t)a.B * a.C * a.K * 5 * 8);
+  w.st = o; o += al256c((size_t)a.B * a.n * a.K * a.M * 8);
   w.total = o;
   return w;
 }
@@ -835,27 +1026,6 @@ int carry_threads(int C) { return std::min(chain::kCarryThreads, std::max(64, (C
     }                                                                                                         \
     if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;                                               \
   } while (0)
-
-// the adjoint's LDS (a chunk of states per lane) can exceed the 64 KB a launch gets without asking
-template <int M, bool CPLX>
-int allow_lds(size_t bytes) {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&chain::k_full<M, CPLX>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess
-             ? EWS_OK
-             : EWS_ERR_LAUNCH;
-}
-int allow_full_lds(const CArgs& a, size_t bytes) {
-  switch (a.M * 2 + (a.cplx ? 1 : 0)) {
-    case 2: return allow_lds<1, false>(bytes);
-    case 3: return allow_lds<1, true>(bytes);
-    case 4: return allow_lds<2, false>(bytes);
-    case 5: return allow_lds<2, true>(bytes);
-    case 6: return allow_lds<3, false>(bytes);
-    case 7: return allow_lds<3, true>(bytes);
-    case 8: return allow_lds<4, false>(bytes);
-    default: return allow_lds<4, true>(bytes);
-  }
-}
 
 }  // namespace
 }  // namespace ews
@@ -915,9 +1085,10 @@ int ews_chain_backward(const ews_chain_desc* desc, const void* path, const float
   a.summ = (double*)(ws + w.summ);
   a.mu = (double*)(ws + w.mu);
   a.mt = (double*)(ws + w.mt);
-  a.dv = (float*)(ws + w.dv);
-  a.dh = (float*)(ws + w.dh);
+  a.dvb = (float*)(ws + w.dvb);
+  a.dhb = (float*)(ws + w.dhb);
   a.pp = (double*)(ws + w.pp);
+  a.st = (float2*)(ws + w.st);
   a.gpath = grad_path;
   a.gclock = grad_clock;
   a.gA = grad_A;
@@ -925,20 +1096,13 @@ int ews_chain_backward(const ews_chain_desc* desc, const void* path, const float
   const dim3 grid((a.C + a.CPW - 1) / a.CPW, a.B), blk(64);
   if (a.readout == EWS_READOUT_PREFIX) EWS_CHAIN_LAUNCH(ews::chain::k_local, grid, blk, 0, st, a);
   EWS_CHAIN_LAUNCH(ews::chain::k_carry_bwd, dim3(a.B * a.K), dim3(ews::carry_threads(a.C)), 0, st, a);
-  const size_t lds = (size_t)64 * a.T * a.M * sizeof(float2);
-  if (lds > 65536 && ews::allow_full_lds(a, lds) != EWS_OK) return EWS_ERR_LAUNCH;
-  EWS_CHAIN_LAUNCH(ews::chain::k_full, grid, blk, lds, st, a);
-  if (a.d % 4 == 0 && ((uintptr_t)grad_path & 15) == 0) {  // dv rows sit at 256-byte aligned offsets
-    const size_t kt = (size_t)a.B * a.L * (a.d / 4 + 1);
-    hipLaunchKernelGGL(ews::chain::k_knots4, dim3((unsigned)((kt + 255) / 256)), dim3(256), 0, st, a);
-  } else {
-    const size_t kt = (size_t)a.B * a.L * (a.d + 1);
-    hipLaunchKernelGGL(ews::chain::k_knots, dim3((unsigned)((kt + 255) / 256)), dim3(256), 0, st, a);
-  }
+  EWS_CHAIN_LAUNCH(ews::chain::k_full, grid, blk, 0, st, a);
+  const size_t kt = (size_t)a.B * (a.C + 1) * (a.d + 1);
+  hipLaunchKernelGGL(ews::chain::k_bounds, dim3((unsigned)((kt + 255) / 256)), dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;
   hipLaunchKernelGGL(ews::chain::k_zero_a, dim3((a.d * a.d + 255) / 256), dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;
-  hipLaunchKernelGGL(ews::chain::k_params, dim3(a.K * 3), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(ews::chain::k_params, dim3(a.K * 3), dim3(ews::chain::kParamThreads), 0, st, a);
   return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
 }
 

@@ -332,12 +332,13 @@ typedef struct ews_chain_desc {
   int32_t readout;   /* EWS_READOUT_PREFIX (B, L-1, W) or EWS_READOUT_TERMINAL (B, W), W = level0 + d */
   int32_t level0;    /* 1: the leading level-0 column of the flat format */
   int32_t series_q;  /* 0: the exact level 1 phi(-hA) v; 1..48: the series leaf's order-q truncation */
-  int32_t chunk;     /* intervals per chunk, 0: 32; at most 64 */
+  int32_t chunk;     /* intervals per chunk, 0: 32, down to 8 for few intervals; at most 64 */
 } ews_chain_desc;
 
 /* Residual the forward leaves for the backward: the float64 chunk carries (B, C+1, chains, coordinates). */
 size_t ews_chain_residual_bytes(const ews_chain_desc* desc);
-/* Scratch of both directions: chunk summaries, adjoint carries, per-interval dv and dh, parameter partials. */
+/* Scratch of both directions: chunk summaries, adjoint carries, the chunks' boundary cotangents, parameter partials,
+ * and the states of chunks whose steps are not inverted. */
 size_t ews_chain_workspace_bytes(const ews_chain_desc* desc);
 
 /* Forward: path (B, L, d) f32, clock (B, L) f32, A (d, d) f32 row-major (reference sign; the chains' parameters
