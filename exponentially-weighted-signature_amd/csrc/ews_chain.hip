@@ -924,6 +924,164 @@ __global__ __launch_bounds__(kParamThreads) void k_params(CArgs a) {
   }
 }
 
+// ------------------------------------------------------------------------------------------------ token cache
+// The cached scan's per-token terms at depth 1 (ews/core/token_scan.py:44-88): P (V, d) the level 1 of a token's segment
+// (increment dx_g, step dtheta_g), D (V, d, d) its flow exp(-dtheta_g A), zero outside the chains' blocks. Both are the
+// coefficients of one interval, so one thread per (token, chain) forms them, and their adjoint, directly: on the scan
+// kernels the cache was V one-interval samples and V d basis injections through every pass of both directions, and some
+// forty torch operations around them (V = 8, d = 64: 0.17 ms of kernels, 0.4 ms of a training step's host time).
+struct KArgs {
+  int V, d, K, size, q;
+  const float *dx, *dth, *gP, *gD;
+  float *P, *D, *gdx, *gdth, *gA;
+  double* pp;  // (V, K, 4): partials of Re c, Im c, eps and the token's step
+};
+__device__ __forceinline__ CArgs chain_view(const KArgs& a, const float* A, int M, bool cplx) {
+  CArgs c{};
+  c.d = a.d;
+  c.size = a.size;
+  c.M = M;
+  c.cplx = cplx;
+  c.A = A;
+  return c;
+}
+template <int M, bool CPLX>
+__global__ __launch_bounds__(256) void k_cache(KArgs a, const float* A) {
+  const int g = blockIdx.x, tid = threadIdx.x;
+  float* D = a.D + (size_t)g * a.d * a.d;
+  for (int e = tid; e < a.d * a.d; e += 256)
+    if (e / a.d / a.size != e % a.d / a.size) D[e] = 0.0f;
+  if (tid >= a.K) return;
+  const int f = tid * a.size;
+  zd c;
+  double eps;
+  chain_params(chain_view(a, A, M, CPLX), tid, c, eps);
+  const double h = (double)a.dth[g];
+  Coef<M> k;
+  coefs<M>(c, eps, h, h, a.q, k);
+  zd v[M], S[M];
+  Knot<M, CPLX> x;
+  x.row(a.dx + (size_t)g * a.d + f);
+  x.get(v);
+#pragma unroll
+  for (int i = 0; i < M; ++i) S[i] = Z(0.0);
+  step<M>(k, eps, v, S);
+  st_row<M, CPLX>(a.P + (size_t)g * a.d + f, S);
+  // (E S)_i = sum_p e_p S_{i+p}: a complex coordinate is the 2 x 2 block [[re, -im], [im, re]]
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const zd e = m >= i ? k.e[m >= i ? m - i : 0] : Z(0.0);
+      if (CPLX) {
+        float* r = D + (size_t)(f + 2 * i) * a.d + f + 2 * m;
+        r[0] = (float)e.re;
+        r[1] = -(float)e.im;
+        r[a.d] = (float)e.im;
+        r[a.d + 1] = (float)e.re;
+      } else {
+        D[(size_t)(f + i) * a.d + f + m] = (float)e.re;
+      }
+    }
+}
+// a thread per (token, chain): dx's cotangent and the partials of the chain's parameters and the token's step
+template <int M, bool CPLX>
+__global__ __launch_bounds__(64) void k_cache_bwd(KArgs a, const float* A) {
+  const int e0 = blockIdx.x * 64 + threadIdx.x;
+  if (e0 >= a.V * a.K) return;
+  const int g = e0 / a.K, j = e0 % a.K, f = j * a.size;
+  zd c;
+  double eps;
+  chain_params(chain_view(a, A, M, CPLX), j, c, eps);
+  const double h = (double)a.dth[g];
+  zd v[M], Lam[M], u[M + 1], ex;
+  Knot<M, CPLX> x;
+  x.row(a.dx + (size_t)g * a.d + f);
+  x.get(v);
+  x.row(a.gP + (size_t)g * a.d + f);
+  x.get(Lam);
+  u_table<M>(-h * c, a.q, u, ex);
+  double ew[M];
+  ew[0] = 1.0;
+#pragma unroll
+  for (int p = 1; p < M; ++p) ew[p] = eps * ew[p - 1];
+  zd dv[M], Gc = Z(0.0);
+  double deps = 0.0, dh = 0.0, hp = 1.0, hq = 0.0;
+#pragma unroll
+  for (int i = 0; i < M; ++i) dv[i] = Z(0.0);
+#pragma unroll
+  for (int p = 0; p < M; ++p) {  // the leaf, as in the scan's adjoint
+    const zd zp = hp * u[p];
+    zd Gz = Z(0.0);
+#pragma unroll
+    for (int i = 0; i + p < M; ++i) {
+      Gz += cjm(ew[p] * v[i + p], Lam[i]);
+      dv[i + p] += ew[p] * cjm(zp, Lam[i]);
+      if (p > 0) deps += (double)p * ew[p - 1] * redot(Lam[i], zp * v[i + p]);
+    }
+    Gc += cjm((-h * (double)(p + 1) * hp) * u[p + 1], Gz);
+    dh += redot(Gz, (-(double)p * hq) * u[p] - ((double)(p + 1) * hp) * (c * u[p + 1]));
+    hq = hp;
+    hp *= -h;
+  }
+  st_row<M, CPLX>(a.gdx + (size_t)g * a.d + f, dv);
+  // the flow: its coefficients' cotangents are sums over the block's diagonals
+  const float* D = a.gD + (size_t)g * a.d * a.d;
+  zd e[M];
+  e[0] = a.q == 0 ? ex : zexp(-h * c);
+#pragma unroll
+  for (int p = 1; p < M; ++p) e[p] = (-h * eps / (double)p) * e[p - 1];
+  double xp = 1.0, fp = 1.0;
+#pragma unroll
+  for (int p = 0; p < M; ++p) {
+    zd Ge = Z(0.0);
+#pragma unroll
+    for (int i = 0; i + p < M; ++i) {
+      if (CPLX) {
+        const float* r = D + (size_t)(f + 2 * i) * a.d + f + 2 * (i + p);
+        Ge += Z((double)r[0] + (double)r[a.d + 1], (double)r[a.d] - (double)r[1]);
+      } else {
+        Ge += Z((double)D[(size_t)(f + i) * a.d + f + i + p]);
+      }
+    }
+    Gc += cjm(-h * e[p], Ge);
+    zd deh = Z(0.0) - c * e[p];
+    if (p > 0) {
+      deh += (-eps * xp / fp) * e[0];
+      deps += redot(Ge, (-h * xp / fp) * e[0]);
+      xp *= -h * eps;
+      fp *= (double)p;
+    }
+    dh += redot(Ge, deh);
+  }
+  double* pp = a.pp + (size_t)e0 * 4;
+  pp[0] = Gc.re;
+  pp[1] = Gc.im;
+  pp[2] = deps;
+  pp[3] = dh;
+}
+// the sums in order: a chain's parameters over the tokens, a token's step over the chains; grad_A's other entries zero
+__global__ __launch_bounds__(1024) void k_cache_sums(KArgs a, int M, int cplx) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x > 0) {  // the tokens' steps
+    const int g = (blockIdx.x - 1) * 1024 + tid;
+    if (g >= a.V) return;
+    double s = 0.0;
+    for (int j = 0; j < a.K; ++j) s += a.pp[((size_t)g * a.K + j) * 4 + 3];
+    a.gdth[g] = (float)s;
+    return;
+  }
+  for (int e = tid; e < a.d * a.d; e += 1024) a.gA[e] = 0.0f;
+  __syncthreads();
+  const int j = tid / 3, comp = tid % 3;
+  if (j >= a.K || (comp == 1 && !cplx) || (comp == 2 && M == 1)) return;
+  double s = 0.0;
+  for (int g = 0; g < a.V; ++g) s += a.pp[((size_t)g * a.K + j) * 4 + comp];
+  const int f = j * a.size;
+  const int r = comp == 1 ? f + 1 : f, col = comp < 2 ? f : (cplx ? f + 2 : f + 1);
+  a.gA[(size_t)r * a.d + col] = (float)s;
+}
+
 }  // namespace chain
 
 namespace {
@@ -1027,6 +1185,30 @@ int carry_threads(int C) { return std::min(chain::kCarryThreads, std::max(64, (C
     if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;                                               \
   } while (0)
 
+#define EWS_CHAIN_LAUNCH2(KERNEL, GRID, BLK, ST, A, ARG, PTR)                                                  \
+  do {                                                                                                        \
+    const bool cp = (A).cplx != 0;                                                                            \
+    switch ((A).M) {                                                                                          \
+      case 1:                                                                                                 \
+        if (cp) hipLaunchKernelGGL((KERNEL<1, true>), GRID, BLK, 0, ST, ARG, PTR);                             \
+        else hipLaunchKernelGGL((KERNEL<1, false>), GRID, BLK, 0, ST, ARG, PTR);                               \
+        break;                                                                                                \
+      case 2:                                                                                                 \
+        if (cp) hipLaunchKernelGGL((KERNEL<2, true>), GRID, BLK, 0, ST, ARG, PTR);                             \
+        else hipLaunchKernelGGL((KERNEL<2, false>), GRID, BLK, 0, ST, ARG, PTR);                               \
+        break;                                                                                                \
+      case 3:                                                                                                 \
+        if (cp) hipLaunchKernelGGL((KERNEL<3, true>), GRID, BLK, 0, ST, ARG, PTR);                             \
+        else hipLaunchKernelGGL((KERNEL<3, false>), GRID, BLK, 0, ST, ARG, PTR);                               \
+        break;                                                                                                \
+      default:                                                                                                \
+        if (cp) hipLaunchKernelGGL((KERNEL<4, true>), GRID, BLK, 0, ST, ARG, PTR);                             \
+        else hipLaunchKernelGGL((KERNEL<4, false>), GRID, BLK, 0, ST, ARG, PTR);                               \
+        break;                                                                                                \
+    }                                                                                                         \
+    if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;                                               \
+  } while (0)
+
 }  // namespace
 }  // namespace ews
 
@@ -1103,6 +1285,44 @@ int ews_chain_backward(const ews_chain_desc* desc, const void* path, const float
   hipLaunchKernelGGL(ews::chain::k_zero_a, dim3((a.d * a.d + 255) / 256), dim3(256), 0, st, a);
   if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;
   hipLaunchKernelGGL(ews::chain::k_params, dim3(a.K * 3), dim3(ews::chain::kParamThreads), 0, st, a);
+  return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
+}
+
+size_t ews_chain_cache_workspace_bytes(const ews_chain_desc* desc) {
+  if (ews::chain_check(desc) != EWS_OK) return 0;
+  return ews::al256c((size_t)desc->batch * (desc->dim / desc->size) * 4 * 8);
+}
+
+int ews_chain_cache(const ews_chain_desc* desc, const float* dx, const float* dtheta, const float* A, float* P_cache,
+                    float* D_cache, ews_stream_t stream) {
+  const int rc = ews::chain_check(desc);
+  if (rc != EWS_OK) return rc;
+  if (!dx || !dtheta || !A || !P_cache || !D_cache) return EWS_ERR_NULL;
+  const ews::chain::CArgs a = ews::chain_args(desc);
+  ews::chain::KArgs k{};
+  k.V = a.B; k.d = a.d; k.K = a.K; k.size = a.size; k.q = a.q;
+  k.dx = dx; k.dth = dtheta; k.P = P_cache; k.D = D_cache;
+  hipStream_t st = (hipStream_t)stream;
+  EWS_CHAIN_LAUNCH2(ews::chain::k_cache, dim3(a.B), dim3(256), st, a, k, A);
+  return EWS_OK;
+}
+
+int ews_chain_cache_backward(const ews_chain_desc* desc, const float* dx, const float* dtheta, const float* A,
+                             const float* grad_P, const float* grad_D, float* grad_dx, float* grad_dtheta,
+                             float* grad_A, void* workspace, ews_stream_t stream) {
+  const int rc = ews::chain_check(desc);
+  if (rc != EWS_OK) return rc;
+  if (!dx || !dtheta || !A || !grad_P || !grad_D || !grad_dx || !grad_dtheta || !grad_A || !workspace)
+    return EWS_ERR_NULL;
+  const ews::chain::CArgs a = ews::chain_args(desc);
+  ews::chain::KArgs k{};
+  k.V = a.B; k.d = a.d; k.K = a.K; k.size = a.size; k.q = a.q;
+  k.dx = dx; k.dth = dtheta; k.gP = grad_P; k.gD = grad_D;
+  k.gdx = grad_dx; k.gdth = grad_dtheta; k.gA = grad_A;
+  k.pp = (double*)workspace;
+  hipStream_t st = (hipStream_t)stream;
+  EWS_CHAIN_LAUNCH2(ews::chain::k_cache_bwd, dim3((unsigned)(((size_t)a.B * a.K + 63) / 64)), dim3(64), st, a, k, A);
+  hipLaunchKernelGGL(ews::chain::k_cache_sums, dim3(1 + (a.B + 1023) / 1024), dim3(1024), 0, st, k, a.M, a.cplx);
   return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
 }
 

@@ -81,6 +81,9 @@ EXPORTED = (
     "ews_chain_workspace_bytes",
     "ews_chain_forward",
     "ews_chain_backward",
+    "ews_chain_cache",
+    "ews_chain_cache_workspace_bytes",
+    "ews_chain_cache_backward",
     "ews_token1_workspace_bytes",
     "ews_token1_scan",
     "ews_token1_scan_backward",
@@ -365,6 +368,12 @@ def load():
     lib.ews_chain_forward.restype = i32
     lib.ews_chain_backward.argtypes = [chp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.ews_chain_backward.restype = i32
+    lib.ews_chain_cache.argtypes = [chp, vp, vp, vp, vp, vp, vp]
+    lib.ews_chain_cache.restype = i32
+    lib.ews_chain_cache_workspace_bytes.argtypes = [chp]
+    lib.ews_chain_cache_workspace_bytes.restype = sz
+    lib.ews_chain_cache_backward.argtypes = [chp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+    lib.ews_chain_cache_backward.restype = i32
     lib.ews_diag_mixer_forward.argtypes = [dp, ctypes.POINTER(MixerDesc), vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.ews_diag_mixer_forward.restype = i32
     lib.ews_diag_suited_chunk.argtypes = [dp]

@@ -86,11 +86,51 @@ def _chain_structure(A):
     return ("complex", 2)
 
 
+class _ChainCacheFn(torch.autograd.Function):
+    """P_cache (V, d), D_cache (V, d, d) of a chain-structured generator at depth 1 (ews_chain_cache)."""
+
+    @staticmethod
+    def forward(ctx, dx, dtheta, A, kind, size, q):
+        lib = nat.load()
+        for nm, t in (("vocab_dx", dx), ("vocab_dtheta", dtheta), ("A", A)):
+            if not t.is_cuda:
+                raise RuntimeError("ews_mi355x runs on a HIP device only: move the vocabulary and A to the GPU (no CPU "
+                                   f"path), {nm} is on {t.device}")
+        dx, dtheta, A = dx.contiguous(), dtheta.contiguous(), A.contiguous()
+        V, d = dx.shape
+        desc = nat.ChainDesc(V, 2, d, nat.JORDAN_KINDS[kind], int(size), nat.FLOW_PER_INTERVAL, nat.FLOW_PER_INTERVAL,
+                             nat.READOUTS["prefix"], 0, int(q), 0)
+        if tuple(dtheta.shape) != (V,) or tuple(A.shape) != (d, d):
+            raise ValueError(f"vocab_dtheta must be {(V,)} and A {(d, d)}, got {tuple(dtheta.shape)} and "
+                             f"{tuple(A.shape)}")
+        if int(lib.ews_chain_cache_workspace_bytes(ctypes.byref(desc))) == 0:
+            raise ValueError(f"unsupported chain configuration: d={d}, kind={kind!r}, size={size}, series_q={q}")
+        P = torch.empty((V, d), device=dx.device, dtype=torch.float32)
+        D = torch.empty((V, d, d), device=dx.device, dtype=torch.float32)
+        nat.check(lib.ews_chain_cache(ctypes.byref(desc), dx.data_ptr(), dtheta.data_ptr(), A.data_ptr(), P.data_ptr(),
+                                      D.data_ptr(), _stream_handle(dx.device)), "ews_chain_cache")
+        ctx.save_for_backward(dx, dtheta, A)
+        ctx.desc = desc
+        return P, D
+
+    @staticmethod
+    def backward(ctx, gP, gD):
+        lib = nat.load()
+        dx, dtheta, A = ctx.saved_tensors
+        gP, gD = gP.to(torch.float32).contiguous(), gD.to(torch.float32).contiguous()
+        gdx, gdth, gA = torch.empty_like(dx), torch.empty_like(dtheta), torch.empty_like(A)
+        ws = torch.empty(int(lib.ews_chain_cache_workspace_bytes(ctypes.byref(ctx.desc))), device=dx.device,
+                         dtype=torch.uint8)
+        nat.check(lib.ews_chain_cache_backward(ctypes.byref(ctx.desc), dx.data_ptr(), dtheta.data_ptr(), A.data_ptr(),
+                                               gP.data_ptr(), gD.data_ptr(), gdx.data_ptr(), gdth.data_ptr(),
+                                               gA.data_ptr(), ws.data_ptr(), _stream_handle(dx.device)),
+                  "ews_chain_cache_backward")
+        return gdx, gdth, gA, None, None, None
+
+
 def _wide_cache(vocab_dx, vocab_dtheta, A, N, expm_method, chen_method, leaf, series_q, chain):
-    """Depth-1 caches wider than the dense kernels for a chain-structured A, on the chain kernels: a token's level 1
-    is the one-interval row of the knots (0, dx_g) at clock (0, dtheta_g); column i of its flow is the state after a
-    zero-step injection of e_i and one step of dtheta_g (knots 0, e_i, e_i at clock 0, 0, dtheta_g). Both are
-    differentiable through the chain kernels' adjoint."""
+    """Depth-1 caches wider than the dense kernels for a chain-structured A: a token's level 1 and its flow are the
+    chains' coefficients of one interval of step dtheta_g (ews_chain_cache)."""
     if N != 1:
         raise NotImplementedError("token caches wider than 16 coordinates are built at depth 1 (the banked "
                                   "formal-language blocks); deeper ones need the dense kernels (d <= 16)")
@@ -105,19 +145,8 @@ def _wide_cache(vocab_dx, vocab_dtheta, A, N, expm_method, chen_method, leaf, se
                                   "uniform Jordan chains (pass chain=(kind, size))")
     kind, size = chain
     q = int(series_q) if leaf == "series" else 0
-    V, d = vocab_dx.shape
-    A = A.to(torch.float32).contiguous()
-    zero = torch.zeros_like(vocab_dtheta)
-    path = torch.stack([torch.zeros_like(vocab_dx), vocab_dx], 1).to(torch.float32)
-    clock = torch.stack([zero, vocab_dtheta], 1).to(torch.float32)
-    P = ops.chain_scan(path, clock, A, kind, size, readout="prefix", level0=False, series_q=q)[:, 0]
-    eye = torch.eye(d, device=vocab_dx.device, dtype=torch.float32)
-    basis = eye[None].expand(V, d, d).reshape(V * d, 1, d)
-    kp = torch.cat([torch.zeros_like(basis), basis, basis], 1)
-    th = vocab_dtheta.to(torch.float32).repeat_interleave(d)
-    kc = torch.stack([torch.zeros_like(th), torch.zeros_like(th), th], 1)
-    cols = ops.chain_scan(kp, kc, A, kind, size, readout="prefix", level0=False, series_q=q)[:, 1]  # (V d, d)
-    D = cols.reshape(V, d, d).transpose(1, 2).contiguous()  # column i of token g's flow
+    P, D = _ChainCacheFn.apply(vocab_dx.to(torch.float32), vocab_dtheta.to(torch.float32), A.to(torch.float32), kind,
+                               int(size), q)
     D._ews_block = int(size)  # block-diagonal with blocks of `size` coordinates: the cached scan's sparse route
     return P, D
 

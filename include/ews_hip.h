@@ -356,6 +356,20 @@ int ews_chain_backward(const ews_chain_desc* desc, const void* path, const float
                        const void* residual, const float* grad_out, float* grad_path, float* grad_clock,
                        float* grad_A, void* workspace, ews_stream_t stream);
 
+/* The cached scan's per-token terms at depth 1 for a generator of uniform chains (ews/core/token_scan.py:44-88 with N
+ * = 1 and exact exponentials): P_cache (V, d), the level 1 of each token's segment (increment dx (V, d), step dtheta
+ * (V)), and D_cache (V, d, d), its flow exp(-dtheta_g A), zero outside the chains' blocks. desc: batch = V, dim, kind,
+ * size and series_q as in ews_chain_forward (length is not read, 2 serves). */
+int ews_chain_cache(const ews_chain_desc* desc, const float* dx, const float* dtheta, const float* A, float* P_cache,
+                    float* D_cache, ews_stream_t stream);
+
+/* Gradients of ews_chain_cache: grad_dx (V, d), grad_dtheta (V) and grad_A (d, d), which is nonzero only at the entries
+ * each chain is read from. workspace: ews_chain_cache_workspace_bytes. */
+size_t ews_chain_cache_workspace_bytes(const ews_chain_desc* desc);
+int ews_chain_cache_backward(const ews_chain_desc* desc, const float* dx, const float* dtheta, const float* A,
+                             const float* grad_P, const float* grad_D, float* grad_dx, float* grad_dtheta,
+                             float* grad_A, void* workspace, ews_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------------------
  * Token-cached scan at depth 1 for any width up to 64 (ews/core/token_scan.py:91-118 with trunc 1): from dense
  * per-token caches, P_cache (V, d) the level 1 of each token's segment and D_cache (V, d, d) its flow,
