@@ -10,6 +10,8 @@
 // (the states), in per-chunk partials reduced in a fixed order (deterministic).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ews_hip.h"
 #include "ews_lanes.h"
 
@@ -171,6 +173,15 @@ __global__ void k_reduce(TArgs a) {
 // cotangent lam_{t-1} = D_g^T lam_t (+ the row cotangent), and accumulates the token gradients per lane in LDS
 // (lane i owns dP_g[i] and row i of dD_g's block): per-sample partials, then a fixed-order sum over the samples.
 // Entries of D outside the blocks are taken as zero and their gradients are written as zero.
+//
+// A sample's steps are one dependent chain, and one wavefront per sample leaves most of the chip idle, so the NW
+// wavefronts of a sample's workgroup take one span of steps each: first the span's affine map of the state (its effect
+// from zero, and on the BS unit states of a block, all BS + 1 chains side by side in registers, in float64: the spans'
+// start states are then more exact than the float32 chain's), then, the maps of the spans before it applied in order,
+// the span again from its own start state with the rows written. The adjoint does the
+// same from the last span, with the transposed flows, before the sweep that accumulates the gradients. (BS + 2) / NW of
+// the steps are on the chain for 1. B = 256 x 512 tokens, d = 64, BS = 2: forward 50 -> 28 us, backward 110 -> 39 us at
+// NW = 8. Blocks of 6 and 8, whose lane exchanges go through LDS, keep NW = 1.
 constexpr int kStageFloats = 12288;  // caches staged in LDS up to 48 KB
 
 template <bool STAGED>
@@ -182,8 +193,8 @@ __device__ __forceinline__ float blk_d(const TArgs& a, const float* sD, int BS, 
 // v of lane base + r, the r-th lane of this lane's block (base = BS floor(lane / BS)); every lane of the wavefront
 // takes part. Blocks of 2 and 4 lie inside a quad of lanes: one DPP quad permutation (a VALU operand, no memory
 // round trip); blocks of 3, 6 and 8 go through an LDS permute.
-template <int BS>
-__device__ __forceinline__ float blk_lane(float v, int base, int r) {
+template <int BS, class T>
+__device__ __forceinline__ T blk_lane(T v, int base, int r) {
   if constexpr (BS == 1) {
     return v;
   } else if constexpr (BS == 2) {
@@ -202,68 +213,94 @@ __device__ __forceinline__ float blk_lane(float v, int base, int r) {
 
 // the block caches into LDS (row i of token g's block at (g d + i) BS, then P), eight loads in flight per lane
 template <int BS>
-__device__ __forceinline__ void stage_blk(const TArgs& a, float* sP, float* sD, bool with_p, int i) {
-  const int nd = a.V * a.d * BS;
-  for (int q0 = i; q0 < nd; q0 += 8 * 64) {
+__device__ __forceinline__ void stage_blk(const TArgs& a, float* sP, float* sD, bool with_p) {
+  const int nd = a.V * a.d * BS, i = threadIdx.x, nt = blockDim.x;
+  for (int q0 = i; q0 < nd; q0 += 8 * nt) {
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int q = min(q0 + 64 * u, nd - 1);  // clamped: every load unconditional
+      const int q = min(q0 + nt * u, nd - 1);  // clamped: every load unconditional
       const int gr = q / BS, r = q - gr * BS, g = gr / a.d, row = gr - g * a.d;
       v[u] = a.D[((size_t)g * a.d + row) * a.d + (row / BS) * BS + r];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      if (q0 + 64 * u < nd) sD[q0 + 64 * u] = v[u];
+      if (q0 + nt * u < nd) sD[q0 + nt * u] = v[u];
     }
   }
   if (with_p) {
     const int np = a.V * a.d;
-    for (int q0 = i; q0 < np; q0 += 8 * 64) {
+    for (int q0 = i; q0 < np; q0 += 8 * nt) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = a.P[min(q0 + 64 * u, np - 1)];
+      for (int u = 0; u < 8; ++u) v[u] = a.P[min(q0 + nt * u, np - 1)];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        if (q0 + 64 * u < np) sP[q0 + 64 * u] = v[u];
+        if (q0 + nt * u < np) sP[q0 + nt * u] = v[u];
       }
     }
   }
 }
 
-// The step loops take the caches from LDS (STAGED) or from global memory, a compile-time choice: one load kind each
-template <int BS, bool STAGED>
-__device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, const float* sD, int b, int i) {
+// The spans: wavefront w of NW takes steps [w span, (w + 1) span), whole groups of eight.
+__device__ __forceinline__ int span_len(const TArgs& a, int nw) { return ((a.n + nw - 1) / nw + 7) / 8 * 8; }
+// x + sum_c U[c] y_{base + c}: a span's map applied to the state (cotangent) y of the lane's block. A zero of y adds
+// nothing (the map of a span of growing flows may have overflowed).
+template <int BS>
+__device__ __forceinline__ double span_apply(double x, const double* U, int stride, double y, int base) {
+#pragma unroll
+  for (int c = 0; c < BS; ++c) {
+    const double yc = blk_lane<BS>(y, base, c);
+    x = yc != 0.0 ? fma(U[c * stride], yc, x) : x;
+  }
+  return x;
+}
+template <bool MAP> using span_t = std::conditional_t<MAP, double, float>;
+
+// The step loops take the caches from LDS (STAGED) or from global memory, a compile-time choice: one load kind each.
+// MAP: the span's map instead of its rows: S from zero and U[c], the states from the units of the lane's block.
+template <int BS, bool STAGED, bool MAP>
+__device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, const float* sD, int b, int i, int tb,
+                                              int te, span_t<MAP>& S, span_t<MAP>* U) {
+  using T = span_t<MAP>;
   const bool on = i < a.d;
   const int base = (i / BS) * BS;
   const int row = on ? i : 0;  // lanes past d read row 0 and keep S = 0
-  float S = 0.0f;
-  for (int t0 = 0; t0 < a.n; t0 += 64) {
+  for (int t0 = tb; t0 < te; t0 += 64) {
     int tokv = 0, livev = 0;
-    if (t0 + i < a.n) {
+    if (t0 + i < te) {
       bool live;
       tokv = tok_at(a, (size_t)b * a.n + t0 + i, live);
       livev = live ? 1 : 0;
     }
-    const int cnt = min(64, a.n - t0);
+    const int cnt = min(64, te - t0);
     // groups of eight steps without a branch (the lane reads are convergent, so only a constant trip count is
     // unrolled; the states are stored after the group), so that the group's cache reads are issued ahead of the
-    // state chain; steps past n carry token 0 and no mask bit
-    for (int s0 = 0; s0 < 64; s0 += 8) {
+    // state chain; steps past the span carry token 0 and no mask bit
+    for (int s0 = 0; s0 < cnt; s0 += 8) {
       float Sv[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int g = __builtin_amdgcn_readlane(tokv, s0 + u), live = __builtin_amdgcn_readlane(livev, s0 + u);
-        float acc = STAGED ? sP[g * a.d + row] : a.P[(size_t)g * a.d + row];
-        float dr[BS];
+        T acc = STAGED ? sP[g * a.d + row] : a.P[(size_t)g * a.d + row];
+        T dr[BS];
 #pragma unroll
         for (int r = 0; r < BS; ++r) dr[r] = blk_d<STAGED>(a, sD, BS, g, row, r);
 #pragma unroll
-        for (int r = 0; r < BS; ++r) acc = fmaf(dr[r], blk_lane<BS>(S, base, r), acc);
+        for (int r = 0; r < BS; ++r) acc = fma(dr[r], blk_lane<BS>(S, base, r), acc);
+        if constexpr (MAP) {
+#pragma unroll
+          for (int c = 0; c < BS; ++c) {
+            T ua = 0;
+#pragma unroll
+            for (int r = 0; r < BS; ++r) ua = fma(dr[r], blk_lane<BS>(U[c], base, r), ua);
+            if (live) U[c] = ua;
+          }
+        }
         if (live && on) S = acc;
-        Sv[u] = S;
+        Sv[u] = (float)S;
       }
-      if (on) {
+      if (!MAP && on) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
           if (s0 + u < cnt) a.out[((size_t)b * a.n + t0 + s0 + u) * a.d + i] = Sv[u];
@@ -273,142 +310,215 @@ __device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, c
   }
 }
 
-template <int BS>
-__global__ __launch_bounds__(64) void k_fwd_blk(TArgs a) {
-  extern __shared__ float s_c[];
-  const int b = blockIdx.x, i = threadIdx.x;
-  float* sP = s_c;
-  float* sD = s_c + (size_t)a.V * a.d;
-  if ((size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats) {
-    stage_blk<BS>(a, sP, sD, true, i);
+template <int BS, bool STAGED>
+__device__ __forceinline__ void fwd_blk_body(const TArgs& a, const float* sP, const float* sD, double* sX) {
+  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
+  double S = 0.0, U[BS];
+  if (nw > 1) {
+    if (w + 1 < nw) {
+#pragma unroll
+      for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
+      fwd_blk_steps<BS, STAGED, true>(a, sP, sD, b, i, tb, te, S, U);
+      double* x = sX + (size_t)w * (BS + 1) * 64 + i;
+#pragma unroll
+      for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
+      x[BS * 64] = S;
+    }
     __syncthreads();
-    fwd_blk_steps<BS, true>(a, sP, sD, b, i);
+    S = 0.0;
+    for (int u = 0; u < w; ++u) {
+      const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
+      S = span_apply<BS>(x[BS * 64], x, 64, S, base);
+    }
+  }
+  float S0 = (float)S;
+  fwd_blk_steps<BS, STAGED, false>(a, sP, sD, b, i, tb, te, S0, nullptr);
+}
+
+template <int BS>
+__global__ __launch_bounds__(512) void k_fwd_blk(TArgs a) {
+  extern __shared__ double s_c[];
+  double* sX = s_c;  // (NW, BS + 1, 64): the spans' maps
+  float* sP = reinterpret_cast<float*>(sX + (size_t)(blockDim.x >> 6) * (BS + 1) * 64);
+  float* sD = sP + (size_t)a.V * a.d;
+  if ((size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats) {
+    stage_blk<BS>(a, sP, sD, true);
+    __syncthreads();
+    fwd_blk_body<BS, true>(a, sP, sD, sX);
   } else {
-    fwd_blk_steps<BS, false>(a, sP, sD, b, i);
+    fwd_blk_body<BS, false>(a, sP, sD, sX);
   }
 }
 
-template <int BS, bool STAGED>
-__device__ __forceinline__ void bwd_blk_steps(const TArgs& a, const float* sD, float* sAcc, float* sG, float* sR,
-                                              int b, int i) {
+// kStage steps' row cotangents (and, ROWS, the states before them) from step u1 - 1 down: lane i's column, loads
+// unconditional from clamped addresses and zeroed afterwards
+template <bool ROWS>
+__device__ __forceinline__ void load_stage(const TArgs& a, int b, int ic, int tb, int u1, float* gv, float* rv) {
+#pragma unroll
+  for (int k = 0; k < kStage; ++k) {
+    const int t = max(u1 - 1 - k, tb);
+    gv[k] = a.gout[((size_t)b * a.n + t) * a.d + ic];
+    if (ROWS) rv[k] = a.rows[((size_t)b * a.n + max(t - 1, 0)) * a.d + ic];  // S_{t-1}
+  }
+}
+
+// MAP: the span's adjoint map: lam from zero at its end and U[c] from the unit cotangents; else the sweep from lam at
+// the span's end, the token gradients added to sAcc.
+template <int BS, bool STAGED, bool MAP>
+__device__ __forceinline__ void bwd_blk_steps(const TArgs& a, const float* sD, float* sAcc, int b, int i, int tb, int te,
+                                              span_t<MAP>& lam, span_t<MAP>* U) {
+  using T = span_t<MAP>;
   const bool on = i < a.d;
   const int base = (i / BS) * BS;
   // lanes past d read block row 0 (their products are dropped); their lam, state and accumulators stay zero
   const int rowb = on ? base : 0, col = on ? i - base : 0, ic = on ? i : 0;
-  float lam = 0.0f;
-  for (int t1 = a.n; t1 > 0; t1 -= 64) {
-    const int t0 = max(0, t1 - 64);
-    int tokv = 0, livev = 0;
-    if (t0 + i < t1) {
+  if (tb >= te) return;
+  float gv[kStage], rv[kStage], gn[kStage], rn[kStage];
+  load_stage<!MAP>(a, b, ic, tb, te, gn, rn);
+  for (int t1 = te; t1 > tb; t1 -= 64) {
+    const int t0 = max(tb, t1 - 64);
+    int tokv = 0, livev = 0;  // lane l: step t1 - 1 - l
+    if (t1 - 1 - i >= t0) {
       bool live;
-      tokv = tok_at(a, (size_t)b * a.n + t0 + i, live);
+      tokv = tok_at(a, (size_t)b * a.n + t1 - 1 - i, live);
       livev = live ? 1 : 0;
     }
-    for (int u1 = t1; u1 > t0; u1 -= kStage) {
-      const int u0 = max(t0, u1 - kStage);
-      {  // the stage's inputs: unconditional loads from clamped (valid) addresses, all issued before the first
-         // store, zeroed afterwards
-        float gv[kStage], rv[kStage];
+    for (int q0 = 0; q0 < t1 - t0; q0 += kStage) {
+      const int u1 = t1 - q0;
 #pragma unroll
-        for (int k = 0; k < kStage; ++k) {
-          const int t = min(u0 + k, u1 - 1), tp = max(t - 1, 0);
-          gv[k] = a.gout[((size_t)b * a.n + t) * a.d + ic];
-          rv[k] = a.rows[((size_t)b * a.n + tp) * a.d + ic];  // S_{t-1}
-        }
-#pragma unroll
-        for (int k = 0; k < kStage; ++k) {
-          const int t = u0 + k;
-          sG[k * 64 + i] = (on && t < u1) ? gv[k] : 0.0f;
-          sR[k * 64 + i] = (on && t < u1 && t > 0) ? rv[k] : 0.0f;
-        }
+      for (int k = 0; k < kStage; ++k) {
+        gv[k] = gn[k];
+        if (!MAP) rv[k] = rn[k];
       }
-      // steps u1 - 1 down to u0, unrolled and without a branch (see the forward): a step past u1 or without its
-      // mask bit adds zero to the accumulators (exact: they start at +0 and never become -0) and keeps lam
+      load_stage<!MAP>(a, b, ic, tb, max(u1 - kStage, tb + 1), gn, rn);  // the next stage's, in flight meanwhile
+      // unrolled and without a branch (see the forward): a step before the span or without its mask bit adds zero to
+      // the accumulators (exact: they start at +0 and never become -0) and keeps lam
 #pragma unroll
-      for (int k = kStage - 1; k >= 0; --k) {
-        const int t = u0 + k;  // t - t0 < 64
-        // uniform over the wavefront: the step's token and mask bit from lane t - t0
-        const int g = __builtin_amdgcn_readlane(tokv, t - t0);
-        const bool live = __builtin_amdgcn_readlane(livev, t - t0) && t < u1;
-        lam += sG[k * 64 + i];
-        const float sp = sR[k * 64 + i];
-        const float lw = live ? lam : 0.0f;
-        float* acc = sAcc + (size_t)g * (BS + 1) * 64 + i;
-        float ln = 0.0f;
+      for (int k = 0; k < kStage; ++k) {
+        const int t = u1 - 1 - k;
+        const bool in = t >= t0;
+        // uniform over the wavefront: the step's token and mask bit from lane t1 - 1 - t
+        const int g = __builtin_amdgcn_readlane(tokv, q0 + k);
+        const bool live = __builtin_amdgcn_readlane(livev, q0 + k) && in;
+        lam += on && in ? gv[k] : 0.0f;
+        T dc[BS], ln = 0;
 #pragma unroll
-        for (int r = 0; r < BS; ++r) {
-          const float s_r = blk_lane<BS>(sp, base, r), l_r = blk_lane<BS>(lam, base, r);
-          acc[r * 64] += lw * s_r;                                              // dD_g[i][base + r]
-          ln = fmaf(blk_d<STAGED>(a, sD, BS, g, rowb + r, col), l_r, ln);       // (D_g^T lam)_i
+        for (int r = 0; r < BS; ++r) dc[r] = blk_d<STAGED>(a, sD, BS, g, rowb + r, col);
+        if constexpr (MAP) {
+#pragma unroll
+          for (int c = 0; c < BS; ++c) {
+            T ua = 0;
+#pragma unroll
+            for (int r = 0; r < BS; ++r) ua = fma(dc[r], blk_lane<BS>(U[c], base, r), ua);
+            if (live) U[c] = ua;
+          }
+#pragma unroll
+          for (int r = 0; r < BS; ++r) ln = fma(dc[r], blk_lane<BS>(lam, base, r), ln);
+        } else {
+          const float sp = on && in && t > 0 ? rv[k] : 0.0f;
+          const float lw = live ? lam : 0.0f;
+          float* acc = sAcc + (size_t)g * (BS + 1) * 64 + i;
+#pragma unroll
+          for (int r = 0; r < BS; ++r) {
+            const float s_r = blk_lane<BS>(sp, base, r), l_r = blk_lane<BS>(lam, base, r);
+            acc[r * 64] += lw * s_r;        // dD_g[i][base + r]
+            ln = fmaf(dc[r], l_r, ln);      // (D_g^T lam)_i
+          }
+          acc[BS * 64] += lw;  // dP_g[i]
         }
-        acc[BS * 64] += lw;  // dP_g[i]
-        lam = live ? (on ? ln : 0.0f) : lam;
+        lam = live ? (on ? ln : (T)0) : lam;
       }
     }
   }
+}
+
+template <int BS, bool STAGED>
+__device__ __forceinline__ void bwd_blk_body(const TArgs& a, const float* sD, float* sAcc, double* sX) {
+  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
+  double lam = 0.0, U[BS];
+  if (nw > 1) {
+    if (w > 0) {
+#pragma unroll
+      for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
+      bwd_blk_steps<BS, STAGED, true>(a, sD, nullptr, b, i, tb, te, lam, U);
+      double* x = sX + (size_t)w * (BS + 1) * 64 + i;
+#pragma unroll
+      for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
+      x[BS * 64] = lam;
+    }
+    __syncthreads();
+    lam = 0.0;
+    for (int u = nw - 1; u > w; --u) {
+      const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
+      lam = span_apply<BS>(x[BS * 64], x, 64, lam, base);
+    }
+  }
+  float lam0 = (float)lam;
+  bwd_blk_steps<BS, STAGED, false>(a, sD, sAcc + (size_t)w * a.V * (BS + 1) * 64, b, i, tb, te, lam0, nullptr);
 }
 
 template <int BS>
-__global__ __launch_bounds__(64) void k_bwd_blk(TArgs a) {
-  extern __shared__ float s_c[];
-  const int b = blockIdx.x, i = threadIdx.x;
-  const bool on = i < a.d;
+__global__ __launch_bounds__(512) void k_bwd_blk(TArgs a) {
+  extern __shared__ double s_c[];
+  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const bool staged = (size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats;
-  float* sD = s_c + (size_t)a.V * a.d;  // the same layout as the forward's (P's slot unused)
-  float* sAcc = staged ? sD + (size_t)a.V * a.d * BS : s_c;  // (V, BS + 1, 64): lane i's column
-  // kStage steps' row cotangents and previous states, lane i's column of each (only lane i reads it: no barrier)
-  float* sG = sAcc + (size_t)a.V * (BS + 1) * 64;
-  float* sR = sG + kStage * 64;
-  if (staged) stage_blk<BS>(a, nullptr, sD, false, i);
-  for (int q = 0; q < a.V * (BS + 1); ++q) sAcc[q * 64 + i] = 0.0f;
+  const int na = a.V * (BS + 1);
+  double* sX = s_c;  // (NW, BS + 1, 64): the spans' maps
+  float* sAcc = reinterpret_cast<float*>(sX + (size_t)nw * (BS + 1) * 64);  // (NW, V, BS + 1, 64): lane i's column
+  float* sD = sAcc + (size_t)nw * na * 64;
+  if (staged) stage_blk<BS>(a, nullptr, sD, false);
+  for (int q = 0; q < na; ++q) sAcc[((size_t)w * na + q) * 64 + i] = 0.0f;
   __syncthreads();
-  if (staged) bwd_blk_steps<BS, true>(a, sD, sAcc, sG, sR, b, i);
-  else bwd_blk_steps<BS, false>(a, sD, sAcc, sG, sR, b, i);
-  if (on) {
-    for (int q = 0; q < a.V * (BS + 1); ++q)
-      a.part[(((size_t)b * a.V * (BS + 1)) + q) * a.d + i] = sAcc[q * 64 + i];
+  if (staged) bwd_blk_body<BS, true>(a, sD, sAcc, sX);
+  else bwd_blk_body<BS, false>(a, sD, sAcc, sX);
+  __syncthreads();
+  if (i < a.d) {  // the sample's partial: its spans in order
+    for (int q = w; q < na; q += nw) {
+      double s = 0.0;
+      for (int u = 0; u < nw; ++u) s += (double)sAcc[((size_t)u * na + q) * 64 + i];
+      a.part[((size_t)b * na + q) * a.d + i] = (float)s;
+    }
   }
 }
 
-// gP and gD from the per-sample partials (samples in order, float64); gD's entries outside the blocks are zero
-__global__ void k_reduce_blk(TArgs a, int BS) {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t dd = (size_t)a.d * a.d, tot = (size_t)a.V * (dd + a.d);
-  if (e >= tot) return;
-  int g, i, r;
-  bool isP;
-  if (e < (size_t)a.V * dd) {
-    g = (int)(e / dd);
-    const int rc = (int)(e - (size_t)g * dd);
-    i = rc / a.d;
-    const int col = rc - i * a.d;
-    r = col - (i / BS) * BS;
-    isP = false;
-    if (r < 0 || r >= BS) {
-      a.gD[e] = 0.0f;
-      return;
-    }
-  } else {
-    const size_t q = e - (size_t)a.V * dd;
-    g = (int)(q / a.d);
-    i = (int)(q - (size_t)g * a.d);
-    r = BS;
-    isP = true;
+// gP and gD from the per-sample partials, in float64: 16 threads per entry sum a run of samples each, eight loads in
+// flight, and thread 0 adds the runs in order (one thread per entry took 16 us at 256 samples). The workgroups past the
+// entries write gD's zeros outside the blocks.
+constexpr int kRedEnt = 16, kRedRun = 16;
+__global__ __launch_bounds__(kRedEnt* kRedRun) void k_reduce_blk(TArgs a, int BS, int nent_wg) {
+  __shared__ double red[kRedRun][kRedEnt];
+  const size_t dd = (size_t)a.d * a.d;
+  if ((int)blockIdx.x >= nent_wg) {
+    const size_t e = (size_t)(blockIdx.x - nent_wg) * blockDim.x + threadIdx.x;
+    if (e >= (size_t)a.V * dd) return;
+    const int rc = (int)(e % dd);
+    if (rc / a.d / BS != rc % a.d / BS) a.gD[e] = 0.0f;
+    return;
   }
-  // the samples in order; eight loads in flight before their adds (the same order of additions)
-  const size_t off = ((size_t)g * (BS + 1) + r) * a.d + i, stride = (size_t)a.V * (BS + 1) * a.d;
+  const int x = threadIdx.x % kRedEnt, y = threadIdx.x / kRedEnt;
+  const size_t nent = (size_t)a.V * (BS + 1) * a.d, off = (size_t)blockIdx.x * kRedEnt + x;
+  const int per = (a.B + kRedRun - 1) / kRedRun, b1 = min(a.B, (y + 1) * per);
   double s = 0.0;
-  int b = 0;
-  for (; b + 8 <= a.B; b += 8) {
-    float v[8];
+  if (off < nent) {
+    int b = y * per;
+    for (; b + 8 <= b1; b += 8) {
+      float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = a.part[(size_t)(b + u) * stride + off];
+      for (int u = 0; u < 8; ++u) v[u] = a.part[(size_t)(b + u) * nent + off];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s += (double)v[u];
+      for (int u = 0; u < 8; ++u) s += (double)v[u];
+    }
+    for (; b < b1; ++b) s += (double)a.part[(size_t)b * nent + off];
   }
-  for (; b < a.B; ++b) s += (double)a.part[(size_t)b * stride + off];
-  if (isP) a.gP[(size_t)g * a.d + i] = (float)s;
-  else a.gD[e] = (float)s;
+  red[y][x] = s;
+  __syncthreads();
+  if (y > 0 || off >= nent) return;
+  for (int u = 1; u < kRedRun; ++u) s += red[u][x];
+  const int i = (int)(off % a.d), q = (int)(off / a.d), g = q / (BS + 1), r = q % (BS + 1);
+  if (r == BS) a.gP[(size_t)g * a.d + i] = (float)s;
+  else a.gD[((size_t)g * a.d + i) * a.d + (i / BS) * BS + r] = (float)s;
 }
 
 }  // namespace tok1
@@ -419,28 +529,42 @@ int tok1_check(const ews_token1_desc* s) {
   if (s->batch < 1 || s->steps < 1 || s->dim < 1 || s->dim > tok1::kMaxD || s->vocab < 1) return EWS_ERR_SHAPE;
   const int bs = s->block;
   if (bs < 0 || bs > 8 || bs == 5 || bs == 7 || (bs > 0 && s->dim % bs != 0)) return EWS_ERR_OPTION;
-  // the backward's per-lane accumulators (16 KB at most) and its staged steps (8 KB) sit in LDS beside the staged
-  // caches (48 KB at most)
+  // the backward's per-lane accumulators (16 KB per wavefront at most) sit in LDS beside the staged caches (48 KB at
+  // most)
   if (bs > 0 && (size_t)s->vocab * (bs + 1) > 64) return EWS_ERR_SHAPE;
   return EWS_OK;
 }
-// launch of a block-diagonal kernel for the descriptor's block size
-#define EWS_TOK1_BLK(KERNEL, BS, GRID, LDS, ST, A)                                                    \
-  do {                                                                                               \
-    switch (BS) {                                                                                    \
-      case 1: hipLaunchKernelGGL((KERNEL<1>), GRID, dim3(64), LDS, ST, A); break;                  \
-      case 2: hipLaunchKernelGGL((KERNEL<2>), GRID, dim3(64), LDS, ST, A); break;                  \
-      case 3: hipLaunchKernelGGL((KERNEL<3>), GRID, dim3(64), LDS, ST, A); break;                  \
-      case 4: hipLaunchKernelGGL((KERNEL<4>), GRID, dim3(64), LDS, ST, A); break;                  \
-      case 6: hipLaunchKernelGGL((KERNEL<6>), GRID, dim3(64), LDS, ST, A); break;                  \
-      default: hipLaunchKernelGGL((KERNEL<8>), GRID, dim3(64), LDS, ST, A); break;                 \
-    }                                                                                                \
-  } while (0)
-size_t blk_lds_bytes(const ews_token1_desc* s, bool bwd) {
+// Wavefronts per sample (spans of its steps): eight while that stays under 4096 wavefronts, at least 32 steps each, and
+// while their accumulators fit the LDS; one for blocks of 6 and 8.
+size_t blk_lds_bytes(const ews_token1_desc* s, int nw, bool bwd) {
   const size_t stage = (size_t)s->vocab * s->dim * (s->block + 1);
   const size_t staged = stage <= (size_t)tok1::kStageFloats ? stage : 0;
-  return (staged + (bwd ? (size_t)s->vocab * (s->block + 1) * 64 + 2 * tok1::kStage * 64 : 0)) * 4;
+  const size_t maps = (size_t)nw * (s->block + 1) * 64;
+  return (staged + 2 * maps + (bwd ? maps * s->vocab : 0)) * 4;
 }
+int blk_waves(const ews_token1_desc* s) {
+  int nw = s->block <= 4 ? 8 : 1;
+  while (nw > 1 && ((long)s->batch * nw > 4096 || s->steps < 32 * nw || blk_lds_bytes(s, nw, true) > 160 * 1024)) nw /= 2;
+  return nw;
+}
+// launch of a block-diagonal kernel for the descriptor's block size
+template <class K>
+int blk_launch(K* kern, const ews_token1_desc* s, bool bwd, hipStream_t st, const tok1::TArgs& a) {
+  const int nw = blk_waves(s);
+  const size_t lds = blk_lds_bytes(s, nw, bwd);
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return EWS_ERR_LAUNCH;
+  hipLaunchKernelGGL(kern, dim3(a.B), dim3(64 * nw), lds, st, a);
+  return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
+}
+#define EWS_TOK1_BLK(KERNEL, S, BWD, ST, A)                                         \
+  ((S)->block == 1   ? blk_launch(&KERNEL<1>, S, BWD, ST, A)                        \
+   : (S)->block == 2 ? blk_launch(&KERNEL<2>, S, BWD, ST, A)                        \
+   : (S)->block == 3 ? blk_launch(&KERNEL<3>, S, BWD, ST, A)                        \
+   : (S)->block == 4 ? blk_launch(&KERNEL<4>, S, BWD, ST, A)                        \
+   : (S)->block == 6 ? blk_launch(&KERNEL<6>, S, BWD, ST, A)                        \
+                     : blk_launch(&KERNEL<8>, S, BWD, ST, A))
 size_t al256t(size_t x) { return (x + 255) & ~(size_t)255; }
 tok1::TArgs tok1_args(const ews_token1_desc* s) {
   tok1::TArgs a{};
@@ -479,8 +603,8 @@ int ews_token1_scan(const ews_token1_desc* desc, const int32_t* tokens, const ui
   a.out = out;
   hipStream_t st = (hipStream_t)stream;
   if (desc->block > 0) {
-    EWS_TOK1_BLK(ews::tok1::k_fwd_blk, desc->block, dim3(a.B), ews::blk_lds_bytes(desc, false), st, a);
-    return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
+    using ews::blk_launch;
+    return EWS_TOK1_BLK(ews::tok1::k_fwd_blk, desc, false, st, a);
   }
   const size_t nd = (size_t)a.V * a.d * a.d;
   hipLaunchKernelGGL(ews::tok1::k_transpose, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, st, a);
@@ -508,11 +632,13 @@ int ews_token1_scan_backward(const ews_token1_desc* desc, const int32_t* tokens,
   hipStream_t st = (hipStream_t)stream;
   if (desc->block > 0) {
     a.part = (float*)workspace;
-    EWS_TOK1_BLK(ews::tok1::k_bwd_blk, desc->block, dim3(a.B), ews::blk_lds_bytes(desc, true), st, a);
-    if (hipGetLastError() != hipSuccess) return EWS_ERR_LAUNCH;
-    const size_t tot = (size_t)a.V * (dd + a.d);
-    hipLaunchKernelGGL(ews::tok1::k_reduce_blk, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, a,
-                       desc->block);
+    using ews::blk_launch;
+    const int brc = EWS_TOK1_BLK(ews::tok1::k_bwd_blk, desc, true, st, a);
+    if (brc != EWS_OK) return brc;
+    constexpr int rt = ews::tok1::kRedEnt * ews::tok1::kRedRun;
+    const int ne = (int)(((size_t)a.V * (desc->block + 1) * a.d + ews::tok1::kRedEnt - 1) / ews::tok1::kRedEnt);
+    const int nz = (int)(((size_t)a.V * dd + rt - 1) / rt);
+    hipLaunchKernelGGL(ews::tok1::k_reduce_blk, dim3(ne + nz), dim3(rt), 0, st, a, desc->block, ne);
     return hipGetLastError() == hipSuccess ? EWS_OK : EWS_ERR_LAUNCH;
   }
   char* w = (char*)workspace;
