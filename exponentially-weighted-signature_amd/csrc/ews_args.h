@@ -44,6 +44,7 @@ struct DiagArgs {
   float* chbar;     // (B, C)
   float* ctab;      // pair-group coefficient table at one reference step (residual)
   int fast_ok;      // 1 if this configuration has pair-group kernels (flags are valid), else 0
+  int pw;           // 1 if it has wave-per-chunk plane kernels (ews_planes.hip), which own the strictly uniform chunks
   // quad carry scan of the pair-group path (quads of four chunks)
   int NQ;           // quads per sample
   float* qagg;      // (B, NQ, D) quad summaries (forward) / quad adjoint aggregates (backward)

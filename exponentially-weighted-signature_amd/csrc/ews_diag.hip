@@ -32,6 +32,7 @@
 #include "ews_lanes.h"
 #include "ews_numerics.h"
 #include "ews_pairs.h"
+#include "ews_planes.h"
 #include "ews_seq.h"
 
 namespace ews {
@@ -277,8 +278,14 @@ __device__ __forceinline__ void fwd_step(const Coef<T>& c, T pj, T pk, T& S1, T&
 
 // Chunk setup shared by all chunk kernels: the chunk's class and its reference step. The class is decided once, by the
 // forward's first summary pass (or the pair-group forward), and kept in the residual: flag bit 0 uniform steps, bit 1
-// the steps may be inverted, bit 3 small steps (the polynomial model applies), and the mean step hbar.
-constexpr int kFlagUniform = 1, kFlagInvert = 2, kFlagSmall = 8;
+// the steps may be inverted, bit 3 small steps (the polynomial model applies), bit 4 steps uniform enough for constant
+// coefficients (set where the wave-per-chunk plane kernels run: a.pw), and the mean step hbar.
+constexpr int kFlagUniform = 1, kFlagInvert = 2, kFlagSmall = 8, kFlagStrict = 16;
+// a chunk whose summary, prefix rows (not log rows) and local adjoint the wave-per-chunk kernels take, and, where it may be
+// inverted and no clock gradient is wanted, its full adjoint
+__device__ __forceinline__ bool pw_owns(const DiagArgs& a, int f) {
+  return a.pw && (f & (kFlagUniform | kFlagStrict)) == (kFlagUniform | kFlagStrict);
+}
 struct ChunkClock {
   float hbar, href;
   bool fast, per_int;
@@ -453,15 +460,20 @@ __global__ __launch_bounds__(MAXT) void k_chunk_fwd(DiagArgs a) {
   const int c = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
   // the first summary pass (FAST) classifies every chunk and writes its class; every later kernel reads it and leaves
   // a chunk it does not own before staging anything
+  // (where the wave-per-chunk plane kernels run, theirs has classified them and taken the strictly uniform ones)
   constexpr bool kClassify = MODE == MODE_SUMMARY && FAST;
-  if (!kClassify && ((a.cflag[b * a.C + c] & kFlagUniform) != 0) != FAST) return;
+  if (!kClassify || a.pw) {
+    const int fl = a.cflag[b * a.C + c];
+    if (((fl & kFlagUniform) != 0) != FAST || (MODE != MODE_REDUCE && !(MODE == MODE_PREFIX && a.log) && pw_owns(a, fl)))
+      return;
+  }
   const int t0 = c * a.T;
   const int Tc = min(a.T, a.n_int - t0);
   load_chunk(a, b, t0, Tc, s_v, s_h);
   __syncthreads();
   const LaneMap m = lane_map(a, tid);
   ChunkClock cc;
-  if constexpr (kClassify) {
+  if (kClassify && !a.pw) {
     cc = chunk_classify<T>(a, b, Tc, s_h);
     if (tid == 0) {
       a.cflag[b * a.C + c] = (cc.fast ? kFlagUniform : 0) | (cc.inv_ok ? kFlagInvert : 0) | (cc.small ? kFlagSmall : 0);
@@ -1070,34 +1082,52 @@ __global__ __launch_bounds__(MAXT) void k_fwd_group(DiagArgs a) {
   }
 }
 
+// The flows of up to kScanBlk groups over their clock spans into LDS, a lane per (group, coordinate): group(i) is the
+// i-th of the block. Every lane of a scan needs two of them a step; evaluated in the scan's own chain (two float64
+// exponentials, sines and cosines a step) they were most of it (49 groups at d = 24: 55 and 83 us).
+constexpr int kScanBlk = 16, kScanMaxK = 32;
+template <class TD, int CW, class G>
+__device__ __forceinline__ void stage_flows(const DiagArgs& a, int b, int n, double* s_F, G&& group) {
+  TD dummy{};
+  for (int i = threadIdx.x; i < n * a.K; i += blockDim.x) {
+    const int q = i / a.K, j = i % a.K, t0 = group(q) * a.scan_cb * a.T, t1 = min(t0 + a.scan_cb * a.T, a.n_int);
+    stD(s_F + (size_t)i * CW, dexp(mul_s(load_ud(a.params, j, &dummy), span_tau(a, b, t0, t1))));
+  }
+}
+
 template <bool CPLX, int N, int MAXT>
 __global__ __launch_bounds__(MAXT) void k_fwd_group_scan(DiagArgs a) {
   using TD = typename Types<CPLX>::TD;
+  constexpr int CW = CPLX ? 2 : 1;
+  __shared__ double s_F[kScanBlk * kScanMaxK * CW];
   const int b = blockIdx.x;
   const LaneMap m = lane_map(a, threadIdx.x);
-  if (!m.active) return;
   TD dummy{};
-  const TD uj = load_ud(a.params, m.j, &dummy), uk = load_ud(a.params, m.k, &dummy);
   // group g's span and aggregate are loaded one group ahead and issued before the group's carry is stored (the
   // memory counter is in order: a load issued after a store is waited for together with the store)
   struct Pre {
-    double tau;
     TD l1j, l1k, l2A, l2B;
   };
   auto load = [&](int g, Pre& p) {
-    const int t0 = g * a.scan_cb * a.T, t1 = min(t0 + a.scan_cb * a.T, a.n_int);
-    p.tau = span_tau(a, b, t0, t1);
     lane_summary_d<CPLX>(a, m, a.gagg + ((size_t)b * a.NG + g) * a.D, p.l1j, p.l1k, p.l2A, p.l2B);
   };
   TD S1{}, SA{}, SB{};
   Pre cur{}, nxt{};
-  if (a.NG > 0) load(0, cur);
-  for (int g = 0; g < a.NG; ++g) {
-    if (g + 1 < a.NG) load(g + 1, nxt);
-    store_lane_d<CPLX, N>(a, m, a.gcar + ((size_t)b * a.NG + g) * a.D, S1, SA, SB);
-    chen_fwd_lane<CPLX, N>(S1, SA, SB, dexp(mul_s(uj, cur.tau)), dexp(mul_s(uk, cur.tau)), cur.l1j, cur.l1k, cur.l2A,
-                           cur.l2B);
-    cur = nxt;
+  if (m.active && a.NG > 0) load(0, cur);
+  for (int g0 = 0; g0 < a.NG; g0 += kScanBlk) {
+    const int n = min(kScanBlk, a.NG - g0);
+    __syncthreads();  // the block before has been read
+    stage_flows<TD, CW>(a, b, n, s_F, [&](int q) { return g0 + q; });
+    __syncthreads();
+    if (!m.active) continue;
+    for (int q = 0; q < n; ++q) {
+      const int g = g0 + q;
+      if (g + 1 < a.NG) load(g + 1, nxt);
+      store_lane_d<CPLX, N>(a, m, a.gcar + ((size_t)b * a.NG + g) * a.D, S1, SA, SB);
+      const TD Fj = ldDD(s_F + (size_t)(q * a.K + m.j) * CW, &dummy), Fk = ldDD(s_F + (size_t)(q * a.K + m.k) * CW, &dummy);
+      chen_fwd_lane<CPLX, N>(S1, SA, SB, Fj, Fk, cur.l1j, cur.l1k, cur.l2A, cur.l2B);
+      cur = nxt;
+    }
   }
 }
 
@@ -1204,21 +1234,18 @@ __global__ __launch_bounds__(MAXT) void k_bwd_group_scan(DiagArgs a) {
   using TD = typename Types<CPLX>::TD;
   constexpr int CW = CPLX ? 2 : 1;
   __shared__ double s_red[MAXT * CW];
+  __shared__ double s_F[kScanBlk * kScanMaxK * CW];
   const int b = blockIdx.x;
   const LaneMap m = lane_map(a, threadIdx.x);
   TD dummy{};
-  const TD uj = load_ud(a.params, m.j, &dummy), uk = load_ud(a.params, m.k, &dummy);
-  // Group g's operands (its span, the level-1 carries at its ends, its aggregate) are loaded one group ahead and
+  // Group g's operands (the level-1 carries at its ends, its aggregate) are loaded one group ahead and
   // issued before the group's carry is stored: the memory counter is in order, so a load issued after a store could
   // not be waited for without waiting for the store as well.
   struct Pre {
-    double tau;
     TD cek, csk, a1, aA, aB;
   };
   auto load = [&](int g, Pre& p) {
     const int c0 = g * a.scan_cb, c1 = min(c0 + a.scan_cb, a.C);
-    const int t0 = c0 * a.T, t1 = min(c1 * a.T, a.n_int);
-    p.tau = span_tau(a, b, t0, t1);
     const double* cs = a.carries + ((size_t)b * (a.C + 1) + c0) * a.D;
     const double* ce = a.carries + ((size_t)b * (a.C + 1) + c1) * a.D;
     p.cek = ldDD(ce + st1<CPLX>(m.k), &dummy);
@@ -1241,9 +1268,15 @@ __global__ __launch_bounds__(MAXT) void k_bwd_group_scan(DiagArgs a) {
   Pre cur{}, nxt{};
   if (a.NG > 0) load(a.NG - 1, cur);
   for (int g = a.NG - 1; g >= 0; --g) {
+    const int q = (a.NG - 1 - g) % kScanBlk;
+    if (q == 0) {
+      __syncthreads();  // the block before has been read
+      stage_flows<TD, CW>(a, b, min(kScanBlk, g + 1), s_F, [&](int i) { return g - i; });
+      __syncthreads();
+    }
     if (g > 0) load(g - 1, nxt);
     if (m.active) store_lane_d<CPLX, N>(a, m, a.gcar + ((size_t)b * a.NG + g) * a.D, X1, XA, XB);
-    const TD Fj = dexp(mul_s(uj, cur.tau)), Fk = dexp(mul_s(uk, cur.tau));
+    const TD Fj = ldDD(s_F + (size_t)(q * a.K + m.j) * CW, &dummy), Fk = ldDD(s_F + (size_t)(q * a.K + m.k) * CW, &dummy);
     const TD l1k = cur.cek - Fk * cur.csk;
     adj_lane<CPLX, N>(a, m, X1, XA, XB, Fj, Fk, l1k, s_red);
     if (m.plane) X1 = X1 + cur.a1;
@@ -1474,7 +1507,8 @@ __global__ __launch_bounds__(MAXT) void k_chunk_bwd_local(DiagArgs a) {
   int* s_am = reinterpret_cast<int*>(smem + Lo.am);
   float* s_red = smem + Lo.g;
   const int c = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  if (((a.cflag[b * a.C + c] & kFlagUniform) != 0) != FAST) return;  // the forward's chunk class
+  const int fl = a.cflag[b * a.C + c];  // the forward's chunk class
+  if (((fl & kFlagUniform) != 0) != FAST || pw_owns(a, fl)) return;
   const int t0 = c * a.T;
   const int Tc = min(a.T, a.n_int - t0);
   const bool prefix = a.readout == EWS_READOUT_PREFIX;
@@ -2027,6 +2061,7 @@ __device__ __forceinline__ void chunk_bwd_inv(const DiagArgs& a, const int c, co
 
 template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
 __global__ __launch_bounds__(MAXT) void k_chunk_bwd_inv(DiagArgs a) {
+  if (!DH && pw_owns(a, a.cflag[blockIdx.y * a.C + blockIdx.x])) return;
   chunk_bwd_inv<CPLX, N, MAXT, WAVE, DH, false>(a, blockIdx.x, blockIdx.y);
 }
 // Chunks blockIdx.x, blockIdx.x + gridDim.x, ... of sample blockIdx.y whose class OWNS accepts: the classes of 64
@@ -2587,6 +2622,7 @@ DiagArgs make_args(const ews_diag_desc* s, const Plan& p, const void* path, cons
   a.cflow = (double*)(ws + w.cflow);
   a.lbflag = (int*)(ws + w.lbflag); a.lbagg = (double*)(ws + w.lbagg);
   if (p.log && !fwd_only) a.gcot = (float*)(ws + w.gcot);
+  a.pw = p.cplx && planes_eligible(a) ? 1 : 0;
   return a;
 }
 
@@ -2608,6 +2644,7 @@ int forward_pass(const ews_diag_desc* s, const Plan& p, DiagArgs a, hipStream_t 
         if (pairs_forward(a, st, false) != 0) return EWS_ERR_LAUNCH;
         return EWS_OK;
       }
+      if (a.pw && planes_summary(a, st) != 0) return EWS_ERR_LAUNCH;
       hipLaunchKernelGGL((k_chunk_fwd<CPLX, N, MODE_SUMMARY, MAXT, true>), grid, blk, fwd_lds(p), st, a);
       EWS_LAUNCH_CHECK();
       hipLaunchKernelGGL((k_chunk_fwd<CPLX, N, MODE_SUMMARY, MAXT, false>), grid, blk, fwd_lds(p), st, a);
@@ -2628,6 +2665,7 @@ int forward_pass(const ews_diag_desc* s, const Plan& p, DiagArgs a, hipStream_t 
           if (pairs_forward(a, st, true) != 0) return EWS_ERR_LAUNCH;
           return EWS_OK;
         }
+        if (a.pw && planes_rows(a, st) != 0) return EWS_ERR_LAUNCH;
         hipLaunchKernelGGL((k_chunk_fwd<CPLX, N, MODE_PREFIX, MAXT, true>), grid, blk, fwd_lds(p), st, a);
         EWS_LAUNCH_CHECK();
         hipLaunchKernelGGL((k_chunk_fwd<CPLX, N, MODE_PREFIX, MAXT, false>), grid, blk, fwd_lds(p), st, a);
@@ -2693,6 +2731,7 @@ int backward_pass(const Plan& p, DiagArgs a, hipStream_t st, int pass) {
   switch (pass) {
     case 0:
       if (p.fast && pairs_backward(a, st, false) != 0) return EWS_ERR_LAUNCH;
+      if (a.pw && planes_local(a, st) != 0) return EWS_ERR_LAUNCH;
       if (set_lds(&k_chunk_bwd_local<CPLX, N, MAXT, WAVE, true>, p.lds_bwd_local) != EWS_OK) return EWS_ERR_LAUNCH;
       if (set_lds(&k_chunk_bwd_local<CPLX, N, MAXT, WAVE, false>, p.lds_bwd_local) != EWS_OK) return EWS_ERR_LAUNCH;
       if (!p.fast) {  // with the pair kernels active no chunk is left to the FAST instantiation
@@ -2718,6 +2757,7 @@ int backward_pass(const Plan& p, DiagArgs a, hipStream_t st, int pass) {
       break;
     case 2:
       if (p.fast && pairs_backward(a, st, true) != 0) return EWS_ERR_LAUNCH;
+      if (a.pw && !a.dclock && planes_full(a, st) != 0) return EWS_ERR_LAUNCH;
       // the clock gradient's dh terms only when it is requested (grad_clock non-null)
       if (a.dclock) return full_adjoints<CPLX, N, MAXT, WAVE, true>(p, a, st);
       return full_adjoints<CPLX, N, MAXT, WAVE, false>(p, a, st);
