@@ -2150,50 +2150,321 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
   pb[HP * 256 + tid] = dAl;
 }
 
-// Van Loan leaf adjoint (one workgroup per interval, grid-stride). The forward's recompute saved per interval the
-// step matrices P, V and the knot increments Delta_m (Delta_{M-1} = V w, Delta_{m-1} = P Delta_m); from them
-// Pre_m, R_m, Y_m, X_m (see k_vl), then:
+// Van Loan leaf adjoint. The forward's recompute saved per interval the step matrices P, V and the knot increments
+// Delta_m (Delta_{M-1} = V w, Delta_{m-1} = P Delta_m); from them Pre_m, R_m, Y_m, X_m (see k_vl), then:
 //   level adjoints:  dDelta_m += dS1;  dY_m = dS2 Delta_m, dDelta_m += dS2^T Y_m;
 //     depth 3 (S3 = sum_m Delta_m[b] G_m[a][c], G_m = Y_m (x) R_m + X_m (x) Delta_m / 2), with
 //     Q_m = dS3 ._2 Delta_m:  dY_m += Q_m R_m,  dX_m = Q_m Delta_m / 2,  dR_m = Q_m^T Y_m,
 //     dDelta_m += Q_m^T X_m / 2 (last index) and dDelta_m[b] += <dS3[:, b, :], G_m> (middle index);
-//     each thread keeps its column dS3[a][:][c] and its row dS3[a][b][:] in registers across the segments;
 //   Y = Pre + Delta/2, X = Pre + Delta/3, Pre_m = sum_{j<m} Delta_j, R_m = sum_{j>m} Delta_j;
-//   chain (one wavefront): lambda_0 = dDelta_0, lambda_m = dDelta_m + P^T lambda_{m-1},
-//   GP = sum_m lambda_{m-1} (x) Delta_m, GV = lambda_{M-1} (x) w, dw = V^T lambda_{M-1}, dv = dw / M;
-//   step matrices: block_exp_adjoint (exact) or block_rational_adjoint, for the step delta = h / M.
-// Then the flow's adjoint as in k_leaf_bwd.
-constexpr int VMAX = 64;  // knots per interval at most
+//   chain: lambda_0 = dDelta_0, lambda_m = dDelta_m + P^T lambda_{m-1},
+//   GP = sum_m lambda_{m-1} (x) Delta_m, GV = lambda_{M-1} (x) w, dw = V^T lambda_{M-1}, dv = dw / M.
+// k_vl_knots_bwd does this with a wavefront per interval (no workgroup barrier); it leaves GP over the saved P and
+// lambda_{M-1} over the first saved knot for k_vl_mats_bwd: the adjoints of the step matrices (block_exp_adjoint or
+// block_rational_adjoint, for the step delta = h / M) and of the flow, a workgroup per interval.
+//
+// Depth 3 is three contractions of the 16 KB dS3 with the knots, on fp32 MFMA over tiles of 16 knots (rows m; up to 8
+// knots past the last full tile in quads, v_mfma_f32_4x4x1_16b, whose blocks split the contraction over the lane groups
+// g): per first index a, Q^a[m][c] = sum_b Delta_m[b] dS3[a][b][c]; over all (a, c), sum G_m[a][c] dS3[a][b][c]; per last
+// index c, Q^c[m][a] (the first one again, for sums over c that then need no lane exchange). Each reads dS3 in its own
+// order into 64 registers, loaded one contraction ahead (the second and third time from the caches). One workgroup per
+// interval, with these sums on the vector units and behind barriers, left 2 workgroups per CU: B = 16, L = 4096, d = 16,
+// M = 20, 2434 us (this kernel and k_vl_mats_bwd: 662 + 506).
 
-template <int N, bool EXACTF>
-__global__ __launch_bounds__(256) void k_vl_bwd(Args a, LeafBwd o) {
+
+__host__ __device__ constexpr int vlk_rows(int M) { return (M & 15) > 8 ? (M + 15) / 16 * 16 : (M + 3) / 4 * 4; }
+__host__ __device__ constexpr int vlk_wave(int M) { return 8 * 16 * vlk_rows(M); }  // floats of LDS per wavefront
+
+// n, unknown to the compiler from here on: the tables' row addresses, invariant over the intervals, are then formed as they
+// are used (hoisted, a few hundred of them spill)
+__device__ __forceinline__ int opaque(int n) {
+  asm volatile("" : "+s"(n));
+  return n;
+}
+template <bool QUAD> __device__ __forceinline__ f4 mfma_k(float x, float y, f4 c) {
+  if constexpr (QUAD) return __builtin_amdgcn_mfma_f32_4x4x1f32(x, y, c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+}
+// the quads' partial sums over the lane groups
+template <bool QUAD> __device__ __forceinline__ void quad_sum(f4& v) {
+  if constexpr (QUAD) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = lanes::add_xor32(lanes::add_xor16(v[r]));
+  }
+}
+// f(row, r): the lane's result rows of the block of knots at mb (a quad's sums are in every lane group: group 0 stores)
+template <bool QUAD, class F> __device__ __forceinline__ void own_rows(int mb, int g, F&& f) {
+  if (!QUAD || g == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f(QUAD ? mb + r : mb + 4 * g + r, r);
+  }
+}
+
+template <int N>
+__global__ __launch_bounds__(256, 2) void k_vl_knots_bwd(Args a, LeafBwd o) {
+  extern __shared__ __align__(16) float lds[];
   constexpr int LW = lw_of(N);
-  __shared__ __align__(16) float sp[HP][256];
-  __shared__ __align__(16) float Pm[256], Vm[256], W1[256], W2[256], W3[256 + 32], GPm[256], GVm[256], Gm[256];
-  // The knot arrays and dS3 are dead once the chain has run; the squarings of the step-matrix and flow adjoints
-  // (Esq, Fsq) then reuse their space, which keeps the workgroup at two per CU.
-  constexpr int UL = 7 * VMAX * 16 + (N >= 3 ? 4096 : 4), UE = 2 * SQMAX * 256;
-  __shared__ __align__(16) float U[UL > UE ? UL : UE];
-  __shared__ __align__(16) float dS2[256];
-  typedef float Row16[16];
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, c16 = l & 15;
+  const int Mv = a.vm, MP = vlk_rows(Mv), vs = 512 + 16 * Mv, TS = 16 * MP;
+  float* D = lds + w * vlk_wave(Mv);  // Delta[m][c]
+  float* R = D + TS;                  // R[m][c]
+  float* DT = R + TS;                 // transposed: Delta, R, Y, X
+  float* RT = DT + TS;
+  float* YT = RT + TS;
+  float* XT = YT + TS;
+  float* oD = XT + TS;                // dDelta, then lambda; dR; dPre (over Y)
+  float* oR = oD + TS;
+  float* oP = YT;
+  const long total = (long)a.B * a.n_int, first = (long)blockIdx.x * 4 + w, stride = (long)gridDim.x * 4;
+  f4 pd[4];                          // the next interval's knots
+  f4 A3[N >= 3 ? 16 : 1];            // dS3 in the order of the contraction
+  auto prefetch = [&](long it) {
+    const float* kn = a.vlsave + (size_t)it * vs + 512;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (l + 64 * u < 4 * Mv) pd[u] = reinterpret_cast<const f4*>(kn)[l + 64 * u];
+    if constexpr (N >= 3) {  // A3[a][s] = dS3[a][4g + s][c16]
+      const float* r3 = a.loc + (size_t)it * LW + 272;
+#pragma unroll
+      for (int aa = 0; aa < 16; ++aa)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) A3[aa][s] = r3[aa * 256 + (4 * g + s) * 16 + c16];
+    }
+  };
+  if (first < total) prefetch(first);
+  for (long it = first; it < total; it += stride) {
+    const int b = (int)(it / a.n_int), t = (int)(it - (long)b * a.n_int);
+    float* sv = a.vlsave + (size_t)it * vs;
+    const float* row = a.loc + (size_t)it * LW;
+    wave_order_d();
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (l + 64 * u < 4 * Mv) reinterpret_cast<f4*>(D)[l + 64 * u] = pd[u];
+    f4 pr[4], vc;  // columns of P; rows 4g .. of V's column c16
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pr[q][r] = sv[(4 * q + r) * 16 + c16];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) vc[r] = sv[256 + (4 * g + r) * 16 + c16];
+    const float s1 = row[c16];
+    f4 s2r, s2c;  // dS2[c16][4g + s], dS2[4g + s][c16]
+    if constexpr (N >= 2) {
+      s2r = *reinterpret_cast<const f4*>(row + 16 + c16 * 16 + 4 * g);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) s2c[s] = row[16 + (4 * g + s) * 16 + c16];
+    }
+    wave_order_d();
+    // R, Y, X: lane (c16, g) walks a quarter of the column's knots
+    const int S = (Mv + 3) >> 2, m0 = min(Mv, g * S), m1 = min(Mv, m0 + S);
+    {
+      float own = 0.0f;
+      for (int m = m0; m < m1; ++m) own += D[m * 16 + c16];
+      float pre = 0.0f, all = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float x = __shfl(own, c16 + 16 * k, 64);
+        if (k < g) pre += x;
+        all += x;
+      }
+      for (int m = m0; m < m1; ++m) {
+        const float dm = D[m * 16 + c16], rm = all - pre - dm;
+        R[m * 16 + c16] = rm;
+        DT[c16 * MP + m] = dm;
+        RT[c16 * MP + m] = rm;
+        YT[c16 * MP + m] = fmaf(0.5f, dm, pre);
+        XT[c16 * MP + m] = fmaf(1.0f / 3.0f, dm, pre);
+        pre += dm;
+      }
+      for (int m = Mv + g; m < MP; m += 4) {
+        D[m * 16 + c16] = R[m * 16 + c16] = 0.0f;
+        DT[c16 * MP + m] = RT[c16 * MP + m] = YT[c16 * MP + m] = XT[c16 * MP + m] = 0.0f;
+      }
+    }
+    wave_order_d();
+    // ---- dR and the last index's dDelta (per first index a); dS2^T Y
+    auto first_index = [&](auto quad, int mb) {
+      constexpr bool QUAD = decltype(quad)::value;
+      const int mr = mb + (QUAD ? l & 3 : c16), me = QUAD ? mb : mb + 4 * g;
+      f4 aR = {0.0f, 0.0f, 0.0f, 0.0f}, aD = aR;
+      if constexpr (N >= 3) {
+        const f4 dm = *reinterpret_cast<const f4*>(D + mr * 16 + 4 * g);
+        const int mp = opaque(MP);
+        const float* ty = YT + me;
+#pragma unroll
+        for (int aa = 0; aa < 16; ++aa) {
+          f4 q = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) q = mfma_k<QUAD>(dm[s], A3[aa][s], q);
+          const f4 y = *reinterpret_cast<const f4*>(ty), x = *reinterpret_cast<const f4*>(ty + TS);
+          ty += mp;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            aR[r] = fmaf(y[r], q[r], aR[r]);
+            aD[r] = fmaf(x[r], q[r], aD[r]);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) aD[r] *= 0.5f;
+      }
+      if constexpr (N >= 2) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) aD = mfma_k<QUAD>(YT[(4 * g + s) * MP + mr], s2c[s], aD);
+      }
+      quad_sum<QUAD>(aR);
+      quad_sum<QUAD>(aD);
+      own_rows<QUAD>(mb, g, [&](int m, int r) {
+        oR[m * 16 + c16] = aR[r];
+        oD[m * 16 + c16] = aD[r];
+      });
+    };
+    // ---- the middle index's dDelta: sum over (a, c) of G_m[a][c] dS3[a][b][c]
+    auto middle_index = [&](auto quad, int mb) {
+      constexpr bool QUAD = decltype(quad)::value;
+      const int mr = mb + (QUAD ? l & 3 : c16);
+      const f4 rm = *reinterpret_cast<const f4*>(R + mr * 16 + 4 * g);
+      f4 dh = *reinterpret_cast<const f4*>(D + mr * 16 + 4 * g);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) dh[s] *= 0.5f;
+      const int mp = opaque(MP);
+      const float* ty = YT + mr;
+      f4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+      for (int aa = 0; aa < 16; ++aa) {
+        const float y = ty[0], x = ty[TS];
+        ty += mp;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[s & 1] = mfma_k<QUAD>(fmaf(y, rm[s], x * dh[s]), A3[aa][s], acc[s & 1]);
+      }
+      f4 aD;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) aD[r] = acc[0][r] + acc[1][r];
+      quad_sum<QUAD>(aD);
+      own_rows<QUAD>(mb, g, [&](int m, int r) { oD[m * 16 + c16] += aD[r]; });
+    };
+    // ---- dY, dX (per last index c) -> dPre and dDelta
+    auto last_index = [&](auto quad, int mb) {
+      constexpr bool QUAD = decltype(quad)::value;
+      const int mr = mb + (QUAD ? l & 3 : c16), me = QUAD ? mb : mb + 4 * g;
+      const f4 dm = *reinterpret_cast<const f4*>(D + mr * 16 + 4 * g);
+      f4 aY = {0.0f, 0.0f, 0.0f, 0.0f}, aX = aY;
+      if constexpr (N >= 3) {
+        const int mp = opaque(MP);
+        const float* td = DT + me;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+          f4 q = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) q = mfma_k<QUAD>(dm[s], A3[4 * s + (c >> 2)][c & 3], q);
+          const f4 dd = *reinterpret_cast<const f4*>(td), rr = *reinterpret_cast<const f4*>(td + TS);
+          td += mp;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            aY[r] = fmaf(rr[r], q[r], aY[r]);
+            aX[r] = fmaf(dd[r], q[r], aX[r]);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) aX[r] *= 0.5f;
+        quad_sum<QUAD>(aX);
+      }
+      if constexpr (N >= 2) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) aY = mfma_k<QUAD>(dm[s], s2r[s], aY);
+      }
+      quad_sum<QUAD>(aY);
+      own_rows<QUAD>(mb, g, [&](int m, int r) {
+        oP[m * 16 + c16] = aY[r] + aX[r];
+        oD[m * 16 + c16] += fmaf(0.5f, aY[r], aX[r] * (1.0f / 3.0f));
+      });
+    };
+    auto blocks = [&](auto&& f) {
+      int mb = 0;
+      for (; mb + 16 <= MP; mb += 16) f(std::integral_constant<bool, false>{}, mb);
+      for (; mb < MP; mb += 4) f(std::integral_constant<bool, true>{}, mb);
+    };
+    blocks(first_index);
+    if constexpr (N >= 3) {
+      // A3[a][s] = dS3[a][c16][4g + s]
+#pragma unroll
+      for (int aa = 0; aa < 16; ++aa) A3[aa] = *reinterpret_cast<const f4*>(row + 272 + aa * 256 + c16 * 16 + 4 * g);
+      wave_order_d();
+      blocks(middle_index);
+      // A3[4 s + q][r] = dS3[c16][4g + s][4q + r]
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          A3[4 * s + q] = *reinterpret_cast<const f4*>(row + 272 + c16 * 256 + (4 * g + s) * 16 + 4 * q);
+    }
+    wave_order_d();  // dPre goes over Y
+    blocks(last_index);
+    if (it + stride < total) prefetch(it + stride);
+    wave_order_d();
+    // ---- Pre and R -> Delta: dDelta_m += sum_{m' > m} dPre_m' + sum_{m' < m} dR_m'
+    {
+      float ownP = 0.0f, ownR = 0.0f;
+      for (int m = m0; m < m1; ++m) {
+        ownP += oP[m * 16 + c16];
+        ownR += oR[m * 16 + c16];
+      }
+      float accP = 0.0f, accR = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float xp = __shfl(ownP, c16 + 16 * k, 64), xr = __shfl(ownR, c16 + 16 * k, 64);
+        if (k > g) accP += xp;
+        if (k < g) accR += xr;
+      }
+      for (int m = m1 - 1; m >= m0; --m) {
+        oD[m * 16 + c16] += s1 + accP;
+        accP += oP[m * 16 + c16];
+      }
+      for (int m = m0; m < m1; ++m) {
+        oD[m * 16 + c16] += accR;
+        accR += oR[m * 16 + c16];
+      }
+    }
+    wave_order_d();
+    // ---- the chain: lambda_m over dDelta_m; every lane forms the whole product from the broadcast vector
+    for (int m = 1; m < Mv; ++m) {
+      f4 xv[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xv[q] = *reinterpret_cast<const f4*>(oD + (m - 1) * 16 + 4 * q);
+      const float u = oD[m * 16 + c16] + dot16(pr, xv);
+      wave_order_d();
+      if (g == 0) oD[m * 16 + c16] = u;
+      wave_order_d();
+    }
+    f4 gp = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < Mv - 1; k += 4) {  // GP[i][j] = sum_m lambda_m[i] Delta_{m+1}[j]
+      const int m = k + g;
+      const bool ok = m + 1 < Mv;
+      gp = mfma(ok ? oD[m * 16 + c16] : 0.0f, ok ? D[(m + 1) * 16 + c16] : 0.0f, gp);
+    }
+    const f4 lm = *reinterpret_cast<const f4*>(oD + (Mv - 1) * 16 + 4 * g);
+    float u = fmaf(vc.x, lm.x, fmaf(vc.y, lm.y, fmaf(vc.z, lm.z, vc.w * lm.w)));  // (V^T lambda)[c16]
+    u = lanes::add_xor32(lanes::add_xor16(u));
+    if (g == 0) {
+      o.dv[(size_t)it * 16 + c16] = u / (float)Mv;
+      sv[512 + c16] = oD[(Mv - 1) * 16 + c16];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sv[(4 * g + r) * 16 + c16] = gp[r];
+  }
+}
+
+// One workgroup per interval, grid-stride. exact: the knots' scheme is the exponential (Fsq in dynamic LDS).
+template <bool EXACTF>  // EXACTF: exact flows (the other schemes' code is left out)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 : 1))) void k_vl_mats_bwd(Args a,
+                                                                                                      LeafBwd o) {
+  extern __shared__ __align__(16) float lds[];
   typedef float Mat[256];
-  Row16* Dl = reinterpret_cast<Row16*>(U);
-  Row16* Rs = Dl + VMAX;
-  Row16* Ys = Rs + VMAX;
-  Row16* Xs = Ys + VMAX;
-  Row16* dD = Xs + VMAX;
-  Row16* dP = dD + VMAX;
-  Row16* dR = dP + VMAX;
-  float* dS3 = U + 7 * VMAX * 16;
-  Mat* Esq = reinterpret_cast<Mat*>(U);
-  Mat* Fsq = Esq + SQMAX;
-  __shared__ __align__(16) float dS1[16], wv[16], lam[16], red[8];
-  // depth 3: per-wavefront partial sums of the column cotangents of a block of VB knots, summed in a fixed order
-  // once per block
-  constexpr int VB = 8;
-  __shared__ float wR[VB][4][16], wD[VB][4][16], rowD[VB][16];
-  const int tid = threadIdx.x, i = tid >> 4, j = tid & 15, l = tid & 63, g = l >> 4, c16 = l & 15;
-  const int wv_id = tid >> 6;
+  __shared__ __align__(16) float sp[HP][256];
+  __shared__ __align__(16) float Vm[256], W1[256], W2[256], W3[256 + 32], GPm[256], GVm[256], Gm[256];
+  __shared__ __align__(16) float Esq[SQMAX][256];
+  __shared__ float red[8];
+  Mat* Fsq = reinterpret_cast<Mat*>(lds);
+  const int tid = threadIdx.x, i = tid >> 4, j = tid & 15;
   const int Mv = a.vm, vs = 512 + 16 * Mv;
 #pragma unroll
   for (int p = 0; p < HP; ++p) sp[p][tid] = a.apow[p * 256 + tid];
@@ -2202,43 +2473,26 @@ __global__ __launch_bounds__(256) void k_vl_bwd(Args a, LeafBwd o) {
 #pragma unroll
   for (int p = 0; p < HP; ++p) H[p] = 0.0f;
   float dAl = 0.0f;
-  __syncthreads();
   const long total = (long)a.B * a.n_int;
-  // ---- saved step matrices and increments, loaded into registers during the interval before (issued once the
-  // depth-3 sums are done): P, V, the knots (one float4 per thread: M <= 64), ds1, ds2, ds3 (four float4), dM and the
-  // increment's coordinates; all of them before the first store to LDS
-  const bool dl_own = tid < Mv * 4;
-  float in_p = 0.0f, in_v = 0.0f, in_g = 0.0f, in_s2 = 0.0f, in_s1 = 0.0f, in_x0 = 0.0f, in_x1 = 0.0f;
-  f4 in_d = {0.0f, 0.0f, 0.0f, 0.0f};
-  f4 in_s3[N >= 3 ? 4 : 1];
+  // the interval's inputs, loaded during the one before: GP, V, dM, lambda[i], the increment's coordinate j
+  float in_p = 0.0f, in_v = 0.0f, in_g = 0.0f, in_l = 0.0f, in_x0 = 0.0f, in_x1 = 0.0f;
   auto prefetch = [&](long i2) {
-    const size_t r2 = (size_t)i2;  // = b2 n_int + t2
     const int b2 = (int)(i2 / a.n_int), t2 = (int)(i2 - (long)b2 * a.n_int);
-    const float* sv2 = a.vlsave + r2 * vs;
-    const float* dr2 = a.loc + r2 * LW;
+    const float* sv2 = a.vlsave + (size_t)i2 * vs;
     in_p = sv2[tid];
     in_v = sv2[256 + tid];
-    in_g = a.fl[r2 * 256 + tid];  // dM_t
-    if (dl_own) in_d = reinterpret_cast<const f4*>(sv2 + 512)[tid];
-    if constexpr (N >= 2) in_s2 = dr2[16 + tid];
-    if constexpr (N >= 3) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) in_s3[m] = reinterpret_cast<const f4*>(dr2 + 272)[tid + 256 * m];
-    }
-    if (tid < 16) {
-      in_s1 = dr2[tid];
-      if (tid < a.d) {
-        const float* x = a.path + ((size_t)b2 * a.L + t2) * a.d;
-        in_x0 = x[tid];
-        in_x1 = x[a.d + tid];
-      }
+    in_l = sv2[512 + i];
+    in_g = a.fl[(size_t)i2 * 256 + tid];
+    if (j < a.d) {
+      const float* x = a.path + ((size_t)b2 * a.L + t2) * a.d;
+      in_x0 = x[j];
+      in_x1 = x[a.d + j];
     }
   };
   if (blockIdx.x < total) prefetch(blockIdx.x);
   for (long it = blockIdx.x; it < total; it += gridDim.x) {
     const int b = (int)(it / a.n_int), t = (int)(it - (long)b * a.n_int);
     const float* th = a.clock + (size_t)b * a.L;
-    const float in_w = (tid < 16 && tid < a.d) ? (in_x1 - in_x0) / (float)Mv : 0.0f;
     bool fixed = false;  // delta = 0: P = V = I (the jump / basepoint interval), no dependence on A or the clock
     float delta;
     if (a.vl_mode == EWS_FLOW_PER_INTERVAL) {
@@ -2247,176 +2501,11 @@ __global__ __launch_bounds__(256) void k_vl_bwd(Args a, LeafBwd o) {
       delta = vl_shared_step(a, th);
       fixed = delta == 0.0f || (a.vl_mode == EWS_FLOW_CACHED_BASEPOINT && t == 0);
     }
-    Pm[tid] = in_p;
     Vm[tid] = in_v;
-    if (dl_own) reinterpret_cast<f4*>(U)[tid] = in_d;  // Dl[m][c] at U[16 m + c]
-    if (tid < 16) {
-      wv[tid] = in_w;
-      dS1[tid] = in_s1;
-    }
-    if constexpr (N >= 2) dS2[tid] = in_s2;
-    if constexpr (N >= 3) {
-#pragma unroll
-      for (int m = 0; m < 4; ++m) reinterpret_cast<f4*>(dS3)[tid + 256 * m] = in_s3[m];
-    }
+    GPm[tid] = in_p;
+    GVm[tid] = in_l * ((in_x1 - in_x0) / (float)Mv);
     Gm[tid] = in_g;
-    __syncthreads();
-    {  // Pre, R, Y, X; level-1 cotangent; zero the other accumulators. 16 lanes per column, a segment of
-       // ceil(M / 16) knots each: the segments' sums scanned across the lanes, then each lane walks its segment
-      const int col = tid >> 4, seg = tid & 15, S = (Mv + 15) >> 4, m0 = min(Mv, seg * S), m1 = min(Mv, m0 + S);
-      float own = 0.0f;
-      for (int m = m0; m < m1; ++m) own += Dl[m][col];
-      float inc = own;
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        const float v = __shfl_up(inc, o, 16);
-        if (seg >= o) inc += v;
-      }
-      const float total = __shfl(inc, 15, 16);
-      float pre = inc - own, suf = total - inc;
-      for (int m = m0; m < m1; ++m) {
-        const float dm = Dl[m][col];
-        Ys[m][col] = fmaf(0.5f, dm, pre);
-        Xs[m][col] = fmaf(1.0f / 3.0f, dm, pre);
-        pre += dm;
-        dD[m][col] = dS1[col];
-        dP[m][col] = 0.0f;
-        dR[m][col] = 0.0f;
-      }
-      for (int m = m1 - 1; m >= m0; --m) {  // R_m: the knots after m
-        Rs[m][col] = suf;
-        suf += Dl[m][col];
-      }
-    }
-    __syncthreads();
-    // ---- level adjoints
-    if constexpr (N >= 2) {
-      for (int e = tid; e < Mv * 16; e += 256) {  // dY_m = dS2 Delta_m;  dDelta_m += dS2^T Y_m
-        const int m = e >> 4, r = e & 15;
-        float y1 = 0.0f, y2 = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          y1 = fmaf(dS2[r * 16 + k], Dl[m][k], y1);
-          y2 = fmaf(dS2[k * 16 + r], Ys[m][k], y2);
-        }
-        dP[m][r] += y1;
-        dD[m][r] += fmaf(0.5f, y1, y2);
-      }
-      __syncthreads();
-    }
-    if constexpr (N >= 3) {
-      float colb[16];  // dS3[i][.][j]
-      f4 rowc[4];      // dS3[i][j][.]
-#pragma unroll
-      for (int k = 0; k < 16; ++k) colb[k] = dS3[i * 256 + k * 16 + j];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) rowc[k] = *reinterpret_cast<const f4*>(dS3 + i * 256 + j * 16 + 4 * k);
-      for (int mb = 0; mb < Mv; mb += VB) {
-      const int me = min(Mv, mb + VB);
-      for (int m = mb; m < me; ++m) {
-        // the knot's Delta_m and R_m: the same 16 floats in every lane (broadcast float4 reads)
-        float q = 0.0f, e1 = 0.0f, f1 = 0.0f;
-#pragma unroll
-        for (int k4 = 0; k4 < 4; ++k4) {
-          const f4 dk = *reinterpret_cast<const f4*>(&Dl[m][4 * k4]);
-          const f4 rk = *reinterpret_cast<const f4*>(&Rs[m][4 * k4]);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            q = fmaf(colb[4 * k4 + c], dk[c], q);
-            e1 = fmaf(rowc[k4][c], rk[c], e1);
-            f1 = fmaf(rowc[k4][c], dk[c], f1);
-          }
-        }
-        const float yi = Ys[m][i], xi = Xs[m][i];
-        // over the last index (lanes j of a row i): dY_m[i], dX_m[i]
-        float py = q * Rs[m][j], px = 0.5f * q * Dl[m][j];
-        py = lanes::sum16(py);
-        px = lanes::sum16(px);
-        // over the first index (rows i of the wave, then the four wavefronts' partials in a fixed order):
-        // dR_m[j], dDelta_m[j]
-        float pr2 = q * yi, pd = fmaf(0.5f * q, xi, fmaf(yi, e1, 0.5f * xi * f1));
-        pr2 = lanes::add_xor32(lanes::add_xor16(pr2));
-        pd = lanes::add_xor32(lanes::add_xor16(pd));
-        const int sb = m - mb;
-        if (j == 0) {  // row i lives in one wavefront: a single writer
-          dP[m][i] += py + px;
-          rowD[sb][i] = fmaf(0.5f, py, px * (1.0f / 3.0f));
-        }
-        if (l < 16) {
-          wR[sb][wv_id][j] = pr2;
-          wD[sb][wv_id][j] = pd;
-        }
-      }
-      __syncthreads();
-      {  // the block's partials: thread (knot mb + tid / 16, column tid % 16)
-        const int sb = tid >> 4, c = tid & 15;
-        if (sb < me - mb) {
-          const int m = mb + sb;
-          dR[m][c] += ((wR[sb][0][c] + wR[sb][1][c]) + wR[sb][2][c]) + wR[sb][3][c];
-          dD[m][c] += rowD[sb][c] + (((wD[sb][0][c] + wD[sb][1][c]) + wD[sb][2][c]) + wD[sb][3][c]);
-        }
-      }
-      __syncthreads();  // before the next block's partials
-      }
-    }
-    if (it + gridDim.x < total) prefetch(it + gridDim.x);  // the next interval's inputs
-    // Pre and R -> Delta (dP holds dPre): dDelta_m += sum_{m' > m} dPre_m' + sum_{m' < m} dR_m', segments as above
-    {
-      const int col = tid >> 4, seg = tid & 15, S = (Mv + 15) >> 4, m0 = min(Mv, seg * S), m1 = min(Mv, m0 + S);
-      float ownP = 0.0f, ownR = 0.0f;
-      for (int m = m0; m < m1; ++m) {
-        ownP += dP[m][col];
-        ownR += dR[m][col];
-      }
-      float incP = ownP, incR = ownR;
-#pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        const float vp = __shfl_up(incP, o, 16), vr = __shfl_up(incR, o, 16);
-        if (seg >= o) {
-          incP += vp;
-          incR += vr;
-        }
-      }
-      float accP = __shfl(incP, 15, 16) - incP, accR = incR - ownR;
-      for (int m = m1 - 1; m >= m0; --m) {
-        dD[m][col] += accP;
-        accP += dP[m][col];
-      }
-      for (int m = m0; m < m1; ++m) {
-        dD[m][col] += accR;
-        accR += dR[m][col];
-      }
-      if (seg == 0) lam[col] = dD[0][col];
-    }
-    __syncthreads();
-    // ---- the chain in reverse, one wavefront
-    if (tid < 64) {
-      f4 pc;  // P[4g + r][c16]
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pc[r] = Pm[(4 * g + r) * 16 + c16];
-      const int gi = l >> 2, gj = 4 * (l & 3);
-      f4 gp = {0.0f, 0.0f, 0.0f, 0.0f};
-      for (int m = 1; m < Mv; ++m) {
-        const f4 lv = *reinterpret_cast<const f4*>(lam + 4 * g);
-        const float li = lam[gi];
-        const f4 dm = *reinterpret_cast<const f4*>(&Dl[m][gj]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) gp[r] = fmaf(li, dm[r], gp[r]);
-        float u = fmaf(pc.x, lv.x, fmaf(pc.y, lv.y, fmaf(pc.z, lv.z, pc.w * lv.w)));
-        u = lanes::add_xor32(lanes::add_xor16(u));
-        wave_order_d();
-        if (g == 0) lam[c16] = dD[m][c16] + u;
-        wave_order_d();
-      }
-      *reinterpret_cast<f4*>(GPm + 4 * l) = gp;
-    }
-    __syncthreads();
-    GVm[tid] = lam[i] * wv[j];
-    {
-      float u = Vm[j * 16 + i] * lam[j];  // (V^T lambda)[i]
-      u = lanes::sum16(u);
-      if (j == 0) o.dv[((size_t)b * a.n_int + t) * 16 + i] = u / (float)Mv;
-    }
+    if (it + gridDim.x < total) prefetch(it + gridDim.x);
     __syncthreads();
     // ---- step matrices' adjoint
     float ddelta = 0.0f;
@@ -3467,9 +3556,23 @@ int dense_leaf_adjoint(const ews_dense_desc* desc, const DPlan& p, const Args& a
     else hipLaunchKernelGGL((KER<NN, false>), dim3(grid), dim3(256), lshm, st, a, o);                        \
   } while (0)
   if (p.leaf == EWS_LEAF_VAN_LOAN) {
-    if (p.N == 1) EWS_LEAF_BWD(k_vl_bwd, 1);
-    else if (p.N == 2) EWS_LEAF_BWD(k_vl_bwd, 2);
-    else EWS_LEAF_BWD(k_vl_bwd, 3);
+    const size_t kshm = (size_t)4 * vlk_wave(p.vm) * 4, mshm = p.vl_expm == EWS_EXPM_EXACT ? (size_t)SQMAX * 1024 : 0;
+    const int kgrid = (int)((total + 3) / 4 < 512 ? (total + 3) / 4 : 512);  // two workgroups per CU
+#define EWS_VL_KNOTS(NN)                                                                                            \
+  do {                                                                                                              \
+    if (kshm > 65536 &&                                                                                             \
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_vl_knots_bwd<NN>),                                     \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kshm) != hipSuccess)                    \
+      return EWS_ERR_LAUNCH;                                                                                        \
+    hipLaunchKernelGGL((k_vl_knots_bwd<NN>), dim3(kgrid), dim3(256), kshm, st, a, o);                                \
+  } while (0)
+    if (p.N == 1) EWS_VL_KNOTS(1);
+    else if (p.N == 2) EWS_VL_KNOTS(2);
+    else EWS_VL_KNOTS(3);
+#undef EWS_VL_KNOTS
+    DENSE_CHECK();
+    if (p.chen_expm == EWS_EXPM_EXACT) hipLaunchKernelGGL(k_vl_mats_bwd<true>, dim3(grid), dim3(256), mshm, st, a, o);
+    else hipLaunchKernelGGL(k_vl_mats_bwd<false>, dim3(grid), dim3(256), mshm, st, a, o);
   } else {
     if (p.N == 1) EWS_LEAF_BWD(k_leaf_bwd, 1);
     else if (p.N == 2) EWS_LEAF_BWD(k_leaf_bwd, 2);
