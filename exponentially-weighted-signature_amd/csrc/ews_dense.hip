@@ -1681,12 +1681,11 @@ __device__ __forceinline__ float block_sum(float v, float* red, int tid) {
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// Adjoint of E = exp(-c A) and Phi = phi(-c A) as the kernels evaluate them (wave_expm / series_mats: Taylor
-// polynomials of degree PM in y = -c / 2^s, then s doublings E <- E E, Phi <- (Phi + Phi E) / 2). GE and GPhi
-// (GPhi may be null) are the cotangents in LDS, overwritten. Adds the cotangents of the powers A^p to H (entry
-// tid) and returns the cotangent of c. Esq, Fsq: SQMAX matrices of LDS each (Fsq unused without GPhi).
-__device__ float block_exp_adjoint(const LdsTable* sp, float norm1, float c, float* GE, float* GPhi,
-                                   float (*Esq)[256], float (*Fsq)[256], float* red, float* H, int tid) {
+// Adjoint of E = exp(-c A) as the kernels evaluate it (wave_expm: a Taylor polynomial of degree PM in y = -c / 2^s, then
+// s doublings E <- E E). GE is the cotangent in LDS, overwritten. Adds the cotangents of the powers A^p to H (entry tid)
+// and returns the cotangent of c. Esq: SQMAX matrices of LDS.
+__device__ float block_exp_adjoint(const LdsTable* sp, float norm1, float c, float* GE, float (*Esq)[256], float* red,
+                                   float* H, int tid) {
   const int i = tid >> 4, j = tid & 15;
   int s = 0;
   float x = fabsf(c) * norm1;
@@ -1695,56 +1694,37 @@ __device__ float block_exp_adjoint(const LdsTable* sp, float norm1, float c, flo
     ++s;
   }
   const float y = -c * ldexpf(1.0f, -s);
-  float e = sp[PM][tid], f = e * (1.0f / (float)(PM + 1));
+  float e = sp[PM][tid];
 #pragma unroll
-  for (int p = PM - 1; p >= 0; --p) {
-    e = fmaf(e, y, sp[p][tid]);
-    f = fmaf(f, y, sp[p][tid] * (1.0f / (float)(p + 1)));
-  }
-  if (s > 0) {
-    Esq[0][tid] = e;
-    if (GPhi) Fsq[0][tid] = f;
-  }
+  for (int p = PM - 1; p >= 0; --p) e = fmaf(e, y, sp[p][tid]);
+  if (s > 0) Esq[0][tid] = e;
   __syncthreads();
   for (int r = 1; r < s; ++r) {
-    float e2 = 0.0f, f2 = 0.0f;
+    float e2 = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const float ekj = Esq[r - 1][k * 16 + j];
-      e2 = fmaf(Esq[r - 1][i * 16 + k], ekj, e2);
-      if (GPhi) f2 = fmaf(Fsq[r - 1][i * 16 + k], ekj, f2);
-    }
+    for (int k = 0; k < 16; ++k) e2 = fmaf(Esq[r - 1][i * 16 + k], Esq[r - 1][k * 16 + j], e2);
     Esq[r][tid] = e2;
-    if (GPhi) Fsq[r][tid] = 0.5f * (Fsq[r - 1][tid] + f2);
     __syncthreads();
   }
-  for (int r = s - 1; r >= 0; --r) {
-    // E' = E E, Phi' = (Phi + Phi E) / 2:  GE <- GE' E^T + E^T GE' + Phi^T GPhi' / 2,  GPhi <- (GPhi' + GPhi' E^T) / 2
-    float ge = 0.0f, gf = 0.0f, gfe = 0.0f;
+  for (int r = s - 1; r >= 0; --r) {  // E' = E E:  GE <- GE' E^T + E^T GE'
+    float ge = 0.0f;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       ge = fmaf(GE[i * 16 + k], Esq[r][j * 16 + k], ge);
       ge = fmaf(Esq[r][k * 16 + i], GE[k * 16 + j], ge);
-      if (GPhi) {
-        gf = fmaf(Fsq[r][k * 16 + i], GPhi[k * 16 + j], gf);
-        gfe = fmaf(GPhi[i * 16 + k], Esq[r][j * 16 + k], gfe);
-      }
     }
-    const float gp = GPhi ? GPhi[tid] : 0.0f;
     __syncthreads();
-    GE[tid] = fmaf(0.5f, gf, ge);
-    if (GPhi) GPhi[tid] = 0.5f * (gp + gfe);
+    GE[tid] = ge;
     __syncthreads();
   }
-  const float g0 = GE[tid], p0 = GPhi ? GPhi[tid] : 0.0f;
+  const float g0 = GE[tid];
   float yp = 1.0f, ifact = 1.0f, dy = 0.0f, ypm1 = 1.0f;  // ifact = 1/p! (compile-time constants)
 #pragma unroll
   for (int p = 0; p < HP; ++p) {
     if (p) ifact *= 1.0f / (float)p;
-    const float gsum = g0 + p0 * (1.0f / (float)(p + 1));
-    H[p] = fmaf(yp * ifact, gsum, H[p]);
+    H[p] = fmaf(yp * ifact, g0, H[p]);
     if (p) {
-      dy = fmaf((float)p * ypm1 * sp[p][tid], gsum, dy);
+      dy = fmaf((float)p * ypm1 * sp[p][tid], g0, dy);
       ypm1 *= y;
     }
     yp *= y;
@@ -1753,16 +1733,16 @@ __device__ float block_exp_adjoint(const LdsTable* sp, float norm1, float c, flo
 }
 
 // Adjoint of the rational schemes' matrices (wave_matfn): V = N^{-1}, N = I + alpha A + beta A^2, and P = 2V - I
-// (cayley), V (euler), I - c V A (pade), with (alpha, beta) = (c/2, 0), (c, 0), (c/2, c^2/12). V, GP and GV (GV may
-// be null) in LDS; dN = -V^T GV' V^T for the total cotangent GV' of V. Adds the direct dA terms to dAl (entry tid)
+// (cayley), V (euler), I - c V A (pade), with (alpha, beta) = (c/2, 0), (c, 0), (c/2, c^2/12). V and GP in LDS;
+// dN = -V^T GV' V^T for the total cotangent GV' of V. Adds the direct dA terms to dAl (entry tid)
 // and returns the cotangent of c. W1, W2: 256 floats of LDS scratch each.
 __device__ float block_rational_adjoint(const LdsTable* sp, int scheme, float c, const float* V, const float* GP,
-                                        const float* GV, float* W1, float* W2, float* red, float& dAl, int tid) {
+                                        float* W1, float* W2, float* red, float& dAl, int tid) {
   const int i = tid >> 4, j = tid & 15;
   const float* A = sp[1];
-  float gv = GV ? GV[tid] : 0.0f, dc = 0.0f;
-  if (scheme == EWS_EXPM_CAYLEY) gv = fmaf(2.0f, GP[tid], gv);
-  else if (scheme == EWS_EXPM_EULER) gv += GP[tid];
+  float gv = 0.0f, dc = 0.0f;
+  if (scheme == EWS_EXPM_CAYLEY) gv = 2.0f * GP[tid];
+  else if (scheme == EWS_EXPM_EULER) gv = GP[tid];
   else {  // pade: P = I - c V A
     float gpa = 0.0f, vtg = 0.0f, va = 0.0f;
 #pragma unroll
@@ -1813,14 +1793,14 @@ __device__ float block_flow_adjoint(const Args& a, const LdsTable* sp, float nor
                                    float (*Esq)[256], float* W1, float* W2, float* W3, float* red, float* H,
                                    float& dAl, int tid) {
   if (ident) return 0.0f;
-  if (a.chen_expm == EWS_EXPM_EXACT) return block_exp_adjoint(sp, norm1, hf, G, nullptr, Esq, Esq, red, H, tid);
+  if (a.chen_expm == EWS_EXPM_EXACT) return block_exp_adjoint(sp, norm1, hf, G, Esq, red, H, tid);
   if (a.chen_expm == EWS_EXPM_EULER) {  // M = I - hf A
     dAl = fmaf(-hf, G[tid], dAl);
     return block_sum(-G[tid] * sp[1][tid], red, tid);
   }
   if (tid < 64) wave_matfn(sp, norm1, a.chen_expm, hf, false, W1, W2, W3, tid);  // V (and P, unused) of the step
   __syncthreads();
-  return block_rational_adjoint(sp, a.chen_expm, hf, W2, G, nullptr, W1, W3, red, dAl, tid);
+  return block_rational_adjoint(sp, a.chen_expm, hf, W2, G, W1, W3, red, dAl, tid);
 }
 
 // Coefficient of a letter from its stage's base (series-leaf adjoint): b_{a+m} = c P_m b_a with
@@ -2121,7 +2101,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
     // ---- flow adjoint
     bool ident = false;
     const float hf = a.flow_mode == EWS_FLOW_PER_INTERVAL ? h : flow_step(a, th, t, ident);
-    const float dhf = EXACTF ? (ident ? 0.0f : block_exp_adjoint(sp, norm1, hf, Gm, nullptr, Esq, Esq, red, H, tid))
+    const float dhf = EXACTF ? (ident ? 0.0f : block_exp_adjoint(sp, norm1, hf, Gm, Esq, red, H, tid))
                              : block_flow_adjoint(a, sp, norm1, hf, ident, Gm, Esq, W1, W2, W3, red, H, dAl, tid);
     // ---- outputs
     if (tid < 16) o.dv[((size_t)b * a.n_int + t) * 16 + tid] = dB[0][tid];
@@ -2160,8 +2140,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
 //   chain: lambda_0 = dDelta_0, lambda_m = dDelta_m + P^T lambda_{m-1},
 //   GP = sum_m lambda_{m-1} (x) Delta_m, GV = lambda_{M-1} (x) w, dw = V^T lambda_{M-1}, dv = dw / M.
 // k_vl_knots_bwd does this with a wavefront per interval (no workgroup barrier); it leaves GP over the saved P and
-// lambda_{M-1} over the first saved knot for k_vl_mats_bwd: the adjoints of the step matrices (block_exp_adjoint or
-// block_rational_adjoint, for the step delta = h / M) and of the flow, a workgroup per interval.
+// lambda_{M-1} over the first saved knot for k_vl_mats_bwd: the adjoints of the step matrices (for the step delta = h / M)
+// and of the flow.
 //
 // Depth 3 is three contractions of the 16 KB dS3 with the knots, on fp32 MFMA over tiles of 16 knots (rows m; up to 8
 // knots past the last full tile in quads, v_mfma_f32_4x4x1_16b, whose blocks split the contraction over the lane groups
@@ -2169,7 +2149,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
 // index c, Q^c[m][a] (the first one again, for sums over c that then need no lane exchange). Each reads dS3 in its own
 // order into 64 registers, loaded one contraction ahead (the second and third time from the caches). One workgroup per
 // interval, with these sums on the vector units and behind barriers, left 2 workgroups per CU: B = 16, L = 4096, d = 16,
-// M = 20, 2434 us (this kernel and k_vl_mats_bwd: 662 + 506).
+// M = 20, 2434 us (this kernel and k_vl_mats_bwd: 662 + 143).
 
 
 __host__ __device__ constexpr int vlk_rows(int M) { return (M & 15) > 8 ? (M + 15) / 16 * 16 : (M + 3) / 4 * 4; }
@@ -2453,44 +2433,191 @@ __global__ __launch_bounds__(256, 2) void k_vl_knots_bwd(Args a, LeafBwd o) {
   }
 }
 
-// One workgroup per interval, grid-stride. exact: the knots' scheme is the exponential (Fsq in dynamic LDS).
-template <bool EXACTF>  // EXACTF: exact flows (the other schemes' code is left out)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 : 1))) void k_vl_mats_bwd(Args a,
-                                                                                                      LeafBwd o) {
+// The adjoints of the matrix functions with a wavefront per interval. A 16 x 16 matrix X is held four entries a lane
+// ("own": X[c16][4g .. 4g + 3]) or, for the other operand of a product, as X[4g + s][c16], s = 0..3 ("tr"; from own
+// through an LDS slot of pitch TP). own(X Y) = wave_mul(own(X), tr(Y)), and since own and tr exchange under transposition
+// a transposed factor costs nothing: own(X Y^T) = wave_mul(own(X), own(Y)), own(X^T Y) = wave_mul(tr(X), tr(Y)).
+constexpr int TP = 20, TSL = 16 * TP;
+constexpr int SQK = 4;  // squarings kept in LDS; the matrices of later ones (|c| ||A||_1 > 2^SQK) are formed again
+__device__ __forceinline__ f4 wave_mul(f4 x, f4 y) {
+  f4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) z = mfma(y[s], x[s], z);
+  return z;
+}
+__device__ __forceinline__ f4 slot_own(const float* q, int g, int c16) {
+  return *reinterpret_cast<const f4*>(q + c16 * TP + 4 * g);
+}
+__device__ __forceinline__ f4 slot_tr(const float* q, int g, int c16) {
+  return f4{q[(4 * g) * TP + c16], q[(4 * g + 1) * TP + c16], q[(4 * g + 2) * TP + c16], q[(4 * g + 3) * TP + c16]};
+}
+__device__ __forceinline__ f4 slot_put(float* q, f4 x, int g, int c16) {  // returns tr(x)
+  wave_order_d();
+  *reinterpret_cast<f4*>(q + c16 * TP + 4 * g) = x;
+  wave_order_d();
+  return slot_tr(q, g, c16);
+}
+
+// block_exp_adjoint for one wavefront, with PHI for Phi = phi(-c A) as well (Phi <- (Phi + Phi E) / 2 in a doubling): GE,
+// GPhi own; H own entries of the powers' cotangents. q: SQK + 2 slots, with PHI 2 SQK + 4.
+template <bool PHI>
+__device__ __forceinline__ float wave_exp_adjoint(const LdsTable* sp, float norm1, float c, f4 GE, f4 GPhi, float* q, f4* H,
+                                                  int g, int c16) {
+  const int ow = c16 * 16 + 4 * g;
+  float* const sc = q + SQK * TSL;  // scratch of the squarings formed again
+  float* const gs = sc + TSL;
+  float* const fq = gs + TSL;
+  int s = 0;
+  float x = fabsf(c) * norm1;
+  while (x > 1.0f && s < SQMAX) {
+    x *= 0.5f;
+    ++s;
+  }
+  const float y = -c * ldexpf(1.0f, -s);
+  if (s > 0) {
+    f4 e = *reinterpret_cast<const f4*>(&sp[PM][ow]), f = e * (1.0f / (float)(PM + 1));
+#pragma unroll
+    for (int p = PM - 1; p >= 0; --p) {
+      const f4 t = *reinterpret_cast<const f4*>(&sp[p][ow]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        e[r] = fmaf(e[r], y, t[r]);
+        if (PHI) f[r] = fmaf(f[r], y, t[r] * (1.0f / (float)(p + 1)));
+      }
+    }
+    const int kept = min(s, SQK);
+    for (int r = 0; r < kept; ++r) {
+      const f4 et = slot_put(q + r * TSL, e, g, c16);
+      if (PHI) slot_put(fq + r * TSL, f, g, c16);
+      if (r + 1 < kept) {
+        if (PHI) f = 0.5f * (f + wave_mul(f, et));
+        e = wave_mul(e, et);
+      }
+    }
+    for (int r = s - 1; r >= 0; --r) {
+      const int k = min(r, SQK - 1);
+      f4 eo = slot_own(q + k * TSL, g, c16), et = slot_tr(q + k * TSL, g, c16), fo = eo, ft = et;
+      if (PHI) {
+        fo = slot_own(fq + k * TSL, g, c16);
+        ft = slot_tr(fq + k * TSL, g, c16);
+      }
+      for (int m = k; m < r; ++m) {
+        if (PHI) {
+          fo = 0.5f * (fo + wave_mul(fo, et));
+          ft = slot_put(fq + SQK * TSL, fo, g, c16);
+        }
+        eo = wave_mul(eo, et);
+        et = slot_put(sc, eo, g, c16);
+      }
+      // E' = E E, Phi' = (Phi + Phi E) / 2:  GE <- GE' E^T + E^T GE' + Phi^T GPhi' / 2,  GPhi <- (GPhi' + GPhi' E^T) / 2
+      const f4 gt = slot_put(gs, GE, g, c16);
+      GE = wave_mul(GE, eo) + wave_mul(et, gt);
+      if (PHI) {
+        const f4 pt = slot_put(fq + (SQK + 1) * TSL, GPhi, g, c16);
+        GE += 0.5f * wave_mul(ft, pt);
+        GPhi = 0.5f * (GPhi + wave_mul(GPhi, eo));
+      }
+    }
+  }
+  float yp = 1.0f, ifact = 1.0f, dy = 0.0f, ypm1 = 1.0f;  // ifact = 1/p! (compile-time constants)
+#pragma unroll
+  for (int p = 0; p < HP; ++p) {
+    if (p) ifact *= 1.0f / (float)p;
+    f4 gsum = GE;
+    if (PHI) gsum += GPhi * (1.0f / (float)(p + 1));
+    const float hc = yp * ifact;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) H[p][r] = fmaf(hc, gsum[r], H[p][r]);
+    if (p) {
+      const f4 t = *reinterpret_cast<const f4*>(&sp[p][ow]);
+      const float w = (float)p * ypm1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dy = fmaf(w * t[r], gsum[r], dy);
+      ypm1 *= y;
+    }
+    yp *= y;
+  }
+  return -lanes::sum64(dy) * ldexpf(1.0f, -s);
+}
+
+// block_rational_adjoint for one wavefront: V own (vo) and tr (vt), GP and GV own, one slot.
+__device__ __forceinline__ float wave_rational_adjoint(const LdsTable* sp, int scheme, float c, f4 vo, f4 vt, f4 GP, f4 GV,
+                                                       float* gs, f4& dAl, int g, int c16) {
+  const f4 ao = *reinterpret_cast<const f4*>(&sp[1][c16 * 16 + 4 * g]);
+  f4 gv = GV, at = ao;
+  float dc = 0.0f;
+  if (scheme == EWS_EXPM_CAYLEY) gv += 2.0f * GP;
+  else if (scheme == EWS_EXPM_EULER) gv += GP;
+  else {  // pade: P = I - c V A
+#pragma unroll
+    for (int s = 0; s < 4; ++s) at[s] = sp[1][(4 * g + s) * 16 + c16];
+    gv -= c * wave_mul(GP, ao);
+    dAl -= c * wave_mul(vt, slot_put(gs, GP, g, c16));
+    const f4 va = wave_mul(vo, at);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dc -= GP[r] * va[r];
+  }
+  const f4 xv = wave_mul(vt, slot_put(gs, gv, g, c16));  // V^T GV'
+  f4 dN = wave_mul(xv, vo);                              // (V^T GV') V^T
+  dN = -dN;
+  const bool pade = scheme == EWS_EXPM_PADE;
+  const float alpha = scheme == EWS_EXPM_EULER ? c : 0.5f * c, dalpha = scheme == EWS_EXPM_EULER ? 1.0f : 0.5f;
+  const f4 a2 = *reinterpret_cast<const f4*>(&sp[2][c16 * 16 + 4 * g]);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    dAl[r] = fmaf(alpha, dN[r], dAl[r]);
+    dc = fmaf(dN[r], dalpha * ao[r] + (pade ? c * (1.0f / 6.0f) * 2.0f * a2[r] : 0.0f), dc);
+  }
+  if (pade) {  // beta (dN A^T + A^T dN), beta = c^2 / 12
+    const f4 t2 = wave_mul(dN, ao) + wave_mul(at, slot_put(gs, dN, g, c16));
+    dAl += (c * c * (1.0f / 12.0f)) * t2;
+  }
+  return lanes::sum64(dc);
+}
+
+__host__ __device__ constexpr int vlm_wave(bool phi) { return (phi ? 2 * SQK + 4 : SQK + 2) * TSL; }
+
+// Adjoints of the Van Loan step matrices and of the flow, a wavefront per interval; PHI: the knots' scheme is the
+// exponential, EXACTF: the flows' is (the other schemes' code is left out). The matrices stay in registers and meet in
+// MFMA products; a workgroup per interval (a barrier or two per product, its sums on the vector units) took 506 us at
+// B = 16, L = 4096, d = 16 with exact flows and cayley knots, this 143.
+template <bool PHI, bool EXACTF>
+__global__ __launch_bounds__(256, EXACTF && !PHI ? 3 : 2) void k_vl_mats_bwd(Args a, LeafBwd o) {
   extern __shared__ __align__(16) float lds[];
-  typedef float Mat[256];
-  __shared__ __align__(16) float sp[HP][256];
-  __shared__ __align__(16) float Vm[256], W1[256], W2[256], W3[256 + 32], GPm[256], GVm[256], Gm[256];
-  __shared__ __align__(16) float Esq[SQMAX][256];
-  __shared__ float red[8];
-  Mat* Fsq = reinterpret_cast<Mat*>(lds);
-  const int tid = threadIdx.x, i = tid >> 4, j = tid & 15;
+  LdsTable* sp = reinterpret_cast<LdsTable*>(lds);  // HP tables; at the end HP + 1 sums
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, c16 = l & 15, ow = c16 * 16 + 4 * g;
+  float* q = lds + (HP + 1) * 256 + w * vlm_wave(PHI);
   const int Mv = a.vm, vs = 512 + 16 * Mv;
-#pragma unroll
-  for (int p = 0; p < HP; ++p) sp[p][tid] = a.apow[p * 256 + tid];
+  stage_lds(lds, a.apow, HP * 256, tid, blockDim.x);
   const float norm1 = a.apow[a.npow * 256];
-  float H[HP];
+  f4 H[HP], dAl = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int p = 0; p < HP; ++p) H[p] = 0.0f;
-  float dAl = 0.0f;
-  const long total = (long)a.B * a.n_int;
-  // the interval's inputs, loaded during the one before: GP, V, dM, lambda[i], the increment's coordinate j
-  float in_p = 0.0f, in_v = 0.0f, in_g = 0.0f, in_l = 0.0f, in_x0 = 0.0f, in_x1 = 0.0f;
+  for (int p = 0; p < HP; ++p) H[p] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  __syncthreads();
+  const long total = (long)a.B * a.n_int, first = (long)blockIdx.x * 4 + w, stride = (long)gridDim.x * 4;
+  // the interval's inputs, loaded during the one before: GP, V (own and tr), dM, lambda[c16], the increment's
+  // coordinates 4g .. 4g + 3
+  f4 in_p, in_v, in_vt, in_g, in_x0 = {0.0f, 0.0f, 0.0f, 0.0f}, in_x1 = in_x0;
+  float in_l = 0.0f;
   auto prefetch = [&](long i2) {
     const int b2 = (int)(i2 / a.n_int), t2 = (int)(i2 - (long)b2 * a.n_int);
     const float* sv2 = a.vlsave + (size_t)i2 * vs;
-    in_p = sv2[tid];
-    in_v = sv2[256 + tid];
-    in_l = sv2[512 + i];
-    in_g = a.fl[(size_t)i2 * 256 + tid];
-    if (j < a.d) {
-      const float* x = a.path + ((size_t)b2 * a.L + t2) * a.d;
-      in_x0 = x[j];
-      in_x1 = x[a.d + j];
-    }
+    in_p = *reinterpret_cast<const f4*>(sv2 + ow);
+    in_v = *reinterpret_cast<const f4*>(sv2 + 256 + ow);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) in_vt[s] = sv2[256 + (4 * g + s) * 16 + c16];
+    in_l = sv2[512 + c16];
+    in_g = *reinterpret_cast<const f4*>(a.fl + (size_t)i2 * 256 + ow);
+    const float* x = a.path + ((size_t)b2 * a.L + t2) * a.d;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * g + r < a.d) {
+        in_x0[r] = x[4 * g + r];
+        in_x1[r] = x[a.d + 4 * g + r];
+      }
   };
-  if (blockIdx.x < total) prefetch(blockIdx.x);
-  for (long it = blockIdx.x; it < total; it += gridDim.x) {
+  if (first < total) prefetch(first);
+  for (long it = first; it < total; it += stride) {
     const int b = (int)(it / a.n_int), t = (int)(it - (long)b * a.n_int);
     const float* th = a.clock + (size_t)b * a.L;
     bool fixed = false;  // delta = 0: P = V = I (the jump / basepoint interval), no dependence on A or the clock
@@ -2501,41 +2628,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
       delta = vl_shared_step(a, th);
       fixed = delta == 0.0f || (a.vl_mode == EWS_FLOW_CACHED_BASEPOINT && t == 0);
     }
-    Vm[tid] = in_v;
-    GPm[tid] = in_p;
-    GVm[tid] = in_l * ((in_x1 - in_x0) / (float)Mv);
-    Gm[tid] = in_g;
-    if (it + gridDim.x < total) prefetch(it + gridDim.x);
-    __syncthreads();
-    // ---- step matrices' adjoint
-    float ddelta = 0.0f;
-    if (!fixed) {
-      if (a.vl_expm == EWS_EXPM_EXACT)
-        ddelta = block_exp_adjoint(sp, norm1, delta, GPm, GVm, Esq, Fsq, red, H, tid);
-      else
-        ddelta = block_rational_adjoint(sp, a.vl_expm, delta, Vm, GPm, GVm, W1, W2, red, dAl, tid);
-    }
-    // ---- flow adjoint
     bool ident;
     const float hf = flow_step(a, th, t, ident);
-    const float dhf = EXACTF ? (ident ? 0.0f : block_exp_adjoint(sp, norm1, hf, Gm, nullptr, Esq, Esq, red, H, tid))
-                             : block_flow_adjoint(a, sp, norm1, hf, ident, Gm, Esq, W1, W2, W3, red, H, dAl, tid);
-    if (tid == 0) {
+    const f4 vo = in_v, vt = in_vt, gp = in_p, gm = in_g;
+    f4 gv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gv[r] = in_l * ((in_x1[r] - in_x0[r]) / (float)Mv);
+    if (it + stride < total) prefetch(it + stride);
+    // ---- step matrices' adjoint
+    float ddelta = 0.0f, dhf = 0.0f;
+    if (!fixed) {
+      if constexpr (PHI) ddelta = wave_exp_adjoint<true>(sp, norm1, delta, gp, gv, q, H, g, c16);
+      else ddelta = wave_rational_adjoint(sp, a.vl_expm, delta, vo, vt, gp, gv, q, dAl, g, c16);
+    }
+    // ---- flow adjoint
+    if (!ident) {
+      if constexpr (EXACTF) {
+        dhf = wave_exp_adjoint<false>(sp, norm1, hf, gm, gm, q, H, g, c16);
+      } else if (a.chen_expm == EWS_EXPM_EULER) {  // M = I - hf A
+        const f4 ao = *reinterpret_cast<const f4*>(&sp[1][ow]);
+        dAl -= hf * gm;
+        dhf = -lanes::sum64(gm[0] * ao[0] + gm[1] * ao[1] + gm[2] * ao[2] + gm[3] * ao[3]);
+      } else {
+        float* V = q + TSL;  // V (and P, unused) of the step, pitch 16
+        wave_order_d();
+        wave_matfn(sp, norm1, a.chen_expm, hf, false, q, V, q + 2 * TSL, l);
+        wave_order_d();
+        const f4 fo = *reinterpret_cast<const f4*>(V + ow);
+        const f4 ft = {V[(4 * g) * 16 + c16], V[(4 * g + 1) * 16 + c16], V[(4 * g + 2) * 16 + c16],
+                       V[(4 * g + 3) * 16 + c16]};
+        dhf = wave_rational_adjoint(sp, a.chen_expm, hf, fo, ft, gm, f4{0.0f, 0.0f, 0.0f, 0.0f}, q + 2 * TSL, dAl, g, c16);
+      }
+    }
+    if (l == 0) {
       float dh = 0.0f, s_flow = 0.0f, s_vl = 0.0f;  // shared steps: summed in a fixed order by k_dsh_reduce
       if (a.vl_mode == EWS_FLOW_PER_INTERVAL) dh += ddelta / (float)Mv;
       else if (!fixed) s_vl = ddelta / (float)Mv;
       if (a.flow_mode == EWS_FLOW_PER_INTERVAL) dh += dhf;
       else if (!ident) s_flow = dhf;
-      o.dh[(size_t)b * a.n_int + t] = dh;
-      o.dshi[2 * ((size_t)b * a.n_int + t)] = s_flow;
-      o.dshi[2 * ((size_t)b * a.n_int + t) + 1] = s_vl;
+      o.dh[(size_t)it] = dh;
+      o.dshi[2 * (size_t)it] = s_flow;
+      o.dshi[2 * (size_t)it + 1] = s_vl;
     }
-    __syncthreads();
   }
-  float* pb = o.part + (size_t)blockIdx.x * (HP + 1) * 256;
+  // the wavefronts' sums in order, over the tables
+  for (int k = 0; k < 4; ++k) {
+    __syncthreads();
+    if (w == k) {
 #pragma unroll
-  for (int p = 0; p < HP; ++p) pb[p * 256 + tid] = H[p];
-  pb[HP * 256 + tid] = dAl;
+      for (int p = 0; p <= HP; ++p) {
+        f4* s4 = reinterpret_cast<f4*>(lds + p * 256 + ow);
+        const f4 v = p < HP ? H[p < HP ? p : 0] : dAl;
+        *s4 = k == 0 ? v : *s4 + v;
+      }
+    }
+  }
+  __syncthreads();
+  float* pb = o.part + (size_t)blockIdx.x * (HP + 1) * 256;
+  for (int p = 0; p <= HP; ++p) pb[p * 256 + tid] = lds[p * 256 + tid];
 }
 
 // sums of the workgroups' partials (float64): workgroup (p, c) sums row p of the partial sets c, c + PRS, ...
@@ -3540,7 +3690,7 @@ int dense_leaf_adjoint(const ews_dense_desc* desc, const DPlan& p, const Args& a
   o.dshi = (float*)(ws + w.dshi);
   double* hsum = (double*)(ws + w.hsum);
   const long total = (long)p.B * p.n_int;
-  const int grid = (int)(total < kLeafBwdBlocks ? total : kLeafBwdBlocks);
+  int grid = (int)(total < kLeafBwdBlocks ? total : kLeafBwdBlocks);
   const size_t lshm = p.leaf == EWS_LEAF_VAN_LOAN ? 0 : (size_t)6 * (p.q + 1) * 16 * 4;  // k_leaf_bwd's letters
   const bool bs = p.leaf == EWS_LEAF_BLOCK_SERIES;
   float* bsdv = (float*)(ws + w.bsdv);
@@ -3556,7 +3706,7 @@ int dense_leaf_adjoint(const ews_dense_desc* desc, const DPlan& p, const Args& a
     else hipLaunchKernelGGL((KER<NN, false>), dim3(grid), dim3(256), lshm, st, a, o);                        \
   } while (0)
   if (p.leaf == EWS_LEAF_VAN_LOAN) {
-    const size_t kshm = (size_t)4 * vlk_wave(p.vm) * 4, mshm = p.vl_expm == EWS_EXPM_EXACT ? (size_t)SQMAX * 1024 : 0;
+    const size_t kshm = (size_t)4 * vlk_wave(p.vm) * 4;
     const int kgrid = (int)((total + 3) / 4 < 512 ? (total + 3) / 4 : 512);  // two workgroups per CU
 #define EWS_VL_KNOTS(NN)                                                                                            \
   do {                                                                                                              \
@@ -3571,8 +3721,23 @@ int dense_leaf_adjoint(const ews_dense_desc* desc, const DPlan& p, const Args& a
     else EWS_VL_KNOTS(3);
 #undef EWS_VL_KNOTS
     DENSE_CHECK();
-    if (p.chen_expm == EWS_EXPM_EXACT) hipLaunchKernelGGL(k_vl_mats_bwd<true>, dim3(grid), dim3(256), mshm, st, a, o);
-    else hipLaunchKernelGGL(k_vl_mats_bwd<false>, dim3(grid), dim3(256), mshm, st, a, o);
+    const bool phi = p.vl_expm == EWS_EXPM_EXACT, exf = p.chen_expm == EWS_EXPM_EXACT;
+    const size_t mshm = ((size_t)(HP + 1) * 256 + (size_t)4 * vlm_wave(phi)) * 4;
+    const long mgrid = exf && !phi ? 768 : 512;  // three workgroups per CU, or two
+    grid = (int)((total + 3) / 4 < mgrid ? (total + 3) / 4 : mgrid);
+#define EWS_VL_MATS(PP, EE)                                                                                         \
+  do {                                                                                                              \
+    if (mshm > 65536 &&                                                                                             \
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_vl_mats_bwd<PP, EE>),                                  \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)mshm) != hipSuccess)                    \
+      return EWS_ERR_LAUNCH;                                                                                        \
+    hipLaunchKernelGGL((k_vl_mats_bwd<PP, EE>), dim3(grid), dim3(256), mshm, st, a, o);                              \
+  } while (0)
+    if (phi && exf) EWS_VL_MATS(true, true);
+    else if (phi) EWS_VL_MATS(true, false);
+    else if (exf) EWS_VL_MATS(false, true);
+    else EWS_VL_MATS(false, false);
+#undef EWS_VL_MATS
   } else {
     if (p.N == 1) EWS_LEAF_BWD(k_leaf_bwd, 1);
     else if (p.N == 2) EWS_LEAF_BWD(k_leaf_bwd, 2);
