@@ -1213,8 +1213,8 @@ __global__ __launch_bounds__(N >= 3 ? 256 : 64) void k_scan(Seq s) {
 //   dM = rho_1 (x) S1 + rho_2 M S2^T + rho_2^T M S2 + T1 + T2 + T3,
 // where T1 + T2 + T3 is the derivative of <l_3, M^(x)3 S3> along each tensor axis:
 //   T1 = <l_3 x_3 M^T x_2 M^T, S3>_{23},  T2 = <l_3 x_3 M^T, S3 x_1 M>_{13},  T3 = <l_3, S3 x_1 M x_2 M>_{12}
-// (<X, Y>_{jk}[p][q] contracts the two named axes of X[.., p, ..] and Y[.., q, ..]). S3 of the state is read from
-// its row in global memory (L2-resident), which keeps the workgroup within half of the LDS.
+// (<X, Y>_{jk}[p][q] contracts the two named axes of X[.., p, ..] and Y[.., q, ..]). S3 of the state goes into
+// the LDS that S3 x_1 M then takes, which keeps the workgroup within half of the LDS.
 // Passes: LOCAL (each chunk from lambda = 0: the chunk's own part of the cotangent of its entry state),
 // CARRY (one sample's chunks in reverse, on the chunk summaries: Lambda_c = local_c + R(chunk c)^T Lambda_{c+1}),
 // EMIT (each chunk from Lambda_{c+1}, writing ds_t over the local terms and dM_t over the flows).
@@ -1259,24 +1259,44 @@ __device__ __forceinline__ float adj_g(const AdjSeq& s, int b, int t, int e, int
   return s.amax[(long)b * LWN(N) + e] == t ? s.g[(long)b * s.W + col] : 0.0f;
 }
 
-// The inputs of one adjoint step of thread tid: the flow entry M[tid / 16][tid % 16], the local terms' level 1
-// (tid < 16) and level-2 entry tid, the row added this step (entries tid, 16 + tid and the sixteen level-3 entries
-// 272 + 16 tid + i: the readout cotangent g_t, or for CARRY the chunk's local part), and for EMIT the state before
-// the step (levels 1-2).
-// LDS row of 16 floats (16-byte aligned) += v
-__device__ __forceinline__ void add_row16(float* row, const float* v) {
+// Level 3 of a row (4096 floats) is moved with thread tid taking the float4s 4 tid + 1024 i, i = 0..3: entries
+// (4 i + tid / 64, (tid / 4) % 16, 4 (tid % 4) ..), so that a wavefront's load or store is one contiguous kilobyte. (With
+// sixteen consecutive entries a thread it touched 64 cache lines, and EMIT read the state's level 3 in the step that uses
+// it, by 32 strided loads a lane. B = 16, L = 4096, with the state's row now loaded a step ahead into LDS: EMIT 1479 ->
+// 1256 us; LOCAL, bound by its chain of barriers, stays at 465 to 476.) Rows of W floats have any alignment.
+typedef float f4w __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_level3(const float* row3, int tid, f4* x) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    f4 x = *reinterpret_cast<const f4*>(row + 4 * i);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] += v[4 * i + r];
-    *reinterpret_cast<f4*>(row + 4 * i) = x;
+    const f4w v = *reinterpret_cast<const f4w*>(row3 + 4 * tid + 1024 * i);
+    x[i] = f4{v.x, v.y, v.z, v.w};
   }
 }
+__device__ __forceinline__ float* at_level3(float* m, int tid, int i) {
+  return m + (4 * i + (tid >> 6)) * SP + ((tid >> 2) & 15) * RP + 4 * (tid & 3);
+}
+__device__ __forceinline__ void add_level3(float* m, int tid, const f4* x) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f4* q = reinterpret_cast<f4*>(at_level3(m, tid, i));
+    *q = *q + x[i];
+  }
+}
+__device__ __forceinline__ void store_level3(float* row3, int tid, const float* m) {  // row3: 16-byte aligned
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<f4*>(row3 + 4 * tid + 1024 * i) =
+        *reinterpret_cast<const f4*>(at_level3(const_cast<float*>(m), tid, i));
+}
+
+// The inputs of one adjoint step of thread tid: the flow entry M[tid / 16][tid % 16], the local terms' level 1
+// (tid < 16) and level-2 entry tid, the row added this step (entries tid, 16 + tid and level 3 as above: the readout
+// cotangent g_t, or for CARRY the chunk's local part), and for EMIT the state before the step.
 template <int N, int MODE> struct AdjIn {
   float M, s1, s2, r1, r2;
-  float r3[N >= 3 ? 16 : 1];
+  f4 r3[N >= 3 ? 4 : 1];
   float S1, S2;
+  f4 S3[MODE == ADJ_EMIT && N >= 3 ? 4 : 1];
 };
 template <int N, int MODE>
 __device__ __forceinline__ void adj_load(const AdjSeq& s, int b, int t, int tid, AdjIn<N, MODE>& x) {
@@ -1288,29 +1308,17 @@ __device__ __forceinline__ void adj_load(const AdjSeq& s, int b, int t, int tid,
   if constexpr (N >= 2) x.s2 = lrow[16 + tid];
   x.r1 = x.r2 = 0.0f;
 #pragma unroll
-  for (int i = 0; i < (N >= 3 ? 16 : 1); ++i) x.r3[i] = 0.0f;
+  for (int i = 0; i < (N >= 3 ? 4 : 1); ++i) x.r3[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   if constexpr (MODE == ADJ_CARRY) {
     const float* lo = s.lloc + b * s.lloc_bs + (long)t * LW;
     if (tid < 16) x.r1 = lo[tid];
     if constexpr (N >= 2) x.r2 = lo[16 + tid];
-    if constexpr (N >= 3) {
-      const f4* q = reinterpret_cast<const f4*>(lo + 272 + 16 * tid);  // rows of LW floats: 16-byte aligned
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f4 v = q[i];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x.r3[4 * i + r] = v[r];
-      }
-    }
+    if constexpr (N >= 3) load_level3(lo + 272, tid, x.r3);
   } else if (s.gmode == G_PREFIX && s.d == 16) {  // unpadded rows: the cotangent row is the state layout
     const float* grow = s.g + ((long)b * s.n + t) * s.W + s.glvl0;
     if (tid < 16) x.r1 = grow[tid];
     if constexpr (N >= 2) x.r2 = grow[16 + tid];
-    if constexpr (N >= 3) {
-      const float* q = grow + 272 + 16 * tid;  // any alignment (rows of W floats)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x.r3[i] = q[i];
-    }
+    if constexpr (N >= 3) load_level3(grow + 272, tid, x.r3);
   }  // the other readouts' cotangents (index mapping, mean, max) are read inside the step
   x.S1 = x.S2 = 0.0f;
   if constexpr (MODE == ADJ_EMIT) {
@@ -1318,6 +1326,10 @@ __device__ __forceinline__ void adj_load(const AdjSeq& s, int b, int t, int tid,
       const float* srow = s.st + ((long)b * s.n + t - 1) * s.st_ld;
       if (tid < 16) x.S1 = srow[tid];
       if constexpr (N >= 2) x.S2 = srow[16 + tid];
+      if constexpr (N >= 3) load_level3(srow + 272, tid, x.S3);
+    } else if constexpr (N >= 3) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x.S3[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
   }
 }
@@ -1372,12 +1384,7 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
       if (s.lam && t + 1 < s.lam_lim) {
         if (tid < 16) o[tid] = L1[tid];
         if constexpr (N >= 2) o[16 + tid] = L2[ri * RP + rj];
-        if constexpr (N >= 3) {
-          const float* src = L3 + (tid >> 4) * SP + (tid & 15) * RP;
-          f4* dst = reinterpret_cast<f4*>(o + 272 + 16 * tid);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dst[i] = *reinterpret_cast<const f4*>(src + 4 * i);
-        }
+        if constexpr (N >= 3) store_level3(o + 272, tid, L3);
       }
     }
     // ---- inputs of the step; lambda += g_t
@@ -1388,7 +1395,7 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
       if (s.gmode == G_PREFIX && s.d == 16) {
         if (tid < 16) L1[tid] += cur.r1;
         if constexpr (N >= 2) L2[ri * RP + rj] += cur.r2;
-        if constexpr (N >= 3) add_row16(L3 + (tid >> 4) * SP + (tid & 15) * RP, cur.r3);
+        if constexpr (N >= 3) add_level3(L3, tid, cur.r3);
       } else if (s.gmode != G_NONE) {
         if (tid < 16) L1[tid] += adj_g(s, b, t, tid, N);
         if constexpr (N >= 2) L2[ri * RP + rj] += adj_g(s, b, t, 16 + tid, N);
@@ -1402,21 +1409,9 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
       if (tid < 16) S1s[tid] = cur.S1;
       if constexpr (N >= 2) S2s[ri * RP + rj] = cur.S2;
     }
-    // EMIT, depth 3: the lane's operands of S3 (state before the step) for V1 = S3 x_1 M (s3v) and for T1 (s3t),
-    // issued before the next step's inputs so that their wait does not cover those
-    constexpr int NS3 = EMIT && N >= 3 ? 16 : 1;
-    float s3v[NS3], s3t[NS3];
-    if constexpr (EMIT && N >= 3) {
-      const float* s3g = t > 0 ? s.st + ((long)b * s.n + t - 1) * s.st_ld + 272 : nullptr;
-      // S3[4g + k2][4w + jj][c16] and S3[c16][4w + q / 4][4 (q % 4) + g]: one base each, offsets within 4 KB
-      const float* pv = s3g + (4 * g * 256 + 4 * w * 16 + c16);
-      const float* pt = s3g + (c16 * 256 + 4 * w * 16 + g);
+    if constexpr (EMIT && N >= 3) {  // S3 of the state before the step; B3 was last read before the step's last barriers
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-        for (int k2 = 0; k2 < 4; ++k2) s3v[4 * jj + k2] = s3g ? pv[k2 * 256 + jj * 16] : 0.0f;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) s3t[q] = s3g ? pt[(q >> 2) * 16 + 4 * (q & 3)] : 0.0f;
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<f4*>(at_level3(B3, tid, i)) = cur.S3[i];
     }
     if (MODE != ADJ_CARRY && k > 0) adj_load<N, MODE>(s, b, t - 1, tid, nxt);  // the next step's inputs
     __syncthreads();
@@ -1508,6 +1503,7 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
     // ---- level-3 mode products and the T contractions
     f4 tacc = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (N >= 3) {
+      float s3t[EMIT ? 16 : 1];
       f4 a23[4];
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) {
@@ -1524,13 +1520,15 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
         a23[ii] = y;
       }
       if constexpr (EMIT) {
-        // V1 = S3 x_1 M, tiles j, with S3 read from the state row (L2-resident; zero before the first interval)
+        // V1 = S3 x_1 M, tiles j, in place; the wavefront's S3[c16][4w + q / 4][4 (q % 4) + g] are kept for T1
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s3t[q] = B3[c16 * SP + (4 * w + (q >> 2)) * RP + 4 * (q & 3) + g];
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
           const int j = 4 * w + jj;
           f4 z = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-          for (int k2 = 0; k2 < 4; ++k2) z = mfma(M4[k2], s3v[4 * jj + k2], z);
+          for (int k2 = 0; k2 < 4; ++k2) z = mfma(M4[k2], B3[(4 * g + k2) * SP + j * RP + c16], z);
 #pragma unroll
           for (int r = 0; r < 4; ++r) B3[(4 * g + r) * SP + j * RP + c16] = z[r];
         }
@@ -1573,12 +1571,7 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) Tw[w][(4 * g + r) * 16 + c16] = tacc[r];
         // ds3 = l_3 (the step's cotangent of its level-3 local term); L3 is rewritten after the next barrier
-        {
-          const float* src = L3 + (tid >> 4) * SP + (tid & 15) * RP;
-          f4* dst = reinterpret_cast<f4*>(drow + 272 + 16 * tid);  // padded rows of LW floats: 16-byte aligned
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dst[i] = *reinterpret_cast<const f4*>(src + 4 * i);
-        }
+        store_level3(drow + 272, tid, L3);
       }
       __syncthreads();
       // l_3 <- C3 x_1 M^T (tiles j)
@@ -1630,7 +1623,7 @@ __global__ __launch_bounds__(256, 2) void k_adj(AdjSeq s) {
       __syncthreads();
       if (tid < 16) L1[tid] += cur.r1;
       if constexpr (N >= 2) L2[ri * RP + rj] += cur.r2;
-      if constexpr (N >= 3) add_row16(L3 + (tid >> 4) * SP + (tid & 15) * RP, cur.r3);
+      if constexpr (N >= 3) add_level3(L3, tid, cur.r3);
     }
     __syncthreads();
     cur = nxt;
