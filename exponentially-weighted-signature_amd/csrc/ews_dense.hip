@@ -275,8 +275,10 @@ __global__ __launch_bounds__(256) void k_local(Args a) {
   }
 }
 
-// Depth-3 local terms on MFMA, one wavefront per interval (four per workgroup, grid-stride). The letters come
-// from the recursion b_p = (-h/p) A b_{p-1} (lane (c16, g) holds A[c16][4g .. 4g+3]); the degree-N blocks
+// Depth-3 local terms on MFMA, one wavefront per interval (four per workgroup, grid-stride). The letters come a dozen at
+// a time from the power table and the bt_N from two or three tiles of MFMA: the recursion b_p = (-h/p) A b_{p-1} and the
+// sums over p, letter by letter, were 24 and about 80 dependent LDS round trips an interval (B = 16, L = 4096, q = 24:
+// 648 -> 591 us; rows 5.4e-7 -> 2e-7 off the float64 result). The degree-N blocks
 // g2_N = 1/(N+2) sum_{p <= N} b_p (x) g1_{N-p} are MFMAs with the contraction over p; four degree slices at a
 // time go through LDS and feed the level-3 contraction s3[a][i][j] = sum_N bt_N[a] g2_N[i][j] (one k-step of
 // four degrees per slice set, sixteen output tiles, tile i holding s3[.][i][.]). Rows p > q of the letter
@@ -302,7 +304,6 @@ __global__ __launch_bounds__(256, QB <= 24 ? 3 : 2) void k_local3(Args a) {
   float* G2 = g2b[w];
   for (int e = l; e < QB4 * 16; e += 64) L[e] = G1[e] = 0.0f;
   __syncthreads();
-  const f4 a4 = *reinterpret_cast<const f4*>(&sp[1][c16 * 16 + 4 * g]);  // A[c16][4g .. 4g+3]
   const long total = (long)a.B * a.n_int;
   // the interval's clock values and increment coordinates are loaded one interval ahead into registers, so that no
   // memory round trip sits at the top of an interval
@@ -333,13 +334,24 @@ __global__ __launch_bounds__(256, QB <= 24 ? 3 : 2) void k_local3(Args a) {
       G1[l] = v;
     }
     wave_order_d();
-    for (int pp = 1; pp <= q; ++pp) {
-      const f4 bp = *reinterpret_cast<const f4*>(L + (pp - 1) * 16 + 4 * g);
-      float sm = fmaf(a4.x, bp.x, fmaf(a4.y, bp.y, fmaf(a4.z, bp.z, a4.w * bp.w)));
-      sm = lanes::add_xor32(lanes::add_xor16(sm));
-      const float bv = sm * (-h * inv[pp]);
-      if (g == 0) L[pp * 16 + c16] = bv;
-      if (g == 1) G1[pp * 16 + c16] = bv * inv[pp + 1];
+    // the letters, PM at a time from a base letter: b_{a+m} = (prod_{j=1..m} -h j / (a + j)) P_m b_a, the products of
+    // a stage independent of each other
+    for (int a0 = 0; a0 < q; a0 += PM) {
+      const f4 bp = *reinterpret_cast<const f4*>(L + a0 * 16 + 4 * g);
+      float cf = 1.0f;
+#pragma unroll
+      for (int m = 1; m <= PM; ++m) {
+        const int pp = a0 + m;
+        if (pp <= q) {
+          const f4 pm = *reinterpret_cast<const f4*>(&sp[m][c16 * 16 + 4 * g]);
+          float sm = fmaf(pm.x, bp.x, fmaf(pm.y, bp.y, fmaf(pm.z, bp.z, pm.w * bp.w)));
+          sm = lanes::add_xor32(lanes::add_xor16(sm));
+          cf *= -h * ((float)m * inv[pp]);
+          const float bv = sm * cf;
+          if (g == 0) L[pp * 16 + c16] = bv;
+          if (g == 1) G1[pp * 16 + c16] = bv * inv[pp + 1];
+        }
+      }
       wave_order_d();
     }
     float* row = a.loc + ((size_t)b * a.n_int + t) * a.LW;
@@ -353,13 +365,33 @@ __global__ __launch_bounds__(256, QB <= 24 ? 3 : 2) void k_local3(Args a) {
     for (int i = 0; i < 16; ++i) acc3[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     f4 s2acc = {0.0f, 0.0f, 0.0f, 0.0f};
     const int nks = (q + 4) / 4;  // k-steps that hold a degree <= q
+    // bt_N = sum_{p <= q - N} b_p / (p + N + 3) for all degrees, tiles of 16 N (rows): lane (g, c16) holds
+    // bt_{16 T + 4g + r}[c16]
+    constexpr int NT = (QB + 16) / 16;
+    f4 bt[NT];
+#pragma unroll
+    for (int T = 0; T < NT; ++T) {
+      bt[T] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int kp = 0; 16 * T + 4 * kp <= q; ++kp) {
+        const int pp = 4 * kp + g, N = 16 * T + c16;
+        bt[T] = mfma(pp + N <= q ? inv[pp + N + 3] : 0.0f, L[pp * 16 + c16], bt[T]);
+      }
+    }
 #pragma unroll 1
     for (int ks = 0; ks < nks; ++ks) {
-      // A operand of this level-3 k-step: bt_N[c16] = sum_{p <= q - N} b_p[c16] / (p + N + 3), N = 4 ks + g
+      // A operand of this level-3 k-step: bt_N[c16], N = 4 ks + g
       float btv = 0.0f;
       {
-        const int N = 4 * ks + g;
-        for (int pp = 0; pp + N <= q; ++pp) btv = fmaf(L[pp * 16 + c16], inv[pp + N + 3], btv);
+        f4 x = bt[0];
+#pragma unroll
+        for (int T = 1; T < NT; ++T)
+          if ((ks >> 2) == T) x = bt[T];
+        const int src = 16 * (ks & 3) + c16;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float y = __shfl(x[r], src, 64);
+          if (g == r) btv = y;
+        }
       }
       // the four degrees N = 4 ks + nn as independent accumulators: one letter column b_p (p = 4 kp + g) per
       // k-step serves all four (g1_{N-p} is zero for p > N; degrees above q come out zero)
