@@ -230,26 +230,35 @@ __device__ __forceinline__ f4 ld_seg4(const float* p, int c, int nc, bool ok) {
   return f4{p[c], c + 1 < nc ? p[c + 1] : 0.0f, c + 2 < nc ? p[c + 2] : 0.0f, 0.0f};
 }
 
-template <int N, int NH, int RT>
-__global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
-  constexpr int SEG = 128 / RT, PITCH = SEG + 4, RW = 16 * RT;  // 16-byte LDS rows, 4 banks apart
-  constexpr int NV = RW * SEG / 4 / 64;                         // 16-byte loads per lane per segment
-  __shared__ __align__(16) float s_x[4][RW][PITCH];
+// WL: c_down in LDS in fragment order (per 16 entries of a level and hidden tile, a float4 a lane), staged once by 16
+// wavefronts that walk the row tiles. Loaded from memory where it is used, each fragment waited for the row segment
+// prefetched before it (the memory counter is in order), so only other wavefronts covered a segment's round trip:
+// 399,352 rows, D = 600, hidden 24: 415 -> 308 us. It takes (blocks of 16 entries) x NH KB beside 68 KB of row tiles.
+constexpr int FW_WAVES = 16, FW_SEG = 64;
+__host__ __device__ inline int fw_blocks(const MArgs& a) {
+  int n = 0;
+  for (int k = 0; k < a.N; ++k) n += (a.n[k] + 15) / 16;
+  return n;
+}
+__host__ __device__ inline size_t fw_lds(const MArgs& a, int NH) {
+  return (size_t)fw_blocks(a) * NH * 1024 + (size_t)FW_WAVES * 16 * (FW_SEG + 4) * 4;
+}
+
+template <int N, int NH, int RT, bool WL>
+__global__ __launch_bounds__(WL ? 64 * FW_WAVES : 256) void k_mix_fwd_s(MArgs a) {
+  constexpr int SEG = WL ? FW_SEG : 128 / RT, PITCH = SEG + 4, RW = 16 * RT;  // 16-byte LDS rows, 4 banks apart
+  constexpr int NV = RW * SEG / 4 / 64;                                      // 16-byte loads per lane per segment
+  constexpr int NW = WL ? FW_WAVES : 4;
+  extern __shared__ __align__(16) float s_dyn[];  // the row tiles, then (WL) c_down
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, g = l >> 4;
   const int M = a.B * a.R;
-  const int row0 = (blockIdx.x * 4 + w) * RW;
-  if (row0 >= M) return;  // uniform over the wavefront; no workgroup barrier below
-  float(*sx)[PITCH] = s_x[w];
-  f4 acc[N][NH][RT];
-  float ssq[N][RT];
+  int row0 = (blockIdx.x * NW + w) * RW;
+  float(*sx)[PITCH] = reinterpret_cast<float(*)[PITCH]>(s_dyn + w * RW * PITCH);
+  const float* wl = s_dyn + NW * RW * PITCH;
+  int lb[N];  // a level's first block of 16 entries
+  lb[0] = 0;
 #pragma unroll
-  for (int k = 0; k < N; ++k)
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      ssq[k][rt] = 0.0f;
-#pragma unroll
-      for (int h = 0; h < NH; ++h) acc[k][h][rt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+  for (int k = 1; k < N; ++k) lb[k] = lb[k - 1] + (a.n[k - 1] + 15) / 16;
   // the (level, segment) walk: segment q of level k covers entries [st_k + SEG q, ...)
   auto seg_load = [&](int k, int q, f4 (&v)[NV]) {
     const int base = a.lvl0 + a.st[k] + SEG * q, nc = a.n[k] - SEG * q;
@@ -260,8 +269,31 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
     }
   };
   f4 nx[NV];
+  if (row0 < M) seg_load(0, 0, nx);
+  if constexpr (WL) {
+    f4* dst = reinterpret_cast<f4*>(s_dyn + NW * RW * PITCH);
+    for (int k = 0; k < N; ++k)
+      for (int f = w; f < (a.n[k] + 15) / 16 * NH; f += NW) {
+        const int hrow = 16 * (f % NH) + i;
+        const bool hok = hrow < a.hidden;
+        dst[(lb[k] * NH + f) * 64 + l] = load4(a.weight + (size_t)(hok ? hrow : 0) * a.D,
+                                               a.st[k] + 16 * (f / NH) + 4 * g, a.st[k] + a.n[k], hok);
+      }
+    __syncthreads();
+  }
+  while (row0 < M) {  // uniform over the wavefront; no workgroup barrier below
+  f4 acc[N][NH][RT];
+  float ssq[N][RT];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      ssq[k][rt] = 0.0f;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) acc[k][h][rt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
   int k = 0, q = 0;
-  seg_load(0, 0, nx);
+  const int tile0 = row0;
   while (k < N) {
     wave_lds_sync();  // the previous segment's reads of the LDS tile are done
 #pragma unroll
@@ -275,7 +307,8 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
       ++k;
       q = 0;
     }
-    if (k < N) seg_load(k, q, nx);  // the next segment, in flight during the contraction
+    if (k == N) row0 = WL ? row0 + (int)gridDim.x * NW * RW : M;  // the next tile's first segment
+    if (row0 < M) seg_load(k < N ? k : 0, q, nx);  // the next segment, in flight during the contraction
     const int st = a.st[kc] + SEG * qc, nb = min(SEG, a.n[kc] - SEG * qc);
     sfor<0, N>([&](auto lc) {
       constexpr int lv = lc;
@@ -295,7 +328,8 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
         for (int h = 0; h < NH; ++h) {
           const int hrow = 16 * h + i;
           const bool hok = hrow < a.hidden;
-          const f4 wb = load4(a.weight + (size_t)(hok ? hrow : 0) * a.D, kk, en, hok);
+          const f4 wb = WL ? reinterpret_cast<const f4*>(wl)[((lb[lv] + (st - a.st[lv] + cb) / 16) * NH + h) * 64 + l]
+                           : load4(a.weight + (size_t)(hok ? hrow : 0) * a.D, kk, en, hok);
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) {
             acc[lv][h][rt] = mfma(xa[rt].x, wb.x, acc[lv][h][rt]);
@@ -311,7 +345,7 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
   for (int rt = 0; rt < RT; ++rt) {
     // per-row factors: lanes (i, g) hold partial sums of squares of row i; every lane of row i ends with the sum
     float fr[N];
-    const int gi = row0 + 16 * rt + i;
+    const int gi = tile0 + 16 * rt + i;
     const bool vi = gi < M;
     sfor<0, N>([&](auto kc) {
       constexpr int kx = kc;
@@ -352,7 +386,7 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
     });
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 4 * g + r, grow = row0 + 16 * rt + row;
+      const int row = 4 * g + r, grow = tile0 + 16 * rt + row;
       float fk[N];
 #pragma unroll
       for (int kx = 0; kx < N; ++kx) fk[kx] = __shfl(fr[kx], row, 64);  // lane `row` holds row `row`'s factors
@@ -372,7 +406,7 @@ __global__ __launch_bounds__(256) void k_mix_fwd_s(MArgs a) {
         }
       }
     }
-  }
+  }  }
 }
 
 // the leading zero rows of the levels map to the bias alone
@@ -788,7 +822,20 @@ int ews_mixer_forward(const ews_mixer_desc* desc, const float* rows, const float
   if (a.hidden <= 64) {  // streamed rows, every hidden column in one wavefront
     // one row tile per wavefront: two (half the c_down loads, 64-entry segments, fewer waves per SIMD) measured
     // 0.433 ms against 0.418 ms on the c5 epilogue (depth 2, 24 columns, 399K rows)
-#define MIX_FWD_S(NN, H) hipLaunchKernelGGL((k_mix_fwd_s<NN, H, 1>), dim3((M + 63) / 64), blk, 0, st, a)
+    // c_down in LDS where it fits beside the row tiles and every CU has a full workgroup of tiles
+    const size_t wlds = fw_lds(a, NH);
+    const bool wl = wlds <= 160 * 1024 && M >= 256 * FW_WAVES * 16;
+#define MIX_FWD_S(NN, H)                                                                                            \
+  do {                                                                                                              \
+    if (wl) {                                                                                                       \
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mix_fwd_s<NN, H, 1, true>),                          \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds) != hipSuccess)                 \
+        return EWS_ERR_LAUNCH;                                                                                      \
+      hipLaunchKernelGGL((k_mix_fwd_s<NN, H, 1, true>), dim3(256), dim3(64 * FW_WAVES), wlds, st, a);               \
+    } else {                                                                                                        \
+      hipLaunchKernelGGL((k_mix_fwd_s<NN, H, 1, false>), dim3((M + 63) / 64), blk, 4 * 16 * 132 * 4, st, a);        \
+    }                                                                                                               \
+  } while (0)
     if (a.N == 1) {
       if (NH == 2) MIX_FWD_S(1, 2);
       else MIX_FWD_S(1, 4);
