@@ -1251,18 +1251,25 @@ constexpr int LX_PHI = 64 * (PW + 1), LX_U = (PW + 1) * 32;
 constexpr int LF_EXTRA = LX_PHI + LX_U;
 
 // knots Delta_1 .. Delta_M into D (rows 0 .. M-1) on the series path: Delta_{r+1} = sum_k phi[r][k] c^k u_k from
-// u_k = A^k w (rows of U, formed per interval by k_wmat_series)
+// u_k = A^k w (rows of U, formed per interval by k_wmat_series): tiles of 16 knots x 16 entries on MFMA (a wavefront:
+// entries 16 (w % 2) .., knot tiles w / 2, w / 2 + 2, ..)
 __device__ void series_knots(int M, const float* phi, const float* U, float* D, float c) {
-  const int tid = threadIdx.x;
-  for (int e = tid; e < M * 32; e += NT) {
-    const int r = e >> 5, row = e & 31;
-    float x = 0.0f, ck = 1.0f;
-#pragma unroll 4
-    for (int k = 0; k <= PW; ++k) {
-      x = fmaf(phi[r * (PW + 1) + k] * ck, U[k * 32 + row], x);
-      ck *= c;
+  const int w = (int)threadIdx.x >> 6, g = tile_g(), c16 = tile_i(), ii = 16 * (w & 1) + c16;
+  const float c2 = c * c, c4 = c2 * c2, cg = (g & 1 ? c : 1.0f) * (g & 2 ? c2 : 1.0f);
+  for (int r0 = 16 * (w >> 1); r0 < M; r0 += 32) {
+    const float* pr = phi + min(r0 + c16, M - 1) * (PW + 1);  // a row past the last one is not stored
+    v4f x = zero4();
+    float ck = cg;  // c^k
+#pragma unroll
+    for (int u = 0; u <= PW / 4; ++u) {
+      const int k = 4 * u + g;
+      x = __builtin_amdgcn_mfma_f32_16x16x4f32(k <= PW ? pr[min(k, PW)] * ck : 0.0f, k <= PW ? U[min(k, PW) * 32 + ii] : 0.0f,
+                                               x, 0, 0, 0);
+      ck *= c4;
     }
-    D[e] = x;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (r0 + 4 * g + q < M) D[(r0 + 4 * g + q) * 32 + ii] = x[q];
   }
   __syncthreads();
 }
@@ -1929,7 +1936,7 @@ __global__ __launch_bounds__(NT) void k_wadj_carry(WArgs a) {
 // one instantiation each so that each carries only its own registers
 constexpr int LK_SERIES = 0, LK_VL_SHARED = 1, LK_VL_INT = 2;
 template <int N, int LK>
-__global__ __launch_bounds__(NT) void k_wleaf_bwd(WArgs a) {
+__global__ __launch_bounds__(NT, 4) void k_wleaf_bwd(WArgs a) {
   extern __shared__ __align__(16) float sm[];  // lf_floats(rows, 4) (+ LF_EXTRA, per-interval Van Loan)
   float* A = sm + LF_A;
   float* S2b = sm + LF_S2;  // ds2
@@ -2019,40 +2026,55 @@ __global__ __launch_bounds__(NT) void k_wleaf_bwd(WArgs a) {
       else vl_knots(a, P, V, wv, T1);
       knot_sums(M, T1, T3, T2, nullptr);  // Z_m = R_m + Delta_m / 2 (T2), Y_m = Pre_m + Delta_m / 2 (T3)
       __syncthreads();
-      // dDelta_m = ds1 + ds2 Z_m + ds2^T Y_m (rows of T4), a thread per entry
-      for (int e = tid; e < M * 32; e += NT) {
-        const int m = e >> 5, ii = e & 31;
-        float v = ds1[ii];
+      // dDelta_m = ds1 + ds2 Z_m + ds2^T Y_m (rows of T4), tiles of 16 knots x 16 entries: wavefront w takes the entries
+      // 16 (w % 2) .. and the knot tiles w / 2, w / 2 + 2, ... A thread per entry read 64 floats of each operand from LDS
+      // for it, 0.4 MB an interval (B = 32, L = 896, d = 24, M = 20: the kernel 333 -> 179 us).
+      {
+        const int w = tid >> 6, l = tid & 63, g = l >> 4, c16 = l & 15, ii = 16 * (w & 1) + c16;
+        const float d1 = ds1[ii];
+        v4f sr[2], sc[2];  // ds2[ii][16 h + 4g + s], ds2[16 h + 4g + s][ii]
         if constexpr (N >= 2) {
-          const float* z = T2 + m * 32;
-          const float* y = T3 + m * 32;
-          const float* srow = S2b + ii * P32;
-#pragma unroll 2
-          for (int j = 0; j < 32; j += 4) {
-            const float4 zz = *reinterpret_cast<const float4*>(z + j);
-            const float4 yy = *reinterpret_cast<const float4*>(y + j);
-            const float4 sr = *reinterpret_cast<const float4*>(srow + j);
-            v = fmaf(sr.x, zz.x, v);
-            v = fmaf(sr.y, zz.y, v);
-            v = fmaf(sr.z, zz.z, v);
-            v = fmaf(sr.w, zz.w, v);
-            v = fmaf(S2b[j * P32 + ii], yy.x, v);
-            v = fmaf(S2b[(j + 1) * P32 + ii], yy.y, v);
-            v = fmaf(S2b[(j + 2) * P32 + ii], yy.z, v);
-            v = fmaf(S2b[(j + 3) * P32 + ii], yy.w, v);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            sr[h] = *reinterpret_cast<const v4f*>(S2b + ii * P32 + 16 * h + 4 * g);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) sc[h][s] = S2b[(16 * h + 4 * g + s) * P32 + ii];
           }
         }
-        T4[e] = v;
+        for (int m0 = 16 * (w >> 1); m0 < M; m0 += 32) {
+          v4f v = {d1, d1, d1, d1};
+          if constexpr (N >= 2) {
+            const int mr = min(m0 + c16, M - 1) * 32 + 4 * g;  // a row past the last one is not stored
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const v4f z = *reinterpret_cast<const v4f*>(T2 + mr + 16 * h), y = *reinterpret_cast<const v4f*>(T3 + mr + 16 * h);
+#pragma unroll
+              for (int s = 0; s < 4; ++s) {
+                v = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s], sr[h][s], v, 0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x4f32(y[s], sc[h][s], v, 0, 0, 0);
+              }
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (m0 + 4 * g + r < M) T4[(m0 + 4 * g + r) * 32 + ii] = v[r];
+        }
       }
       __syncthreads();
       if (ser) {
         // e_k = sum_r phi[r][k] dDelta_r, to ebuf: the powers' cotangent c^k e_k w^T, dw = sum_k c^k (A^k)^T e_k
         // and dc = sum_k k c^(k-1) <e_k, u_k> are k_wmat_bwd_series's (it holds the powers)
-        for (int e = tid; e < (PW + 1) * 32; e += NT) {
-          const int k = e >> 5, row = e & 31;
-          float x = 0.0f;
-          for (int m = 0; m < M; ++m) x = fmaf(phi[m * (PW + 1) + k], T4[m * 32 + row], x);
-          a.ebuf[r * (PW + 1) * 32 + e] = x;
+        const int w = tid >> 6, l = tid & 63, g = l >> 4, c16 = l & 15, ii = 16 * (w & 1) + c16;
+        for (int k0 = 16 * (w >> 1); k0 <= PW; k0 += 32) {
+          v4f x = zero4();
+          for (int mb = 0; mb < M; mb += 4) {
+            const int m = min(mb + g, M - 1);
+            const float p = mb + g < M ? phi[m * (PW + 1) + min(k0 + c16, PW)] : 0.0f;
+            x = __builtin_amdgcn_mfma_f32_16x16x4f32(p, mb + g < M ? T4[m * 32 + ii] : 0.0f, x, 0, 0, 0);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (k0 + 4 * g + q <= PW) a.ebuf[(r * (PW + 1) + k0 + 4 * g + q) * 32 + ii] = x[q];
         }
         dv_done = true;
       } else {
