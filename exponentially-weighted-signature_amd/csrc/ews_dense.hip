@@ -335,14 +335,16 @@ __global__ __launch_bounds__(256, QB <= 24 ? 3 : 2) void k_local3(Args a) {
     }
     wave_order_d();
     // the letters, PM at a time from a base letter: b_{a+m} = (prod_{j=1..m} -h j / (a + j)) P_m b_a, the products of
-    // a stage independent of each other
-    for (int a0 = 0; a0 < q; a0 += PM) {
+    // a stage independent of each other. With a large ||A||_1 one at a time: A^m / m! leaves the float32 range near 8e3
+    // (at 256 it is 2e20) where the letters, times h^m, need not.
+    const int stage = norm1 <= 256.0f ? PM : 1;
+    for (int a0 = 0; a0 < q; a0 += stage) {
       const f4 bp = *reinterpret_cast<const f4*>(L + a0 * 16 + 4 * g);
       float cf = 1.0f;
 #pragma unroll
       for (int m = 1; m <= PM; ++m) {
         const int pp = a0 + m;
-        if (pp <= q) {
+        if (m <= stage && pp <= q) {
           const f4 pm = *reinterpret_cast<const f4*>(&sp[m][c16 * 16 + 4 * g]);
           float sm = fmaf(pm.x, bp.x, fmaf(pm.y, bp.y, fmaf(pm.z, bp.z, pm.w * bp.w)));
           sm = lanes::add_xor32(lanes::add_xor16(sm));
