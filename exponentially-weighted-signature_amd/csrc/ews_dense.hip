@@ -275,6 +275,15 @@ __global__ __launch_bounds__(256) void k_local(Args a) {
   }
 }
 
+// Letters per stage of an interval with step h: b_{a+m} = (prod_{j=1..m} -h j / (a + j)) P_m b_a from a base letter a for
+// m = 1 .. PM at once, P_m = A^m / m!, or one at a time, which is the recursion b_p = (-h/p) A b_{p-1}. A stage's factors
+// grow like h^m and ||A||^m apart while the letters only have (h ||A||)^m, so a dozen at a time needs both bounded: at
+// ||A||_1 = 256 P_12 is 2e20 at most (above 8e3 it leaves the float32 range), at |h| = 64 h^12 is 5e21 (above 1.6e3 it does;
+// a clock in raw seconds has such steps), and what underflows of the other factor is then below 2^-77 of the base letter.
+__device__ __forceinline__ int letter_stage(float norm1, float h) {
+  return norm1 <= 256.0f && fabsf(h) <= 64.0f ? PM : 1;
+}
+
 // Depth-3 local terms on MFMA, one wavefront per interval (four per workgroup, grid-stride). The letters come a dozen at
 // a time from the power table and the bt_N from two or three tiles of MFMA: the recursion b_p = (-h/p) A b_{p-1} and the
 // sums over p, letter by letter, were 24 and about 80 dependent LDS round trips an interval (B = 16, L = 4096, q = 24:
@@ -334,10 +343,8 @@ __global__ __launch_bounds__(256, QB <= 24 ? 3 : 2) void k_local3(Args a) {
       G1[l] = v;
     }
     wave_order_d();
-    // the letters, PM at a time from a base letter: b_{a+m} = (prod_{j=1..m} -h j / (a + j)) P_m b_a, the products of
-    // a stage independent of each other. With a large ||A||_1 one at a time: A^m / m! leaves the float32 range near 8e3
-    // (at 256 it is 2e20) where the letters, times h^m, need not.
-    const int stage = norm1 <= 256.0f ? PM : 1;
+    // the letters by stages (letter_stage), the products of a stage independent of each other
+    const int stage = letter_stage(norm1, h);
     for (int a0 = 0; a0 < q; a0 += stage) {
       const f4 bp = *reinterpret_cast<const f4*>(L + a0 * 16 + 4 * g);
       float cf = 1.0f;
