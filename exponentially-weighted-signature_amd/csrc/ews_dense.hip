@@ -1951,14 +1951,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
     }
     __syncthreads();
     // ---- letters b_p = (-h)^p A^p v / p!, by stages from the powers table P_m = A^m / m!: the letters a + m of
-    // the stage on base letter a (a = 0, PM, 2 PM, ...; m = 1 .. PM) are b_{a+m} = c_{a,m} P_m b_a with
+    // the stage on base letter a (a = 0, stage, 2 stage, ...; m = 1 .. stage) are b_{a+m} = c_{a,m} P_m b_a with
     // c_{a,m} = (-h)^m / C(a + m, m), all of a stage at once (thread: power m, row r)
-    for (int a0 = 0; a0 < q; a0 += PM) {
+    const int stage = letter_stage(norm1, h);
+    for (int a0 = 0; a0 < q; a0 += stage) {
       if (tid < PM) s_lc[tid] = letter_coef(h, a0, tid + 1);
       __syncthreads();
+      const int pe = min(q, a0 + stage);  // the stage's last letter
       for (int e = tid; e < PM * 16; e += 256) {
         const int m = 1 + (e >> 4), r = e & 15, p = a0 + m;
-        if (p <= q) {
+        if (p <= pe) {
           float x = 0.0f;
 #pragma unroll 4
           for (int k = 0; k < 16; ++k) {
@@ -2097,12 +2099,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
     // (c_{a,m} / m!) db_p (x) b_a (H_m, turned into dA once per launch with the flows' terms)
     float dhl = 0.0f;  // partial dh in threads 0 .. 15
     Row16* Zt = dBT;   // free after the degree sums
-    for (int a0 = q > 0 ? ((q - 1) / PM) * PM : -1; a0 >= 0; a0 -= PM) {
+    for (int a0 = q > 0 ? ((q - 1) / stage) * stage : -1; a0 >= 0; a0 -= stage) {
+      const int pe = min(q, a0 + stage);
       if (tid < PM) s_lc[tid] = letter_coef(h, a0, tid + 1);
       for (int e = tid; e < PM * 16; e += 256) {
         const int m = 1 + (e >> 4), jj = e & 15, p = a0 + m;
         float z = 0.0f;
-        if (p <= q) {
+        if (p <= pe) {
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) z = fmaf(sp[m][i2 * 16 + jj], dB[p][i2], z);
         }
@@ -2116,12 +2119,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
         for (int m = 1; m <= PM; ++m) {
           ifact *= 1.0f / (float)m;
           const int p = a0 + m;
-          if (p <= q) H[m] = fmaf(s_lc[m - 1].x * ifact * dB[p][i], bj, H[m]);
+          if (p <= pe) H[m] = fmaf(s_lc[m - 1].x * ifact * dB[p][i], bj, H[m]);
         }
       }
       if (tid < 16) {
         float acc = dB[a0][tid], dz = 0.0f;
-        for (int m = 1; m <= PM && a0 + m <= q; ++m) {
+        for (int m = 1; m <= PM && a0 + m <= pe; ++m) {
           const float2 cc = s_lc[m - 1];
           const float z = Zt[m - 1][tid];
           acc = fmaf(cc.x, z, acc);

@@ -32,3 +32,24 @@ def test_letters(q, scale):
     err = float((out.cpu().double() - ref).abs().max() / ref.abs().max())
     print(f"q={q} scale={scale} {err:.1e}", flush=True)
     assert err < 1e-5
+
+
+@pytest.mark.parametrize("q", [1, 12, 24, 40])
+@pytest.mark.parametrize("scale", [1.0, 2e4, 4e-4, 1e-4])
+def test_gradients_in_units_of_the_clock(q, scale):
+    rng = np.random.default_rng(q)
+    d, L = 5, 7
+    path = torch.tensor(np.cumsum(rng.normal(size=(2, L, d)) * 0.3, 1), dtype=torch.float32)
+    clock = torch.tensor(np.cumsum(rng.uniform(0.6, 0.9, size=(2, L)) / scale, 1), dtype=torch.float32)
+    A = torch.tensor((rng.normal(size=(d, d)) / np.sqrt(d) + np.eye(d)) * scale, dtype=torch.float32)
+    leaf = ops.DenseLeaf("series", q=q, chen_expm="cayley")
+    p, c, a = (x.to(DEV).requires_grad_() for x in (path, clock, A))
+    out = ops.dense_scan(p, c, a, 3, q, "per_interval", "prefix", True, leaf=leaf)
+    g = torch.tensor(rng.normal(size=tuple(out.shape)), dtype=torch.float32)
+    got = torch.autograd.grad(out, [p, c, a], g.to(DEV))
+    r = [x.double().requires_grad_() for x in (path, clock, A)]
+    ref = O.ews(*r, 3, "prefix", leaf="series", series_q=q, chen_expm="cayley", terminal_reduce="assoc")
+    want = torch.autograd.grad(ref, r, g.double())
+    errs = [float((x.cpu().double() - y).abs().max() / y.abs().max()) for x, y in zip(got, want)]
+    print(f"q={q} scale={scale} {['%.1e' % e for e in errs]}", flush=True)
+    assert max(errs) < 1e-4, errs
