@@ -2104,12 +2104,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXACTF ? 3 
       if (tid < PM) s_lc[tid] = letter_coef(h, a0, tid + 1);
       for (int e = tid; e < PM * 16; e += 256) {
         const int m = 1 + (e >> 4), jj = e & 15, p = a0 + m;
-        float z = 0.0f;
-        if (p <= pe) {
+        if (p <= pe) {  // (the array has q + 1 rows)
+          float z = 0.0f;
 #pragma unroll
           for (int i2 = 0; i2 < 16; ++i2) z = fmaf(sp[m][i2 * 16 + jj], dB[p][i2], z);
+          Zt[m - 1][jj] = z;
         }
-        Zt[m - 1][jj] = z;
       }
       __syncthreads();  // the stage's coefficients and z
       {
