@@ -480,6 +480,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
   __shared__ __align__(16) float s_v[GPW][kMaxT * 8 * KP];
   __shared__ __align__(16) float s_w[GPW][NW > NP ? NW : NP];  // w[s][k][j] (complex); at the end the parameter terms
   __shared__ __align__(16) float s_dvp[GPW][NB * R * 2];       // plane part of dv[s][j] (complex)
+  __shared__ float s_h[GPW][kMaxT];                            // clock steps
   const int b = blockIdx.y;
   const Lane<R, KP> l(a, b, kUniform | kInvert | kStrict);
   if (!__any(l.owns)) return;
@@ -493,6 +494,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     ring[s] = load_g<R, KP>(grow + (size_t)max(min((nblk - 1) * NB + s, l.Tc - 1), 0) * a.W, o1, o2, a.d, l);
   });
   stage<R>(a, b, l.gl, l.t0, l.Tc, vg);
+  float* hg = s_h[l.gi];
+  {
+    const float* th = a.clock + (size_t)b * a.L + l.t0;
+    for (int t = l.gl; t < l.Tc; t += G) hg[t] = th[t + 1] - th[t];
+  }
   const float hb = a.chbar[l.ci];
   const bool small = (a.cflag[l.ci] & kSmall) != 0;
   Coefs<KP, true> f;
@@ -512,7 +518,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       lB[q] = cf{2.0f * mp[e + 2], 2.0f * mp[e + 3]};
     });
   }
-  // the coefficient cotangents summed over the steps (times the mean step at the end: the steps agree to 2^-21)
+  // The coefficient cotangents, summed with each step's own h: the coefficients are constant where |u| times the steps'
+  // deviation is below 2^-21, but for a small |u| or a fine clock the deviation may be as large as the step (float32
+  // values near 1 leave steps of 2e-5 off by 3e-3 of themselves), and a sum times the mean step is then off as much.
   cf kIB[KP], kIA[KP], kLB[KP], kLA[KP], kph[KP], krho{0.0f, 0.0f}, kphj{0.0f, 0.0f};
   static_for<0, KP>([&](auto qc) {
     constexpr int q = qc;
@@ -531,6 +539,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       if (t >= l.Tc) return;
       cf pj, pk[KP];
       load_p<R, KP>(vg + t * a.d, l, pj, pk);
+      const float h = hg[t];
       const cf cj = S1 - f.phi * pj;  // c_j = rho S1(t-1)
       const cf H1 = f.rhoi * cj;
       cf toC{0.0f, 0.0f}, toP{0.0f, 0.0f};
@@ -567,17 +576,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         const float wr = fmaf(ph.re, tSr, fmaf(ph.im, tSi, fmaf(pj.re, Fr, pj.im * Fi)));
         const float wi = fmaf(ph.re, tSi, fmaf(-ph.im, tSr, fmaf(pj.re, Ei, -pj.im * Er)));
         if (l.counts(q)) *reinterpret_cast<float2*>(w_g + ((s * 4 * KP + l.k[q]) * RP + l.j) * 2) = float2{wr, wi};
-        // coefficient cotangents conj(p_k) tS, conj(pi) B, conj(pic) A, conj(HB) B, conj(HA) A
-        kph[q].re = fmaf(pkq.re, tSr, fmaf(pkq.im, tSi, kph[q].re));
-        kph[q].im = fmaf(pkq.re, tSi, fmaf(-pkq.im, tSr, kph[q].im));
-        kIB[q].re = fmaf(pir, Br, fmaf(pii, Bi, kIB[q].re));
-        kIB[q].im = fmaf(pir, Bi, fmaf(-pii, Br, kIB[q].im));
-        kIA[q].re = fmaf(pcr, Ar, fmaf(pci, Ai, kIA[q].re));
-        kIA[q].im = fmaf(pcr, Ai, fmaf(-pci, Ar, kIA[q].im));
-        kLB[q].re = fmaf(HBr, Br, fmaf(HBi, Bi, kLB[q].re));
-        kLB[q].im = fmaf(HBr, Bi, fmaf(-HBi, Br, kLB[q].im));
-        kLA[q].re = fmaf(HAr, Ar, fmaf(HAi, Ai, kLA[q].re));
-        kLA[q].im = fmaf(HAr, Ai, fmaf(-HAi, Ar, kLA[q].im));
+        // coefficient cotangents times h: conj(p_k) tS, conj(pi) B, conj(pic) A, conj(HB) B, conj(HA) A
+        const float tSrh = h * tSr, tSih = h * tSi, Arh = h * Ar, Aih = h * Ai, Brh = h * Br, Bih = h * Bi;
+        kph[q].re = fmaf(pkq.re, tSrh, fmaf(pkq.im, tSih, kph[q].re));
+        kph[q].im = fmaf(pkq.re, tSih, fmaf(-pkq.im, tSrh, kph[q].im));
+        kIB[q].re = fmaf(pir, Brh, fmaf(pii, Bih, kIB[q].re));
+        kIB[q].im = fmaf(pir, Bih, fmaf(-pii, Brh, kIB[q].im));
+        kIA[q].re = fmaf(pcr, Arh, fmaf(pci, Aih, kIA[q].re));
+        kIA[q].im = fmaf(pcr, Aih, fmaf(-pci, Arh, kIA[q].im));
+        kLB[q].re = fmaf(HBr, Brh, fmaf(HBi, Bih, kLB[q].re));
+        kLB[q].im = fmaf(HBr, Bih, fmaf(-HBi, Brh, kLB[q].im));
+        kLA[q].re = fmaf(HAr, Arh, fmaf(HAi, Aih, kLA[q].re));
+        kLA[q].im = fmaf(HAr, Aih, fmaf(-HAi, Arh, kLA[q].im));
         const cf LB = f.LB[q], LA = f.LA[q];
         lB[q] = cf{fmaf(LB.re, Br, LB.im * Bi), fmaf(LB.re, Bi, -LB.im * Br)};
         lA[q] = cf{fmaf(LA.re, Ar, LA.im * Ai), fmaf(LA.re, Ai, -LA.im * Ar)};
@@ -591,8 +601,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         const cf dvp = cjm(f.phi, l1) + toP;
         *reinterpret_cast<float2*>(dvp_g + (s * R + l.j) * 2) = float2{dvp.re, dvp.im};
       }
-      kphj += cjm(pj, l1);
-      krho += cjm(H1, gc);
+      kphj += cjm(pj, h * l1);
+      krho += cjm(H1, h * gc);
       l1 = cjm(f.rho, gc);
       S1 = H1;
     });
@@ -619,7 +629,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     }
     wave_order();
   }
-  // parameter partials: node cotangents -> (d_j, w_j) per plane. A node h u contributes (-Re G, Im G) to its plane for
+  // parameter partials (a moment's further powers of h at the mean step): node cotangents -> (d_j, w_j) per plane. A node h u contributes (-Re G, Im G) to its plane for
   // u = -conj(z) and (-Re G, -Im G) for u = -z (the conj(u_k) of the A pairs).
   const cf uj = load_u(a.params, l.j);
   const cf xj = hb * uj;
@@ -635,7 +645,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     if (small) {
       cf m[kPolyD];
       auto moments = [&](cf k0) {
-        m[0] = hb * k0;
+        m[0] = k0;
 #pragma unroll
         for (int i = 1; i < kPolyD; ++i) m[i] = hb * m[i - 1];
       };
@@ -647,14 +657,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
       gk = poly_phi_node(uk, m);
     } else {
       const DD3<cf> db = dd3q<cf, true>(xj, hb * ub, a.sq2), da = dd3q<cf, true>(xj, hb * ua, a.sq2);
-      gxB = hb * (kIB[q] * conj(db.dx));
-      gyB = hb * (kIB[q] * conj(db.dy));
-      gxA = hb * (kIA[q] * conj(da.dx));
-      gyA = hb * (kIA[q] * conj(da.dy));
-      gk = hb * (kph[q] * conj(node1q(hb * uk, a.sq1).dp));
+      gxB = kIB[q] * conj(db.dx);
+      gyB = kIB[q] * conj(db.dy);
+      gxA = kIA[q] * conj(da.dx);
+      gyA = kIA[q] * conj(da.dy);
+      gk = kph[q] * conj(node1q(hb * uk, a.sq1).dp);
     }
-    const cf GyB = 0.5f * gyB + hb * (kLB[q] * conj(f.LB[q]));
-    const cf GyA = 0.5f * gyA + hb * (kLA[q] * conj(f.LA[q]));
+    const cf GyB = 0.5f * gyB + kLB[q] * conj(f.LB[q]);
+    const cf GyA = 0.5f * gyA + kLA[q] * conj(f.LA[q]);
     const cf Gk = 0.5f * gk;
     if (l.live[q]) {
       Gx += 0.5f * (gxB + gxA);
@@ -670,14 +680,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     cf gp;
     if (small) {
       cf m[kPolyPhi];
-      m[0] = hb * kphj;
+      m[0] = kphj;
 #pragma unroll
       for (int i = 1; i < kPolyPhi; ++i) m[i] = hb * m[i - 1];
       gp = poly_phi_node(uj, m);
     } else {
-      gp = hb * (kphj * conj(node1q(xj, a.sq1).dp));
+      gp = kphj * conj(node1q(xj, a.sq1).dp);
     }
-    gp += hb * (krho * conj(f.rho));
+    gp += krho * conj(f.rho);
     *reinterpret_cast<float2*>(rowp + 2 * l.j) = float2{rd - gp.re, rw + gp.im};
   }
   wave_order();

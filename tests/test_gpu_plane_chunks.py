@@ -20,14 +20,14 @@ def _rel(a, b):
     return float((a - b).abs().max() / b.abs().max().clamp_min(1e-300))
 
 
-def _check(d, B, steps, damp, readout="prefix", chunk=0, bf16=False, clock_grad=True):
-    """steps (L,): the clock's steps (the first is its start)."""
+def _check(d, B, steps, damp, readout="prefix", chunk=0, bf16=False, clock_grad=True, freq=3.0):
+    """steps (L,): the clock's steps (the first is its start). Planes: damping in damp, frequencies in [0, freq]."""
     L = len(steps)
     rng = np.random.default_rng(L + d)
     path = torch.tensor(np.cumsum(rng.normal(size=(B, L, d)) * 0.2, 1), dtype=torch.float32)
     path = path.to(torch.bfloat16) if bf16 else path
     clock = torch.tensor(np.cumsum(steps)[None].repeat(B, 0), dtype=torch.float32)
-    w = torch.tensor(np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, 3.0, d // 2)], -1), dtype=torch.float32)
+    w = torch.tensor(np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, freq, d // 2)], -1), dtype=torch.float32)
     p, c, q = path.to(DEV).requires_grad_(), clock.to(DEV).requires_grad_(clock_grad), w.to(DEV).requires_grad_()
     out = ops.diag_scan(p, c, q, 2, "planes", "per_interval", readout, readout != "log_prefix", chunk=chunk)
     g = torch.tensor(rng.normal(size=tuple(out.shape)), dtype=torch.float32)
@@ -77,6 +77,24 @@ def test_strict_and_loose_chunks(d):
     steps[100:200] *= 1.0 + 2e-4 * np.random.default_rng(0).uniform(-1, 1, 100)
     steps[300:330] *= np.random.default_rng(1).uniform(0.2, 3.0, 30)
     _check(d, 2, steps, (0.1, 1.0), clock_grad=False)
+
+
+def _irregular(L, h, start=0.0):
+    return np.r_[start, np.random.default_rng(2).uniform(0.2, 1.8, L - 1) * h]
+
+
+@pytest.mark.parametrize("d", [8, 12, 16, 24, 32])
+@pytest.mark.parametrize("rate,h", [(0.0, 2.0**-4), (1e-5, 2.0**-8), (2e-2, 2e-5)])
+def test_steps_that_differ_within_constant_coefficients(d, rate, h):
+    # max|u| times the steps' deviation is far below the bound of constant coefficients, the deviation itself 80% of a
+    # step: the parameter gradients weigh each step's cotangents with its own length
+    _check(d, 2, _irregular(140, h), (0.0, rate), clock_grad=False, freq=rate)
+
+
+@pytest.mark.parametrize("d", [12, 16, 24])
+def test_float32_uniform_clock(d):
+    # a uniform clock whose float32 values near 1 leave steps of 2e-5 off by 3e-3 of themselves
+    _check(d, 2, _uniform(300, 2.0e-5) + np.r_[0.9, np.zeros(299)], (0.1, 1.0), clock_grad=False)
 
 
 @pytest.mark.parametrize("d", [12, 24])
