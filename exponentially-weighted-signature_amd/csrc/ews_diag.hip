@@ -326,16 +326,17 @@ __device__ __forceinline__ ChunkClock chunk_classify(const DiagArgs& a, int b, i
   for (int t = lane; t < Tc; t += 64) s += s_h[t];
   s = lanes::sum64(s);
   cc.hbar = s / (float)Tc;
-  float dmax = 0.0f, hmax = 0.0f, bad = 0.0f;
+  float dmax = 0.0f, hmax = 0.0f, bad = 0.0f, back = 0.0f;
   for (int t = lane; t < Tc; t += 64) {
     const float dl = fabsf(s_h[t] - cc.hbar);
     dmax = fmaxf(dmax, dl);
     hmax = fmaxf(hmax, fabsf(s_h[t]));
+    back += fmaxf(-s_h[t], 0.0f);
     if (!(dl <= 3.0e38f)) bad = 1.0f;
   }
   // R: largest |u|; Dmax: largest contraction rate Re(-u_j) (the damping d_j of a plane, lambda_j of a real channel);
-  // a level-2 element contracts at most at twice that rate, so the inverse step grows errors by e^{2 Dmax tau}
-  float R = 0.0f, Dmax = 0.0f;
+  // Gmax: largest growth rate Re(u_j), which only backward steps ask for
+  float R = 0.0f, Dmax = 0.0f, Gmax = 0.0f;
   T dummy{};
   for (int j = lane; j < a.K; j += 64) {
     const T u = load_u(a.params, j, &dummy);
@@ -343,17 +344,26 @@ __device__ __forceinline__ ChunkClock chunk_classify(const DiagArgs& a, int b, i
     if (!(au <= 3.0e38f)) bad = 1.0f;
     R = fmaxf(R, au);
     Dmax = fmaxf(Dmax, -re(u));
+    Gmax = fmaxf(Gmax, re(u));
   }
   dmax = wave_max(dmax);
   hmax = wave_max(hmax);
   bad = wave_max(bad);
   R = wave_max(R);
   Dmax = wave_max(Dmax);
+  if (__any(back > 0.0f) || cc.href < 0.0f) {
+    Gmax = wave_max(Gmax);
+    back = lanes::sum64(back);
+  }
   const bool finite = bad == 0.0f && isfinite(s);
   cc.fast = finite && (dmax * 2.0f * R < 1.52587890625e-5f);  // 2^-16
   cc.small = finite && poly_order_ok(a.sq1, a.sq2) && 2.0f * R * hmax <= kPolyR;
-  const float tau = cc.per_int ? s : fabsf(cc.href) * (float)Tc;
-  cc.inv_ok = finite && (2.0f * Dmax * tau <= 0.69314718f);
+  if (!cc.per_int) {  // cached flows: every step flows over href (a backward one at either rate)
+    s = fabsf(cc.href) * (float)Tc;
+    back = 0.0f;
+    if (cc.href < 0.0f) Dmax = fmaxf(Dmax, Gmax);
+  }
+  cc.inv_ok = finite && invert_growth(s, back, Dmax, Gmax) <= 0.69314718f;
   return cc;
 }
 // The class as the forward left it.

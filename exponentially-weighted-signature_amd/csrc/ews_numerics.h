@@ -271,6 +271,14 @@ template <class T, bool DERIV> EWS_HD DD3<T> dd3q(T x, T y, int q) {
 constexpr float kPolyR = 0.4f;
 constexpr int kPolyPhi = 6, kPolyD = 7;
 
+// Log of the largest growth of an error when a chunk's steps are taken backwards: net their sum, back the length of the
+// backward ones (the sum of -h over h < 0), decay and growth the largest max(0, -Re u) and max(0, Re u); a level-2 element
+// moves at most at twice a rate. A forward step contracts at the decay, a backward one at the growth: on a clock that turns
+// the net step alone says nothing (32 steps of 0.17 forward and back at rate 1 contract level 2 by e^11 on the way).
+EWS_HD float invert_growth(float net, float back, float decay, float growth) {
+  return 2.0f * (decay * (net + back) + growth * back);
+}
+
 EWS_HD bool poly_order_ok(int q1, int q2) { return (q1 == 0 || q1 >= kPolyPhi) && (q2 == 0 || q2 >= kPolyD); }
 
 template <class T> EWS_HD void poly_phi(T u, T* c) {  // c[m] = u^m / (m+1)!

@@ -354,15 +354,17 @@ __global__ __launch_bounds__(192) void k_coef_table(DiagArgs a) {
   const cf xj = h0 * uj;
   const cf ub = uj + uk, ua = uj + conj(uk);
   if (role == 0) {
-    if (l == 0) {  // header: the reference step, max |u_j| and max d_j (the chunk classification's bounds)
-      float R = 0.0f, Dm = 0.0f;
+    if (l == 0) {  // header: the reference step, max |u_j|, max d_j and max -d_j (the chunk classification's bounds)
+      float R = 0.0f, Dm = 0.0f, Gm = 0.0f;
       for (int p = 0; p < K; ++p) {
         R = fmaxf(R, absv(load_u(a.params, p)));
         Dm = fmaxf(Dm, a.params[2 * p]);
+        Gm = fmaxf(Gm, -a.params[2 * p]);
       }
       tab[0] = h0;
       tab[1] = R;
       tab[2] = Dm;
+      tab[4] = Gm;
       reinterpret_cast<int*>(tab)[kCtabStatus] = 0;  // the look-back forward's error word
     }
     if (k == 0) {
@@ -449,7 +451,7 @@ __device__ __forceinline__ void fwd_coef(const DiagArgs& a, const Lane& l, float
 
 // ------------------------------------------------------------------------------------------------ classification
 // Chunk c of sample b: flag bit 0 = uniform steps (coefficients at the mean step hbar), bit 1 = the steps may be
-// inverted backwards (stepping back amplifies errors by e^{2 Dmax tau} <= 2 over the chunk), bit 2 = the coefficient
+// inverted backwards (stepping back grows errors by at most 2 over the chunk: invert_growth), bit 2 = the coefficient
 // table applies, bit 3 = small steps (2 max|u| |h| <= kPolyR: the coefficients as polynomials in h). Evaluated by the 16
 // lanes of the chunk's group, each over every 16th step, then combined with DPP inside the group.
 __device__ __forceinline__ float row_max16(float v) {
@@ -463,7 +465,7 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   constexpr int U = kMaxT / 16;
   const int t0 = c * a.T, Tc = min(a.T, a.n_int - t0);
   const float* th = a.clock + (size_t)b * a.L + t0;
-  const float R = a.ctab[1], Dm = a.ctab[2];  // max |u_j| and max d_j, from the coefficient table's header
+  const float R = a.ctab[1], Dm = a.ctab[2], Gm = a.ctab[4];  // max |u_j|, d_j and -d_j, from the table's header
   float x0[U], x1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {  // every clock load in flight before the first use
@@ -474,7 +476,7 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   const float th0 = th[0];
   const float tau = th[Tc] - th0;
   hb = tau / (float)Tc;
-  float dev = 0.0f, drift = 0.0f, bad = 0.0f, hmax = 0.0f;
+  float dev = 0.0f, drift = 0.0f, bad = 0.0f, hmax = 0.0f, back = 0.0f;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int t = gl + 16 * u;
@@ -482,6 +484,7 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
       const float h = x1[u] - x0[u];
       if (!isfinite(h)) bad = 1.0f;
       hmax = fmaxf(hmax, fabsf(h));
+      back += fmaxf(-h, 0.0f);
       dev = fmaxf(dev, fabsf(h - hb));
       drift = fmaxf(drift, fabsf((x1[u] - th0) - (float)(t + 1) * hb));
     }
@@ -490,10 +493,11 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   drift = row_max16(drift);
   bad = row_max16(bad);
   hmax = row_max16(hmax);
+  back = lanes::sum16(back);
   const bool fin = bad == 0.0f && isfinite(tau) && isfinite(R);
   const float lim = 4.76837158e-7f;  // 2^-21
   const bool uni = fin && R * dev <= lim && R * drift <= lim;
-  const bool inv = fin && 2.0f * Dm * fabsf(tau) <= 0.69314718f;
+  const bool inv = fin && 2.0f * Dm * fabsf(tau) <= 0.69314718f && invert_growth(tau, back, Dm, Gm) <= 0.69314718f;
   const bool tab = uni && R * fabsf(hb - a.ctab[0]) <= 0.5f * lim;  // the coefficient table applies
   const bool small = fin && 2.0f * R * hmax <= kPolyR;
   return (uni ? 1 : 0) | (inv ? 2 : 0) | (tab ? 4 : 0) | (small ? 8 : 0);

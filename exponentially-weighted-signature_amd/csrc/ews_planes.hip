@@ -234,18 +234,20 @@ __device__ __forceinline__ int classify(const DiagArgs& a, int b, int t0, int Tc
   const float* th = a.clock + (size_t)b * a.L + t0;
   const float th0 = th[0], tau = th[Tc] - th0;
   hb = tau / (float)Tc;
-  float dev = 0.0f, drift = 0.0f, hmax = 0.0f, bad = 0.0f, R = 0.0f, Dm = 0.0f;
+  float dev = 0.0f, drift = 0.0f, hmax = 0.0f, bad = 0.0f, back = 0.0f, R = 0.0f, Dm = 0.0f, Gm = 0.0f;
   for (int t = gl; t < Tc; t += G) {
     const float x0 = th[t], x1 = th[t + 1], h = x1 - x0;
     if (!isfinite(h)) bad = 1.0f;
     dev = fmaxf(dev, fabsf(h - hb));
     drift = fmaxf(drift, fabsf((x1 - th0) - (float)(t + 1) * hb));
     hmax = fmaxf(hmax, fabsf(h));
+    back += fmaxf(-h, 0.0f);
   }
   if (gl < a.K) {
     const cf u = load_u(a.params, gl);
     R = absv(u);
     Dm = fmaxf(0.0f, -u.re);
+    Gm = fmaxf(0.0f, u.re);
     if (!isfinite(R)) bad = 1.0f;
   }
   dev = group_max<G>(dev);
@@ -254,11 +256,13 @@ __device__ __forceinline__ int classify(const DiagArgs& a, int b, int t0, int Tc
   bad = group_max<G>(bad);
   R = group_max<G>(R);
   Dm = group_max<G>(Dm);
+  Gm = group_max<G>(Gm);
+  back = lanes::sum_n(back, G);
   const bool fin = bad == 0.0f && isfinite(tau);
   const float lim = 4.76837158e-7f;  // 2^-21
   const bool uni = fin && dev * 2.0f * R < 1.52587890625e-5f;
   const bool strict = uni && R * dev <= lim && R * drift <= lim;
-  const bool inv = fin && 2.0f * Dm * tau <= 0.69314718f;
+  const bool inv = fin && invert_growth(tau, back, Dm, Gm) <= 0.69314718f;
   const bool small = fin && poly_order_ok(a.sq1, a.sq2) && 2.0f * R * hmax <= kPolyR;
   return (uni ? kUniform : 0) | (inv ? kInvert : 0) | (small ? kSmall : 0) | (strict ? kStrict : 0);
 }

@@ -23,20 +23,23 @@ def _rel(a, b):
     return float((a - b).abs().max() / b.abs().max().clamp_min(1e-300))
 
 
-def _check(structure, d, N, B, L, steps, damp, readout="prefix", chunk=0, bf16=False, flow="per_interval"):
-    """steps (L,): the clock's steps (the first unused)."""
+def _check(structure, d, N, B, L, steps, damp, readout="prefix", chunk=0, bf16=False, flow="per_interval", freq=3.0,
+           rows=None, clock_grad=True):
+    """steps (L,): the clock's steps (the first unused). rows: the prefix rows that the loss sees (all)."""
     rng = np.random.default_rng(L + d)
     path = torch.tensor(np.cumsum(rng.normal(size=(B, L, d)) * 0.2, 1), dtype=torch.float32)
     path = path.to(torch.bfloat16) if bf16 else path
     clock = torch.tensor(np.cumsum(np.stack([steps * rng.uniform(0.9, 1.1) for _ in range(B)]), 1), dtype=torch.float32)
     if structure == "planes":
-        w = torch.tensor(np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, 3.0, d // 2)], -1), dtype=torch.float32)
+        w = torch.tensor(np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, freq, d // 2)], -1), dtype=torch.float32)
     else:
         w = torch.tensor(rng.uniform(*damp, d), dtype=torch.float32)
-    p, c, q = path.to(DEV).requires_grad_(), clock.to(DEV).requires_grad_(), w.to(DEV).requires_grad_()
+    p, c, q = path.to(DEV).requires_grad_(), clock.to(DEV).requires_grad_(clock_grad), w.to(DEV).requires_grad_()
     out = ops.diag_scan(p, c, q, N, structure, flow, readout, True, chunk=chunk)
     g = torch.tensor(rng.normal(size=tuple(out.shape)), dtype=torch.float32)
-    got = torch.autograd.grad(out, [p, c, q], g.to(DEV))
+    if rows is not None:
+        g[:, rows:] = 0.0
+    got = torch.autograd.grad(out, [p, q] + ([c] if clock_grad else []), g.to(DEV))
     rp, rc, rq = (x.double().requires_grad_() for x in (path, clock, w))
     if structure == "planes":
         A = torch.block_diag(*[torch.stack([torch.stack([r[0], r[1]]), torch.stack([-r[1], r[0]])]) for r in rq])
@@ -45,11 +48,11 @@ def _check(structure, d, N, B, L, steps, damp, readout="prefix", chunk=0, bf16=F
     mode = {"per_interval": "displacement", "cached": "displacement_uniform"}[flow]
     ref = O.ews(rp, rc, A, N, readout, leaf="plane_closed" if structure == "planes" else "diag_closed",
                 reweighting_mode=mode, terminal_reduce="assoc")
-    want = torch.autograd.grad(ref, [rp, rc, rq], g.double())
+    want = torch.autograd.grad(ref, [rp, rq] + ([rc] if clock_grad else []), g.double())
     errs = [_rel(out, ref)] + [_rel(a, b) for a, b in zip(got, want)]
     print(f"{structure} d={d} N={N} B={B} L={L} {readout} chunk={chunk} errs={['%.1e' % e for e in errs]}", flush=True)
     assert errs[0] < 1e-5, errs
-    assert errs[1] < (1e-2 if bf16 else 1e-4) and errs[2] < 1e-4 and errs[3] < 1e-4, errs
+    assert errs[1] < (1e-2 if bf16 else 1e-4) and max(errs[2:]) < 1e-4, errs
 
 
 def _steps(L, lo, hi, seed=0):
@@ -89,6 +92,18 @@ def test_small_steps_bf16_path(d):
 
 def test_small_steps_cached_flow():
     _check("planes", 6, 2, 2, 70, _steps(70, 0.002, 0.02), (0.01, 1.0), flow="cached")
+
+
+@pytest.mark.parametrize("structure,d,N", [("planes", 16, 2), ("planes", 12, 2), ("planes", 24, 2), ("planes", 10, 1),
+                                           ("real_diag", 9, 2), ("real_diag", 5, 1)])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_clock_that_turns(structure, d, N, sign):
+    """A clock that turns inside a chunk: its net step is near zero, but the states contract by e^11 on the way (sign -1:
+    a growing generator on a clock that starts backwards), so that the steps cannot be inverted from the chunk's end.
+    The loss sees the first rows only, or all of them."""
+    s = sign * np.r_[0.0, np.full(32, 0.17), np.full(32, -0.17), _steps(60, 0.1, 0.17)]
+    for rows in (8, None):
+        _check(structure, d, N, 2, len(s), s, sorted((0.9 * sign, sign)), chunk=64, freq=0.2, rows=rows)
 
 
 def test_suited_chunk_lengths():
