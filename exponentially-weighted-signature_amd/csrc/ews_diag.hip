@@ -20,7 +20,7 @@
 //            checkpoints) -> B4 knot gradients and parameter reductions.
 // Per-step coefficients: when every clock step of a chunk is within 2^-16 / (2 max|mu|) of the chunk mean
 // (a uniform clock in float32), coefficients are first-order Taylor models in h around the mean (error
-// below float32 rounding); else, while every step is small (2 max|u| |h| <= kPolyR), they are polynomials in h whose
+// below float32 rounding); else, while every step is small (poly_small), they are polynomials in h whose
 // coefficients each lane forms once (PolyCoef); otherwise they are evaluated exactly per step.
 #include <hip/hip_runtime.h>
 
@@ -357,7 +357,7 @@ __device__ __forceinline__ ChunkClock chunk_classify(const DiagArgs& a, int b, i
   }
   const bool finite = bad == 0.0f && isfinite(s);
   cc.fast = finite && (dmax * 2.0f * R < 1.52587890625e-5f);  // 2^-16
-  cc.small = finite && poly_order_ok(a.sq1, a.sq2) && 2.0f * R * hmax <= kPolyR;
+  cc.small = finite && poly_order_ok(a.sq1, a.sq2) && poly_small(R, hmax);
   if (!cc.per_int) {  // cached flows: every step flows over href (a backward one at either rate)
     s = fabsf(cc.href) * (float)Tc;
     back = 0.0f;

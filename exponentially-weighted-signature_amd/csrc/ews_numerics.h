@@ -279,6 +279,14 @@ EWS_HD float invert_growth(float net, float back, float decay, float growth) {
   return 2.0f * (decay * (net + back) + growth * back);
 }
 
+// The powers of u and of h are formed apart: up to these bounds (a clock in raw seconds has steps of thousands) the largest,
+// (2u)^7 < 2^119 and h^7 = 2^84, stay in the float32 range, and where the other factor's underflow its terms are far below
+// rounding. Outside them the closed forms in h u serve (|u| above 9e5 gave inf times 0, |h| above 3e5 in the moments).
+constexpr float kPolyMaxU = 65536.0f, kPolyMaxH = 4096.0f;
+EWS_HD bool poly_small(float umax, float hmax) {  // a NaN is not small
+  return 2.0f * umax * hmax <= kPolyR && umax <= kPolyMaxU && hmax <= kPolyMaxH;
+}
+
 EWS_HD bool poly_order_ok(int q1, int q2) { return (q1 == 0 || q1 >= kPolyPhi) && (q2 == 0 || q2 >= kPolyD); }
 
 template <class T> EWS_HD void poly_phi(T u, T* c) {  // c[m] = u^m / (m+1)!

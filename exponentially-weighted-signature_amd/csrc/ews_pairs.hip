@@ -452,7 +452,7 @@ __device__ __forceinline__ void fwd_coef(const DiagArgs& a, const Lane& l, float
 // ------------------------------------------------------------------------------------------------ classification
 // Chunk c of sample b: flag bit 0 = uniform steps (coefficients at the mean step hbar), bit 1 = the steps may be
 // inverted backwards (stepping back grows errors by at most 2 over the chunk: invert_growth), bit 2 = the coefficient
-// table applies, bit 3 = small steps (2 max|u| |h| <= kPolyR: the coefficients as polynomials in h). Evaluated by the 16
+// table applies, bit 3 = small steps (poly_small: the coefficients as polynomials in h). Evaluated by the 16
 // lanes of the chunk's group, each over every 16th step, then combined with DPP inside the group.
 __device__ __forceinline__ float row_max16(float v) {
   v = fmaxf(v, EWS_ROR(v, 8));
@@ -499,7 +499,7 @@ __device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int c, i
   const bool uni = fin && R * dev <= lim && R * drift <= lim;
   const bool inv = fin && 2.0f * Dm * fabsf(tau) <= 0.69314718f && invert_growth(tau, back, Dm, Gm) <= 0.69314718f;
   const bool tab = uni && R * fabsf(hb - a.ctab[0]) <= 0.5f * lim;  // the coefficient table applies
-  const bool small = fin && 2.0f * R * hmax <= kPolyR;
+  const bool small = fin && poly_small(R, hmax);
   return (uni ? 1 : 0) | (inv ? 2 : 0) | (tab ? 4 : 0) | (small ? 8 : 0);
 }
 

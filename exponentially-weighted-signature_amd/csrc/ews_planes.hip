@@ -263,7 +263,7 @@ __device__ __forceinline__ int classify(const DiagArgs& a, int b, int t0, int Tc
   const bool uni = fin && dev * 2.0f * R < 1.52587890625e-5f;
   const bool strict = uni && R * dev <= lim && R * drift <= lim;
   const bool inv = fin && invert_growth(tau, back, Dm, Gm) <= 0.69314718f;
-  const bool small = fin && poly_order_ok(a.sq1, a.sq2) && 2.0f * R * hmax <= kPolyR;
+  const bool small = fin && poly_order_ok(a.sq1, a.sq2) && poly_small(R, hmax);
   return (uni ? kUniform : 0) | (inv ? kInvert : 0) | (small ? kSmall : 0) | (strict ? kStrict : 0);
 }
 

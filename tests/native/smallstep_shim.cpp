@@ -6,6 +6,8 @@ using ews::cf;
 extern "C" {
 int shim_degrees(int which) { return which == 0 ? ews::kPolyPhi : ews::kPolyD; }
 float shim_radius() { return ews::kPolyR; }
+int shim_small(float umax, float hmax) { return ews::poly_small(umax, hmax); }
+float shim_max(int which) { return which == 0 ? ews::kPolyMaxU : ews::kPolyMaxH; }
 // phi(h u), its d/dh, exp[0, h u, h v] and its d/dh: out n x 8 (re, im)
 void shim_poly(int n, const float* h, const float* u, const float* v, float* out) {
   for (int i = 0; i < n; ++i) {

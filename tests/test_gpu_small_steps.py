@@ -106,6 +106,17 @@ def test_clock_that_turns(structure, d, N, sign):
         _check(structure, d, N, 2, len(s), s, sorted((0.9 * sign, sign)), chunk=64, freq=0.2, rows=rows)
 
 
+@pytest.mark.parametrize("structure,d", [("planes", 16), ("planes", 12), ("planes", 24), ("real_diag", 9)])
+@pytest.mark.parametrize("unit", [2.0**-20, 2.0**26, 2.0**13])
+@pytest.mark.parametrize("regular", [False, True])
+def test_units_of_the_clock(structure, d, unit, regular):
+    """The same problem with the clock in other units: steps near 1e-8 or 1e6, generators near 1e6 or 1e-8, whose powers
+    leave the float32 range where h u does not."""
+    L = 83
+    s = np.full(L, 2.0**-6) if regular else _steps(L, 0.002, 0.028)
+    _check(structure, d, 2, 2, L, s * unit, (0.01 / unit, 1.0 / unit), freq=3.0 / unit, clock_grad=not regular)
+
+
 def test_suited_chunk_lengths():
     """The library's choice: 64 intervals where there are many, 16 where few, 0 on the sequential kernels, and an
     error code (never a choice) for a descriptor it refuses."""

@@ -20,7 +20,8 @@ def shim(tmp_path_factory):
     subprocess.check_call(["g++", "-O2", "-shared", "-fPIC", "-I", CSRC, "-o", str(out),
                            os.path.join(HERE, "native", "smallstep_shim.cpp")])
     lib = ctypes.CDLL(str(out))
-    lib.shim_radius.restype = ctypes.c_float
+    lib.shim_radius.restype = lib.shim_max.restype = ctypes.c_float
+    lib.shim_small.argtypes = [ctypes.c_float, ctypes.c_float]
     return lib
 
 
@@ -79,3 +80,30 @@ def test_node_cotangents_through_moments(shim):
     size = float(np.sum(h * np.abs(g)))
     for k in range(3):  # float32 sums of 64 terms: 64 roundings of the summed magnitudes at most
         assert abs(got[k] - ref[k]) <= 64 * 6e-8 * size, (k, got[k], ref[k])
+
+
+@pytest.mark.parametrize("side", [0, 1])
+def test_at_the_bounds_of_u_and_h(shim, side):
+    """At the largest generator with its steps, and at the largest step with its generators: the values and the node
+    cotangents are those of the same h u in moderate units; past either bound the model is refused."""
+    R = shim.shim_radius()
+    U, H = (shim.shim_max(0), R / 2 / shim.shim_max(0)) if side == 0 else (R / 2 / shim.shim_max(1), shim.shim_max(1))
+    assert shim.shim_small(U * (1 - 1e-6), H * (1 - 1e-6))
+    assert not shim.shim_small(U * (1.01 if side == 0 else 1.0), H / 2 if side == 0 else H * 1.01)
+    assert not shim.shim_small(float("nan"), H) and not shim.shim_small(U, float("nan"))
+    rng = np.random.default_rng(9)
+    n, k = 40, 2.0 ** (round(math.log2(U)))  # a power of two: the same problem in moderate units
+    u = (U * np.exp(1j * rng.uniform(0, 2 * np.pi, n))).astype(np.complex64)
+    v = (2 * U * np.exp(1j * rng.uniform(0, 2 * np.pi, n))).astype(np.complex64)
+    h = (rng.uniform(0.1, 1.0, n) * H).astype(np.float32)
+    g = (rng.normal(size=n) + 1j * rng.normal(size=n)).astype(np.complex64)
+    outs = []
+    for f in (1.0, k):
+        uf, vf, hf = (u / f).astype(np.complex64), (v / f).astype(np.complex64), (h * f).astype(np.float32)
+        a, b = np.zeros((n, 8), np.float32), np.zeros(6, np.float32)
+        shim.shim_poly(n, _ptr(hf), _ptr(_f(uf)), _ptr(_f(vf)), _ptr(a))
+        shim.shim_moments(n, _ptr(hf), _ptr(_f(g)), _ptr(_f(uf[:1])), _ptr(_f(vf[:1])), _ptr(b))
+        a = a.reshape(n, 4, 2) * np.array([1.0, f, 1.0, f])[None, :, None]  # d/dh scales with u
+        outs.append((a, b / f))
+    for x, y in zip(*outs):
+        assert np.isfinite(x).all() and np.max(np.abs(x - y)) <= 1e-6 * np.max(np.abs(y))
