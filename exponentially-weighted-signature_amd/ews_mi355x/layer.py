@@ -158,9 +158,10 @@ class EWS(torch.nn.Module):
 
     def _diag_params(self, device, a_scale):
         """Kernel parameters as ews/core/leaf.py:130-131 reads them off the materialised A times a_scale: straight from
-        the parametrisation where it holds them, else off A (row 0 of every 2 x 2 block, or the diagonal). a_scale
-        None: unscaled, moved to the path's device."""
-        rows = kernel_rows(self.A_param)
+        the parametrisation where it holds them, else off A (row 0 of every 2 x 2 block, or the diagonal); a scale
+        with dimensions of its own broadcasts against A. a_scale None: unscaled, moved to the path's device."""
+        one = a_scale is None or isinstance(a_scale, (int, float)) or torch.as_tensor(a_scale).dim() == 0
+        rows = kernel_rows(self.A_param) if one else None
         A = self.A_param() if rows is None else rows
         A = A.to(device, torch.float32) if a_scale is None else self._scaled(A, a_scale, device)
         if rows is not None:
