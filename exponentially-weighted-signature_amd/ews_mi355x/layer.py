@@ -146,14 +146,17 @@ class EWS(torch.nn.Module):
 
     @staticmethod
     def _scaled(A, a_scale, device):
-        """A times a_scale in float32 (a plain number needs no tensor on the device, and 1 no product). A has to be on
-        the path's device."""
+        """A times a_scale in float32 (a plain number needs no tensor on the device). A has to be on the path's device.
+        A scale of 1 needs no product where A is an operation's own output or nothing is recorded; a parameter or buffer
+        is copied, so that a step taken on it in place leaves the operand saved for the backward as it was."""
         A = A.to(torch.float32)
         if device.type != "cpu" and A.device != device:
             raise RuntimeError("Expected all tensors to be on the same device, but found the generator on "
                                f"{A.device} and the path on {device}")
         if isinstance(a_scale, (int, float)):
-            return A if a_scale == 1 else A * float(a_scale)
+            if a_scale == 1 and (not torch.is_grad_enabled() or (A.grad_fn is not None and not A._is_view())):
+                return A
+            return A * float(a_scale)
         return A * torch.as_tensor(a_scale, dtype=torch.float32, device=device)
 
     def _diag_params(self, device, a_scale):

@@ -1,5 +1,6 @@
 """How a layer hands its generator to the kernels: a_scale of every shape that broadcasts against A, numbers on the
-parameters' rows and tensors of A's shape on the entries read off A."""
+parameters' rows and tensors of A's shape on the entries read off A, and a generator that is the module's own storage
+(the kernels' operand, saved for the backward, is no alias of it while gradients are recorded)."""
 
 import numpy as np
 import pytest
@@ -45,3 +46,12 @@ def test_learned_scale_gets_its_gradient():
             layer._diag_params(CPU, s).square().sum().backward()
             _read(layer.structure, layer.A_param() * r).square().sum().backward()
             assert torch.allclose(s.grad, r.grad, rtol=1e-6)
+
+
+def test_no_alias_of_the_modules_own_storage():
+    for p in (E.AParamConstant(torch.randn(4, 4)), E.AParamGeneral(torch.randn(4, 4))):
+        own = next(iter(p.state_dict().values()))
+        A = E.EWS._scaled(p(), 1.0, CPU)
+        assert A.data_ptr() != own.data_ptr()
+        with torch.no_grad():  # nothing is saved: the tensor itself serves
+            assert E.EWS._scaled(p(), 1.0, CPU).data_ptr() == own.data_ptr()
