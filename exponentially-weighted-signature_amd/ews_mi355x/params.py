@@ -304,9 +304,9 @@ def _hooked(module):
 
 def kernel_rows(a_param):
     """The diagonal kernels' parameters, (d/2, 2) plane rows (d_j, w_j) or the (d,) diagonal, straight from a
-    parametrisation whose forward is one of this module's own (the exact class, no hooks), without forming A; None
-    for any other, whose A has to be read."""
-    if _hooked(a_param):
+    parametrisation whose forward is one of this module's own (the exact class, no hooks, no forward set on the
+    instance), without forming A; None for any other, whose A has to be read."""
+    if _hooked(a_param) or "forward" in vars(a_param):
         return None
     if type(a_param) in (AParamBoundedRotation, AParamDampedRotation):
         return a_param.plane_params()

@@ -1,12 +1,14 @@
 """How a layer hands its generator to the kernels: a_scale of every shape that broadcasts against A, numbers on the
-parameters' rows and tensors of A's shape on the entries read off A, and a generator that is the module's own storage
-(the kernels' operand, saved for the backward, is no alias of it while gradients are recorded)."""
+parameters' rows and tensors of A's shape on the entries read off A; a generator that is the module's own storage (the
+kernels' operand, saved for the backward, is no alias of it while gradients are recorded); a parametrisation whose
+forward was replaced on the instance."""
 
 import numpy as np
 import pytest
 import torch
 
 import ews_mi355x as E
+from ews_mi355x.params import kernel_rows
 
 CPU = torch.device("cpu")
 D = 6
@@ -55,3 +57,10 @@ def test_no_alias_of_the_modules_own_storage():
         assert A.data_ptr() != own.data_ptr()
         with torch.no_grad():  # nothing is saved: the tensor itself serves
             assert E.EWS._scaled(p(), 1.0, CPU).data_ptr() == own.data_ptr()
+
+
+def test_forward_replaced_on_the_instance():
+    p = E.AParamEFM(torch.randn(D))
+    assert kernel_rows(p) is not None
+    p.forward = lambda: torch.diag(p.theta.exp())
+    assert kernel_rows(p) is None
