@@ -643,15 +643,19 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
     tot += fabs(mode_step(th, a.L, t, (double)th[t + 1] - (double)th[t], a.flow_mode));
   }
   for (int o = 1; o < a.KP; o <<= 1) tot += __shfl_xor(tot, o, 64);
-  const bool invert = !__any(live && !((fabs(c.re) + fabs(eps)) * tot <= kInvert));
   zd S[M], v[M], xc[M], xn[M];
+  double end = 0.0;  // finite if the chunk's end state is: padding with NaN must not reach the rows before it
+  if (live) {
+    ld_state<M>(a.carries + st_off(a, l.b, l.c + 1, l.j), S);
+#pragma unroll
+    for (int i = 0; i < M; ++i) end += fabs(S[i].re) + fabs(S[i].im);
+  }
+  const bool invert = !__any(live && !((fabs(c.re) + fabs(eps)) * tot <= kInvert && isfinite(end)));
   Knot<M, CPLX> x1, x2;
   // the states of the lane's steps, (B, n, K, M) pairs
   float2* my = a.st + (((size_t)l.b * a.n + l.t0) * a.K + l.j) * M;
   const size_t my_step = (size_t)a.K * M;
-  if (invert) {
-    if (live) ld_state<M>(a.carries + st_off(a, l.b, l.c + 1, l.j), S);
-  } else if (live) {
+  if (!invert && live) {
     Coef<M> k;
     zd x0[M];
     ld_state<M>(a.carries + st_off(a, l.b, l.c, l.j), S);

@@ -79,3 +79,26 @@ def test_reference_step_shares(chunk):
         errs = [_rel(out, ref), _rel(gp, wp), _rel(gc, wc)]
         print(flow, chunk, errs)
         assert errs[0] < 1e-5 and errs[1] < 1e-4 and errs[2] < 1e-4, errs
+
+
+@pytest.mark.parametrize("kind,size,K", [("real", 1, 5), ("real", 2, 3), ("complex", 2, 4), ("complex", 4, 4)])
+@pytest.mark.parametrize("chunk", [0, 32, 64])
+def test_rows_before_missing_values(kind, size, K, chunk):
+    """Recordings padded with NaN, the loss on rows before the padding: the path's and the clock's gradients there are
+    those of the recordings cut before it (the states before a step never come from a chunk's end that is not finite)."""
+    rng = np.random.default_rng(8)
+    B, L, cut, seen = 2, 64, 45, 40
+    path = torch.tensor(np.cumsum(rng.normal(size=(B, L, K * size)) * 0.3, 1), dtype=torch.float32)
+    path[:, cut:] = float("nan")
+    clock = torch.tensor(np.cumsum(rng.uniform(0.0, 0.02, size=(B, L)), 1), dtype=torch.float32).to(DEV)
+    A = _generator(kind, size, K, (0.3, 0.01), 3).to(DEV)
+    g = torch.tensor(rng.normal(size=(B, seen, 1 + K * size)), dtype=torch.float32).to(DEV)
+    res = []
+    for n in (L, cut):
+        p, c = path[:, :n].to(DEV).requires_grad_(), clock[:, :n].clone().requires_grad_()
+        out = ops.chain_scan(p, c, A, kind, size, chunk=chunk)
+        res.append(torch.autograd.grad((out[:, :seen] * g).sum(), [p, c]))
+    (gp, gc), (wp, wc) = res
+    errs = [_rel(gp[:, :cut], wp.cpu()), _rel(gc[:, :cut - 1], wc[:, :cut - 1].cpu())]
+    print(kind, size, chunk, errs)
+    assert errs[0] < 1e-5 and errs[1] < 1e-5, errs
