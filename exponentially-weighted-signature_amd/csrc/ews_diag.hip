@@ -485,6 +485,13 @@ __global__ __launch_bounds__(MAXT) void k_chunk_fwd(DiagArgs a) {
   ChunkClock cc;
   if (kClassify && !a.pw) {
     cc = chunk_classify<T>(a, b, Tc, s_h);
+    if constexpr (N == 1) {
+      // A chunk with a NaN or infinite increment is not inverted (it takes exact coefficients and the recomputing adjoint):
+      // at depth 1 the gradients of the rows before the increment do not depend on it, unless through the chunk's end
+      bool ok = true;
+      for (int i = tid & 63; i < Tc * a.d; i += 64) ok = ok && isfinite(s_v[i]);
+      cc.small = cc.small && __all(ok);
+    }
     if (tid == 0) {
       a.cflag[b * a.C + c] = (cc.fast ? kFlagUniform : 0) | (cc.inv_ok ? kFlagInvert : 0) | (cc.small ? kFlagSmall : 0);
       a.chbar[b * a.C + c] = cc.hbar;

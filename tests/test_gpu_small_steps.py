@@ -131,3 +131,26 @@ def test_suited_chunk_lengths():
     assert suited(256, 512, 32, nat.STRUCT_REAL_DIAG, readout="log_prefix") == 0
     assert suited(2, 100, 16, chunk=40) == 40
     assert suited(2, 100, 34) < 0
+
+
+@pytest.mark.parametrize("structure,d", [("planes", 10), ("real_diag", 5)])
+@pytest.mark.parametrize("chunk", [16, 64])
+def test_depth1_rows_before_missing_values(structure, d, chunk):
+    """Recordings padded with NaN at depth 1, the loss on rows before the padding: the path's and the clock's gradients
+    there are those of the recordings cut before it."""
+    rng = np.random.default_rng(8)
+    B, L, cut, seen = 2, 64, 45, 40
+    path = torch.tensor(np.cumsum(rng.normal(size=(B, L, d)) * 0.3, 1), dtype=torch.float32)
+    path[:, cut:] = float("nan")
+    clock = torch.tensor(np.cumsum(rng.uniform(0.001, 0.02, size=(B, L)), 1), dtype=torch.float32).to(DEV)
+    w = torch.tensor(rng.uniform(0.01, 0.4, size=(d // 2, 2) if structure == "planes" else d), dtype=torch.float32)
+    g = torch.tensor(rng.normal(size=(B, seen, 1 + d)), dtype=torch.float32).to(DEV)
+    res = []
+    for n in (L, cut):
+        p, c = path[:, :n].to(DEV).requires_grad_(), clock[:, :n].clone().requires_grad_()
+        out = ops.diag_scan(p, c, w.to(DEV), 1, structure, "per_interval", "prefix", True, chunk=chunk)
+        res.append(torch.autograd.grad((out[:, :seen] * g).sum(), [p, c]))
+    (gp, gc), (wp, wc) = res
+    errs = [_rel(gp[:, :cut], wp.cpu()), _rel(gc[:, :cut - 1], wc[:, :cut - 1].cpu())]
+    print(structure, chunk, errs)
+    assert errs[0] < 1e-5 and errs[1] < 1e-5, errs
