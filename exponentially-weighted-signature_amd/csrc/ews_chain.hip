@@ -91,7 +91,7 @@ struct CArgs {
   double* mt;       // (B, C, K, M) complex: the cotangent at the chunk's end from the later chunks
   float* dvb;       // (B, C, 2, d) increment cotangents of each chunk's first and last interval
   float* dhb;       // (B, C, 2) step cotangents of those (every chain's)
-  float2* st;       // (B, n, K, M) states before each step, of the chunks whose steps are not inverted
+  float* st;        // (B, n, d) states before each step, of the chunks whose steps are not inverted
   double* pp;       // (B, C, K, 5): partials of Re c, Im c, eps, and of the reference steps theta1-theta0, theta2-theta1
   float* gpath;
   float* gclock;
@@ -620,11 +620,12 @@ __global__ __launch_bounds__(kCarryThreads) void k_carry_bwd(CArgs a) {
 // Each chunk from the cotangent at its end: the steps in reverse with the increment and step cotangents and the
 // chain-parameter partials. The states S_{t-1} come from inverting each step from the chunk's end state in float64
 // while the whole chunk contracts by less than e^kInvert (errors then stay below 1e-12, where states kept in float32
-// had 6e-8); a wavefront with a stronger contraction first recomputes its states from the carry into st. The sweep keeps the interval after in registers, so
-// a chunk's interior knot gradients dX_{t+1} = dv_t - dv_{t+1} (and the clock's) are written here; the cotangents of
-// its first and last interval go to dvb / dhb for the boundary knots (k_bounds). Bound by float64 issue: at B = 8,
-// L = 49,920, 16 complex chains of two coordinates, 543 us with the 28-term series at every step, the states
-// recomputed into LDS (one wavefront per SIMD) and dv, dh through memory; 171 us now (the step 1.12 -> 0.60 ms).
+// had 6e-8); a wavefront with a stronger contraction, or an end state that is not finite, first recomputes its states from
+// the carry into st. The sweep keeps the interval after in registers, so a chunk's interior knot gradients
+// dX_{t+1} = dv_t - dv_{t+1} (and the clock's) are written here; the cotangents of its first and last interval go to dvb /
+// dhb for the boundary knots (k_bounds). Bound by float64 issue: at B = 8, L = 49,920, 16 complex chains of two
+// coordinates, 543 us with the 28-term series at every step, the states recomputed into LDS (one wavefront per SIMD) and
+// dv, dh through memory; 171 us now (the step 1.12 -> 0.60 ms).
 template <int M, bool CPLX>
 __global__ __launch_bounds__(64) void k_full(CArgs a) {
   constexpr int NX = CPLX ? 2 * M : M;
@@ -652,9 +653,7 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
   }
   const bool invert = !__any(live && !((fabs(c.re) + fabs(eps)) * tot <= kInvert && isfinite(end)));
   Knot<M, CPLX> x1, x2;
-  // the states of the lane's steps, (B, n, K, M) pairs
-  float2* my = a.st + (((size_t)l.b * a.n + l.t0) * a.K + l.j) * M;
-  const size_t my_step = (size_t)a.K * M;
+  float* my = a.st + ((size_t)l.b * a.n + l.t0) * a.d + (size_t)l.j * NX;  // the states of the lane's steps
   if (!invert && live) {
     Coef<M> k;
     zd x0[M];
@@ -665,8 +664,7 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
     float th1 = th[l.t0 + 1];
     for (int s = 0; s < l.Tc; ++s) {
       const int t = l.t0 + s, tn = l.t0 + min(s + 2, l.Tc);
-#pragma unroll
-      for (int i = 0; i < M; ++i) my[s * my_step + i] = float2{(float)S[i].re, (float)S[i].im};
+      st_row<M, CPLX>(my + (size_t)s * a.d, S);
       if (s == l.Tc - 1) break;
       x2.load(a, l.b, tn, l.j);
       const float th2 = th[tn];
@@ -777,11 +775,9 @@ __global__ __launch_bounds__(64) void k_full(CArgs a) {
           Sp[i] = ei * r;
         }
       } else {
-#pragma unroll
-        for (int i = 0; i < M; ++i) {
-          const float2 w = my[s * my_step + i];
-          Sp[i] = Z((double)w.x, (double)w.y);
-        }
+        Knot<M, CPLX> w;
+        w.row(my + (size_t)s * a.d);
+        w.get(Sp);
       }
 #pragma unroll
       for (int i = 0; i < M; ++i) S[i] = Sp[i];
@@ -1157,7 +1153,7 @@ WsOff ws_off(const CArgs& a) {
   w.dvb = o; o += al256c((size_t)a.B * a.C * 2 * a.d * 4);
   w.dhb = o; o += al256c((size_t)a.B * a.C * 2 * 4);
   w.pp = o; o += al256c((size_t)a.B * a.C * a.K * 5 * 8);
-  w.st = o; o += al256c((size_t)a.B * a.n * a.K * a.M * 8);
+  w.st = o; o += al256c((size_t)a.B * a.n * a.d * 4);
   w.total = o;
   return w;
 }
@@ -1274,7 +1270,7 @@ int ews_chain_backward(const ews_chain_desc* desc, const void* path, const float
   a.dvb = (float*)(ws + w.dvb);
   a.dhb = (float*)(ws + w.dhb);
   a.pp = (double*)(ws + w.pp);
-  a.st = (float2*)(ws + w.st);
+  a.st = (float*)(ws + w.st);
   a.gpath = grad_path;
   a.gclock = grad_clock;
   a.gA = grad_A;
