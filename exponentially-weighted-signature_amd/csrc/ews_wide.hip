@@ -1125,8 +1125,8 @@ __global__ __launch_bounds__(NT) void k_wmat_bwd_series_smp(WArgs a, int hslot0)
   if (do_vl) {
     bool fixed;
     const float c = vl_step(a, th, 1, fixed);
+    sv = true;  // a fixed pair (zero shared step): zero, which the clock's gradient reads
     if (!fixed) {
-      sv = true;
       float4 GP = float4{0.0f, 0.0f, 0.0f, 0.0f}, GV = GP;
 #pragma unroll 8
       for (int s2 = 0; s2 < a.NSL; ++s2) {
