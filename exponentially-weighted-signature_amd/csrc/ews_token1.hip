@@ -183,6 +183,7 @@ __global__ void k_reduce(TArgs a) {
 // the steps are on the chain for 1. B = 256 x 512 tokens, d = 64, BS = 2: forward 50 -> 28 us, backward 110 -> 39 us at
 // NW = 8. Blocks of 6 and 8, whose lane exchanges go through LDS, keep NW = 1.
 constexpr int kStageFloats = 12288;  // caches staged in LDS up to 48 KB
+template <int BS> constexpr bool kSpans = BS <= 4;  // block sizes whose samples are split into spans
 
 template <bool STAGED>
 __device__ __forceinline__ float blk_d(const TArgs& a, const float* sD, int BS, int g, int row, int r) {
@@ -314,22 +315,25 @@ template <int BS, bool STAGED>
 __device__ __forceinline__ void fwd_blk_body(const TArgs& a, const float* sP, const float* sD, double* sX) {
   const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
-  double S = 0.0, U[BS];
-  if (nw > 1) {
-    if (w + 1 < nw) {
+  double S = 0.0;
+  if constexpr (kSpans<BS>) {
+    if (nw > 1) {
+      double U[BS];
+      if (w + 1 < nw) {
 #pragma unroll
-      for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
-      fwd_blk_steps<BS, STAGED, true>(a, sP, sD, b, i, tb, te, S, U);
-      double* x = sX + (size_t)w * (BS + 1) * 64 + i;
+        for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
+        fwd_blk_steps<BS, STAGED, true>(a, sP, sD, b, i, tb, te, S, U);
+        double* x = sX + (size_t)w * (BS + 1) * 64 + i;
 #pragma unroll
-      for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
-      x[BS * 64] = S;
-    }
-    __syncthreads();
-    S = 0.0;
-    for (int u = 0; u < w; ++u) {
-      const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
-      S = span_apply<BS>(x[BS * 64], x, 64, S, base);
+        for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
+        x[BS * 64] = S;
+      }
+      __syncthreads();
+      S = 0.0;
+      for (int u = 0; u < w; ++u) {
+        const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
+        S = span_apply<BS>(x[BS * 64], x, 64, S, base);
+      }
     }
   }
   float S0 = (float)S;
@@ -337,7 +341,7 @@ __device__ __forceinline__ void fwd_blk_body(const TArgs& a, const float* sP, co
 }
 
 template <int BS>
-__global__ __launch_bounds__(512) void k_fwd_blk(TArgs a) {
+__global__ __launch_bounds__(kSpans<BS> ? 512 : 64) void k_fwd_blk(TArgs a) {
   extern __shared__ double s_c[];
   double* sX = s_c;  // (NW, BS + 1, 64): the spans' maps
   float* sP = reinterpret_cast<float*>(sX + (size_t)(blockDim.x >> 6) * (BS + 1) * 64);
@@ -437,22 +441,25 @@ template <int BS, bool STAGED>
 __device__ __forceinline__ void bwd_blk_body(const TArgs& a, const float* sD, float* sAcc, double* sX) {
   const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
-  double lam = 0.0, U[BS];
-  if (nw > 1) {
-    if (w > 0) {
+  double lam = 0.0;
+  if constexpr (kSpans<BS>) {
+    if (nw > 1) {
+      double U[BS];
+      if (w > 0) {
 #pragma unroll
-      for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
-      bwd_blk_steps<BS, STAGED, true>(a, sD, nullptr, b, i, tb, te, lam, U);
-      double* x = sX + (size_t)w * (BS + 1) * 64 + i;
+        for (int c = 0; c < BS; ++c) U[c] = i - base == c ? 1.0 : 0.0;
+        bwd_blk_steps<BS, STAGED, true>(a, sD, nullptr, b, i, tb, te, lam, U);
+        double* x = sX + (size_t)w * (BS + 1) * 64 + i;
 #pragma unroll
-      for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
-      x[BS * 64] = lam;
-    }
-    __syncthreads();
-    lam = 0.0;
-    for (int u = nw - 1; u > w; --u) {
-      const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
-      lam = span_apply<BS>(x[BS * 64], x, 64, lam, base);
+        for (int c = 0; c < BS; ++c) x[c * 64] = U[c];
+        x[BS * 64] = lam;
+      }
+      __syncthreads();
+      lam = 0.0;
+      for (int u = nw - 1; u > w; --u) {
+        const double* x = sX + (size_t)u * (BS + 1) * 64 + i;
+        lam = span_apply<BS>(x[BS * 64], x, 64, lam, base);
+      }
     }
   }
   float lam0 = (float)lam;
@@ -460,7 +467,7 @@ __device__ __forceinline__ void bwd_blk_body(const TArgs& a, const float* sD, fl
 }
 
 template <int BS>
-__global__ __launch_bounds__(512) void k_bwd_blk(TArgs a) {
+__global__ __launch_bounds__(kSpans<BS> ? 512 : 64) void k_bwd_blk(TArgs a) {
   extern __shared__ double s_c[];
   const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const bool staged = (size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats;
@@ -543,7 +550,7 @@ size_t blk_lds_bytes(const ews_token1_desc* s, int nw, bool bwd) {
   return (staged + 2 * maps + (bwd ? maps * s->vocab : 0)) * 4;
 }
 int blk_waves(const ews_token1_desc* s) {
-  int nw = s->block <= 4 ? 8 : 1;
+  int nw = s->block <= 4 ? 8 : 1;  // kSpans
   while (nw > 1 && ((long)s->batch * nw > 4096 || s->steps < 32 * nw || blk_lds_bytes(s, nw, true) > 160 * 1024)) nw /= 2;
   return nw;
 }
