@@ -282,131 +282,132 @@ __global__ __launch_bounds__(WL ? 64 * FW_WAVES : 256) void k_mix_fwd_s(MArgs a)
     __syncthreads();
   }
   while (row0 < M) {  // uniform over the wavefront; no workgroup barrier below
-  f4 acc[N][NH][RT];
-  float ssq[N][RT];
+    f4 acc[N][NH][RT];
+    float ssq[N][RT];
 #pragma unroll
-  for (int k = 0; k < N; ++k)
+    for (int k = 0; k < N; ++k)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      ssq[k][rt] = 0.0f;
+      for (int rt = 0; rt < RT; ++rt) {
+        ssq[k][rt] = 0.0f;
 #pragma unroll
-      for (int h = 0; h < NH; ++h) acc[k][h][rt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-  int k = 0, q = 0;
-  const int tile0 = row0;
-  while (k < N) {
-    wave_lds_sync();  // the previous segment's reads of the LDS tile are done
+        for (int h = 0; h < NH; ++h) acc[k][h][rt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    int k = 0, q = 0;
+    const int tile0 = row0;
+    while (k < N) {
+      wave_lds_sync();  // the previous segment's reads of the LDS tile are done
 #pragma unroll
-    for (int u = 0; u < NV; ++u) {
-      const int e = l + 64 * u;
-      *reinterpret_cast<f4*>(&sx[e / (SEG / 4)][4 * (e % (SEG / 4))]) = nx[u];
-    }
-    wave_lds_sync();
-    const int kc = k, qc = q;  // the segment in LDS
-    if (++q * SEG >= a.n[k]) {
-      ++k;
-      q = 0;
-    }
-    if (k == N) row0 = WL ? row0 + (int)gridDim.x * NW * RW : M;  // the next tile's first segment
-    if (row0 < M) seg_load(k < N ? k : 0, q, nx);  // the next segment, in flight during the contraction
-    const int st = a.st[kc] + SEG * qc, nb = min(SEG, a.n[kc] - SEG * qc);
-    sfor<0, N>([&](auto lc) {
-      constexpr int lv = lc;
-      if (lv != kc) return;
-      const int en = a.st[lv] + a.n[lv];
+      for (int u = 0; u < NV; ++u) {
+        const int e = l + 64 * u;
+        *reinterpret_cast<f4*>(&sx[e / (SEG / 4)][4 * (e % (SEG / 4))]) = nx[u];
+      }
+      wave_lds_sync();
+      const int kc = k, qc = q;  // the segment in LDS
+      if (++q * SEG >= a.n[k]) {
+        ++k;
+        q = 0;
+      }
+      if (k == N) row0 = WL ? row0 + (int)gridDim.x * NW * RW : M;  // the next tile's first segment
+      if (row0 < M) seg_load(k < N ? k : 0, q, nx);  // the next segment, in flight during the contraction
+      const int st = a.st[kc] + SEG * qc, nb = min(SEG, a.n[kc] - SEG * qc);
+      sfor<0, N>([&](auto lc) {
+        constexpr int lv = lc;
+        if (lv != kc) return;
+        const int en = a.st[lv] + a.n[lv];
 #pragma unroll 2
-      for (int cb = 0; cb < nb; cb += 16) {
-        f4 xa[RT];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          xa[rt] = *reinterpret_cast<const f4*>(&sx[16 * rt + i][cb + 4 * g]);  // zero past the level's end
-          ssq[lv][rt] = fmaf(xa[rt].x, xa[rt].x,
-                             fmaf(xa[rt].y, xa[rt].y, fmaf(xa[rt].z, xa[rt].z, fmaf(xa[rt].w, xa[rt].w, ssq[lv][rt]))));
-        }
-        const int kk = st + cb + 4 * g;
-#pragma unroll
-        for (int h = 0; h < NH; ++h) {
-          const int hrow = 16 * h + i;
-          const bool hok = hrow < a.hidden;
-          const f4 wb = WL ? reinterpret_cast<const f4*>(wl)[((lb[lv] + (st - a.st[lv] + cb) / 16) * NH + h) * 64 + l]
-                           : load4(a.weight + (size_t)(hok ? hrow : 0) * a.D, kk, en, hok);
+        for (int cb = 0; cb < nb; cb += 16) {
+          f4 xa[RT];
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) {
-            acc[lv][h][rt] = mfma(xa[rt].x, wb.x, acc[lv][h][rt]);
-            acc[lv][h][rt] = mfma(xa[rt].y, wb.y, acc[lv][h][rt]);
-            acc[lv][h][rt] = mfma(xa[rt].z, wb.z, acc[lv][h][rt]);
-            acc[lv][h][rt] = mfma(xa[rt].w, wb.w, acc[lv][h][rt]);
+            xa[rt] = *reinterpret_cast<const f4*>(&sx[16 * rt + i][cb + 4 * g]);  // zero past the level's end
+            const f4 x = xa[rt];
+            ssq[lv][rt] = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, fmaf(x.w, x.w, ssq[lv][rt]))));
+          }
+          const int kk = st + cb + 4 * g;
+#pragma unroll
+          for (int h = 0; h < NH; ++h) {
+            const int hrow = 16 * h + i;
+            const bool hok = hrow < a.hidden;
+            const f4 wb = WL ? reinterpret_cast<const f4*>(wl)[((lb[lv] + (st - a.st[lv] + cb) / 16) * NH + h) * 64 + l]
+                             : load4(a.weight + (size_t)(hok ? hrow : 0) * a.D, kk, en, hok);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+              acc[lv][h][rt] = mfma(xa[rt].x, wb.x, acc[lv][h][rt]);
+              acc[lv][h][rt] = mfma(xa[rt].y, wb.y, acc[lv][h][rt]);
+              acc[lv][h][rt] = mfma(xa[rt].z, wb.z, acc[lv][h][rt]);
+              acc[lv][h][rt] = mfma(xa[rt].w, wb.w, acc[lv][h][rt]);
+            }
           }
         }
-      }
-    });
-  }
+      });
+    }
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    // per-row factors: lanes (i, g) hold partial sums of squares of row i; every lane of row i ends with the sum
-    float fr[N];
-    const int gi = tile0 + 16 * rt + i;
-    const bool vi = gi < M;
-    sfor<0, N>([&](auto kc) {
-      constexpr int kx = kc;
-      float v = ssq[kx][rt];
-      v = lanes::add_xor32(lanes::add_xor16(v));
-      const int t = vi ? gi % a.R : 0;
-      const int K = kx + 1;
-      float c = 1.0f;
-      if (a.prescale) {  // 1 / C(max(t + 1 + prepend, K), K), K <= 3: the exact product
-        const double tl = fmax((double)(t + 1 + a.prepend), (double)K);
-        c = (float)(K == 1 ? 1.0 / tl : (K == 2 ? 2.0 / (tl * (tl - 1.0)) : 6.0 / (tl * (tl - 1.0) * (tl - 2.0))));
-      }
-      float f, beta = 0.0f, dfdg;
-      if (a.variant == EWS_GRADED_LIVE_RMS) {
-        const float gk = a.gains[kx];
-        const float ms = v / (float)a.n[kx];
-        const float rho = ms > 0.0f ? sqrtf(ms) : 0.0f;
-        const float den = fmaf(c, rho, a.eps[kx]);
-        dfdg = c / den;
-        f = gk * dfdg;
-        if (rho > 0.0f) beta = gk * c * c / (den * den * (float)a.n[kx] * rho);
-      } else if (a.variant == EWS_GRADED_STATIC_GAIN) {
-        dfdg = c;
-        f = a.gains[kx] * c;
-      } else {
-        const float lam = a.gains[0];
-        const float lk1 = powf(lam, (float)(K - 1));
-        dfdg = (float)K * lk1 * c;
-        f = lk1 * lam * c;
-      }
-      fr[kx] = f;
-      if (vi && g == kx) {  // one lane per (row, level) writes the residual's factors
-        float* fp = a.F + ((size_t)gi * N + kx) * 3;
-        fp[0] = f;
-        fp[1] = beta;
-        fp[2] = dfdg;
-      }
-    });
+    for (int rt = 0; rt < RT; ++rt) {
+      // per-row factors: lanes (i, g) hold partial sums of squares of row i; every lane of row i ends with the sum
+      float fr[N];
+      const int gi = tile0 + 16 * rt + i;
+      const bool vi = gi < M;
+      sfor<0, N>([&](auto kc) {
+        constexpr int kx = kc;
+        float v = ssq[kx][rt];
+        v = lanes::add_xor32(lanes::add_xor16(v));
+        const int t = vi ? gi % a.R : 0;
+        const int K = kx + 1;
+        float c = 1.0f;
+        if (a.prescale) {  // 1 / C(max(t + 1 + prepend, K), K), K <= 3: the exact product
+          const double tl = fmax((double)(t + 1 + a.prepend), (double)K);
+          c = (float)(K == 1 ? 1.0 / tl : (K == 2 ? 2.0 / (tl * (tl - 1.0)) : 6.0 / (tl * (tl - 1.0) * (tl - 2.0))));
+        }
+        float f, beta = 0.0f, dfdg;
+        if (a.variant == EWS_GRADED_LIVE_RMS) {
+          const float gk = a.gains[kx];
+          const float ms = v / (float)a.n[kx];
+          const float rho = ms > 0.0f ? sqrtf(ms) : 0.0f;
+          const float den = fmaf(c, rho, a.eps[kx]);
+          dfdg = c / den;
+          f = gk * dfdg;
+          if (rho > 0.0f) beta = gk * c * c / (den * den * (float)a.n[kx] * rho);
+        } else if (a.variant == EWS_GRADED_STATIC_GAIN) {
+          dfdg = c;
+          f = a.gains[kx] * c;
+        } else {
+          const float lam = a.gains[0];
+          const float lk1 = powf(lam, (float)(K - 1));
+          dfdg = (float)K * lk1 * c;
+          f = lk1 * lam * c;
+        }
+        fr[kx] = f;
+        if (vi && g == kx) {  // one lane per (row, level) writes the residual's factors
+          float* fp = a.F + ((size_t)gi * N + kx) * 3;
+          fp[0] = f;
+          fp[1] = beta;
+          fp[2] = dfdg;
+        }
+      });
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 4 * g + r, grow = tile0 + 16 * rt + row;
-      float fk[N];
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * g + r, grow = tile0 + 16 * rt + row;
+        float fk[N];
 #pragma unroll
-      for (int kx = 0; kx < N; ++kx) fk[kx] = __shfl(fr[kx], row, 64);  // lane `row` holds row `row`'s factors
+        for (int kx = 0; kx < N; ++kx) fk[kx] = __shfl(fr[kx], row, 64);  // lane `row` holds row `row`'s factors
 #pragma unroll
-      for (int h = 0; h < NH; ++h) {
-        const int col = 16 * h + i;
-        if (grow < M && col < a.hidden) {
-          float v = a.bias[col];
+        for (int h = 0; h < NH; ++h) {
+          const int col = 16 * h + i;
+          if (grow < M && col < a.hidden) {
+            float v = a.bias[col];
 #pragma unroll
-          for (int kx = 0; kx < N; ++kx) {
-            const f4 qv = acc[kx][h][rt];
-            const float pv = r == 0 ? qv.x : (r == 1 ? qv.y : (r == 2 ? qv.z : qv.w));
-            v = fmaf(fk[kx], pv, v);
-            a.P[((size_t)grow * N + kx) * a.hidden + col] = pv;
+            for (int kx = 0; kx < N; ++kx) {
+              const f4 qv = acc[kx][h][rt];
+              const float pv = r == 0 ? qv.x : (r == 1 ? qv.y : (r == 2 ? qv.z : qv.w));
+              v = fmaf(fk[kx], pv, v);
+              a.P[((size_t)grow * N + kx) * a.hidden + col] = pv;
+            }
+            a.out[out_row(a, grow) * a.hidden + col] = v;
           }
-          a.out[out_row(a, grow) * a.hidden + col] = v;
         }
       }
     }
-  }  }
+  }
 }
 
 // the leading zero rows of the levels map to the bias alone
