@@ -154,8 +154,9 @@ class EWS(torch.nn.Module):
             raise RuntimeError("Expected all tensors to be on the same device, but found the generator on "
                                f"{A.device} and the path on {device}")
         if isinstance(a_scale, (int, float)):
-            if a_scale == 1 and (not torch.is_grad_enabled() or (A.grad_fn is not None and not A._is_view())):
-                return A
+            if a_scale == 1:
+                own = torch.is_grad_enabled() and (A.grad_fn is None or A._is_view())
+                return A.clone() if own else A
             return A * float(a_scale)
         return A * torch.as_tensor(a_scale, dtype=torch.float32, device=device)
 
