@@ -8,7 +8,7 @@
 // and the KP = ceil(K / 4) pairs (j, KP kg ..), so a row sum is KP additions and a quad exchange, the plane's own work is
 // shared by KP pairs, column terms wait in LDS for a block of NB steps, and nothing waits on another wavefront. The
 // cotangent rows come straight into registers NB steps ahead. B = 8, L = 49,920, d = 24, bfloat16 path (399k intervals):
-// full adjoint 964 -> 402 us, chunk-local adjoints 377 -> 298, rows 305 -> 225, summaries 160 -> 121. The full adjoint is
+// full adjoint 964 -> 403 us, chunk-local adjoints 377 -> 298, rows 305 -> 225, summaries 160 -> 121. The full adjoint is
 // bound by instruction issue, the local one by its 0.96 GB of cotangents.
 //
 // States, coefficients and cotangents are kept halved or doubled (half SA, SB, phi_k, IB, IA; twice the pair cotangents),

@@ -1,7 +1,7 @@
 """Uniform clocks on rotation planes of every lane map of the wave-per-chunk kernels (two chunks or one per wavefront,
 rows whose pair count is no multiple of four), against the float64 oracle: short and ragged last chunks, chunks that
-cannot be stepped backwards, chunks that are uniform only to the looser bound next to strict ones, with and without the
-clock's gradient, rows, log rows and reductions. Bars as the repository's: forward 1e-5, gradients 1e-4."""
+cannot be stepped backwards, chunks that are uniform only to the looser bound next to strict ones, steps that differ by as much as they are long
+within the strict bound, with and without the clock's gradient, rows, log rows and reductions. Bars as the repository's: forward 1e-5, gradients 1e-4."""
 
 import numpy as np
 import pytest

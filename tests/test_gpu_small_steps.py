@@ -1,7 +1,8 @@
 """Irregular clocks under the small-step coefficient model, forward and every gradient, against the float64 oracle:
 chunks whose steps can be inverted and chunks too contractive for it, planes and real diagonals on every lane map, the
 d = 16 pair-group forward with chunks of every class in one call, the chunk lengths the library suits to few intervals,
-and steps on both sides of the model's radius. Bars as the repository's: forward 1e-5, gradients 1e-4."""
+steps on both sides of the model's radius, clocks that turn inside a chunk, in other units, and recordings padded with
+NaN. Bars as the repository's: forward 1e-5, gradients 1e-4."""
 
 import ctypes
 
