@@ -281,7 +281,7 @@ __global__ __launch_bounds__(WL ? 64 * FW_WAVES : 256) void k_mix_fwd_s(MArgs a)
       }
     __syncthreads();
   }
-  while (row0 < M) {  // uniform over the wavefront; no workgroup barrier below
+  while (row0 < M) {  // uniform over the wavefront; no workgroup barrier below. One tile a wavefront without WL
     f4 acc[N][NH][RT];
     float ssq[N][RT];
 #pragma unroll
@@ -307,8 +307,13 @@ __global__ __launch_bounds__(WL ? 64 * FW_WAVES : 256) void k_mix_fwd_s(MArgs a)
         ++k;
         q = 0;
       }
-      if (k == N) row0 = WL ? row0 + (int)gridDim.x * NW * RW : M;  // the next tile's first segment
-      if (row0 < M) seg_load(k < N ? k : 0, q, nx);  // the next segment, in flight during the contraction
+      // the next segment, in flight during the contraction (WL: past the last one the next tile's first)
+      if constexpr (WL) {
+        if (k == N) row0 += (int)gridDim.x * NW * RW;
+        if (row0 < M) seg_load(k < N ? k : 0, q, nx);
+      } else if (k < N) {
+        seg_load(k, q, nx);
+      }
       const int st = a.st[kc] + SEG * qc, nb = min(SEG, a.n[kc] - SEG * qc);
       sfor<0, N>([&](auto lc) {
         constexpr int lv = lc;
@@ -407,6 +412,7 @@ __global__ __launch_bounds__(WL ? 64 * FW_WAVES : 256) void k_mix_fwd_s(MArgs a)
         }
       }
     }
+    if constexpr (!WL) return;
   }
 }
 
