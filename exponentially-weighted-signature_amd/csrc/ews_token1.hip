@@ -181,7 +181,10 @@ __global__ void k_reduce(TArgs a) {
 // the span again from its own start state with the rows written. The adjoint does the
 // same from the last span, with the transposed flows, before the sweep that accumulates the gradients. (BS + 2) / NW of
 // the steps are on the chain for 1. B = 256 x 512 tokens, d = 64, BS = 2: forward 50 -> 28 us, backward 110 -> 39 us at
-// NW = 8. Blocks of 6 and 8, whose lane exchanges go through LDS, keep NW = 1.
+// NW = 8. Blocks of 6 and 8, whose lane exchanges go through LDS, keep NW = 1, a constant for them: with the span and the
+// LDS offsets from the launch's size their kernels took a quarter longer than without spans at all (1 x 1000 tokens, blocks
+// of 6: 163 and 371 us; 130 and 263 as constants). The new state is a select: as a branch around each step it held back the
+// loads of the steps after it.
 constexpr int kStageFloats = 12288;  // caches staged in LDS up to 48 KB
 template <int BS> constexpr bool kSpans = BS <= 4;  // block sizes whose samples are split into spans
 
@@ -278,7 +281,7 @@ __device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, c
     // groups of eight steps without a branch (the lane reads are convergent, so only a constant trip count is
     // unrolled; the states are stored after the group), so that the group's cache reads are issued ahead of the
     // state chain; steps past the span carry token 0 and no mask bit
-    for (int s0 = 0; s0 < cnt; s0 += 8) {
+    for (int s0 = 0; s0 < (kSpans<BS> ? cnt : 64); s0 += 8) {
       float Sv[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
@@ -298,7 +301,7 @@ __device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, c
             if (live) U[c] = ua;
           }
         }
-        if (live && on) S = acc;
+        S = live && on ? acc : S;
         Sv[u] = (float)S;
       }
       if (!MAP && on) {
@@ -313,8 +316,10 @@ __device__ __forceinline__ void fwd_blk_steps(const TArgs& a, const float* sP, c
 
 template <int BS, bool STAGED>
 __device__ __forceinline__ void fwd_blk_body(const TArgs& a, const float* sP, const float* sD, double* sX) {
-  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
+  const int b = blockIdx.x, i = threadIdx.x & 63;
+  const int w = kSpans<BS> ? threadIdx.x >> 6 : 0, nw = kSpans<BS> ? (int)(blockDim.x >> 6) : 1;
+  const int span = kSpans<BS> ? span_len(a, nw) : a.n, tb = kSpans<BS> ? min(a.n, w * span) : 0;
+  const int te = min(a.n, tb + span), base = (i / BS) * BS;
   double S = 0.0;
   if constexpr (kSpans<BS>) {
     if (nw > 1) {
@@ -341,10 +346,10 @@ __device__ __forceinline__ void fwd_blk_body(const TArgs& a, const float* sP, co
 }
 
 template <int BS>
-__global__ __launch_bounds__(kSpans<BS> ? 512 : 64) void k_fwd_blk(TArgs a) {
+__global__ __launch_bounds__(512) void k_fwd_blk(TArgs a) {
   extern __shared__ double s_c[];
   double* sX = s_c;  // (NW, BS + 1, 64): the spans' maps
-  float* sP = reinterpret_cast<float*>(sX + (size_t)(blockDim.x >> 6) * (BS + 1) * 64);
+  float* sP = reinterpret_cast<float*>(sX + (size_t)(kSpans<BS> ? blockDim.x >> 6 : 1) * (BS + 1) * 64);
   float* sD = sP + (size_t)a.V * a.d;
   if ((size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats) {
     stage_blk<BS>(a, sP, sD, true);
@@ -439,8 +444,10 @@ __device__ __forceinline__ void bwd_blk_steps(const TArgs& a, const float* sD, f
 
 template <int BS, bool STAGED>
 __device__ __forceinline__ void bwd_blk_body(const TArgs& a, const float* sD, float* sAcc, double* sX) {
-  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int span = span_len(a, nw), tb = min(a.n, w * span), te = min(a.n, tb + span), base = (i / BS) * BS;
+  const int b = blockIdx.x, i = threadIdx.x & 63;
+  const int w = kSpans<BS> ? threadIdx.x >> 6 : 0, nw = kSpans<BS> ? (int)(blockDim.x >> 6) : 1;
+  const int span = kSpans<BS> ? span_len(a, nw) : a.n, tb = kSpans<BS> ? min(a.n, w * span) : 0;
+  const int te = min(a.n, tb + span), base = (i / BS) * BS;
   double lam = 0.0;
   if constexpr (kSpans<BS>) {
     if (nw > 1) {
@@ -467,9 +474,10 @@ __device__ __forceinline__ void bwd_blk_body(const TArgs& a, const float* sD, fl
 }
 
 template <int BS>
-__global__ __launch_bounds__(kSpans<BS> ? 512 : 64) void k_bwd_blk(TArgs a) {
+__global__ __launch_bounds__(512) void k_bwd_blk(TArgs a) {
   extern __shared__ double s_c[];
-  const int b = blockIdx.x, i = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int b = blockIdx.x, i = threadIdx.x & 63;
+  const int w = kSpans<BS> ? threadIdx.x >> 6 : 0, nw = kSpans<BS> ? (int)(blockDim.x >> 6) : 1;
   const bool staged = (size_t)a.V * a.d * (BS + 1) <= (size_t)kStageFloats;
   const int na = a.V * (BS + 1);
   double* sX = s_c;  // (NW, BS + 1, 64): the spans' maps
