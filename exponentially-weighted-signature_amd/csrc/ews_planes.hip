@@ -267,6 +267,25 @@ __device__ __forceinline__ int classify(const DiagArgs& a, int b, int t0, int Tc
   return (uni ? kUniform : 0) | (inv ? kInvert : 0) | (small ? kSmall : 0) | (strict ? kStrict : 0);
 }
 
+// A clock whose rounding passes the strict bound part way (float32 values double their spacing at every power of two) splits
+// a sample between these kernels and the generic ones, and with few chunks each side only takes the length of its own
+// chains: B = 16, L = 8192, clock from 0 to 8, one training pass 459 us split and 334 us by the generic kernels alone (d = 10;
+// d = 18 714 and 613). Below kFewWaves wavefronts a sample is strict as a whole or not at all: not where its last full chunk
+// is uniform without being strict. With more of them the split gains (B = 8, L = 49,920, 3120 wavefronts, d = 6: 545 us and
+// 622 alone; d = 14 849 and 888), and at 16 planes, where the generic kernels take 256 lanes a chunk, at any number.
+constexpr int kFewWaves = 3072;
+template <int G, int GPW>
+__device__ __forceinline__ int classify_chunk(const DiagArgs& a, int b, int t0, int Tc, int gl, float& hb) {
+  int f = classify<G>(a, b, t0, Tc, gl, hb);
+  const int last = (a.n_int / a.T - 1) * a.T;  // the last full chunk's first step
+  if (a.K < 16 && (long)a.B * ((a.C + GPW - 1) / GPW) < kFewWaves && last >= 0) {
+    float hl;
+    const int fl = classify<G>(a, b, last, a.T, gl, hl);
+    if ((fl & (kUniform | kStrict)) == kUniform) f &= ~kStrict;
+  }
+  return f;
+}
+
 // Level 1 runs in float64: its roundings over a chunk, and that of its flow, are what the states' error at L = 50k came
 // from (level 2 takes them over: rows 5.8e-6 off with float32 here, 2.9e-6 with float64; 114 -> 121 us).
 template <int R, int KP>
@@ -276,7 +295,7 @@ __global__ __launch_bounds__(64) void k_summary(DiagArgs a) {
   const int b = blockIdx.y;
   const Lane<R, KP> l(a, b, 0);
   float hb;
-  const int flag = classify<G>(a, b, l.t0, l.Tc, l.gl, hb);
+  const int flag = classify_chunk<G, GPW>(a, b, l.t0, l.Tc, l.gl, hb);
   if (l.owns && l.gl == 0) {
     a.cflag[l.ci] = flag;
     a.chbar[l.ci] = hb;
