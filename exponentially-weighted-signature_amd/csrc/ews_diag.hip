@@ -2108,8 +2108,11 @@ __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(2))) void 
 // (b) Every other chunk: forward states recomputed from the chunk's float64 carry (checkpoints every kb steps; each
 // block recomputed into a lane-private LDS history before its reverse sweep), with exact per-step coefficients, or
 // the first-order model at the mean step for a uniform chunk.
-// One chunk c of sample b; every early return is uniform over the workgroup.
-template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
+// One chunk c of sample b; every early return is uniform over the workgroup. POLY: a chunk of small steps (too contractive
+// to invert). A body of its own: with the polynomials and moments live beside the other models the kernel took 3 to 15%
+// longer on every class (real diagonals, B = 16, L = 8192, steps of 0.5: d = 3 406 us in one body, 345 in two; d = 24 1843
+// and 1672).
+template <bool CPLX, int N, int MAXT, bool WAVE, bool DH, bool POLY>
 __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, const int b) {
   using T = typename Types<CPLX>::T;
   constexpr int NS = CPLX ? 6 : 2;  // checkpoint floats per lane
@@ -2127,21 +2130,20 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
   const RedLds red{smem + Lo.red, smem + Lo.red + 2 * NT, smem + Lo.red + 4 * NT, smem + Lo.red + 6 * NT};
   float* s_dh = smem + Lo.dh;
   float* s_g = smem + Lo.g;
-  EWS_BWD_PROLOGUE(!(cc.inv_ok && (cc.fast || cc.small)), kb)
+  EWS_BWD_PROLOGUE(POLY ? !cc.inv_ok && !cc.fast && cc.small : cc.fast ? !cc.inv_ok : !cc.small, kb)
   // uniform chunks (too contractive to invert) take the first-order model at the mean step, as every other
   // kernel does for them, small-step chunks the polynomial model; the others evaluate each step's exact coefficients
   Coef<T> c0;
   CoefD<T> q0;
   PolyCoef<T, CPLX, N> pc;
-  const bool poly = !cc.fast && cc.small;
-  if (cc.fast) eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q0);
-  if (poly) pc.init(uj, uk, cc.per_int, cc.href);
+  if (!POLY && cc.fast) eval_coef<T, CPLX, N, true>(a.sq1, a.sq2, cc.hbar, cc.href, cc.per_int, uj, uk, c0, q0);
+  if constexpr (POLY) pc.init(uj, uk, cc.per_int, cc.href);
   PolyMom<T> mom;
   mom.clear();
   // the coefficients of the forward recomputation, and with the derivatives the adjoint needs
   auto coef_fwd = [&](int t, Coef<T>& co) {
     CoefD<T> qq;
-    if (poly) {
+    if constexpr (POLY) {
       pc.template at<false>(s_h[t], co, qq);
     } else if (cc.fast) {
       lin_coef<T, CPLX, N>(c0, q0, s_h[t] - cc.hbar, cc.per_int, co);
@@ -2221,7 +2223,7 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
         st_load(s_hist + (size_t)s * NS * NT, H1, HA, HB);
         Coef<T> co;
         CoefD<T> qq;
-        if (poly) {
+        if constexpr (POLY) {
           pc.template at<DH>(s_h[t], co, qq);
           bwd_step<CPLX, N, WAVE, MAXT == 1024, DH, true>(a, m, gs, s, t, t0 + t, s_h[t], s_v, cc.per_int, co, qq, acc,
                                                           mom, H1, HA, HB, red, s_dh);
@@ -2235,13 +2237,17 @@ __device__ __forceinline__ void chunk_bwd_full(const DiagArgs& a, const int c, c
     if (more) lds_dma_wait();
     __syncthreads();
   }
-  if (poly) fold_moments<CPLX, N>(m, mom, uj, ua, ub, acc);
+  if constexpr (POLY) fold_moments<CPLX, N>(m, mom, uj, ua, ub, acc);
   bwd_epilogue<CPLX, N, WAVE, DH>(a, m, cc, acc, uj, ua, ub, Tc, t0, s_dh, s_g, c, b);
 }
 template <bool CPLX, int N, int MAXT, bool WAVE, bool DH>
 __global__ __launch_bounds__(MAXT) void k_chunk_bwd_full(DiagArgs a) {
   visit_chunks(a, [](int f) { return !inv_lin(f) && !inv_poly(f); },
-               [&](int c, int b) { chunk_bwd_full<CPLX, N, MAXT, WAVE, DH>(a, c, b); });
+               [&](int c, int b) {
+                 const bool poly = (a.cflag[b * a.C + c] & (kFlagUniform | kFlagSmall)) == kFlagSmall;
+                 if (poly) chunk_bwd_full<CPLX, N, MAXT, WAVE, DH, true>(a, c, b);
+                 else chunk_bwd_full<CPLX, N, MAXT, WAVE, DH, false>(a, c, b);
+               });
 }
 
 // ------------------------------------------------------------------------------------------- B0 (log rows)
