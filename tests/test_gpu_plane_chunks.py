@@ -1,7 +1,8 @@
 """Uniform clocks on rotation planes of every lane map of the wave-per-chunk kernels (two chunks or one per wavefront,
 rows whose pair count is no multiple of four), against the float64 oracle: short and ragged last chunks, chunks that
-cannot be stepped backwards, chunks that are uniform only to the looser bound next to strict ones, steps that differ by as much as they are long
-within the strict bound, with and without the clock's gradient, rows, log rows and reductions. Bars as the repository's: forward 1e-5, gradients 1e-4."""
+cannot be stepped backwards, chunks that are uniform only to the looser bound next to strict ones, steps that differ by
+as much as they are long within the strict bound, with and without the clock's gradient, rows, log rows and reductions.
+Bars as the repository's: forward 1e-5, gradients 1e-4."""
 
 import numpy as np
 import pytest
@@ -95,6 +96,13 @@ def test_steps_that_differ_within_constant_coefficients(d, rate, h):
 def test_float32_uniform_clock(d):
     # a uniform clock whose float32 values near 1 leave steps of 2e-5 off by 3e-3 of themselves
     _check(d, 2, _uniform(300, 2.0e-5) + np.r_[0.9, np.zeros(299)], (0.1, 1.0), clock_grad=False)
+
+
+@pytest.mark.parametrize("d", [8, 24, 32])
+@pytest.mark.parametrize("clock_grad", [False, True])
+def test_rounding_that_grows_past_the_strict_bound(d, clock_grad):
+    # steps of 5e-3 on a clock from 1.5 to 8.5: with max|u| near 3 the chunks miss the strict bound from 2 on
+    _check(d, 2, np.r_[1.5, np.full(1400, 5e-3)], (0.1, 1.0), clock_grad=clock_grad)
 
 
 @pytest.mark.parametrize("d", [12, 24])
