@@ -32,7 +32,8 @@ def _check(structure, d, N, B, L, steps, damp, readout="prefix", chunk=0, bf16=F
     path = path.to(torch.bfloat16) if bf16 else path
     clock = torch.tensor(np.cumsum(np.stack([steps * rng.uniform(0.9, 1.1) for _ in range(B)]), 1), dtype=torch.float32)
     if structure == "planes":
-        w = torch.tensor(np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, freq, d // 2)], -1), dtype=torch.float32)
+        w = np.stack([rng.uniform(*damp, d // 2), rng.uniform(0.0, freq, d // 2)], -1)
+        w = torch.tensor(w, dtype=torch.float32)
     else:
         w = torch.tensor(rng.uniform(*damp, d), dtype=torch.float32)
     p, c, q = path.to(DEV).requires_grad_(), clock.to(DEV).requires_grad_(clock_grad), w.to(DEV).requires_grad_()
@@ -99,9 +100,9 @@ def test_small_steps_cached_flow():
                                            ("real_diag", 9, 2), ("real_diag", 5, 1)])
 @pytest.mark.parametrize("sign", [1.0, -1.0])
 def test_clock_that_turns(structure, d, N, sign):
-    """A clock that turns inside a chunk: its net step is near zero, but the states contract by e^11 on the way (sign -1:
-    a growing generator on a clock that starts backwards), so that the steps cannot be inverted from the chunk's end.
-    The loss sees the first rows only, or all of them."""
+    """A clock that turns inside a chunk: its net step is near zero, but the states contract by e^11 on the way (sign
+    -1: a growing generator on a clock that starts backwards), so that the steps cannot be inverted from the chunk's
+    end. The loss sees the first rows only, or all of them."""
     s = sign * np.r_[0.0, np.full(32, 0.17), np.full(32, -0.17), _steps(60, 0.1, 0.17)]
     for rows in (8, None):
         _check(structure, d, N, 2, len(s), s, sorted((0.9 * sign, sign)), chunk=64, freq=0.2, rows=rows)
